@@ -213,10 +213,9 @@ typedef struct rswa_attn_params {
    * whole backward, at the price of 2 bytes per pair written and read once.  The workspace
    * grows by rswa_attn_bwd_workspace_bytes' account of it (about 2.2 bytes per visible pair and
    * q head for a window of thousands of keys).  Honoured when the call has no sink keys under a
-   * bounded window, every sequence spans less than 2 GiB (the first addressing form), one
-   * q head's tiles stay below 2 GiB and, with the value 1, the launch is not one of the small
-   * ones whose key tiles are split over several blocks (the value 2 prefers the hand-off to that
-   * split); silently the recomputing route otherwise -- ask rswa_attn_bwd_handoff_active().  With rswa_attn_bwd_phases the DQ phase of this route reads
+   * bounded window, every sequence spans less than 2 GiB (the first addressing form) and one
+   * q head's tiles stay below 2 GiB (the values 1 and 2 mean the same); silently the recomputing
+   * route otherwise -- ask rswa_attn_bwd_handoff_active().  With rswa_attn_bwd_phases the DQ phase of this route reads
    * what the DKDV phase of the same call parameters left in the same workspace, so DKDV must
    * have run before it.  rswa_attn_bwd_static never uses it.  Same interface replaced:
    * ring_swa/ops/wrap_flash.py:276-429. */
@@ -272,8 +271,7 @@ int rswa_attn_bwd_phases(const rswa_attn_params* p, void* stream, int phases);
  * callers that cannot allocate device memory around the call - code under HIP graph
  * capture, tight serving loops, harnesses that forbid hipMalloc.  Shapes whose statistics
  * (8 bytes per (row, q head) pair) exceed the buffer -- more than 4 194 304 pairs -- are
- * refused with RSWA_ERR_UNSUPPORTED; the dK/dV kernel runs one block per key tile here,
- * whatever the shape (no partial sums).  The buffer's address is looked up on the
+ * refused with RSWA_ERR_UNSUPPORTED.  The buffer's address is looked up on the
  * first call on each device (the device must be current, as for every other call); nothing
  * in it has to be cleared between calls, the statistics kernel rewrites what the others
  * read.  All calls on one GPU share the one buffer: calls that may overlap in time on the
@@ -292,11 +290,8 @@ int rswa_attn_bwd_static(const rswa_attn_params* p, void* stream);
 int rswa_attn_bwd_static_init(void);
 
 /* Scratch rswa_attn_bwd needs for these shapes: two fp32 values per (row, q head) -- the
- * row sum of dout * out and the LSE in base-2 units -- and, for launches with so few key
- * tiles (fewer than 129 blocks of 256 keys x kv head) that the q heads of each GQA group are
- * dealt to 2-4 blocks per tile, one arrival counter per tile and the fp32 partial dK / dV of
- * every part (256 keys x head_dim x 2 x 4 bytes each).  The call leaves the counters at zero;
- * nothing in the workspace has to be initialised by the caller. */
+ * row sum of dout * out and the LSE in base-2 units --, with sink keys under a bounded window the
+ * sink kernel's arrival counters and fp32 sums, and with ds_handoff the dS tiles.  Nothing in the workspace has to be initialised by the caller. */
 uint64_t rswa_attn_bwd_workspace_bytes(const rswa_attn_params* p);
 
 /* 1 when a backward with these parameters takes the dS hand-off route (ds_handoff != 0 and the

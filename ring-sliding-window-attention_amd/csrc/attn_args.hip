@@ -26,27 +26,13 @@ static bool handoff_eligible(const rswa_attn_params* p) {
   return true;
 }
 
-BwdLayout bwd_layout(const rswa_attn_params* p, bool allow_split, bool allow_handoff) {
+BwdLayout bwd_layout(const rswa_attn_params* p, bool allow_handoff) {
   BwdLayout L{};
-  L.nsplit = 1;
   if (!p || p->batch <= 0 || p->heads_q <= 0 || p->heads_kv <= 0 || p->head_dim <= 0) return L;
   L.stats_bytes = delta_bytes(p);
   const bool packed = p->cu_seqlens_q != nullptr;
   const int64_t rows_k = packed ? p->total_k : p->seqlen_k;
-  L.n_tile_k = (int)((rows_k + kDkvKeysPerBlock - 1) / kDkvKeysPerBlock + (packed ? p->batch : 0));
-  const int64_t blocks = (int64_t)L.n_tile_k * p->heads_kv * (packed ? 1 : p->batch);
   const int group = p->heads_q / p->heads_kv;
-  // Splitting pays when one block per key tile leaves compute units without any work (see
-  // kDkvSplitBelow).  The parts of a tile are summed in a fixed order.
-  // (ds_handoff >= 2: the caller prefers the dS hand-off, which the split kernel does not do)
-  const bool prefer_handoff = allow_handoff && p->ds_handoff >= 2 && handoff_eligible(p);
-  if (allow_split && !prefer_handoff && group > 1 && blocks > 0 && blocks < kDkvSplitBelow) {
-    for (int n : {4, 3, 2})
-      if (group % n == 0) {
-        L.nsplit = n;
-        break;
-      }
-  }
   // Sink keys under a bounded window: the sink kernel, one chunk per ~512 rows of an average
   // sequence (at most 64), one arrival counter per (sequence, kv head).
   int64_t sink_units = 0;
@@ -55,24 +41,17 @@ BwdLayout bwd_layout(const rswa_attn_params* p, bool allow_split, bool allow_han
     L.sink_chunks = (int)std::min<int64_t>(64, std::max<int64_t>(1, (rows_q + 511) / 512));
     sink_units = (int64_t)p->batch * p->heads_kv;
   }
-  // workspace: statistics | arrival counters (split key tiles, then sink units) | partial
-  // dK / dV of split key tiles | sums of the sink kernel
-  const int64_t split_units = L.nsplit > 1 ? blocks : 0;
-  L.n_count = (int)(split_units + sink_units);
-  L.sink_count_index = (int)split_units;
+  // workspace: statistics | arrival counters and sums of the sink kernel | dS tiles
+  L.n_count = (int)sink_units;
   L.count_off = 2 * L.stats_bytes;
-  L.part_off = L.count_off + align_up((uint64_t)L.n_count * sizeof(int32_t), 256);
-  const uint64_t per_unit = (uint64_t)kDkvKeysPerBlock * p->head_dim * 2 * sizeof(float);
-  L.sink_off = L.part_off + (uint64_t)split_units * L.nsplit * per_unit;
+  L.sink_off = L.count_off + align_up((uint64_t)L.n_count * sizeof(int32_t), 256);
   L.total_bytes = L.sink_off + (uint64_t)sink_units * L.sink_chunks * p->num_sink * 2 * p->head_dim *
                                    sizeof(float);
   // dS hand-off: one 4 KiB unit per (q head, 32-row tile slot, 256-key block modulo nkb, 64-key
   // group).  A row tile sees keys [i0 + shift - left, i0 + 31 + shift + right]: left + right + 32
   // consecutive keys, which touch at most (left + right + 31) / 256 + 2 blocks of 256, and never
   // more than a sequence has.
-  // (Launches whose key tiles are split over several blocks are small ones; they keep the
-  // recomputing route: the split kernel has no registers left for the hand-off.)
-  if (allow_handoff && p->ds_handoff && L.nsplit == 1 && handoff_eligible(p)) {
+  if (allow_handoff && p->ds_handoff && handoff_eligible(p)) {
     const int64_t rows_q = packed ? p->total_q : (int64_t)p->batch * p->seqlen_q;
     const int64_t blocks_seq = (rows_k + kDkvKeysPerBlock - 1) / kDkvKeysPerBlock;  // rows_k: one sequence's bound
     int64_t nkb = blocks_seq;
@@ -96,7 +75,7 @@ BwdLayout bwd_layout(const rswa_attn_params* p, bool allow_split, bool allow_han
   return L;
 }
 
-uint64_t bwd_workspace_bytes(const rswa_attn_params* p) { return bwd_layout(p, true, true).total_bytes; }
+uint64_t bwd_workspace_bytes(const rswa_attn_params* p) { return bwd_layout(p, true).total_bytes; }
 
 static bool rows_aligned(const void* ptr, const int64_t* st, int elem_bytes = 2) {
   if (((uintptr_t)ptr) % 16) return false;
@@ -105,8 +84,7 @@ static bool rows_aligned(const void* ptr, const int64_t* st, int elem_bytes = 2)
   return true;
 }
 
-int fill_args(const rswa_attn_params* p, bool backward, AttnArgs& a, bool allow_split,
-              bool allow_handoff) {
+int fill_args(const rswa_attn_params* p, bool backward, AttnArgs& a, bool allow_handoff) {
   RSWA_REQUIRE(p != nullptr, RSWA_ERR_INVALID, "attn: null params");
   RSWA_REQUIRE(p->dtype == RSWA_BF16 || p->dtype == RSWA_F16, RSWA_ERR_UNSUPPORTED,
                "attn: dtype %d (only bf16 and fp16)", p->dtype);
@@ -191,9 +169,6 @@ int fill_args(const rswa_attn_params* p, bool backward, AttnArgs& a, bool allow_
   }
   a.delta = nullptr;
   a.lse2 = nullptr;
-  a.dkv_part = nullptr;
-  a.dkv_count = nullptr;
-  a.nsplit = 1;
   a.n_count = 0;
   a.sink_part = nullptr;
   a.sink_count = nullptr;
@@ -272,9 +247,18 @@ int fill_args(const rswa_attn_params* p, bool backward, AttnArgs& a, bool allow_
     a.rev_q = keys_of(lq - 1) > keys_of(0);
     a.rev_k = rows_of(lk - 1) > rows_of(0);
     // keys a query row sees on average (keys_of is piecewise linear: 17 samples)
-    int64_t sum = 0;
-    for (int t = 0; t <= 16; t++) sum += keys_of((lq - 1) * t / 16);
+    int64_t sum = 0, sum_r = 0, max_r = 0;
+    for (int t = 0; t <= 16; t++) {
+      sum += keys_of((lq - 1) * t / 16);
+      // (sink keys under a bounded window are the sink kernel's: band rows only)
+      const int64_t j = std::max<int64_t>((lk - 1) * t / 16, a.wl >= 0 ? std::min<int64_t>(a.n_sink, lk - 1) : 0);
+      const int64_t r = rows_of(j);
+      sum_r += r;
+      max_r = std::max(max_r, r);
+    }
     a.avg_keys = (int32_t)std::min<int64_t>(sum / 17, INT32_MAX);
+    a.avg_rows = (int32_t)std::min<int64_t>(sum_r / 17, INT32_MAX);
+    a.max_rows = (int32_t)std::min<int64_t>(max_r, INT32_MAX);
   }
   a.scale = p->softmax_scale;
   a.scale_log2 = p->softmax_scale * kLog2e;
@@ -288,7 +272,7 @@ int fill_args(const rswa_attn_params* p, bool backward, AttnArgs& a, bool allow_
                  RSWA_ERR_UNSUPPORTED, "attn_bwd: dout/dq/dk/dv rows must start 16-byte aligned");
     RSWA_REQUIRE(p->dout_stride[1] >= 0 && p->dout_stride[1] * 2 < ((1ll << 31) - 65536) / kMaxTileRows,
                  RSWA_ERR_UNSUPPORTED, "attn_bwd: row stride of dout is negative or too large");
-    const BwdLayout L = bwd_layout(p, allow_split, allow_handoff);
+    const BwdLayout L = bwd_layout(p, allow_handoff);
     const uint64_t need = L.total_bytes;
     RSWA_REQUIRE(p->workspace != nullptr || need == 0, RSWA_ERR_INVALID,
                  "attn_bwd: null workspace");
@@ -299,13 +283,10 @@ int fill_args(const rswa_attn_params* p, bool backward, AttnArgs& a, bool allow_
                  "attn_bwd: workspace must be 256-byte aligned");
     a.lse2 = (float*)p->workspace;
     a.delta = (float*)((char*)p->workspace + delta_bytes(p));
-    a.nsplit = L.nsplit;
     a.n_count = L.n_count;
-    a.dkv_count = (int32_t*)((char*)p->workspace + L.count_off);
-    a.dkv_part = (float*)((char*)p->workspace + L.part_off);
     a.sink_chunks = L.sink_chunks;
     a.sink_part = L.sink_chunks ? (float*)((char*)p->workspace + L.sink_off) : nullptr;
-    a.sink_count = a.dkv_count + L.sink_count_index;
+    a.sink_count = (int32_t*)((char*)p->workspace + L.count_off);
     if (L.ds_bytes) {
       a.ds = (char*)p->workspace + L.ds_off;
       a.ds_nkb = L.ds_nkb;
@@ -327,5 +308,5 @@ extern "C" uint64_t rswa_attn_bwd_workspace_bytes(const rswa_attn_params* p) {
 }
 
 extern "C" int rswa_attn_bwd_handoff_active(const rswa_attn_params* p) {
-  return rswa::bwd_layout(p, true, true).ds_bytes != 0;
+  return rswa::bwd_layout(p, true).ds_bytes != 0;
 }

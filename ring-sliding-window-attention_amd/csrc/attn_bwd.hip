@@ -9,7 +9,8 @@
 //          (sequence, kv head) and walks the query tiles (32 rows) that can see them, for
 //          every q head of the GQA group; a wave owns 64 keys: their K and V fragments stay
 //          in registers, dK^T / dV^T accumulate in accumulation registers for the whole
-//          walk and are written once
+//          walk and are written once.  Where such blocks would leave compute units idle a
+//          block owns 64 keys instead and its waves share out the walk (WALK4)
 //   DQ   : one block (8 waves x 32 query rows: 128 rows of two q heads of a GQA group, or
 //          256 rows of one head) walks the key tiles (64 keys) it can see, like the forward
 //          kernel; dQ^T stays in registers
@@ -47,6 +48,8 @@
 // that every access names its buffer statically (see attn_fwd.hip for why).
 #include "attn_common.h"
 
+#include <algorithm>
+#include <cmath>
 #include <mutex>
 
 namespace rswa {
@@ -101,44 +104,54 @@ struct DkvCfg {
   static constexpr int Q_TILE = BM * ROWB;
 };
 
-template <typename T, int D, bool SPLIT, bool FAR, bool HAND>
+// WALK4: the block owns 64 keys, all four waves hold the same K and V fragments and take turns on
+// the walk (q heads dealt to the waves; with fewer than four in the group also query tiles), each
+// fetching its own Q / dO tiles into its own buffers -- no barrier in the walk, and a wave's keys
+// are the block's, so no step is idle for some waves.  The four partial sums are added in LDS at
+// the end, in wave order.  Four times as many, four times as short blocks for launches that would
+// otherwise fill the chip badly (small launches, short sequences, sizes just above a full round),
+// a longer tile fetch per step (four tiles instead of one shared), so blocks that fill the chip by
+// themselves stay wide: see dkv_walk4.  It took the place of blocks of 256 keys whose q heads were
+// split over 2-4 blocks with fp32 partial sums in memory: us, dK/dV alone, bf16, head_dim 128, 32 / 8
+// heads: window 1024, 4001 rows 180 -> 127; full causal attention over 2048 / 4096 rows 111 -> 98 / 261
+// -> 244; 28 / 4 heads (which could not be split evenly), 2000 rows, 368 -> 97.
+template <typename T, int D, bool FAR, bool HAND, bool WALK4>
 __global__ __launch_bounds__(256) void attn_bwd_dkdv_kernel(const AttnArgs a) {
   static_assert(!(HAND && FAR), "dS hand-off in the first addressing form only");
   using C = DkvCfg<D>;
+  constexpr int BN = WALK4 ? C::BN / 4 : C::BN;  // keys of the block
   using M = Mma<T>;
   using V8 = typename M::V8;
   constexpr int KB = C::KB, KS = C::KSTEPS, DB = C::DBLK;
-  __shared__ __attribute__((aligned(1024))) char q_s0[C::Q_TILE];
-  __shared__ __attribute__((aligned(1024))) char q_s1[C::Q_TILE];
-  __shared__ __attribute__((aligned(1024))) char do_s0[C::Q_TILE];
-  __shared__ __attribute__((aligned(1024))) char do_s1[C::Q_TILE];
-  __shared__ __attribute__((aligned(1024))) float st_s0[2 * C::BM];  // -lse2[BM], -delta[BM]
-  __shared__ __attribute__((aligned(1024))) float st_s1[2 * C::BM];
-  __shared__ int arrived_s;
+  // (WALK4: q_s0 holds every wave's own four tile buffers, wave after wave, the st_* every wave's
+  // own statistics)
+  constexpr int W_LDS = 4 * C::Q_TILE;  // LDS bytes of one wave's tile buffers
+  __shared__ __attribute__((aligned(1024))) char q_s0[WALK4 ? 4 * W_LDS : C::Q_TILE];
+  __shared__ __attribute__((aligned(1024))) char q_s1[WALK4 ? 16 : C::Q_TILE];
+  __shared__ __attribute__((aligned(1024))) char do_s0[WALK4 ? 16 : C::Q_TILE];
+  __shared__ __attribute__((aligned(1024))) char do_s1[WALK4 ? 16 : C::Q_TILE];
+  __shared__ __attribute__((aligned(1024))) float st_s0[(WALK4 ? 8 : 2) * C::BM];  // -lse2[BM], -delta[BM]
+  __shared__ __attribute__((aligned(1024))) float st_s1[(WALK4 ? 8 : 2) * C::BM];
 
   const int wid = logical_block_id(a.n_work);
   if (wid < 0) return;
   const int tid = threadIdx.x;
   const int lane = tid & 63;
-  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);  // key group: 64 keys each
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);  // (not WALK4: key group of 64 keys)
   const int l32 = lane & 31;
   const int g = lane >> 5;
   const int i16 = lane & 15;
   const int u = lane >> 4;
 
-  // ---- which (sequence, kv head, key tile) and which part of the GQA group -----------
-  // parts of a tile are neighbours in the launch order; tiles go heaviest first
-  const int part = wid % a.nsplit;
-  const int unit = wid / a.nsplit;
-  const int hpu = a.group / a.nsplit;  // q heads this block walks
-  const int slot = a.rev_k ? a.n_tile - 1 - unit % a.n_tile : unit % a.n_tile;
-  int rest = unit / a.n_tile;
+  // ---- which (sequence, kv head, key tile); tiles go heaviest first -------------------
+  const int slot = a.rev_k ? a.n_tile - 1 - wid % a.n_tile : wid % a.n_tile;
+  int rest = wid / a.n_tile;
   const int hk = rest % a.heads_kv;
   SeqInfo s;
   int kt;
   if (a.cu_q) {
     static_assert(C::BN == 1 << 8, "tile size passed to locate_packed");
-    if (!locate_packed(a, slot, 8, true, s, kt)) return;
+    if (!locate_packed(a, slot, WALK4 ? 6 : 8, true, s, kt)) return;
   } else {
     s.batch_idx = rest / a.heads_kv;
     s.q_row0 = s.k_row0 = 0;
@@ -148,9 +161,9 @@ __global__ __launch_bounds__(256) void attn_bwd_dkdv_kernel(const AttnArgs a) {
   }
   const int b = s.batch_idx;
   const int len_q = s.len_q, len_k = s.len_k;
-  const int j0 = kt * C::BN;
+  const int j0 = kt * BN;
   if (j0 >= len_k) return;
-  const int j_last = min(j0 + C::BN, len_k) - 1;
+  const int j_last = min(j0 + BN, len_k) - 1;
   const int shift = a.shift_explicit ? a.shift_val : len_k - len_q;
 
   // Keys in two row ranges (dense mode; the boundary is a multiple of the block's keys): the
@@ -173,21 +186,28 @@ __global__ __launch_bounds__(256) void attn_bwd_dkdv_kernel(const AttnArgs a) {
       (a.wl >= 0) ? min(len_q - 1, j_last - shift + a.wl) : len_q - 1;
   const int qt_lo = i_min / C::BM;
   const int n_qt = (i_max >= i_min) ? i_max / C::BM - qt_lo + 1 : 0;
-  const int n_iter = n_qt * hpu;
+  // WALK4: the walk is dealt to the waves, 1 << hw_log2 q heads at a time and, of a head's query
+  // tiles, every (1 << tw_log2)-th to each wave on it
+  const int hw_log2 = WALK4 ? ((a.group & 3) == 0 ? 2 : (a.group & 1) == 0 ? 1 : 0) : 0;
+  const int tw_log2 = WALK4 ? 2 - hw_log2 : 0;
+  const int w_tile = WALK4 ? wave >> hw_log2 : 0;  // the wave's first tile of a head's walk
+  const int w_tiles = (n_qt - w_tile + (1 << tw_log2) - 1) >> tw_log2;
+  const int n_iter = WALK4 ? w_tiles * (a.group >> hw_log2) : n_qt * a.group;
 
-  const int jw0 = j0 + wave * (32 * KB);  // first key column of this wave
+  const int jw0 = WALK4 ? j0 : j0 + wave * (32 * KB);  // first key column of this wave
   const int jw1 = jw0 + 32 * KB - 1;
 
   // ---- lane-constant LDS offsets (swizzle folded: varying parts are XOR / immediates) ----
   // 16-byte row fragments: row = l32 (+ 32 per block), chunk = 2 ks + g
   //   offset = (a_row ^ (ks << 5)) + blk * 32 * ROWB
-  const int a_row = l32 * C::ROWB + ((g ^ swz_f<C::CPR>(l32)) << 4);
+  const int w_lds = WALK4 ? wave * W_LDS : 0;  // (a multiple of what the XORs touch)
+  const int a_row = w_lds + l32 * C::ROWB + ((g ^ swz_f<C::CPR>(l32)) << 4);
   // transposing reads of Q / dO: rows 16 ks + 4 g + (i16 >> 2) and + 8, chunk = 4 d + lp
   //   offset = (t_row{0,1} ^ (d << 6)) + ks * 16 * ROWB
   const int rl = 4 * g + (i16 >> 2);
   const int lp = 2 * (u & 1) + ((i16 & 3) >> 1);
-  const int t_row0 = rl * C::ROWB + ((lp ^ swz_f<C::CPR>(rl)) << 4) + (i16 & 1) * 8;
-  const int t_row1 = (rl + 8) * C::ROWB + ((lp ^ swz_f<C::CPR>(rl + 8)) << 4) + (i16 & 1) * 8;
+  const int t_row0 = w_lds + rl * C::ROWB + ((lp ^ swz_f<C::CPR>(rl)) << 4) + (i16 & 1) * 8;
+  const int t_row1 = w_lds + (rl + 8) * C::ROWB + ((lp ^ swz_f<C::CPR>(rl + 8)) << 4) + (i16 & 1) * 8;
 
   // ---- this wave's K fragments stay in registers for the whole walk (B operand of
   // S = Q K^T: lane = key column, 8 consecutive d per k-step); keys past the end are zero
@@ -229,8 +249,17 @@ __global__ __launch_bounds__(256) void attn_bwd_dkdv_kernel(const AttnArgs a) {
         dk_acc[kb][d][i] = 0.f;
         dv_acc[kb][d][i] = 0.f;
       }
+  if constexpr (WALK4) {
+    // (opaque zeros: the compiler takes a loop-carried vector that starts from a constant apart into
+    // scalars, which live in vector registers and are copied to accumulation registers every step)
+#pragma unroll
+    for (int kb = 0; kb < KB; kb++)
+#pragma unroll
+      for (int d = 0; d < DB; d++) asm volatile("" : "+a"(dk_acc[kb][d]), "+a"(dv_acc[kb][d]));
+  }
   // ---- tile DMA (rows past the end of the sequence read as zero) ------------------
-  TileDma<D, C::BM, C::THREADS> q_dma, do_dma;
+  using Dma = std::conditional_t<WALK4, WaveTileDma<D, C::BM>, TileDma<D, C::BM, C::THREADS>>;
+  Dma q_dma, do_dma;
   q_dma.init(a.q_st[1], tid);
   do_dma.init(a.do_st[1], tid);
   const T* q_base = (const T*)a.q + b * a.q_st[0] + s.q_row0 * a.q_st[1];
@@ -258,10 +287,14 @@ __global__ __launch_bounds__(256) void attn_bwd_dkdv_kernel(const AttnArgs a) {
   // rows, and walking them in step lets one L2 fill serve all of them.
   const int qt_start = n_qt > 0 ? (n_qt - qt_lo % n_qt) % n_qt : 0;
   Cursor nxt;  // the tile that the load parts fetch
-  nxt.qt = qt_start;
-  nxt.i0 = i_first + qt_start * C::BM;
+  nxt.qt = WALK4 ? w_tile : qt_start;  // WALK4: position in the walk, counted from qt_start
+  auto row_of = [&](int pos) __attribute__((always_inline)) {
+    const int at = qt_start + pos;
+    return i_first + (at >= n_qt ? at - n_qt : at) * C::BM;
+  };
+  nxt.i0 = row_of(w_tile);
   int nxt_left = n_qt;  // tiles left in the walk of nxt's head, nxt included
-  const int h_first = hk * a.group + part * hpu;
+  const int h_first = hk * a.group + (WALK4 ? wave & ((1 << hw_log2) - 1) : 0);
   nxt.q_head = q_base + (int64_t)h_first * a.q_st[2];
   nxt.do_head = do_base + (int64_t)h_first * a.do_st[2];
   nxt.stat_row = (int)(h_first * a.rows_q + ws_row0);
@@ -276,32 +309,49 @@ __global__ __launch_bounds__(256) void attn_bwd_dkdv_kernel(const AttnArgs a) {
   constexpr int kDsNowhere = 0x7ff00000;
   const int64_t ds_slot0 = a.cu_q ? (s.q_row0 >> 5) + b : (int64_t)b * ((a.seqlen_q + 31) >> 5);
   const int64_t ds_first = HAND ? (int64_t)h_first * ds_head_bytes + (ds_slot0 + qt_lo) * ds_row_bytes +
-                                      (kt % max(a.ds_nkb, 1)) * kDsBlockBytes + wave * kDsUnitBytes
+                                      ((jw0 >> 8) % max(a.ds_nkb, 1)) * kDsBlockBytes +
+                                      ((jw0 >> 6) & 3) * kDsUnitBytes
                                 : 0;
   const __amdgpu_buffer_rsrc_t ds_rsrc = __builtin_amdgcn_make_buffer_rsrc(
       a.ds + ds_first, 0,
-      HAND ? (int)min((int64_t)hpu * ds_head_bytes, (int64_t)a.heads_q * ds_head_bytes - ds_first) : 0,
+      HAND ? (int)min((int64_t)a.group * ds_head_bytes, (int64_t)a.heads_q * ds_head_bytes - ds_first) : 0,
       0x00020000);
   int ds_head_off = 0;  // of the head the cursor is on
-  nxt.ds = qt_start * ds_row_bytes;
+  nxt.ds = ((nxt.i0 - i_first) >> 5) * ds_row_bytes;
   [[maybe_unused]] int cur_ds = nxt.ds;  // the unit of the tile being computed
   // The next tile is fetched by NPART instructions per wave (statistics, Q, dO), issued
   // one at a time between the first MFMAs of a step; advance() then moves the cursor on.
-  constexpr int NQD = TileDma<D, C::BM, C::THREADS>::N;
+  constexpr int NQD = Dma::N;
   constexpr int NPART = 1 + 2 * NQD;
   const int st_voff = ((lane & 31) << 2) + (lane >> 5) * (stat_elems * 4);
-  auto load_part = [&](int part, char* qd, char* dod, float* std_) __attribute__((always_inline)) {
-    if (part == 0) {
-      if (wave == 0) {  // lanes 0-31: lse2 of the 32 rows, lanes 32-63: their delta
+  [[maybe_unused]] int dma_chunk = 0;  // WALK4: see WaveTileDma
+  if constexpr (WALK4) dma_chunk = Dma::chunk(lane);
+  auto load_part = [&](auto part_c, char* qd, char* dod, float* std_) __attribute__((always_inline)) {
+    constexpr int part = decltype(part_c)::value;
+    if constexpr (part == 0) {
+      if (WALK4 || wave == 0) {  // lanes 0-31: lse2 of the 32 rows, lanes 32-63: their delta
         const int first = nxt.stat_row + nxt.i0;
         const __amdgpu_buffer_rsrc_t st_rsrc = __builtin_amdgcn_make_buffer_rsrc(
             (void*)(a.lse2 + first), 0, min(stat_end - first, stat_elems + C::BM) * 4, 0x00020000);
         // the per-lane offset is recomputed here (opaque to the optimiser): kept in a
         // register across the walk it could be spilled, and its reload would wait for
         // every tile load issued before it
-        __builtin_amdgcn_raw_ptr_buffer_load_lds(st_rsrc, (lds_void_t*)std_, 4, st_voff, 0, 0, 0);
+        if constexpr (WALK4) {
+          lds_load_asm<4>(rsrc_words(a.lse2 + first, min(stat_end - first, stat_elems + C::BM) * 4), st_voff,
+                          0, (uint32_t)(uintptr_t)(lds_void_t*)std_);
+        } else {
+          __builtin_amdgcn_raw_ptr_buffer_load_lds(st_rsrc, (lds_void_t*)std_, 4, st_voff, 0, 0, 0);
+        }
       }
-    } else if (part <= NQD) {
+    } else if constexpr (WALK4) {
+      constexpr bool is_q = part <= NQD;
+      const T* head = is_q ? nxt.q_head : nxt.do_head;
+      const int row_bytes = is_q ? q_row_bytes : do_row_bytes;
+      (is_q ? q_dma : do_dma)
+          .template load_one<is_q ? part - 1 : part - 1 - NQD>(
+              tile_words<C::BM, FAR>(head, nxt.i0, len_q, row_bytes, C::ROWB), FAR ? 0 : nxt.i0 * row_bytes,
+              (uint32_t)(uintptr_t)(lds_void_t*)(is_q ? qd : dod) + w_lds, dma_chunk);
+    } else if constexpr (part <= NQD) {
       const TileSrc t = tile_src<C::BM, FAR>(nxt.q_head, nxt.i0, len_q, q_row_bytes, C::ROWB);
       q_dma.load_one(t.rsrc, t.soff, qd, part - 1);
     } else {
@@ -310,6 +360,19 @@ __global__ __launch_bounds__(256) void attn_bwd_dkdv_kernel(const AttnArgs a) {
     }
   };
   auto advance = [&]() __attribute__((always_inline)) {
+    if constexpr (WALK4) {
+      nxt.qt += 1 << tw_log2;
+      if (nxt.qt >= n_qt) {
+        nxt.qt = w_tile;
+        nxt.q_head += a.q_st[2] << hw_log2;
+        nxt.do_head += a.do_st[2] << hw_log2;
+        nxt.stat_row += (int)a.rows_q << hw_log2;
+        if constexpr (HAND) ds_head_off += ds_head_bytes << hw_log2;
+      }
+      nxt.i0 = row_of(nxt.qt);
+      if constexpr (HAND) nxt.ds = ds_head_off + ((nxt.i0 - i_first) >> 5) * ds_row_bytes;
+      return;
+    }
     nxt.qt++;
     nxt.i0 += C::BM;
     if constexpr (HAND) nxt.ds += ds_row_bytes;
@@ -332,15 +395,18 @@ __global__ __launch_bounds__(256) void attn_bwd_dkdv_kernel(const AttnArgs a) {
     }
   };
 
+  // buffers of the even and odd steps
+  char *const qb0 = q_s0, *const qb1 = WALK4 ? q_s0 + 2 * C::Q_TILE : q_s1;
+  char *const dob0 = WALK4 ? q_s0 + C::Q_TILE : do_s0, *const dob1 = WALK4 ? q_s0 + 3 * C::Q_TILE : do_s1;
+  float *const stb0 = WALK4 ? st_s0 + wave * 2 * C::BM : st_s0, *const stb1 = WALK4 ? st_s1 + wave * 2 * C::BM : st_s1;
+  int cur_i0 = nxt.i0;  // first row of the tile being computed
   if (n_iter > 0) {
-#pragma unroll
-    for (int part = 0; part < NPART; part++) load_part(part, q_s0, do_s0, st_s0);
+    static_for<NPART>([&](auto pc) __attribute__((always_inline)) { load_part(pc, qb0, dob0, stb0); });
     if (n_iter > 1) advance();
   }
-  __syncthreads();
+  if constexpr (WALK4) wait_vmem_but<0>();
+  else __syncthreads();
 
-
-  int cur_i0 = i_first + qt_start * C::BM;  // first row of the tile being computed
   // byte of a lane's 16 in a 1 KiB piece of a dS unit: [key l32][query group g]
   const int ds_lane = l32 * 32 + g * 16;
   // dS of a step, packed to 16 bits as the operand of its dK MFMAs.  HAND: the four groups also
@@ -348,13 +414,15 @@ __global__ __launch_bounds__(256) void attn_bwd_dkdv_kernel(const AttnArgs a) {
   // their own step would still be on their way at its end, and the wait for the tile loads
   // there waits for every vector memory operation of the wave: that cost a fifth of the
   // kernel).  ds_pend = where they go: the unit of the last computed step, or nowhere.
+  // (WALK4 has no registers for the carry and stores in the same step.)
+  constexpr bool CARRY = HAND && !WALK4;
   [[maybe_unused]] V8 ds_carry[KB][2];
   [[maybe_unused]] int ds_pend = kDsNowhere;
-  auto store_ds = [&](int pc, int voff) __attribute__((always_inline)) {
+  auto store_ds = [&](const V8(&from)[KB][2], int pc, int voff) __attribute__((always_inline)) {
     // piece [key block][query half] of the unit, 1 KiB per wave instruction: a key's 32 bytes
     // side by side ([query group g][rows 16 ks2 + 4 g .., 16 ks2 + 8 + 4 g ..])
     u32x4 bits;
-    __builtin_memcpy(&bits, &ds_carry[pc >> 1][pc & 1], 16);
+    __builtin_memcpy(&bits, &from[pc >> 1][pc & 1], 16);
     // (aux 2 = non-temporal: the tiles are read once, by another kernel, much later; measured
     // 6 % faster than plain stores on a 2.4 GB hand-off)
     __builtin_amdgcn_raw_buffer_store_b128(bits, ds_rsrc, voff + pc * 1024, ds_pend, 2);
@@ -390,17 +458,18 @@ __global__ __launch_bounds__(256) void attn_bwd_dkdv_kernel(const AttnArgs a) {
     const bool has_next = it + 1 < n_iter;
     const float* lse_lds = stc;
     const float* delta_lds = stc + C::BM;
-    const bool needed = i0 >= need_lo && i0 <= need_hi;
+    // (opaque: the XOR forms of the lane offsets are made where they are used, not kept)
+    if constexpr (WALK4) asm volatile("" : "+v"(dma_chunk));
+    const bool needed = WALK4 || (i0 >= need_lo && i0 <= need_hi);
     if (!needed && has_next) {
-#pragma unroll
-      for (int part = 0; part < NPART; part++) load_part(part, qn, don, stn);
+      static_for<NPART>([&](auto pc) __attribute__((always_inline)) { load_part(pc, qn, don, stn); });
       if (it + 2 < n_iter) advance();
     }
-    if constexpr (HAND) {
+    if constexpr (CARRY) {
       if (!needed) {
         const int voff = ds_voff();
 #pragma unroll
-        for (int pc = 0; pc < 2 * KB; pc++) store_ds(pc, voff);
+        for (int pc = 0; pc < 2 * KB; pc++) store_ds(ds_carry, pc, voff);
         ds_pend = kDsNowhere;
       }
     }
@@ -423,11 +492,11 @@ __global__ __launch_bounds__(256) void attn_bwd_dkdv_kernel(const AttnArgs a) {
       V8 fa[NF];
       auto fetch = [&](auto fc) __attribute__((always_inline)) {
         constexpr int f = decltype(fc)::value;
-        if constexpr (f < KS) {
-          fa[f] = *(const V8*)(qc + (a_row ^ (f << 5)));
-        } else if constexpr (f < 2 * KS) {
-          constexpr int ks = f - KS;
-          fa[f] = *(const V8*)(doc + (a_row ^ (ks << 5)));
+        if constexpr (f < 2 * KS) {
+          constexpr int ks = f % KS;
+          int at = a_row;
+          if constexpr (WALK4 && ks >= KS / 2) asm volatile("" : "+v"(at));
+          fa[f] = *(const V8*)((f < KS ? qc : doc) + (at ^ (ks << 5)));
         } else if constexpr (f < NF) {
           constexpr int j = (f - 2 * KS) % KS, ks2 = j / DB, d = j % DB;
           const char* src = f < 3 * KS ? doc : qc;
@@ -443,7 +512,7 @@ __global__ __launch_bounds__(256) void attn_bwd_dkdv_kernel(const AttnArgs a) {
       f32x4 l4[4];   // -lse2 of the rows
       V8 pb[KB][2], ds_step[KB][2];
       V8(&dsb)[KB][2] = *[&]() __attribute__((always_inline)) {
-        if constexpr (HAND) return &ds_carry;  // lives on into the next step
+        if constexpr (CARRY) return &ds_carry;  // lives on into the next step
         else return &ds_step;
       }();
       // vector work in 2 KB chunks of four rows: chunk order lets the packed operands of
@@ -478,7 +547,7 @@ __global__ __launch_bounds__(256) void attn_bwd_dkdv_kernel(const AttnArgs a) {
       };
 
       [[maybe_unused]] int ds_voff_step = 0;
-      if constexpr (HAND) ds_voff_step = ds_voff();
+      if constexpr (CARRY) ds_voff_step = ds_voff();
       static_for<AH>([&](auto fc) __attribute__((always_inline)) { fetch(fc); });
       fence();
       static_for<4 * NG>([&](auto mc) __attribute__((always_inline)) {
@@ -487,9 +556,11 @@ __global__ __launch_bounds__(256) void attn_bwd_dkdv_kernel(const AttnArgs a) {
         if constexpr (kb == 0) fetch(std::integral_constant<int, f + AH>{});
         // (after the last tile the cursor still names it: its rows are fetched once more, into
         // the idle buffers, rather than branching around every load)
-        if constexpr (m < NPART) load_part(m, qn, don, stn);
-        if constexpr (HAND && m < 2 * KB) {
-          store_ds(m, ds_voff_step);
+        // (WALK4 issues four times as many: one every other MFMA)
+        constexpr int every = WALK4 ? 2 : 1;
+        if constexpr (m % every == 0 && m / every < NPART) load_part(std::integral_constant<int, m / every>{}, qn, don, stn);
+        if constexpr (CARRY && m < 2 * KB) {
+          store_ds(ds_carry, m, ds_voff_step);
           if constexpr (m == 2 * KB - 1) ds_pend = ds_unit;
         }
         // row statistics: -delta early in S (the dP chains start from it), -lse2 at its end
@@ -512,13 +583,18 @@ __global__ __launch_bounds__(256) void attn_bwd_dkdv_kernel(const AttnArgs a) {
               constexpr int kBig = 1 << 29;  // |t| stays below it
               const int rel_lo = (a.wl < 0) ? -kBig : -a.wl;
               const int rel_up = (a.wr < 0) ? kBig : a.wr;
-              const int jc = jw0 + kb * 32 + l32;
+              int lane_m = lane;
+              if constexpr (WALK4) {  // (taken afresh in this rare path: no register for it)
+                lane_m = (int)__builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, 0u));
+                asm volatile("" : "+v"(lane_m));
+              }
+              const int jc = jw0 + kb * 32 + (lane_m & 31);
               const int t = jc - i0 - shift;
               const int rows_ok = (jc < len_k) ? len_q - i0 : 0;  // rows r < rows_ok are real
               const int rmin = t - rel_up;
               const int rmax = min(t - rel_lo, rows_ok - 1);
               const unsigned width = (unsigned)max(rmax - rmin + 1, 0);
-              const int base = 4 * g - rmin;
+              const int base = 4 * (lane_m >> 5) - rmin;
 #pragma unroll
               for (int i = 0; i < 16; i++) {
                 const int c = 8 * (i >> 2) + (i & 3);
@@ -548,22 +624,30 @@ __global__ __launch_bounds__(256) void attn_bwd_dkdv_kernel(const AttnArgs a) {
         } else {
           constexpr int j = f - 3 * KS, ks2 = j / DB, d = j % DB;
           dk_acc[kb][d] = M::mfma32(fa[f], dsb[kb][ks2], dk_acc[kb][d]);
+          if constexpr (HAND && WALK4 && m < 3 * NG + 2 * KB) {
+            if constexpr (m == 3 * NG) {
+              ds_pend = ds_unit;
+              ds_voff_step = ds_voff();
+            }
+            store_ds(dsb, m - 3 * NG, ds_voff_step);
+          }
         }
         fence();
       });
       if (it + 2 < n_iter) advance();
     }
-    __syncthreads();
+    if constexpr (WALK4) wait_vmem_but<0>();  // the wave's own tiles: nobody else reads them
+    else __syncthreads();
   };
 
   for (int it = 0; it < n_iter; it += 2) {
-    step(it, q_s0, do_s0, st_s0, q_s1, do_s1, st_s1);
-    if (it + 1 < n_iter) step(it + 1, q_s1, do_s1, st_s1, q_s0, do_s0, st_s0);
+    step(it, qb0, dob0, stb0, qb1, dob1, stb1);
+    if (it + 1 < n_iter) step(it + 1, qb1, dob1, stb1, qb0, dob0, stb0);
   }
-  if constexpr (HAND) {  // the last computed step's dS
+  if constexpr (CARRY) {  // the last computed step's dS
     const int voff = ds_voff();
 #pragma unroll
-    for (int pc = 0; pc < 2 * KB; pc++) store_ds(pc, voff);
+    for (int pc = 0; pc < 2 * KB; pc++) store_ds(ds_carry, pc, voff);
   }
 
   // ---- write dK, dV (C layout: lane = key, regs = d) -----------------------------------
@@ -572,78 +656,16 @@ __global__ __launch_bounds__(256) void attn_bwd_dkdv_kernel(const AttnArgs a) {
   int lane_e = (int)__builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, 0u));
   asm volatile("" : "+v"(lane_e));
   const int l32_e = lane_e & 31, g_e = lane_e >> 5;
-  // value group (mtx: 0 dK / 1 dV, key block, d block, four consecutive d) of this lane -> memory
-  auto emit = [&](int mtx, int kb, int d, int i4, f32x4 val) __attribute__((always_inline)) {
-    const int jc = jw0 + kb * 32 + l32_e;
-    if (jc < len_k) {
+  if constexpr (WALK4) {
+    // The four waves' sums of the block's 64 keys meet in LDS as fp32, one matrix at a time: a
+    // wave's 64 x D values fill its own tile buffers (row = key, chunk c of 16 bytes at position
+    // c ^ (key mod chunks-per-row)); then all threads add the four parts in wave order, 8 values
+    // each, and store whole rows.
+    static_assert(W_LDS == 64 * D * 4, "a matrix of 64 keys in fp32 fills a wave's tile buffers");
+    constexpr int FPR = D / 4;  // fp32 chunks per row
+#pragma unroll
+    for (int mtx = 0; mtx < 2; mtx++) {
       const float sc = mtx == 0 ? a.scale : 1.f;
-      const int64_t at = (mtx == 0 ? dk_off + (int64_t)jc * a.dk_st[1] : dv_off + (int64_t)jc * a.dv_st[1]) +
-                         d * 32 + 8 * i4 + 4 * g_e;
-      const typename M::V4 h4 = M::pack4(val[0] * sc, val[1] * sc, val[2] * sc, val[3] * sc);
-      if (a.wide_dkv) {
-        float* dst = (float*)(mtx == 0 ? dk_buf : dv_buf) + at;
-        f32x4 y = {(float)h4[0], (float)h4[1], (float)h4[2], (float)h4[3]};
-        if (a.dkv_accumulate) y += *(const f32x4*)dst;
-        *(f32x4*)dst = y;
-      } else {
-        *(typename M::V4*)((T*)(mtx == 0 ? dk_buf : dv_buf) + at) = h4;
-      }
-    }
-  };
-  // Without a split (SPLIT = false, nsplit = 1) the lane's sums go straight out.  Otherwise the
-  // group's q heads were dealt to nsplit blocks: every block stores its fp32 partial sums (16
-  // bytes per lane and value group, lanes contiguous), then counts itself in; the block that
-  // arrives last adds the parts in part order -- the same order whichever block that is, so
-  // the result does not depend on timing -- and writes dK, dV.  Nobody waits for anybody.
-  constexpr int GROUPS = 2 * KB * DB * 4;  // value groups per lane
-  f32x4* part_base = (f32x4*)a.dkv_part + (int64_t)unit * a.nsplit * (GROUPS * C::THREADS);
-  if constexpr (!SPLIT) {
-    // Through LDS, one 32-key block of one matrix at a time: in the accumulator layout a lane
-    // holds 4 consecutive d of one key, so a direct store instruction would touch 32 rows with
-    // 16 bytes each (256 such instructions per block; at short walks -- 40 steps per block at
-    // window 1000 and one q head per kv head -- they took a tenth of the kernel).  Each wave
-    // stages its block in the tile buffer nobody reads any more (rows of 16-byte chunks, chunk
-    // c of row r at position c ^ (r % chunks-per-row)), and stores whole rows, 16 bytes a lane.
-    char* stage = wave == 0 ? q_s0 : wave == 1 ? q_s1 : wave == 2 ? do_s0 : do_s1;
-    static_assert(C::Q_TILE >= 32 * C::ROWB, "a 32-key block fits a tile buffer");
-    const int wr_row = l32_e * C::ROWB + g_e * 8;
-    const int wr_swz = l32_e & (C::CPR - 1);
-#pragma unroll
-    for (int mtx = 0; mtx < 2; mtx++)
-#pragma unroll
-      for (int kb = 0; kb < KB; kb++) {
-        const float sc = mtx == 0 ? a.scale : 1.f;
-#pragma unroll
-        for (int d = 0; d < DB; d++)
-#pragma unroll
-          for (int i4 = 0; i4 < 4; i4++) {
-            const f32x16& acc = mtx == 0 ? dk_acc[kb][d] : dv_acc[kb][d];
-            *(typename M::V4*)(stage + wr_row + (((d * 4 + i4) ^ wr_swz) << 4)) =
-                M::pack4(acc[4 * i4] * sc, acc[4 * i4 + 1] * sc, acc[4 * i4 + 2] * sc,
-                         acc[4 * i4 + 3] * sc);
-          }
-        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // the wave's own writes have landed
-        void* const dst = mtx == 0 ? dk_buf : dv_buf;
-        const int64_t dst_off = mtx == 0 ? dk_off : dv_off;
-        const int64_t dst_st = mtx == 0 ? a.dk_st[1] : a.dv_st[1];
-#pragma unroll
-        for (int n = 0; n < 32 * C::CPR / 64; n++) {
-          const int idx = n * 64 + lane_e;
-          const int row = idx / C::CPR, c = idx % C::CPR;
-          const V8 val = *(const V8*)(stage + row * C::ROWB + ((c ^ (row & (C::CPR - 1))) << 4));
-          const int jc = jw0 + kb * 32 + row;
-          if (jc < len_k)
-            put_grad8<T>(dst, dst_off + (int64_t)jc * dst_st + c * 8, val, a.wide_dkv, a.dkv_accumulate);
-        }
-        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // read before the next block overwrites
-      }
-    return;
-  }
-  {
-    // one running pointer (opaque to the optimiser, or it would keep 64 addresses in registers)
-    f32x4* mine = part_base + (int64_t)part * (GROUPS * C::THREADS) + (wave * 64 + lane_e);
-#pragma unroll
-    for (int mtx = 0; mtx < 2; mtx++)
 #pragma unroll
       for (int kb = 0; kb < KB; kb++)
 #pragma unroll
@@ -652,50 +674,73 @@ __global__ __launch_bounds__(256) void attn_bwd_dkdv_kernel(const AttnArgs a) {
           for (int i4 = 0; i4 < 4; i4++) {
             const f32x16& acc = mtx == 0 ? dk_acc[kb][d] : dv_acc[kb][d];
             const f32x4 val = {acc[4 * i4], acc[4 * i4 + 1], acc[4 * i4 + 2], acc[4 * i4 + 3]};
-            *mine = val;
-            mine += C::THREADS;
-            asm volatile("" : "+v"(mine));
+            const int c = d * 8 + 2 * i4 + g_e;
+            *(f32x4*)(q_s0 + wave * W_LDS + (kb * 32 + l32_e) * (D * 4) + ((c ^ (l32_e & (FPR - 1))) << 4)) = val;
           }
-  }
-  // Release: every wave waits for its own stores, then one thread makes the block's partial
-  // sums visible device-wide and counts the block in.  Acquire on the other side: the block
-  // that finds itself last drops what its compute unit and L2 may hold of those lines.
-  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-  __syncthreads();
-  if (tid == 0) {
-    __threadfence();
-    arrived_s = atomicAdd(a.dkv_count + unit, 1);
-  }
-  __syncthreads();
-  if (arrived_s != a.nsplit - 1) return;
-  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
-  if (tid == 0) a.dkv_count[unit] = 0;  // the next launch on this workspace starts from zero
-  // eight value groups at a time, all their loads in flight before the first sum
-  const f32x4* parts = part_base + (wave * 64 + lane_e);
-  constexpr int GB = 8;
-  static_assert(GROUPS % GB == 0, "batches of value groups");
-  for (int g0 = 0; g0 < GROUPS; g0 += GB) {  // group = ((mtx KB + kb) DB + d) 4 + i4
-    // four loads per group whatever nsplit is (a part past the last reads the last one again
-    // and is left out of the sum): no branch, so nothing waits between the loads
-    f32x4 v[GB][4];
+      __syncthreads();
+      void* const dst = mtx == 0 ? dk_buf : dv_buf;
+      const int64_t dst_off = mtx == 0 ? dk_off : dv_off;
+      const int64_t dst_st = mtx == 0 ? a.dk_st[1] : a.dv_st[1];
 #pragma unroll
-    for (int j = 0; j < GB; j++)
+      for (int n = 0; n < 64 * C::CPR / 256; n++) {
+        const int idx = n * 256 + wave * 64 + lane_e;
+        const int row = idx / C::CPR, c = (idx % C::CPR) * 2;
+        const char* src = q_s0 + row * (D * 4);
+        const int at0 = (c ^ (row & (FPR - 1))) << 4, at1 = ((c + 1) ^ (row & (FPR - 1))) << 4;
+        f32x4 lo = *(const f32x4*)(src + at0), hi = *(const f32x4*)(src + at1);
 #pragma unroll
-      for (int pp = 0; pp < 4; pp++)
-        v[j][pp] = parts[(int64_t)min(pp, a.nsplit - 1) * (GROUPS * C::THREADS) + j * C::THREADS];
-#pragma unroll
-    for (int j = 0; j < GB; j++) {
-      f32x4 sum = v[j][0];
-#pragma unroll
-      for (int pp = 1; pp < 4; pp++) {
-        const float use = pp < a.nsplit ? 1.f : 0.f;
-        sum += v[j][pp] * use;
+        for (int w = 1; w < 4; w++) {
+          lo += *(const f32x4*)(src + w * W_LDS + at0);
+          hi += *(const f32x4*)(src + w * W_LDS + at1);
+        }
+        const float x[8] = {lo[0] * sc, lo[1] * sc, lo[2] * sc, lo[3] * sc,
+                            hi[0] * sc, hi[1] * sc, hi[2] * sc, hi[3] * sc};
+        if (j0 + row < len_k)
+          put_grad8<T>(dst, dst_off + (int64_t)(j0 + row) * dst_st + c * 4, M::pack(x), a.wide_dkv, a.dkv_accumulate);
       }
-      const int grp = g0 + j;
-      emit(grp / (KB * DB * 4), grp / (DB * 4) % KB, grp / 4 % DB, grp % 4, sum);
+      __syncthreads();
     }
-    parts += GB * C::THREADS;
+    return;
   }
+  // Through LDS, one 32-key block of one matrix at a time: in the accumulator layout a lane
+  // holds 4 consecutive d of one key, so a direct store instruction would touch 32 rows with
+  // 16 bytes each (256 such instructions per block; at short walks -- 40 steps per block at
+  // window 1000 and one q head per kv head -- they took a tenth of the kernel).  Each wave
+  // stages its block in the tile buffer nobody reads any more (rows of 16-byte chunks, chunk
+  // c of row r at position c ^ (r % chunks-per-row)), and stores whole rows, 16 bytes a lane.
+  char* stage = wave == 0 ? q_s0 : wave == 1 ? q_s1 : wave == 2 ? do_s0 : do_s1;
+  static_assert(C::Q_TILE >= 32 * C::ROWB, "a 32-key block fits a tile buffer");
+  const int wr_row = l32_e * C::ROWB + g_e * 8;
+  const int wr_swz = l32_e & (C::CPR - 1);
+#pragma unroll
+  for (int mtx = 0; mtx < 2; mtx++)
+#pragma unroll
+    for (int kb = 0; kb < KB; kb++) {
+      const float sc = mtx == 0 ? a.scale : 1.f;
+#pragma unroll
+      for (int d = 0; d < DB; d++)
+#pragma unroll
+        for (int i4 = 0; i4 < 4; i4++) {
+          const f32x16& acc = mtx == 0 ? dk_acc[kb][d] : dv_acc[kb][d];
+          *(typename M::V4*)(stage + wr_row + (((d * 4 + i4) ^ wr_swz) << 4)) =
+              M::pack4(acc[4 * i4] * sc, acc[4 * i4 + 1] * sc, acc[4 * i4 + 2] * sc,
+                       acc[4 * i4 + 3] * sc);
+        }
+      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // the wave's own writes have landed
+      void* const dst = mtx == 0 ? dk_buf : dv_buf;
+      const int64_t dst_off = mtx == 0 ? dk_off : dv_off;
+      const int64_t dst_st = mtx == 0 ? a.dk_st[1] : a.dv_st[1];
+#pragma unroll
+      for (int n = 0; n < 32 * C::CPR / 64; n++) {
+        const int idx = n * 64 + lane_e;
+        const int row = idx / C::CPR, c = idx % C::CPR;
+        const V8 val = *(const V8*)(stage + row * C::ROWB + ((c ^ (row & (C::CPR - 1))) << 4));
+        const int jc = jw0 + kb * 32 + row;
+        if (jc < len_k)
+          put_grad8<T>(dst, dst_off + (int64_t)jc * dst_st + c * 8, val, a.wide_dkv, a.dkv_accumulate);
+      }
+      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // read before the next block overwrites
+    }
 }
 
 // ============================================================================
@@ -1483,9 +1528,9 @@ template <typename T, int D>
 __global__ __launch_bounds__(256) void attn_bwd_prep_kernel(const AttnArgs a) {
   using P = PrepCfg<D>;
   using V8 = typename Mma<T>::V8;
-  // arrival counters of the dK/dV kernel's split blocks start from zero
+  // arrival counters of the sink kernel start from zero
   for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < a.n_count; i += (int64_t)gridDim.x * 256)
-    a.dkv_count[i] = 0;
+    a.sink_count[i] = 0;
   // The delta array starts at the next 256-byte boundary after the lse2 array, and the tile
   // kernels read up to a tile of rows past the last one as statistics: the elements in between
   // get the neutral value (P exactly zero) rather than whatever the workspace held.
@@ -1543,10 +1588,11 @@ __global__ __launch_bounds__(256) void attn_bwd_prep_kernel(const AttnArgs a) {
 // launch stubs of only some of the variants.
 #define RSWA_INSTANTIATE(T, D)                                              \
   template __global__ void attn_bwd_dkdv_kernel<T, D, false, false, false>(const AttnArgs); \
-  template __global__ void attn_bwd_dkdv_kernel<T, D, true, false, false>(const AttnArgs);  \
-  template __global__ void attn_bwd_dkdv_kernel<T, D, false, true, false>(const AttnArgs);  \
-  template __global__ void attn_bwd_dkdv_kernel<T, D, true, true, false>(const AttnArgs);   \
-  template __global__ void attn_bwd_dkdv_kernel<T, D, false, false, true>(const AttnArgs);  \
+  template __global__ void attn_bwd_dkdv_kernel<T, D, false, false, true>(const AttnArgs); \
+  template __global__ void attn_bwd_dkdv_kernel<T, D, true, false, false>(const AttnArgs); \
+  template __global__ void attn_bwd_dkdv_kernel<T, D, true, false, true>(const AttnArgs); \
+  template __global__ void attn_bwd_dkdv_kernel<T, D, false, true, false>(const AttnArgs); \
+  template __global__ void attn_bwd_dkdv_kernel<T, D, false, true, true>(const AttnArgs); \
   template __global__ void attn_bwd_dq_ds_kernel<T, D>(const AttnArgs);                     \
   template __global__ void attn_bwd_dq_kernel<T, D, false, 8>(const AttnArgs);       \
   template __global__ void attn_bwd_dq_kernel<T, D, true, 8>(const AttnArgs);        \
@@ -1559,6 +1605,35 @@ RSWA_INSTANTIATE(__bf16, 64)
 RSWA_INSTANTIATE(_Float16, 128)
 RSWA_INSTANTIATE(_Float16, 64)
 #undef RSWA_INSTANTIATE
+
+// Does the dK/dV launch take blocks of 64 keys whose waves share out the walk (WALK4) instead of
+// blocks of 256 keys?  Both forms keep every compute unit busy with one block; what decides is how
+// evenly the launch's blocks fill the chip.  Estimated time of a form = the larger of its longest
+// block and of rounds x average block, a block being steps x (time of a step) + (prologue and
+// epilogue), with the times measured here (us): head_dim 128, 1.2 + 20 wide, 1.5 + 10 WALK4;
+// head_dim 64, 0.77 + 18 and 0.93 + 7.  Measured on both sides of the line (us, wide / WALK4, bf16,
+// head_dim 128): 32 / 8 heads, window 1024, 4096 rows 217 / 128, 6000 rows 218 / 190, 8192 rows (256
+// wide blocks, one full round) 229 / 255, 9000 rows 368 / 303, 16384 rows 477 / 523; 32 / 32 heads,
+// window 1000, 2 x 8192 rows 545 / 700; full attention over 4096 rows, 32 / 8 heads, 615 / 238.  Of the
+// 117 shapes timed the rule is 2 % behind the better form on average.
+bool dkv_walk4(const AttnArgs& a, int head_dim) {
+  const int64_t nseq = a.batch;
+  const int64_t lq = a.cu_q ? std::max<int64_t>(1, a.rows_q / a.batch) : a.seqlen_q;
+  const int64_t lk = a.cu_q ? std::max<int64_t>(1, a.rows_k / a.batch) : a.seqlen_k;
+  auto estimate = [&](int keys, int walkers, double step, double fixed) {
+    auto walk = [&](int64_t rows) {  // steps of a wave whose keys are seen by `rows` rows each
+      const int64_t r = std::min<int64_t>(lq, rows + std::min<int64_t>(keys, lk) - 1);
+      return std::max((double)a.group * r / (32. * walkers), std::ceil((double)a.group / walkers));
+    };
+    const double avg = walk(a.avg_rows), most = walk(a.max_rows);
+    double rounds = (double)(ceil_div(lk, keys) * a.heads_kv * nseq) / kComputeUnits;
+    // (blocks of equal length run in whole rounds; those of a ramp fill each other's gaps)
+    if (rounds < 4 && avg > 0.7 * most) rounds = std::ceil(rounds);
+    return std::max(most * step + fixed, rounds * (avg * step + fixed));
+  };
+  return head_dim == 128 ? estimate(64, 4, 1.5, 10.) < estimate(256, 1, 1.2, 20.)
+                         : estimate(64, 4, 0.93, 7.) < estimate(256, 1, 0.77, 18.);
+}
 
 template <typename T, int D>
 int launch_bwd(AttnArgs& a, hipStream_t stream, int phases) {
@@ -1573,26 +1648,27 @@ int launch_bwd(AttnArgs& a, hipStream_t stream, int phases) {
   }
   if (phases & RSWA_BWD_DKDV) {
     using C = DkvCfg<D>;
-    if (a.rows_q == 0) a.nsplit = 1;  // nothing to walk (and no statistics launch ran)
+    const bool walk4 = dkv_walk4(a, D);
+    const int bn = walk4 ? C::BN / 4 : C::BN;
     if (a.cu_q) {
-      a.n_tile = (int)(ceil_div(a.rows_k, C::BN) + a.batch);
-      a.n_work = a.n_tile * a.heads_kv * a.nsplit;
+      a.n_tile = (int)(ceil_div(a.rows_k, bn) + a.batch);
+      a.n_work = a.n_tile * a.heads_kv;
     } else {
-      a.n_tile = (int)ceil_div(a.seqlen_k, C::BN);
-      a.n_work = a.n_tile * a.heads_kv * a.batch * a.nsplit;
+      a.n_tile = (int)ceil_div(a.seqlen_k, bn);
+      a.n_work = a.n_tile * a.heads_kv * a.batch;
     }
     if (a.n_work > 0) {
       clear_launch_error();
       const dim3 grid(padded_grid(a.n_work)), block(C::THREADS);
-      if (a.ds) {  // (never with a.far or a.nsplit > 1: see bwd_layout)
-        hipLaunchKernelGGL((attn_bwd_dkdv_kernel<T, D, false, false, true>), grid, block, 0, stream, a);
-      } else if (a.nsplit > 1) {
-        if (a.far) hipLaunchKernelGGL((attn_bwd_dkdv_kernel<T, D, true, true, false>), grid, block, 0, stream, a);
-        else hipLaunchKernelGGL((attn_bwd_dkdv_kernel<T, D, true, false, false>), grid, block, 0, stream, a);
-      } else {
-        if (a.far) hipLaunchKernelGGL((attn_bwd_dkdv_kernel<T, D, false, true, false>), grid, block, 0, stream, a);
-        else hipLaunchKernelGGL((attn_bwd_dkdv_kernel<T, D, false, false, false>), grid, block, 0, stream, a);
-      }
+      auto go = [&](auto far, auto hand, auto w4) {
+        hipLaunchKernelGGL((attn_bwd_dkdv_kernel<T, D, decltype(far)::value, decltype(hand)::value, decltype(w4)::value>),
+                           grid, block, 0, stream, a);
+      };
+      constexpr std::true_type yes{};
+      constexpr std::false_type no{};
+      if (a.ds) walk4 ? go(no, yes, yes) : go(no, yes, no);  // (never with a.far: see bwd_layout)
+      else if (a.far) walk4 ? go(yes, no, yes) : go(yes, no, no);
+      else walk4 ? go(no, no, yes) : go(no, no, no);
       int rc = check_launch("attn_bwd dkdv");
       if (rc != RSWA_OK) return rc;
     }
@@ -1656,10 +1732,9 @@ int launch_bwd(AttnArgs& a, hipStream_t stream, int phases) {
 
 namespace rswa {
 namespace {
-int bwd_entry(const rswa_attn_params* p, void* stream, int phases, bool allow_split,
-              bool allow_handoff) {
+int bwd_entry(const rswa_attn_params* p, void* stream, int phases, bool allow_handoff) {
   AttnArgs a;
-  int rc = fill_args(p, true, a, allow_split, allow_handoff);
+  int rc = fill_args(p, true, a, allow_handoff);
   if (rc != RSWA_OK) return rc;
   hipStream_t st = (hipStream_t)stream;
   if (p->dtype == RSWA_BF16) {
@@ -1673,7 +1748,7 @@ int bwd_entry(const rswa_attn_params* p, void* stream, int phases, bool allow_sp
 }  // namespace rswa
 
 extern "C" int rswa_attn_bwd_phases(const rswa_attn_params* p, void* stream, int phases) {
-  return rswa::bwd_entry(p, stream, phases, true, true);
+  return rswa::bwd_entry(p, stream, phases, true);
 }
 
 extern "C" int rswa_attn_bwd(const rswa_attn_params* p, void* stream) {
@@ -1722,7 +1797,6 @@ extern "C" int rswa_attn_bwd_static_init(void) {
 extern "C" int rswa_attn_bwd_static(const rswa_attn_params* p, void* stream) {
   using namespace rswa;
   RSWA_REQUIRE(p != nullptr, RSWA_ERR_INVALID, "attn_bwd_static: null params");
-  // statistics only: on the built-in buffer the dK/dV kernel never splits its key tiles
   const uint64_t need = bwd_layout(p, false).total_bytes;
   RSWA_REQUIRE(need <= RSWA_BWD_STATIC_MAX_BYTES, RSWA_ERR_UNSUPPORTED,
                "attn_bwd_static: rows * heads_q needs %llu bytes of statistics, the built-in "
@@ -1741,5 +1815,5 @@ extern "C" int rswa_attn_bwd_static(const rswa_attn_params* p, void* stream) {
   void* ptr = scratch_on_current_device();
   if (!ptr) return RSWA_ERR_LAUNCH;
   q.workspace = ptr;
-  return bwd_entry(&q, stream, RSWA_BWD_PREP | RSWA_BWD_DKDV | RSWA_BWD_DQ, false, false);
+  return bwd_entry(&q, stream, RSWA_BWD_PREP | RSWA_BWD_DKDV | RSWA_BWD_DQ, false);
 }

@@ -34,12 +34,7 @@ struct AttnArgs {
   void* dv;
   float* delta;   // fp32 [heads_q, rows_q] packed: -sum_d dO * O         (workspace)
   float* lse2;    // fp32 [heads_q, rows_q] packed: -lse * log2(e); empty rows -inf (workspace)
-  // dK/dV kernel with the q heads of a GQA group split over `nsplit` blocks per key tile:
-  // fp32 partial sums [tile unit][part] and one arrival counter per tile unit (workspace)
-  float* dkv_part;
-  int32_t* dkv_count;
-  int32_t nsplit;     // 1: one block per (key tile, kv head) walks the whole group
-  int32_t n_count;    // arrival counters in the workspace
+  int32_t n_count;    // arrival counters in the workspace (sink kernel)
   const int32_t* cu_q;
   const int32_t* cu_k;
   int64_t q_st[3], k_st[3], v_st[3], o_st[3], do_st[3], dq_st[3], dk_st[3], dv_st[3], lse_st[3];
@@ -73,6 +68,7 @@ struct AttnArgs {
   void* dk2;
   void* dv2;
   int32_t seg;
+  int32_t avg_rows, max_rows;  // query rows that see a key: on average, at most (host estimate, as avg_keys)
   int32_t avg_keys;  // keys a query row sees on average (host estimate; block shapes hang on it)
   int32_t far;  // a sequence of some streamed tensor spans 2 GiB or more: FAR kernels
   // dS hand-off (backward): the dK/dV kernel stores its packed 16-bit dS tiles and the dQ
@@ -398,6 +394,66 @@ struct TileDma {
   }
 };
 
+// The four words of a buffer resource over `bytes` bytes at `base`, for inline assembly.
+__device__ __forceinline__ u32x4 rsrc_words(const void* base, int bytes) {
+  const uint64_t p = (uint64_t)base;
+  return u32x4{(uint32_t)p, (uint32_t)(p >> 32) & 0xffffu, (uint32_t)bytes, 0x00020000u};
+}
+// tile_src in that form: the resource of the tile whose first row is row0 (FAR: based at that row)
+template <int ROWS, bool FAR>
+__device__ __forceinline__ u32x4 tile_words(const void* base, int row0, int rows, int stride_bytes,
+                                            int row_bytes) {
+  if constexpr (FAR) {
+    const int n = min(rows - row0, ROWS);
+    const uint64_t off = (uint64_t)(uint32_t)row0 * (uint64_t)(uint32_t)stride_bytes;
+    return rsrc_words((const char*)base + off, n > 0 ? (n - 1) * stride_bytes + row_bytes : 0);
+  } else {
+    return rsrc_words(base, (rows - 1) * stride_bytes + row_bytes);
+  }
+}
+// A load that lands in LDS (lane L of the wave: at `lds` + BYTES L) as inline assembly: the
+// compiler does not see it write LDS and so never waits for it on its own -- the caller waits
+// (wait_dma) before it reads what was loaded.  For tile buffers picked at run time, which the
+// compiler cannot tell apart: with the builtin it would wait for the load in flight before every
+// LDS read.  (One wait state between the write of m0 and its use.)
+template <int BYTES>
+__device__ __forceinline__ void lds_load_asm(u32x4 rsrc, int voff, int soff, uint32_t lds) {
+  static_assert(BYTES == 4 || BYTES == 16, "one dword or four per lane");
+  if constexpr (BYTES == 16) {
+    asm volatile("s_mov_b32 m0, %3\n\ts_nop 0\n\tbuffer_load_dwordx4 %0, %1, %2 offen lds"
+                 :: "v"(voff), "s"(rsrc), "s"(soff), "s"(lds) : "memory");
+  } else {
+    asm volatile("s_mov_b32 m0, %3\n\ts_nop 0\n\tbuffer_load_dword %0, %1, %2 offen lds"
+                 :: "v"(voff), "s"(rsrc), "s"(soff), "s"(lds) : "memory");
+  }
+}
+
+// TileDma for a tile that one wave loads for itself (layout as of TileDma with swz_f): instruction n
+// covers rows n RPI .. n RPI + RPI - 1, fewer than the 16 after which the swizzle repeats, so the
+// chunk part of the lane offset takes one of 16 / RPI forms in turn, made by one XOR-and-add from
+// the lane's chunk in the tile's first rows (`chunk`, the same for every tensor).
+template <int D, int ROWS>
+struct WaveTileDma {
+  static constexpr int CPR = D / 8;
+  static constexpr int RPI = 64 / CPR;
+  static constexpr int N = ROWS * CPR / 64;
+  int row_off;
+  int step_bytes;
+  static __device__ __forceinline__ int chunk(int lane) {
+    return ((lane % CPR) ^ swz_f<CPR>(lane / CPR)) << 4;
+  }
+  __device__ __forceinline__ void init(int64_t stride_elems, int tid) {
+    row_off = (int)((tid & 63) / CPR * stride_elems * 2);
+    step_bytes = (int)(RPI * stride_elems * 2);
+  }
+  template <int NTH>
+  __device__ __forceinline__ void load_one(u32x4 rsrc, int soff, uint32_t lds_tile, int chunk0) const {
+    // rows n RPI + r, r < RPI: swz_f(n RPI + r) = swz_f(r) ^ swz_f(n RPI)
+    constexpr int x = (CPR == 16 ? NTH & 3 : (NTH & 1) << 1) << 4;
+    lds_load_asm<16>(rsrc, (chunk0 ^ x) + row_off, soff + NTH * step_bytes, lds_tile + NTH * 1024);
+  }
+};
+
 // f(integral_constant<int, 0>{}), ..., f(integral_constant<int, N - 1>{}): a loop whose
 // index is a compile-time constant in every iteration (register arrays indexed by it never
 // fall back to dynamic indexing, whatever the unroller thinks of the body's size).
@@ -440,15 +496,7 @@ __device__ __forceinline__ float halfwave_sum(float x) {
   return __uint_as_float(r[0]) + __uint_as_float(r[1]);
 }
 
-// Keys per block of the dK/dV kernel, and how a launch of it is laid out: with so few key
-// tiles that one block per (tile, kv head) would leave half of the 256 compute units without
-// work, the q heads of each GQA group are dealt to `nsplit` blocks, whose fp32 partial sums
-// meet in the workspace.  Measured on the rank share (8192-token chunk, window 4096, 32 / 8
-// heads): the previous-chunk corner (128 blocks) 0.75 -> 0.30 ms; the own-chunk block (256
-// blocks of 32..544 steps) gains 4 % alone and loses 8 % beside the corner launch -- more
-// compute units busy lowers the shader clock (1.92 -> 1.77 GHz), and every part pays its own
-// prologue, partial store and share of the final sum -- so launches that already give every
-// compute unit a block are left alone.
+// Keys per block of the dK/dV kernel
 constexpr int kDkvKeysPerBlock = 256;
 // dS hand-off: bytes one dK/dV block leaves per 32-row query tile (32 x 256 16-bit values) and
 // per wave of it (32 x 64: the unit the dQ kernel of that route fetches)
@@ -457,29 +505,19 @@ constexpr int kDsUnitBytes = kDsBlockBytes / 4;
 constexpr int kMaxTileRows = 256;  // bound on the rows fetched as one tile that the stride checks assume
                                    // (today's largest tile has 64 rows: K / V in the forward and dQ kernels)
 constexpr int kComputeUnits = 256;  // MI355X
-#ifndef RSWA_DKDV_SPLIT_BELOW
-#define RSWA_DKDV_SPLIT_BELOW (kComputeUnits / 2 + 1)
-#endif
-constexpr int kDkvSplitBelow = RSWA_DKDV_SPLIT_BELOW;  // split launches of fewer blocks
 struct BwdLayout {
   uint64_t stats_bytes;    // each of the two statistics arrays
-  int nsplit;
-  int n_tile_k;            // key tile slots per kv head (dense: per batch entry)
-  int n_count;             // arrival counters (one per key tile unit)
-  uint64_t count_off, part_off, total_bytes;
+  int n_count;             // arrival counters of the sink kernel
+  uint64_t count_off, total_bytes;
   int sink_chunks;         // row chunks of the sink kernel per (sequence, kv head); 0: no sink kernel
-  int sink_count_index;    // its first arrival counter
   uint64_t sink_off;       // its fp32 sums
   // dS hand-off (ds_bytes == 0: not used for this call)
   uint64_t ds_off, ds_bytes;
   int ds_nkb, ds_slots;
 };
-BwdLayout bwd_layout(const rswa_attn_params* p, bool allow_split, bool allow_handoff = false);
+BwdLayout bwd_layout(const rswa_attn_params* p, bool allow_handoff);
 
 // Fill an AttnArgs from the public struct; validates what both directions share.
-// `allow_split` = false keeps the dK/dV kernel at one block per key tile, whatever the shape
-// (workspace holds the statistics only).
-int fill_args(const rswa_attn_params* p, bool backward, AttnArgs& a, bool allow_split = true,
-              bool allow_handoff = false);
+int fill_args(const rswa_attn_params* p, bool backward, AttnArgs& a, bool allow_handoff = false);
 
 }  // namespace rswa

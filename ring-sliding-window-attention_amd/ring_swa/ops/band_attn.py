@@ -245,10 +245,8 @@ def attn_bwd(
     tiles in the workspace and dQ comes from a kernel that only multiplies them with K instead
     of recomputing S and dP.  ``None`` (default) takes it when the library accepts the shape and
     the tiles fit ``handoff_max_bytes()`` (0 unless the environment switches the route on: it is
-    not faster at the sizes measured); ``True`` asks for it whatever its size (shapes the
-    library does not accept still take the recomputing route, and so do small launches whose key
-    tiles the dK/dV kernel splits over several blocks -- ``"force"`` prefers the hand-off to that
-    split); ``False`` never.  With
+    not faster at the sizes measured); ``True`` (or ``"force"``) asks for it whatever its size
+    (shapes the library does not accept still take the recomputing route); ``False`` never.  With
     ``phases`` spread over several calls the same value must be passed to each, on the same
     workspace, and the dK/dV phase must run before the dQ phase.  A ``workspace`` the caller
     supplies without room for the dS tiles makes the automatic choice (``None``) recompute."""
@@ -378,8 +376,7 @@ def bwd_workspace_bytes(q: torch.Tensor, k: torch.Tensor,
                         num_sink: int = 0, handoff: Optional[bool] = False) -> int:
     """Scratch size of one backward over ``q`` against ``k`` (dense ``[B,S,H,D]`` or packed
     ``[T,H,D]``), as ``rswa_attn_bwd_workspace_bytes`` computes it: two fp32 values per
-    (row, q head); the partial sums of the dK/dV kernel when the shape makes it deal the q
-    heads of a GQA group to several blocks; the sums of the sink kernel with ``num_sink`` keys
+    (row, q head); the sums of the sink kernel with ``num_sink`` keys
     under a bounded window; the dS tiles with ``handoff`` (which depend on the window).  Pass the
     mask and ``handoff`` of the ``attn_bwd`` call the workspace is for."""
     p = _params(q, k, k, 1.0, window_size, causal, cu_seqlens_q, cu_seqlens_k, num_sink)
