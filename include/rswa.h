@@ -291,7 +291,8 @@ int rswa_attn_bwd_static_init(void);
 
 /* Scratch rswa_attn_bwd needs for these shapes: two fp32 values per (row, q head) -- the
  * row sum of dout * out and the LSE in base-2 units --, with sink keys under a bounded window the
- * sink kernel's arrival counters and fp32 sums, and with ds_handoff the dS tiles.  Nothing in the workspace has to be initialised by the caller. */
+ * sink kernel's arrival counters and fp32 sums, for a pack one int32 per sequence and two more (the
+ * key tile table), and with ds_handoff the dS tiles.  Nothing in the workspace has to be initialised by the caller. */
 uint64_t rswa_attn_bwd_workspace_bytes(const rswa_attn_params* p);
 
 /* 1 when a backward with these parameters takes the dS hand-off route (ds_handoff != 0 and the

@@ -26,7 +26,7 @@ static bool handoff_eligible(const rswa_attn_params* p) {
   return true;
 }
 
-BwdLayout bwd_layout(const rswa_attn_params* p, bool allow_handoff) {
+BwdLayout bwd_layout(const rswa_attn_params* p, bool allow_handoff, uint64_t max_bytes) {
   BwdLayout L{};
   if (!p || p->batch <= 0 || p->heads_q <= 0 || p->heads_kv <= 0 || p->head_dim <= 0) return L;
   L.stats_bytes = delta_bytes(p);
@@ -41,12 +41,20 @@ BwdLayout bwd_layout(const rswa_attn_params* p, bool allow_handoff) {
     L.sink_chunks = (int)std::min<int64_t>(64, std::max<int64_t>(1, (rows_q + 511) / 512));
     sink_units = (int64_t)p->batch * p->heads_kv;
   }
-  // workspace: statistics | arrival counters and sums of the sink kernel | dS tiles
+  // workspace: statistics | arrival counters and sums of the sink kernel | key tile table | dS tiles
   L.n_count = (int)sink_units;
   L.count_off = 2 * L.stats_bytes;
   L.sink_off = L.count_off + align_up((uint64_t)L.n_count * sizeof(int32_t), 256);
   L.total_bytes = L.sink_off + (uint64_t)sink_units * L.sink_chunks * p->num_sink * 2 * p->head_dim *
                                    sizeof(float);
+  if (packed) {
+    const uint64_t off = align_up(L.total_bytes, 256);
+    const uint64_t end = off + ((uint64_t)p->batch + 2) * sizeof(int32_t);
+    if (end <= max_bytes) {
+      L.ktile_off = off;
+      L.total_bytes = end;
+    }
+  }
   // dS hand-off: one 4 KiB unit per (q head, 32-row tile slot, 256-key block modulo nkb, 64-key
   // group).  A row tile sees keys [i0 + shift - left, i0 + 31 + shift + right]: left + right + 32
   // consecutive keys, which touch at most (left + right + 31) / 256 + 2 blocks of 256, and never
@@ -84,7 +92,8 @@ static bool rows_aligned(const void* ptr, const int64_t* st, int elem_bytes = 2)
   return true;
 }
 
-int fill_args(const rswa_attn_params* p, bool backward, AttnArgs& a, bool allow_handoff) {
+int fill_args(const rswa_attn_params* p, bool backward, AttnArgs& a, bool allow_handoff,
+              uint64_t max_bytes) {
   RSWA_REQUIRE(p != nullptr, RSWA_ERR_INVALID, "attn: null params");
   RSWA_REQUIRE(p->dtype == RSWA_BF16 || p->dtype == RSWA_F16, RSWA_ERR_UNSUPPORTED,
                "attn: dtype %d (only bf16 and fp16)", p->dtype);
@@ -170,6 +179,9 @@ int fill_args(const rswa_attn_params* p, bool backward, AttnArgs& a, bool allow_
   a.delta = nullptr;
   a.lse2 = nullptr;
   a.n_count = 0;
+  a.ktile = nullptr;
+  a.ktile_log2 = 0;
+  a.snake = 0;
   a.sink_part = nullptr;
   a.sink_count = nullptr;
   a.sink_chunks = 0;
@@ -247,18 +259,9 @@ int fill_args(const rswa_attn_params* p, bool backward, AttnArgs& a, bool allow_
     a.rev_q = keys_of(lq - 1) > keys_of(0);
     a.rev_k = rows_of(lk - 1) > rows_of(0);
     // keys a query row sees on average (keys_of is piecewise linear: 17 samples)
-    int64_t sum = 0, sum_r = 0, max_r = 0;
-    for (int t = 0; t <= 16; t++) {
-      sum += keys_of((lq - 1) * t / 16);
-      // (sink keys under a bounded window are the sink kernel's: band rows only)
-      const int64_t j = std::max<int64_t>((lk - 1) * t / 16, a.wl >= 0 ? std::min<int64_t>(a.n_sink, lk - 1) : 0);
-      const int64_t r = rows_of(j);
-      sum_r += r;
-      max_r = std::max(max_r, r);
-    }
+    int64_t sum = 0;
+    for (int t = 0; t <= 16; t++) sum += keys_of((lq - 1) * t / 16);
     a.avg_keys = (int32_t)std::min<int64_t>(sum / 17, INT32_MAX);
-    a.avg_rows = (int32_t)std::min<int64_t>(sum_r / 17, INT32_MAX);
-    a.max_rows = (int32_t)std::min<int64_t>(max_r, INT32_MAX);
   }
   a.scale = p->softmax_scale;
   a.scale_log2 = p->softmax_scale * kLog2e;
@@ -272,7 +275,7 @@ int fill_args(const rswa_attn_params* p, bool backward, AttnArgs& a, bool allow_
                  RSWA_ERR_UNSUPPORTED, "attn_bwd: dout/dq/dk/dv rows must start 16-byte aligned");
     RSWA_REQUIRE(p->dout_stride[1] >= 0 && p->dout_stride[1] * 2 < ((1ll << 31) - 65536) / kMaxTileRows,
                  RSWA_ERR_UNSUPPORTED, "attn_bwd: row stride of dout is negative or too large");
-    const BwdLayout L = bwd_layout(p, allow_handoff);
+    const BwdLayout L = bwd_layout(p, allow_handoff, max_bytes);
     const uint64_t need = L.total_bytes;
     RSWA_REQUIRE(p->workspace != nullptr || need == 0, RSWA_ERR_INVALID,
                  "attn_bwd: null workspace");
@@ -284,6 +287,8 @@ int fill_args(const rswa_attn_params* p, bool backward, AttnArgs& a, bool allow_
     a.lse2 = (float*)p->workspace;
     a.delta = (float*)((char*)p->workspace + delta_bytes(p));
     a.n_count = L.n_count;
+    // (no query rows: no statistics launch, which would write it)
+    if (L.ktile_off && a.rows_q > 0) a.ktile = (int32_t*)((char*)p->workspace + L.ktile_off);
     a.sink_chunks = L.sink_chunks;
     a.sink_part = L.sink_chunks ? (float*)((char*)p->workspace + L.sink_off) : nullptr;
     a.sink_count = (int32_t*)((char*)p->workspace + L.count_off);

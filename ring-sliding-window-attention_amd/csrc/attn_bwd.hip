@@ -87,6 +87,8 @@ __device__ __forceinline__ void put_grad8(void* buf, int64_t at, typename Mma<T>
   }
 }
 
+constexpr int kSnakeKeys = 4096;  // longest sequence whose dK/dV blocks take the snake order
+
 // ============================================================================
 // dK / dV
 // ============================================================================
@@ -133,8 +135,28 @@ __global__ __launch_bounds__(256) void attn_bwd_dkdv_kernel(const AttnArgs a) {
   __shared__ __attribute__((aligned(1024))) float st_s0[(WALK4 ? 8 : 2) * C::BM];  // -lse2[BM], -delta[BM]
   __shared__ __attribute__((aligned(1024))) float st_s1[(WALK4 ? 8 : 2) * C::BM];
 
-  const int wid = logical_block_id(a.n_work);
-  if (wid < 0) return;
+  // A pack's exact number of key tiles is known on the device only (ktile, see the statistics
+  // kernel): the tiles come first in the launch, dealt evenly to the XCDs, and the blocks beyond
+  // them end here.  Consecutive blocks of an XCD go to its shader engines in turn and wait for the
+  // engine whose turn it is, so lengths that repeat with an even period leave engines idle: with a
+  // pack's tiles numbered by slots, one of them unused per sequence, as in the other kernels, 64
+  // sequences of 256 tokens (32 / 8 heads, head_dim 128) took 242 us, every other block being empty;
+  // numbered exactly, 129 us.  `snake` reverses every other group of four blocks where the walks
+  // of a short sequence's few tiles, one sequence like the other, are the pattern: 64 sequences of
+  // 1024 tokens 1368 -> 1141 us, dense causal 4096 rows x 32 heads 300 -> 277 us.  (Sequences
+  // longer than 4096 keys keep the plain order: four of 16384 tokens lose 3 % by it.)
+  int n_tile = a.n_tile, n_work = a.n_work, per_xcd = (int)gridDim.x >> 3, snake = a.snake;
+  if (a.ktile) {
+    n_tile = a.ktile[a.batch];
+    snake = a.ktile[a.batch + 1];
+    n_work = n_tile * a.heads_kv;
+    per_xcd = (n_work + 7) >> 3;
+  }
+  int in_xcd = (int)blockIdx.x >> 3;
+  if (in_xcd >= per_xcd) return;
+  if (snake && (in_xcd & 4) && (in_xcd | 3) < per_xcd) in_xcd ^= 3;
+  const int wid = ((int)blockIdx.x & 7) * per_xcd + in_xcd;
+  if (wid >= n_work) return;
   const int tid = threadIdx.x;
   const int lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);  // (not WALK4: key group of 64 keys)
@@ -144,12 +166,14 @@ __global__ __launch_bounds__(256) void attn_bwd_dkdv_kernel(const AttnArgs a) {
   const int u = lane >> 4;
 
   // ---- which (sequence, kv head, key tile); tiles go heaviest first -------------------
-  const int slot = a.rev_k ? a.n_tile - 1 - wid % a.n_tile : wid % a.n_tile;
-  int rest = wid / a.n_tile;
+  const int slot = a.rev_k ? n_tile - 1 - wid % n_tile : wid % n_tile;
+  int rest = wid / n_tile;
   const int hk = rest % a.heads_kv;
   SeqInfo s;
   int kt;
-  if (a.cu_q) {
+  if (a.ktile) {
+    locate_tile(a, slot, s, kt);
+  } else if (a.cu_q) {
     static_assert(C::BN == 1 << 8, "tile size passed to locate_packed");
     if (!locate_packed(a, slot, WALK4 ? 6 : 8, true, s, kt)) return;
   } else {
@@ -1538,8 +1562,48 @@ __global__ __launch_bounds__(256) void attn_bwd_prep_kernel(const AttnArgs a) {
     const int64_t used = a.rows_q * a.heads_q;
     if (used + threadIdx.x < a.delta - a.lse2) a.lse2[used + threadIdx.x] = -__builtin_inff();
   }
-  const int h = (int)(blockIdx.x % (unsigned)a.heads_q);
-  const int64_t row0 = (int64_t)(blockIdx.x / (unsigned)a.heads_q) * P::ROWS + threadIdx.x / P::LPR;
+  // The first block of a pack's launch writes the key tile table: running sums of the sequences'
+  // tile counts, 256 sequences at a time (a scan in each wave, the waves' totals through LDS).
+  if (a.ktile) {
+    if (blockIdx.x == 0) {
+      __shared__ int wave_sum[4];
+      const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+      const int first_n = (a.cu_k[1] - a.cu_k[0] + (1 << a.ktile_log2) - 1) >> a.ktile_log2;
+      int unlike = 0;  // some sequence has another number of tiles than the first
+      int base = 0;
+      for (int b0 = 0; b0 < a.batch; b0 += 256) {
+        const int b = b0 + (int)threadIdx.x;
+        const int len = b < a.batch ? a.cu_k[b + 1] - a.cu_k[b] : 0;
+        const int n = (len + (1 << a.ktile_log2) - 1) >> a.ktile_log2;
+        int sum = n;  // inclusive
+#pragma unroll
+        for (int m = 1; m < 64; m <<= 1) {
+          const int up = __shfl_up(sum, m, 64);
+          if (lane >= m) sum += up;
+        }
+        __syncthreads();  // (wave_sum of the previous pass has been read)
+        if (lane == 63) wave_sum[wave] = sum;
+        __syncthreads();
+        int before = base;
+        for (int w = 0; w < 4; w++) {
+          if (w < wave) before += wave_sum[w];
+          base += wave_sum[w];
+        }
+        if (b < a.batch) a.ktile[b] = before + sum - n;
+        // (the last sequence may be a remainder)
+        unlike |= b < a.batch - 1 && n != first_n;
+      }
+      unlike = __syncthreads_or(unlike);
+      if (threadIdx.x == 0) {
+        a.ktile[a.batch] = base;
+        a.ktile[a.batch + 1] = !unlike && first_n << a.ktile_log2 <= kSnakeKeys;
+      }
+      return;
+    }
+  }
+  const unsigned blk = blockIdx.x - (a.ktile ? 1 : 0);
+  const int h = (int)(blk % (unsigned)a.heads_q);
+  const int64_t row0 = (int64_t)(blk / (unsigned)a.heads_q) * P::ROWS + threadIdx.x / P::LPR;
   const int c = (threadIdx.x % P::LPR) * 8;
   // Packed rows past the last sequence belong to nobody: their out / dout may hold anything
   // (NaN included), and the tile kernels read the statistics of the rows that follow a
@@ -1615,31 +1679,57 @@ RSWA_INSTANTIATE(_Float16, 64)
 // head_dim 128): 32 / 8 heads, window 1024, 4096 rows 217 / 128, 6000 rows 218 / 190, 8192 rows (256
 // wide blocks, one full round) 229 / 255, 9000 rows 368 / 303, 16384 rows 477 / 523; 32 / 32 heads,
 // window 1000, 2 x 8192 rows 545 / 700; full attention over 4096 rows, 32 / 8 heads, 615 / 238.  Of the
-// 117 shapes timed the rule is 2 % behind the better form on average.
+// 78 dense shapes timed the rule is 1 % behind the better form on average.
+// A pack is judged on its average length L, the only one the host knows, as if of sequences of
+// 1.5 L (what a token sees when lengths vary), none longer than 3 L, with half a key tile per
+// sequence wasted.  Packs of 16384 tokens, 32 / 8 heads, window 1024, lengths log-uniform: 16-64
+// 262 / 173, 64-256 193 / 175, 16-1024 260 / 216; all of 512 198 / 204, 32 / 32 heads 16-1024 348 / 475.
+// The 0.9 leans to the wide form where lengths are alike (65536 tokens of 512: 715 / 784).
 bool dkv_walk4(const AttnArgs& a, int head_dim) {
-  const int64_t nseq = a.batch;
-  const int64_t lq = a.cu_q ? std::max<int64_t>(1, a.rows_q / a.batch) : a.seqlen_q;
-  const int64_t lk = a.cu_q ? std::max<int64_t>(1, a.rows_k / a.batch) : a.seqlen_k;
+  const bool pack = a.cu_q != nullptr;
+  const int64_t lk1 = pack ? std::max<int64_t>(1, a.rows_k / a.batch) : a.seqlen_k;
+  const int64_t lq1 = pack ? std::max<int64_t>(1, a.rows_q / a.batch) : a.seqlen_q;
+  const int64_t lq = pack ? std::min(a.rows_q, lq1 * 3 / 2) : lq1, lk = pack ? std::min(a.rows_k, lk1 * 3 / 2) : lk1;
+  // query rows that see a key, of the first the band kernel owns to the last: on average, at most
+  const int64_t sh = a.shift_explicit ? a.shift_val : lk - lq;
+  const int64_t first = a.wl >= 0 ? std::min<int64_t>(a.n_sink, std::max<int64_t>(lk - 1, 0)) : 0;
+  double avg_rows = 0, max_rows = 0;
+  for (int t = 0; t <= 16; t++) {
+    const int64_t j = std::max((lk - 1) * t / 16, first);
+    const int64_t lo = a.wr >= 0 ? std::max<int64_t>(0, j - sh - a.wr) : 0;
+    const int64_t hi = a.wl >= 0 ? std::min(lq - 1, j - sh + a.wl) : lq - 1;
+    const double r = (double)std::max<int64_t>(0, hi - lo + 1);
+    avg_rows += r / 17;
+    max_rows = std::max(max_rows, r);
+  }
+  if (pack) {
+    max_rows = (double)std::min(a.rows_q, 3 * lq1);
+    if (a.wl >= 0 && a.wr >= 0) max_rows = std::min(max_rows, (double)a.wl + a.wr + 1);
+  }
   auto estimate = [&](int keys, int walkers, double step, double fixed) {
-    auto walk = [&](int64_t rows) {  // steps of a wave whose keys are seen by `rows` rows each
-      const int64_t r = std::min<int64_t>(lq, rows + std::min<int64_t>(keys, lk) - 1);
-      return std::max((double)a.group * r / (32. * walkers), std::ceil((double)a.group / walkers));
+    auto walk = [&](double rows, int64_t len) {  // steps of a wave whose keys are seen by `rows` rows each
+      const double r = std::min<double>((double)len, rows + (double)std::min<int64_t>(keys, lk1) - 1);
+      return std::max(a.group * r / (32. * walkers), std::ceil((double)a.group / walkers));
     };
-    const double avg = walk(a.avg_rows), most = walk(a.max_rows);
-    double rounds = (double)(ceil_div(lk, keys) * a.heads_kv * nseq) / kComputeUnits;
+    const double avg = walk(avg_rows, lq), most = walk(max_rows, pack ? 3 * lq1 : lq);
+    const double tiles = pack ? (double)lk1 / keys + 0.5 : (double)ceil_div(lk1, keys);
+    double rounds = tiles * a.heads_kv * a.batch / kComputeUnits;
     // (blocks of equal length run in whole rounds; those of a ramp fill each other's gaps)
     if (rounds < 4 && avg > 0.7 * most) rounds = std::ceil(rounds);
     return std::max(most * step + fixed, rounds * (avg * step + fixed));
   };
-  return head_dim == 128 ? estimate(64, 4, 1.5, 10.) < estimate(256, 1, 1.2, 20.)
-                         : estimate(64, 4, 0.93, 7.) < estimate(256, 1, 0.77, 18.);
+  const double lean = pack ? 0.9 : 1.;
+  return head_dim == 128 ? estimate(64, 4, 1.5, 10.) < lean * estimate(256, 1, 1.2, 20.)
+                         : estimate(64, 4, 0.93, 7.) < lean * estimate(256, 1, 0.77, 18.);
 }
 
 template <typename T, int D>
 int launch_bwd(AttnArgs& a, hipStream_t stream, int phases) {
   const int64_t units = a.rows_q * a.heads_q;
+  const bool walk4 = dkv_walk4(a, D);
+  a.ktile_log2 = walk4 ? 6 : 8;
   if (units > 0 && (phases & RSWA_BWD_PREP)) {
-    const int64_t blocks = ceil_div(a.rows_q, PrepCfg<D>::ROWS) * a.heads_q;
+    const int64_t blocks = ceil_div(a.rows_q, PrepCfg<D>::ROWS) * a.heads_q + (a.ktile ? 1 : 0);
     RSWA_REQUIRE(blocks < (1ll << 31), RSWA_ERR_UNSUPPORTED, "attn_bwd: too many (row, head) pairs");
     clear_launch_error();
     hipLaunchKernelGGL((attn_bwd_prep_kernel<T, D>), dim3((unsigned)blocks), dim3(256), 0, stream, a);
@@ -1648,7 +1738,6 @@ int launch_bwd(AttnArgs& a, hipStream_t stream, int phases) {
   }
   if (phases & RSWA_BWD_DKDV) {
     using C = DkvCfg<D>;
-    const bool walk4 = dkv_walk4(a, D);
     const int bn = walk4 ? C::BN / 4 : C::BN;
     if (a.cu_q) {
       a.n_tile = (int)(ceil_div(a.rows_k, bn) + a.batch);
@@ -1657,6 +1746,7 @@ int launch_bwd(AttnArgs& a, hipStream_t stream, int phases) {
       a.n_tile = (int)ceil_div(a.seqlen_k, bn);
       a.n_work = a.n_tile * a.heads_kv * a.batch;
     }
+    a.snake = !a.cu_q && a.seqlen_k <= kSnakeKeys;
     if (a.n_work > 0) {
       clear_launch_error();
       const dim3 grid(padded_grid(a.n_work)), block(C::THREADS);
@@ -1732,9 +1822,10 @@ int launch_bwd(AttnArgs& a, hipStream_t stream, int phases) {
 
 namespace rswa {
 namespace {
-int bwd_entry(const rswa_attn_params* p, void* stream, int phases, bool allow_handoff) {
+int bwd_entry(const rswa_attn_params* p, void* stream, int phases, bool allow_handoff,
+              uint64_t max_bytes = ~0ull) {
   AttnArgs a;
-  int rc = fill_args(p, true, a, allow_handoff);
+  int rc = fill_args(p, true, a, allow_handoff, max_bytes);
   if (rc != RSWA_OK) return rc;
   hipStream_t st = (hipStream_t)stream;
   if (p->dtype == RSWA_BF16) {
@@ -1797,7 +1888,7 @@ extern "C" int rswa_attn_bwd_static_init(void) {
 extern "C" int rswa_attn_bwd_static(const rswa_attn_params* p, void* stream) {
   using namespace rswa;
   RSWA_REQUIRE(p != nullptr, RSWA_ERR_INVALID, "attn_bwd_static: null params");
-  const uint64_t need = bwd_layout(p, false).total_bytes;
+  const uint64_t need = bwd_layout(p, false, RSWA_BWD_STATIC_MAX_BYTES).total_bytes;
   RSWA_REQUIRE(need <= RSWA_BWD_STATIC_MAX_BYTES, RSWA_ERR_UNSUPPORTED,
                "attn_bwd_static: rows * heads_q needs %llu bytes of statistics, the built-in "
                "buffer holds %llu (use rswa_attn_bwd with a caller workspace)",
@@ -1809,11 +1900,12 @@ extern "C" int rswa_attn_bwd_static(const rswa_attn_params* p, void* stream) {
   q.workspace_bytes = RSWA_BWD_STATIC_MAX_BYTES;
   {
     AttnArgs probe;
-    int rc = fill_args(&q, true, probe, false);
+    int rc = fill_args(&q, true, probe, false, RSWA_BWD_STATIC_MAX_BYTES);
     if (rc != RSWA_OK) return rc;
   }
   void* ptr = scratch_on_current_device();
   if (!ptr) return RSWA_ERR_LAUNCH;
   q.workspace = ptr;
-  return bwd_entry(&q, stream, RSWA_BWD_PREP | RSWA_BWD_DKDV | RSWA_BWD_DQ, false);
+  return bwd_entry(&q, stream, RSWA_BWD_PREP | RSWA_BWD_DKDV | RSWA_BWD_DQ, false,
+                   RSWA_BWD_STATIC_MAX_BYTES);
 }

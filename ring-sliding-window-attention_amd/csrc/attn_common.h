@@ -35,6 +35,12 @@ struct AttnArgs {
   float* delta;   // fp32 [heads_q, rows_q] packed: -sum_d dO * O         (workspace)
   float* lse2;    // fp32 [heads_q, rows_q] packed: -lse * log2(e); empty rows -inf (workspace)
   int32_t n_count;    // arrival counters in the workspace (sink kernel)
+  // backward of a pack (workspace; null: no table): number of dK/dV key tiles before sequence b, for
+  // b = 0 .. batch, then whether all sequences have the same number; written by the statistics
+  // kernel; a tile has 2^ktile_log2 keys
+  int32_t* ktile;
+  int32_t ktile_log2;
+  int32_t snake;    // dK/dV: see the kernel (dense; of a pack the device decides)
   const int32_t* cu_q;
   const int32_t* cu_k;
   int64_t q_st[3], k_st[3], v_st[3], o_st[3], do_st[3], dq_st[3], dk_st[3], dv_st[3], lse_st[3];
@@ -68,7 +74,6 @@ struct AttnArgs {
   void* dk2;
   void* dv2;
   int32_t seg;
-  int32_t avg_rows, max_rows;  // query rows that see a key: on average, at most (host estimate, as avg_keys)
   int32_t avg_keys;  // keys a query row sees on average (host estimate; block shapes hang on it)
   int32_t far;  // a sequence of some streamed tensor spans 2 GiB or more: FAR kernels
   // dS hand-off (backward): the dK/dV kernel stores its packed 16-bit dS tiles and the dQ
@@ -143,6 +148,34 @@ __device__ __forceinline__ bool locate_packed(const AttnArgs& a, int t, int tile
   s.q_base = 0;
   s.k_base = 0;
   return true;
+}
+
+// The same along k from the exact table a.ktile: tile number t (of a.ktile[batch]) is tile
+// tile_in_seq of sequence s.  The search goes 64 ways at a time: each lane tests one entry, the
+// ballot counts those at or below t.  Every lane takes part; the results are wave-uniform.
+__device__ __forceinline__ void locate_tile(const AttnArgs& a, int t, SeqInfo& s, int& tile_in_seq) {
+  const int lane = (int)__builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, 0u));
+  int lo = 0, n = a.batch;  // the sequence is one of lo .. lo + n - 1, and ktile[lo] <= t
+  int c;
+  for (;;) {
+    const int step = (n + 63) >> 6;
+    const int i = lo + lane * step;
+    c = a.ktile[min(i, lo + n - 1)];
+    const int at = __popcll(__builtin_amdgcn_ballot_w64(lane * step < n && c <= t)) - 1;
+    lo += at * step;
+    if (step == 1) {
+      tile_in_seq = t - __builtin_amdgcn_readlane(c, at);
+      break;
+    }
+    n = min(step, n - at * step);
+  }
+  s.batch_idx = lo;
+  s.q_row0 = a.cu_q[lo];
+  s.k_row0 = a.cu_k[lo];
+  s.len_q = a.cu_q[lo + 1] - a.cu_q[lo];
+  s.len_k = a.cu_k[lo + 1] - a.cu_k[lo];
+  s.q_base = 0;
+  s.k_base = 0;
 }
 
 template <typename T>
@@ -509,15 +542,19 @@ struct BwdLayout {
   uint64_t stats_bytes;    // each of the two statistics arrays
   int n_count;             // arrival counters of the sink kernel
   uint64_t count_off, total_bytes;
+  uint64_t ktile_off;      // key tile table of a pack (0: none)
   int sink_chunks;         // row chunks of the sink kernel per (sequence, kv head); 0: no sink kernel
   uint64_t sink_off;       // its fp32 sums
   // dS hand-off (ds_bytes == 0: not used for this call)
   uint64_t ds_off, ds_bytes;
   int ds_nkb, ds_slots;
 };
-BwdLayout bwd_layout(const rswa_attn_params* p, bool allow_handoff);
+// (`max_bytes`: room there is; the key tile table of a pack, which only saves time, is left out
+// where it would not fit)
+BwdLayout bwd_layout(const rswa_attn_params* p, bool allow_handoff, uint64_t max_bytes = ~0ull);
 
 // Fill an AttnArgs from the public struct; validates what both directions share.
-int fill_args(const rswa_attn_params* p, bool backward, AttnArgs& a, bool allow_handoff = false);
+int fill_args(const rswa_attn_params* p, bool backward, AttnArgs& a, bool allow_handoff = false,
+              uint64_t max_bytes = ~0ull);
 
 }  // namespace rswa

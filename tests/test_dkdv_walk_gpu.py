@@ -42,3 +42,37 @@ def test_blocks_whose_waves_share_the_walk(case, dtype, tol):
     for name, x, ref in (("dq", dq, rq), ("dk", dk, rk), ("dv", dv, rv)):
         err = ((x.float().cpu() - ref).norm() / ref.norm().clamp_min(1e-30)).item()
         assert err <= tol, f"{name}: relative norm {err}"
+
+
+PACKS = [
+    # (lengths, Hq, Hkv, D, window): the key tile table the statistics kernel writes and its search
+    ([256] * 9, 8, 8, 128, 100),                      # whole tiles, all alike (blocks in snake order)
+    ([512] * 6 + [77], 4, 4, 64, 300),                # alike but for the last
+    ([0, 64, 0, 1, 700, 0, 129, 0], 4, 1, 128, 50),   # empty sequences everywhere
+    ([1 + i % 3 for i in range(300)], 2, 1, 64, 8),   # more than 256 sequences: two passes of the scan
+    ([40] * 64 + [41], 2, 2, 128, 64),                # 65 sequences: two levels of the search
+]
+
+
+@pytest.mark.parametrize("case", PACKS, ids=lambda c: f"{len(c[0])}seq-{c[1]}x{c[2]}x{c[3]}-w{c[4]}")
+def test_packs_by_their_key_tile_table(case):
+    from ring_swa.ops import attn_bwd, attn_fwd
+
+    lens, hq, hk, d, w = case
+    cu = [0]
+    for n in lens:
+        cu.append(cu[-1] + n)
+    t = cu[-1]
+    g = torch.Generator().manual_seed(8)
+    q, do = (torch.randn(t, hq, d, generator=g).bfloat16() for _ in range(2))
+    k, v = (torch.randn(t, hk, d, generator=g).bfloat16() for _ in range(2))
+    _, _, rq, rk, rv = O.attention_fwd_bwd(
+        lambda q, k, v: O.window_attention_varlen(q, k, v, cu, cu, None, (w, 0), True), q, k, v, do)
+    q, k, v, do = (x.cuda() for x in (q, k, v, do))
+    cu = torch.tensor(cu, dtype=torch.int32, device="cuda")
+    out, lse = attn_fwd(q, k, v, None, (w, 0), True, cu, cu)
+    dq, dk, dv = (torch.full_like(x, float("nan")) for x in (q, k, v))
+    attn_bwd(q, k, v, out, lse, do, dq, dk, dv, None, (w, 0), True, cu, cu)
+    for name, x, ref in (("dq", dq, rq), ("dk", dk, rk), ("dv", dv, rv)):
+        err = ((x.float().cpu() - ref).norm() / ref.norm().clamp_min(1e-30)).item()
+        assert err <= 1e-2, f"{name}: relative norm {err}"
