@@ -1681,8 +1681,8 @@ RSWA_INSTANTIATE(_Float16, 64)
 // window 1000, 2 x 8192 rows 545 / 700; full attention over 4096 rows, 32 / 8 heads, 615 / 238.  Of the
 // 78 dense shapes timed the rule is 1 % behind the better form on average.
 // A pack is judged on its average length L, the only one the host knows, as if of sequences of
-// 1.5 L (what a token sees when lengths vary), none longer than 3 L, with half a key tile per
-// sequence wasted.  Packs of 16384 tokens, 32 / 8 heads, window 1024, lengths log-uniform: 16-64
+// 1.5 L (what a token sees when lengths vary), the longest as long as the pack or the window, with
+// half a key tile per sequence wasted.  Packs of 16384 tokens, 32 / 8 heads, window 1024, lengths log-uniform: 16-64
 // 262 / 173, 64-256 193 / 175, 16-1024 260 / 216; all of 512 198 / 204, 32 / 32 heads 16-1024 348 / 475.
 // The 0.9 leans to the wide form where lengths are alike (65536 tokens of 512: 715 / 784).
 bool dkv_walk4(const AttnArgs& a, int head_dim) {
@@ -1703,7 +1703,7 @@ bool dkv_walk4(const AttnArgs& a, int head_dim) {
     max_rows = std::max(max_rows, r);
   }
   if (pack) {
-    max_rows = (double)std::min(a.rows_q, 3 * lq1);
+    max_rows = (double)a.rows_q;
     if (a.wl >= 0 && a.wr >= 0) max_rows = std::min(max_rows, (double)a.wl + a.wr + 1);
   }
   auto estimate = [&](int keys, int walkers, double step, double fixed) {
@@ -1711,7 +1711,7 @@ bool dkv_walk4(const AttnArgs& a, int head_dim) {
       const double r = std::min<double>((double)len, rows + (double)std::min<int64_t>(keys, lk1) - 1);
       return std::max(a.group * r / (32. * walkers), std::ceil((double)a.group / walkers));
     };
-    const double avg = walk(avg_rows, lq), most = walk(max_rows, pack ? 3 * lq1 : lq);
+    const double avg = walk(avg_rows, lq), most = walk(max_rows, pack ? a.rows_q : lq);
     const double tiles = pack ? (double)lk1 / keys + 0.5 : (double)ceil_div(lk1, keys);
     double rounds = tiles * a.heads_kv * a.batch / kComputeUnits;
     // (blocks of equal length run in whole rounds; those of a ramp fill each other's gaps)

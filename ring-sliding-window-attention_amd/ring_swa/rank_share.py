@@ -102,14 +102,23 @@ class RankShareFunc(torch.autograd.Function):
         plan = plan_nonvarlen(s, window_size, cp_size, rank)
         for (i, _, _, _, _) in plan:
             assert i == 0 or i <= len(prev_kv), f"step {i} needs the chunk of rank {rank - i}"
-        out, lse = _forward_blocks(q, k, v, prev_kv, plan, softmax_scale, None, ring_dtypes,
-                                   one_pass)
-        ctx.save_for_backward(q, k, v, out, lse, *prev_kv)
+        out, lse, joined = _forward_blocks(q, k, v, prev_kv, plan, softmax_scale, None, ring_dtypes,
+                                           one_pass)
         ctx.plan, ctx.scale, ctx.ring_dtypes, ctx.one_pass = plan, softmax_scale, ring_dtypes, one_pass
+        ctx.joined = joined is not None
+        if ctx.joined:
+            ctx.save_for_backward(q, out, lse, joined.kv)
+            ctx.prev_shapes = [p.shape for p in prev_kv]
+        else:
+            ctx.save_for_backward(q, k, v, out, lse, *prev_kv)
         return out
 
     @staticmethod
     def backward(ctx, do):
+        if ctx.joined:
+            q, out, lse, kv = ctx.saved_tensors
+            grads = _backward_joined(q, kv, out, lse, do, ctx.plan, ctx.scale, ctx.prev_shapes)
+            return (grads[0], grads[1], grads[2], None, None, None, None, None, None, *grads[3:])
         q, k, v, out, lse, *prev_kv = ctx.saved_tensors
         grads = _backward_blocks(q, k, v, prev_kv, out, lse, do, ctx.plan, ctx.scale, None,
                                  ctx.ring_dtypes, ctx.one_pass)
@@ -142,17 +151,35 @@ class RankShareVarlenFunc(torch.autograd.Function):
         if softmax_scale is None:
             softmax_scale = d ** (-0.5)
         local_cu, plan = plan_varlen(cu_host, s, window_size, cp_size, rank)
-        cu_dev = _device_cu(local_cu, q.device)
         q4, k4, v4 = q.unsqueeze(0), k.unsqueeze(0), v.unsqueeze(0)
         prev4 = [p.unsqueeze(1) for p in prev_kv]
-        out, lse = _forward_blocks(q4, k4, v4, prev4, plan, softmax_scale, cu_dev, ring_dtypes)
+        ctx.plan, ctx.scale, ctx.ring_dtypes = plan, softmax_scale, ring_dtypes
+        ctx.joined = len(plan) > 1 and not ring_dtypes
+        if ctx.joined:
+            # keys of the pack's first sequence that lie before the chunk
+            start = rank * s
+            before = start - max(c for c in cu_host if c <= start)
+            joined = _join_keys(k4, v4, prev4, plan, window_size, local_cu, before)
+            out, lse = attn_fwd(q, joined.kv[0, 0], joined.kv[1, 0], softmax_scale, plan[0][3], True,
+                                joined.cu_q, joined.cu_k)
+            ctx.save_for_backward(q, out, lse, joined.kv, joined.cu_q, joined.cu_k)
+            ctx.prev_shapes = [p.shape for p in prev4]
+            return out
+        cu_dev = _device_cu(local_cu, q.device)
+        out, lse, _ = _forward_blocks(q4, k4, v4, prev4, plan, softmax_scale, cu_dev, ring_dtypes)
         out, lse = out.squeeze(0), lse.squeeze(0)
         ctx.save_for_backward(q, k, v, out, lse, cu_dev, *prev_kv)
-        ctx.plan, ctx.scale, ctx.ring_dtypes = plan, softmax_scale, ring_dtypes
         return out
 
     @staticmethod
     def backward(ctx, do):
+        if ctx.joined:
+            q, out, lse, kv, cu_q, cu_k = ctx.saved_tensors
+            grads = _backward_joined(q.unsqueeze(0), kv, out.unsqueeze(0), lse.unsqueeze(0),
+                                     do.unsqueeze(0), ctx.plan, ctx.scale, ctx.prev_shapes, cu_q, cu_k)
+            dprev = [g.squeeze(1) for g in grads[3:]]
+            return (grads[0].squeeze(0), grads[1].squeeze(0), grads[2].squeeze(0), None, None, None,
+                    None, None, None, *dprev)
         q, k, v, out, lse, cu_dev, *prev_kv = ctx.saved_tensors
         prev4 = [p.unsqueeze(1) for p in prev_kv]
         grads = _backward_blocks(q.unsqueeze(0), k.unsqueeze(0), v.unsqueeze(0), prev4,
@@ -200,7 +227,7 @@ def blocks_forward(q, kv, kv_of, plan, scale, local_cu, kernels=None, before_res
     device ``cu_seqlens`` of the own-chunk block of a packed chunk (batch 1).  ``before_rest`` is
     called between the own-chunk block and the others (a ring waits for its receives there).
     This one function is what ``ring_rank_share_attn(ring_dtypes=True)``, plans of three and
-    more blocks and the ring over a ``cp_group`` (``ring_swa/ring.py``) all run; on the HIP library
+    more blocks with ``one_pass=False`` and the ring over a ``cp_group`` (``ring_swa/ring.py``) all run; on the HIP library
     the operators work in the kernels' epilogues: the own-chunk block writes the accumulators
     (they are never filled with the merge identity), the others merge into them, no temporary,
     no merge launch."""
@@ -298,8 +325,67 @@ def _one_pass(q, k, v, prev_kv, plan, local_cu):
     return w, kk, vv, tail
 
 
+class _Joined:
+    """The rank's visible keys as one row range: the rows of earlier ranks' chunks that the window
+    reaches, then its own chunk, copied into one buffer, so that every block of the plan is part of
+    one causal band over them.  ``kv``: ``[2, batch, reach + seq, kv_heads, dim]``, ``reach`` rows of it from
+    the ``hops`` chunks before the own one; ``cu_q`` / ``cu_k``: packed chunks.
+
+    Against the blocks one after the other, with merges and fp32 accumulators in between: 2.90 -> 2.45
+    ms for a step on 4096-token chunks, window 10000, 32 / 8 heads (the copies are 35 us of it); against
+    two blocks on two streams, a packed 8192-token chunk, window 2048: 845 -> 834 us."""
+
+    def __init__(self, k, v, prev_kv, hops, reach, cu_q=None, cu_k=None):
+        b, s, hk, d = k.shape
+        self.kv = kv = torch.empty((2, b, reach + s, hk, d), dtype=k.dtype, device=k.device)
+        self.hops, self.cu_q, self.cu_k = hops, cu_q, cu_k
+        for i in range(1, hops + 1):
+            end = reach - (i - 1) * s
+            n = min(end, s)
+            kv[:, :, end - n:end].copy_(prev_kv[i - 1][:, :, s - n:])
+        kv[0, :, reach:].copy_(k)
+        kv[1, :, reach:].copy_(v)
+
+
+def _join_keys(k, v, prev_kv, plan, window, local_cu=None, first_kv_len=0):
+    """``_Joined`` for a plan of two and more blocks.  Of a packed chunk only the first sequence
+    has keys before it, ``first_kv_len`` of them."""
+    hops = plan[-1][0]
+    reach = min(window, hops * k.shape[1])
+    if local_cu is None:
+        return _Joined(k, v, prev_kv, hops, reach)
+    reach = min(reach, first_kv_len)
+    cu_q = _device_cu(local_cu, k.device)
+    cu_k = _device_cu([0] + [reach + c for c in local_cu[1:]], k.device)
+    return _Joined(k, v, prev_kv, hops, reach, cu_q, cu_k)
+
+
+def _backward_joined(q, kv, out, lse, do, plan, scale, prev_shapes, cu_q=None, cu_k=None):
+    """Backward on joined keys.  The gradients of all reached chunks are views of one buffer of
+    whole chunks, zero in the rows that no query sees; chunks beyond get zeros of their own."""
+    if do.stride(-1) != 1:
+        do = do.contiguous()
+    (_, _, _, window, _), hops, s = plan[0], plan[-1][0], q.shape[1]
+    dq = torch.empty_like(q)
+    whole = torch.empty((2, kv.shape[1], (hops + 1) * s) + tuple(kv.shape[3:]), dtype=kv.dtype,
+                        device=kv.device)
+    unseen = whole.shape[2] - kv.shape[2]
+    if unseen:
+        whole[:, :, :unseen].zero_()
+    dk, dv = whole[0, :, unseen:], whole[1, :, unseen:]
+    if cu_q is None:
+        attn_bwd(q, kv[0], kv[1], out, lse, do, dq, dk, dv, scale, window, True)
+    else:
+        attn_bwd(q[0], kv[0, 0], kv[1, 0], out[0], lse[0], do[0], dq[0], dk[0], dv[0], scale, window,
+                 True, cu_q, cu_k)
+    dprev = [whole[:, :, (hops - 1 - i) * s:(hops - i) * s] if i < hops else
+             torch.zeros(shape, dtype=kv.dtype, device=kv.device) for i, shape in enumerate(prev_shapes)]
+    return (dq, whole[0, :, hops * s:], whole[1, :, hops * s:], *dprev)
+
+
 def _forward_blocks(q, k, v, prev_kv, plan, scale, local_cu, ring_dtypes, one_pass=True):
-    """Run the planned blocks and merge them.  Dense 4-d tensors (batch 1 when packed)."""
+    """Run the planned blocks and merge them.  Dense 4-d tensors (batch 1 when packed).  Returns
+    ``(out, lse, joined)``, ``joined`` being the ``_Joined`` keys when that route was taken."""
     assert plan and plan[0][0] == 0, "the diagonal block comes first: it covers every row"
     one = _one_pass(q, k, v, prev_kv, plan, local_cu) if one_pass and not ring_dtypes else None
     if one is not None:
@@ -309,12 +395,15 @@ def _forward_blocks(q, k, v, prev_kv, plan, scale, local_cu, ring_dtypes, one_pa
         # a partial output in between (2.10 -> 2.02 ms per step at 8192-token chunks, window
         # 4096; two launches and a merge remain for every other shape and for ring_dtypes).
         w, kk, vv, _ = one
-        return attn_fwd(q, kk, vv, scale, (w, 0), True, second=(k, v))
+        return (*attn_fwd(q, kk, vv, scale, (w, 0), True, second=(k, v)), None)
+    if one_pass and not ring_dtypes and len(plan) > 1:
+        joined = _join_keys(k, v, prev_kv, plan, plan[0][3][0])
+        return (*attn_fwd(q, joined.kv[0], joined.kv[1], scale, plan[0][3], True), joined)
     if ring_dtypes or len(plan) > 2:
         # With two blocks the 16-bit running output is merged once and rounded once, the same
         # bits as the fp32 accumulator gives; from three blocks on every further merge would
         # add a rounding the reference does not have, so its accumulators are used.
-        return _forward_blocks_accum(q, k, v, prev_kv, plan, scale, local_cu)
+        return (*_forward_blocks_accum(q, k, v, prev_kv, plan, scale, local_cu), None)
     # Own-chunk block first, then the previous-chunk block merged into its rows in the
     # forward kernel's epilogue (same bits as a separate merge).  One stream: two forward
     # launches side by side take longer than one after the other on this hardware (552 against
@@ -329,7 +418,7 @@ def _forward_blocks(q, k, v, prev_kv, plan, scale, local_cu, ring_dtypes, one_pa
         kk, vv = prev_kv[i - 1][0], prev_kv[i - 1][1]
         attn_fwd(q[:, qs], kk[:, ks], vv[:, ks], scale, window, causal,
                  accumulate_into=(out[:, qs], lse[:, :, qs]))
-    return out, lse
+    return out, lse, None
 
 
 def _backward_blocks(q, k, v, prev_kv, out, lse, do, plan, scale, local_cu, ring_dtypes=False,
@@ -484,8 +573,9 @@ def ring_rank_share_attn(
     entry (the gradient a real ring would send back).  ``ring_dtypes=True`` keeps the
     running output in fp32 and the running LSE in fp64 as upstream does.  ``one_pass=False``
     keeps upstream's block structure -- own-chunk block, previous-chunk block, LSE merge
-    (``ring_swa/sliding_window/nonvarlen.py:95-154``) -- where the default computes the two as
-    one band over both key ranges (window shorter than a chunk)."""
+    (``ring_swa/sliding_window/nonvarlen.py:95-154``) -- where the default computes the blocks as
+    one band: over both key ranges where they lie (window shorter than a chunk), or over one
+    buffer that the reached chunks are copied into."""
     assert q.shape[1] == k.shape[1] == v.shape[1], "Sequence length must be the same"
     return RankShareFunc.apply(q, k, v, int(window_size), int(cp_size), int(cp_local_rank),
                                softmax_scale, bool(ring_dtypes), bool(one_pass), *prev_kv)

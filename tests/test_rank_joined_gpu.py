@@ -1,0 +1,66 @@
+"""A rank step whose window reaches over several earlier chunks, or over one whose size the two-range
+pass does not take, runs as one band over the joined keys.  All ranks' shares against the oracle on
+the whole sequence (out <= 2e-2 max-abs, gradients <= 1e-2 relative norm), odd chunk sizes, windows at
+and around multiples of a chunk, batch 2, a pack whose sequences start anywhere, and held chunks
+beyond the window's reach, whose gradient is zero."""
+import pytest
+import torch
+
+from oracle import attention_oracle as O
+
+pytestmark = pytest.mark.gpu
+CP = 4
+
+
+def _rel(x, ref):
+    return ((x - ref).norm() / ref.norm().clamp_min(1e-30)).item()
+
+
+@pytest.mark.parametrize("s,w", [(100, 30), (100, 100), (100, 101), (193, 400), (64, 1000), (256, 511)])
+@pytest.mark.parametrize("packed", [False, True], ids=["dense", "packed"])
+def test_shares_on_joined_keys_match_the_oracle(s, w, packed):
+    import ring_swa
+
+    hq, hk, d, total = 4, 2, 64, s * CP
+    b = 1 if packed else 2
+    cu = [0, s // 2, s // 2 + 1, 2 * s + 7, total]
+    g = torch.Generator().manual_seed(31)
+    q, do = (torch.randn(b, total, hq, d, generator=g).bfloat16() for _ in range(2))
+    k, v = (torch.randn(b, total, hk, d, generator=g).bfloat16() for _ in range(2))
+    if packed:
+        ro, _, rq, rk, rv = O.attention_fwd_bwd(
+            lambda q, k, v: O.window_attention_varlen(q, k, v, cu, cu, None, (w, 0), True),
+            q[0], k[0], v[0], do[0])
+        ro, rq, rk, rv = (t[None] for t in (ro, rq, rk, rv))
+    else:
+        ro, _, rq, rk, rv = O.attention_fwd_bwd(lambda q, k, v: O.sliding_window_attn(q, k, v, w), q, k, v, do)
+    outs, dqs = [], []
+    dk, dv = torch.zeros(b, total, hk, d), torch.zeros(b, total, hk, d)
+    for r in range(CP):
+        sl = slice(r * s, (r + 1) * s)
+        own = [t[:, sl].cuda() for t in (q, k, v)]
+        prev = [torch.stack([t[:, (r - i) * s:(r - i + 1) * s] for t in (k, v)]).cuda() for i in range(1, r + 1)]
+        if packed:
+            own, prev = [t[0] for t in own], [t[:, 0] for t in prev]
+        own, prev = [t.requires_grad_() for t in own], [t.requires_grad_() for t in prev]
+        if packed:
+            out = ring_swa.ring_rank_share_attn_varlen(*own, prev, w, cu, CP, r)
+        else:
+            out = ring_swa.ring_rank_share_attn(*own, prev, w, CP, r)
+        grads = torch.autograd.grad(out, own + prev, do[:, sl].cuda() if not packed else do[0, sl].cuda())
+        cpu = [x.float().cpu() for x in (out.detach(), *grads)]
+        if packed:
+            cpu = [x[None] for x in cpu[:4]] + [x[:, None] for x in cpu[4:]]
+        outs.append(cpu[0])
+        dqs.append(cpu[1])
+        dk[:, sl] += cpu[2]
+        dv[:, sl] += cpu[3]
+        for i, p in enumerate(cpu[4:], 1):
+            ps = slice((r - i) * s, (r - i + 1) * s)
+            dk[:, ps] += p[0]
+            dv[:, ps] += p[1]
+            if (i - 1) * s >= w:
+                assert not p.any()
+    assert (torch.cat(outs, 1) - ro).abs().max().item() <= 2e-2
+    errs = [_rel(torch.cat(dqs, 1), rq), _rel(dk, rk), _rel(dv, rv)]
+    assert max(errs) <= 1e-2, f"dq / dk / dv relative norm {errs}"
