@@ -4,8 +4,8 @@
 // Replaces flash-attn's forward as wrapped at ring_swa/ops/wrap_flash.py:168-273.
 //
 // One block = 4 waves x 32 query rows sharing every K/V tile it loads: either 64 rows of
-// TWO q heads of one GQA group (group size even) or 128 rows of one q head; two blocks fit a
-// compute unit (two waves per SIMD, from independent blocks).  Per 64-key
+// TWO q heads of one GQA group (group size even) or 128 rows of one q head; two blocks (three at
+// head_dim 64) fit a compute unit (waves of a SIMD are from independent blocks).  Per 64-key
 // tile a wave computes S^T = K Q^T (keys x queries) with v_mfma_f32_32x32x16, so each
 // lane owns ONE query column: the row max / sum of the online softmax are in-lane
 // reductions plus a single half-wave exchange, and P^T is already laid out as the B
@@ -38,11 +38,16 @@ struct FwdCfg {
   static constexpr int ROWB = D * 2;  // bytes per row
   static constexpr int TILE = BN * ROWB;
   static constexpr int O_STRIDE = D * 2 + 16;
+  // Blocks per compute unit (a block has one wave per SIMD).  head_dim 128 needs 214 registers, so
+  // two.  head_dim 64 has half the MFMAs per score and is bound by the softmax's vector work and
+  // its latencies; it fits three (148 registers; four would spill): 8000 rows in four sequences,
+  // 28 / 4 heads, window 1000, fp16: 83.6 -> 79.0 us.
+  static constexpr int WAVES_PER_SIMD = D == 64 ? 3 : 2;
   static_assert(TILE >= 32 * O_STRIDE, "one wave's epilogue staging fits one tile buffer");
 };
 
 template <typename T, int D, bool SKIP, bool FAR>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2)))
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(FwdCfg<D>::WAVES_PER_SIMD, FwdCfg<D>::WAVES_PER_SIMD)))
 void attn_fwd_kernel(const AttnArgs a) {
   using C = FwdCfg<D>;
   constexpr int NW = C::THREADS / 64;
