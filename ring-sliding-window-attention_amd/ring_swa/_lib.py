@@ -163,7 +163,18 @@ def dtype_code(t: torch.Tensor) -> int:
 
 
 def stream_ptr(device) -> int:
-    return torch.cuda.current_stream(device).cuda_stream
+    # (the handle alone: building a torch.cuda.Stream around it takes longer than a launch)
+    return torch._C._cuda_getCurrentRawStream(device.index)
+
+
+def launch(device, entry, *args) -> None:
+    """``entry(*args[:1], current stream, *args[1:])`` with ``device`` (with an index) current.
+    Nearly always it is already: entering the guard then costs as much as the call itself."""
+    if torch.cuda.current_device() == device.index:
+        check(entry(args[0], stream_ptr(device), *args[1:]))
+    else:
+        with torch.cuda.device(device):
+            check(entry(args[0], stream_ptr(device), *args[1:]))
 
 
 def require_device(*tensors: torch.Tensor) -> torch.device:
@@ -173,8 +184,9 @@ def require_device(*tensors: torch.Tensor) -> torch.device:
             "ring_swa kernels run on a ROCm GPU only (got a tensor on "
             f"'{dev}'); there is no CPU path"
         )
+    index = dev.index
     for t in tensors:
-        if t.device != dev:
+        if t.get_device() != index or not t.is_cuda:
             raise RuntimeError("all tensors must live on the same device")
     return dev
 

@@ -30,31 +30,26 @@ from .. import _lib
 
 def _check_qkv(q, k, v, packed: bool):
     nd = 3 if packed else 4
-    assert q.dim() == nd and k.dim() == nd and v.dim() == nd, (
+    qs, ks = q.shape, k.shape
+    assert len(qs) == nd and len(ks) == nd and v.dim() == nd, (
         f"expected {nd}-d q/k/v, got {q.dim()}, {k.dim()}, {v.dim()}"
     )
-    assert k.shape == v.shape, "k and v must have the same shape"
-    assert q.shape[-1] == k.shape[-1], "head_dim mismatch"
+    assert ks == v.shape, "k and v must have the same shape"
+    assert qs[-1] == ks[-1], "head_dim mismatch"
     assert q.dtype == k.dtype == v.dtype, "q, k, v must share a dtype"
-    assert q.shape[-2] % k.shape[-2] == 0, (
+    assert qs[-2] % ks[-2] == 0, (
         "Number of query heads must be divisible by number of key/value heads"
     )
     if not packed:
-        assert q.shape[0] == k.shape[0], "batch mismatch"
+        assert qs[0] == ks[0], "batch mismatch"
     for t in (q, k, v):
         assert t.stride(-1) == 1, "last dimension must be contiguous"
 
 
 def _strides3(t: torch.Tensor, packed: bool):
-    if packed:
-        return (0, t.stride(0), t.stride(1))
-    return (t.stride(0), t.stride(1), t.stride(2))
-
-
-def _lse_strides(lse: torch.Tensor, packed: bool):
-    if packed:
-        return (0, lse.stride(0), lse.stride(1))
-    return (lse.stride(0), lse.stride(1), lse.stride(2))
+    """Strides of batch, row and head (of an LSE: batch, head and row) as the ABI takes them."""
+    st = t.stride()
+    return (0, st[0], st[1]) if packed else st[:3]
 
 
 def _same_strides(a, b) -> bool:
@@ -83,11 +78,12 @@ def _second_range(p, k, v, second, packed):
 def _params(q, k, v, softmax_scale, window_size, causal, cu_q, cu_k, num_sink,
             mask_shift=None, second=None) -> "_lib.AttnParams":
     packed = cu_q is not None
-    p = _lib.AttnParams()
+    p = _lib.AttnParams()  # (zero-initialised)
     p.dtype = _lib.dtype_code(q)
-    p.head_dim = q.shape[-1]
-    p.heads_q = q.shape[-2]
-    p.heads_kv = k.shape[-2]
+    qs, ks = q.shape, k.shape
+    p.head_dim = qs[-1]
+    p.heads_q = qs[-2]
+    p.heads_kv = ks[-2]
     if packed:
         assert cu_k is not None, "cu_seqlens_k is required with cu_seqlens_q"
         for cu in (cu_q, cu_k):
@@ -97,28 +93,28 @@ def _params(q, k, v, softmax_scale, window_size, causal, cu_q, cu_k, num_sink,
             assert cu.device == q.device, "cu_seqlens must live on the tensors' device"
         assert cu_q.numel() == cu_k.numel() and cu_q.numel() >= 2
         p.batch = cu_q.numel() - 1
-        p.total_q, p.total_k = q.shape[0], k.shape[0]
         # only upper bounds are needed, so no device->host read of the lengths
-        p.seqlen_q, p.seqlen_k = q.shape[0], k.shape[0]
+        p.total_q, p.total_k = p.seqlen_q, p.seqlen_k = qs[0], ks[0]
         p.cu_seqlens_q, p.cu_seqlens_k = cu_q.data_ptr(), cu_k.data_ptr()
     else:
-        p.batch = q.shape[0]
-        p.seqlen_q, p.seqlen_k = q.shape[1], k.shape[1]
-        p.total_q = p.total_k = 0
-        p.cu_seqlens_q = p.cu_seqlens_k = None
+        p.batch = qs[0]
+        p.seqlen_q, p.seqlen_k = qs[1], ks[1]
     p.softmax_scale = float(softmax_scale)
     p.window_left, p.window_right = int(window_size[0]), int(window_size[1])
-    p.causal = 1 if causal else 0
+    if causal:
+        p.causal = 1
     p.num_sink = int(num_sink)
-    p.shift_explicit = 0 if mask_shift is None else 1
-    p.shift = 0 if mask_shift is None else int(mask_shift)
+    if mask_shift is not None:
+        p.shift_explicit = 1
+        p.shift = int(mask_shift)
     p.q, p.k, p.v = q.data_ptr(), k.data_ptr(), v.data_ptr()
-    p.q_stride = _lib.i64x3(_strides3(q, packed))
-    p.k_stride = _lib.i64x3(_strides3(k, packed))
-    p.v_stride = _lib.i64x3(_strides3(v, packed))
+    p.q_stride = _strides3(q, packed)
+    p.k_stride = _strides3(k, packed)
+    p.v_stride = _strides3(v, packed)
     # RSWA_ADDRESSING=far: the kernels that base every tile fetch at the tile's own first row
     # (picked by the library itself once a sequence spans 2 GiB) whatever the sizes
-    p.addressing = 1 if os.environ.get("RSWA_ADDRESSING", "") == "far" else 0
+    if os.environ.get("RSWA_ADDRESSING", "") == "far":
+        p.addressing = 1
     if second is not None:
         _second_range(p, k, v, second, packed)
     return p
@@ -162,7 +158,8 @@ def attn_fwd(
     dev = _lib.require_device(q, k, v)
     if softmax_scale is None:
         softmax_scale = q.shape[-1] ** (-0.5)
-    lse_shape = (q.shape[1], q.shape[0]) if packed else (q.shape[0], q.shape[2], q.shape[1])
+    qs = q.shape
+    lse_shape = (qs[1], qs[0]) if packed else (qs[0], qs[2], qs[1])
     wide = False
     assert accumulate_into is None or into is None
     if accumulate_into is not None or into is not None:
@@ -182,8 +179,8 @@ def attn_fwd(
             lse.fill_(float("-inf"))
             return out, lse
     else:
-        out = torch.empty(q.shape, dtype=q.dtype, device=dev)
-        lse = torch.empty(lse_shape, dtype=torch.float32, device=dev)
+        out = q.new_empty(q.shape)
+        lse = q.new_empty(lse_shape, dtype=torch.float32)
         if q.numel() == 0:
             return out, lse
         if k.numel() == 0:
@@ -194,13 +191,12 @@ def attn_fwd(
     p = _params(q, k, v, softmax_scale, window_size, causal, cu_seqlens_q, cu_seqlens_k, num_sink,
                 mask_shift, second)
     p.out = out.data_ptr()
-    p.out_stride = _lib.i64x3(_strides3(out, packed))
+    p.out_stride = _strides3(out, packed)
     p.lse = lse.data_ptr()
-    p.lse_stride = _lib.i64x3(_lse_strides(lse, packed))
+    p.lse_stride = _strides3(lse, packed)
     p.out_accumulate = 0 if accumulate_into is None else 1
     p.wide = _lib.WIDE_OUT if wide else 0
-    with torch.cuda.device(dev):
-        _lib.check(_lib.lib().rswa_attn_fwd(p, _lib.stream_ptr(dev)))
+    _lib.launch(dev, _lib.lib().rswa_attn_fwd, p)
     return out, lse
 
 
@@ -254,10 +250,11 @@ def attn_bwd(
     _check_qkv(q, k, v, packed)
     assert second is None or k.numel() > 0, "two key ranges: the first must not be empty"
     dev = _lib.require_device(q, k, v, o, softmax_lse, do, dq, dk, dv)
-    assert o.shape == q.shape and do.shape == q.shape and dq.shape == q.shape
-    assert dk.shape == k.shape and dv.shape == v.shape
-    assert o.dtype == q.dtype and do.dtype == q.dtype
-    assert dq.dtype in (q.dtype, torch.float32) and dk.dtype in (q.dtype, torch.float32) and \
+    qs, ks, dtype = q.shape, k.shape, q.dtype
+    assert o.shape == qs and do.shape == qs and dq.shape == qs
+    assert dk.shape == ks and dv.shape == ks
+    assert o.dtype == dtype and do.dtype == dtype
+    assert dq.dtype in (dtype, torch.float32) and dk.dtype in (dtype, torch.float32) and \
         dv.dtype == dk.dtype, "dq and dk / dv must have the dtype of q, or be fp32 accumulators"
     wide_dq, wide_dkv = dq.dtype == torch.float32, dk.dtype == torch.float32
     assert not dkv_accumulate or wide_dkv, "dkv_accumulate needs fp32 dk / dv"
@@ -265,9 +262,9 @@ def attn_bwd(
     for t in (o, do, dq, dk, dv):
         assert t.stride(-1) == 1, "last dimension must be contiguous"
     if packed:
-        assert softmax_lse.shape == (q.shape[1], q.shape[0])
+        assert softmax_lse.shape == (qs[1], qs[0])
     else:
-        assert softmax_lse.shape == (q.shape[0], q.shape[2], q.shape[1])
+        assert softmax_lse.shape == (qs[0], qs[2], qs[1])
     if softmax_scale is None:
         softmax_scale = q.shape[-1] ** (-0.5)
     if q.numel() == 0 or k.numel() == 0:
@@ -293,20 +290,19 @@ def attn_bwd(
     p.dkv_accumulate = int(bool(dkv_accumulate))
     p.wide = (_lib.WIDE_DQ if wide_dq else 0) | (_lib.WIDE_DKV if wide_dkv else 0)
     p.out = o.data_ptr()
-    p.out_stride = _lib.i64x3(_strides3(o, packed))
+    p.out_stride = _strides3(o, packed)
     p.lse = softmax_lse.data_ptr()
-    p.lse_stride = _lib.i64x3(_lse_strides(softmax_lse, packed))
+    p.lse_stride = _strides3(softmax_lse, packed)
     p.dout = do.data_ptr()
-    p.dout_stride = _lib.i64x3(_strides3(do, packed))
+    p.dout_stride = _strides3(do, packed)
     p.dq, p.dk, p.dv = dq.data_ptr(), dk.data_ptr(), dv.data_ptr()
-    p.dq_stride = _lib.i64x3(_strides3(dq, packed))
-    p.dk_stride = _lib.i64x3(_strides3(dk, packed))
-    p.dv_stride = _lib.i64x3(_strides3(dv, packed))
+    p.dq_stride = _strides3(dq, packed)
+    p.dk_stride = _strides3(dk, packed)
+    p.dv_stride = _strides3(dv, packed)
     L = _lib.lib()
     if static_workspace:
         assert phases == 7 and workspace is None, "the built-in buffer serves whole backward calls"
-        with torch.cuda.device(dev):
-            _lib.check(L.rswa_attn_bwd_static(p, _lib.stream_ptr(dev)))
+        _lib.launch(dev, L.rswa_attn_bwd_static, p)
         return
     _set_handoff(p, handoff)
     need = int(L.rswa_attn_bwd_workspace_bytes(p))
@@ -315,7 +311,7 @@ def attn_bwd(
         p.ds_handoff = 0
         need = int(L.rswa_attn_bwd_workspace_bytes(p))
     if workspace is None:
-        workspace = torch.empty(need, dtype=torch.uint8, device=dev)  # 512-B aligned by torch
+        workspace = q.new_empty(need, dtype=torch.uint8)  # 512-B aligned by torch
     assert workspace.dtype == torch.uint8 and workspace.device == dev
     assert workspace.numel() >= need, (
         f"workspace of {workspace.numel()} bytes, {need} needed: size it with bwd_workspace_bytes "
@@ -323,8 +319,7 @@ def attn_bwd(
     )
     p.workspace = workspace.data_ptr()
     p.workspace_bytes = workspace.numel()
-    with torch.cuda.device(dev):
-        _lib.check(L.rswa_attn_bwd_phases(p, _lib.stream_ptr(dev), int(phases)))
+    _lib.launch(dev, L.rswa_attn_bwd_phases, p, int(phases))
 
 
 def bwd_static_init(device=None) -> None:
@@ -350,16 +345,13 @@ def _set_handoff(p, handoff: Optional[bool]) -> bool:
     """Decide ``p.ds_handoff`` (see ``attn_bwd``); returns whether the library will take it."""
     L = _lib.lib()
     p.ds_handoff = 0
-    if handoff is False:
+    if handoff is False or (handoff is None and handoff_max_bytes() == 0):
         return False
     p.ds_handoff = 2 if handoff == "force" else 1
     if not L.rswa_attn_bwd_handoff_active(p):
         p.ds_handoff = 0
         return False
     if handoff is None:
-        if handoff_max_bytes() == 0:
-            p.ds_handoff = 0
-            return False
         with_ds = int(L.rswa_attn_bwd_workspace_bytes(p))
         p.ds_handoff = 0
         if with_ds - int(L.rswa_attn_bwd_workspace_bytes(p)) > handoff_max_bytes():
