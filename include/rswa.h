@@ -251,7 +251,7 @@ int rswa_attn_fwd(const rswa_attn_params* p, void* stream);
 int rswa_attn_bwd(const rswa_attn_params* p, void* stream);
 
 /*
- * rswa_attn_bwd is three launches: PREP (row statistics into the workspace), DKDV
+ * rswa_attn_bwd has three phases: PREP (row statistics into the workspace), DKDV
  * (dk, dv written; reads the statistics) and DQ (dq written; reads the statistics).
  * This variant enqueues only the phases named in the bit mask, on the same
  * workspace: it lets a profiler or benchmark bracket one kernel alone, and lets a

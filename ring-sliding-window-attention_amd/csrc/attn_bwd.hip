@@ -1,7 +1,9 @@
 // Band / sink attention backward for gfx950, without atomics.
 //
 // Replaces flash-attn's backward as wrapped at ring_swa/ops/wrap_flash.py:276-429.
-// Three launches on the caller's stream:
+// Launches on the caller's stream: DQ (which makes the row statistics, too), then DKDV; for packs
+// and sink keys a one-block kernel ahead of them.  Where the phases are asked for in separate calls,
+// or DQ cannot make the statistics, PREP, then DKDV and DQ:
 //   PREP : per (row, q head): -delta = -sum_d dO * O and -lse2 = -lse * log2(e) (stored negated:
 //          they enter the kernels as addends),
 //          both fp32, into the caller's workspace
@@ -92,9 +94,12 @@ constexpr int kSnakeKeys = 4096;  // longest sequence whose dK/dV blocks take th
 // ============================================================================
 // dK / dV
 // ============================================================================
+// rows of a query tile of the dK/dV kernel, whose statistics it reads together
+constexpr int kStatTileRows = 32;
+
 template <int D>
 struct DkvCfg {
-  static constexpr int BM = 32;        // query rows per step
+  static constexpr int BM = kStatTileRows;  // query rows per step
   static constexpr int KB = 2;         // 32-key blocks per wave
   static constexpr int BN = kDkvKeysPerBlock;  // keys per block: 4 waves x KB x 32
   static_assert(BN == 256, "4 waves x KB x 32 keys");
@@ -981,6 +986,64 @@ struct DqCfg {
   static_assert(TILE >= 32 * O_STRIDE, "one wave's epilogue staging fits one tile buffer");
 };
 
+// The key tile table of a pack, by one block: running sums of the sequences' tile counts, THREADS
+// sequences at a time (a scan in each wave, the waves' totals through LDS).
+template <int THREADS>
+__device__ __forceinline__ void write_ktile(const AttnArgs& a, int* wave_sum) {
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int first_n = (a.cu_k[1] - a.cu_k[0] + (1 << a.ktile_log2) - 1) >> a.ktile_log2;
+  int unlike = 0;  // some sequence has another number of tiles than the first
+  int base = 0;
+  for (int b0 = 0; b0 < a.batch; b0 += THREADS) {
+    const int b = b0 + (int)threadIdx.x;
+    const int len = b < a.batch ? a.cu_k[b + 1] - a.cu_k[b] : 0;
+    const int n = (len + (1 << a.ktile_log2) - 1) >> a.ktile_log2;
+    int sum = n;  // inclusive
+#pragma unroll
+    for (int m = 1; m < 64; m <<= 1) {
+      const int up = __shfl_up(sum, m, 64);
+      if (lane >= m) sum += up;
+    }
+    __syncthreads();  // (wave_sum of the previous pass has been read)
+    if (lane == 63) wave_sum[wave] = sum;
+    __syncthreads();
+    int before = base;
+    for (int w = 0; w < THREADS / 64; w++) {
+      if (w < wave) before += wave_sum[w];
+      base += wave_sum[w];
+    }
+    if (b < a.batch) a.ktile[b] = before + sum - n;
+    // (the last sequence may be a remainder)
+    unlike |= b < a.batch - 1 && n != first_n;
+  }
+  unlike = __syncthreads_or(unlike);
+  if (threadIdx.x == 0) {
+    a.ktile[a.batch] = base;
+    a.ktile[a.batch + 1] = !unlike && first_n << a.ktile_log2 <= kSnakeKeys;
+  }
+}
+
+// What the statistics kernel leaves in the workspace of a pack or a call with sink keys beside the
+// statistics of the rows, by one block: the sink kernel's arrival counters at zero, the neutral
+// value behind a pack's lse2 array, the neutral pair for the rows after a pack's last that the
+// tile kernels read with its last tile, and the key tile table.  (Inside the dQ kernel it would push that kernel's registers into scratch memory.)
+__global__ __launch_bounds__(256) void attn_bwd_rest_kernel(const AttnArgs a) {
+  __shared__ int wave_sum[4];
+  for (int i = threadIdx.x; i < a.n_count; i += 256) a.sink_count[i] = 0;
+  if (a.cu_q) {
+    const int64_t used = a.rows_q * a.heads_q;
+    if (used + threadIdx.x < a.delta - a.lse2) a.lse2[used + threadIdx.x] = -__builtin_inff();
+    const int64_t owned = a.cu_q[a.batch];
+    const int n = (int)min((int64_t)kStatTileRows, a.rows_q - owned);
+    for (int i = threadIdx.x; i < n * a.heads_q; i += 256) {
+      const int64_t at = (int64_t)(i / n) * a.rows_q + owned + i % n;
+      a.lse2[at] = -__builtin_inff();
+      a.delta[at] = -0.f;
+    }
+  }
+  if (a.ktile) write_ktile<256>(a, wave_sum);
+}
+
 // Built on v_mfma_f32_16x16x32 (with random operands the matrix pipes sustain about 14 % more
 // of these than of the 32x32x16 form before the power limit pulls the clock down).  A wave
 // owns 32 query rows as two 16-column blocks: lane l holds query column l % 16 of each block;
@@ -994,11 +1057,18 @@ struct DqCfg {
 // two of them per compute unit -- the same two waves per SIMD, but from independent blocks, so
 // that one block's prologue (three dependent round trips to memory) and epilogue run under the
 // other's tiles; the price is that a K / V tile serves half as many rows.
-template <typename T, int D, bool FAR, int NW>
+//
+// STATS: the kernel also makes the row statistics of the backward, which it has to read dO for
+// anyway, and writes them for the dK/dV kernel, launched after it.  Same bits as the statistics
+// kernel's (same order of sums).  Both kernels are at memory speed there, so what falls away is the
+// second read of dO and a launch; us, statistics + dQ, bf16, head_dim 128: 2 x 8192 rows, 32 / 32 heads,
+// window 1000 461 -> 422; a pack of 16384 tokens in sequences of 16 to 1024, 32 / 8 heads, 217 -> 203.
+template <typename T, int D, bool FAR, int NW, bool STATS>
 __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(2, 2)))
 void attn_bwd_dq_kernel(const AttnArgs a) {
   using C = DqCfg<D>;
   static_assert(NW == 8 || NW == 4, "waves per block");
+  static_assert(!(FAR && STATS), "statistics in the first addressing form only");
   constexpr int HSH = NW == 8 ? 2 : 1;  // waves per q head in pair mode: 1 << HSH
   using M = Mma<T>;
   using V8 = typename M::V8;
@@ -1068,13 +1138,16 @@ void attn_bwd_dq_kernel(const AttnArgs a) {
   const RowBounds wb_first = row_bounds(a, r0, len_q, len_k);
   const RowBounds wb_last = row_bounds(a, min(r0 + 31, len_q - 1), len_q, len_k);
 
-  // Q / dO fragments (B operands) and the statistics of the lane's two query rows.  Q is
-  // multiplied by scale * log2(e) here, once, and the (negated) statistics are the values the
-  // S^T and dP^T accumulator chains start from: the MFMAs then deliver S c - lse2 and
-  // dP - delta, and the vector ALU is left with one exponential, one product and the 16-bit
-  // conversion per score.  Rounding the scaled Q to 16 bits moves a score by about 2^-9 of its
-  // typical magnitude (P by about 0.1 %), a quarter of what rounding P itself to 16 bits does.
+  // Q / dO fragments (B operands) and the (negated) statistics of the lane's two query rows.  The
+  // dP^T accumulator chains start from -delta: the MFMAs then deliver dP - delta, and the vector ALU
+  // is left with a multiply-add, an exponential, a product and the 16-bit conversion per score.
   V8 qf[2][KS], dof[2][KS];
+  if constexpr (STATS) {
+    // the elements behind the lse2 array (see attn_bwd_prep_kernel), where block 0 surely is at
+    // work; for a pack, whose first slot may stand for no tile, attn_bwd_rest_kernel writes them
+    const int64_t used = a.rows_q * a.heads_q;
+    if (!a.cu_q && wid == 0 && used + tid < a.delta - a.lse2) a.lse2[used + tid] = -__builtin_inff();
+  }
   float lse2[2];   // -lse2 of the lane's two queries
   f32x4 delta[2];  // -delta of the same, in all four elements (start value of the dP^T chains)
 #pragma unroll
@@ -1087,13 +1160,50 @@ void attn_bwd_dq_kernel(const AttnArgs a) {
         qf[qb][ks] = *(const V8*)(q_ptr + (int64_t)iq * a.q_st[1] + ks * 32 + u * 8);
         dof[qb][ks] = *(const V8*)(do_ptr + (int64_t)iq * a.do_st[1] + ks * 32 + u * 8);
       }
-      l2 = a.lse2[(int64_t)hq * a.rows_q + ws_row0 + iq];
-      dl = a.delta[(int64_t)hq * a.rows_q + ws_row0 + iq];
+      if constexpr (!STATS) {
+        l2 = a.lse2[(int64_t)hq * a.rows_q + ws_row0 + iq];
+        dl = a.delta[(int64_t)hq * a.rows_q + ws_row0 + iq];
+      }
     } else {
 #pragma unroll
       for (int ks = 0; ks < KS; ks++) {
         qf[qb][ks] = V8{0, 0, 0, 0, 0, 0, 0, 0};
         dof[qb][ks] = V8{0, 0, 0, 0, 0, 0, 0, 0};
+      }
+    }
+    if constexpr (STATS) {
+      // delta = sum over d of dO * O: eight elements a time, then the 16 (8) parts of a row
+      // pairwise from the farthest, as in the statistics kernel
+      float part[KS];
+#pragma unroll
+      for (int ks = 0; ks < KS; ks++) part[ks] = 0.f;
+      if (iq < len_q) {
+        const T* o_ptr = (const T*)a.out + b * a.o_st[0] + (s.q_row0 + iq) * a.o_st[1] + hq * a.o_st[2];
+        const float l = a.lse[b * a.lse_st[0] + hq * a.lse_st[1] + (s.q_row0 + iq) * a.lse_st[2]];
+#pragma unroll
+        for (int ks = 0; ks < KS; ks++) {
+          const V8 o8 = *(const V8*)(o_ptr + ks * 32 + u * 8);
+#pragma unroll
+          for (int j = 0; j < 8; j++) {
+            // (products of 16-bit values are exact; contracted, fp16 becomes v_dot2, which rounds
+            // otherwise than the statistics kernel)
+#pragma clang fp contract(off)
+            part[ks] += (float)o8[j] * (float)dof[qb][ks][j];
+          }
+        }
+        l2 = (l == -__builtin_inff()) ? l : -l * kLog2e;
+      }
+#pragma unroll
+      for (int m = KS / 2; m >= 1; m >>= 1)
+#pragma unroll
+        for (int ks = 0; ks < m; ks++) part[ks] += part[ks + m];
+      float sum = part[0];
+      sum += __shfl_xor(sum, 32, 64);
+      sum += __shfl_xor(sum, 16, 64);
+      dl = -sum;
+      if (u == 0 && iq < len_q) {
+        a.lse2[(int64_t)hq * a.rows_q + ws_row0 + iq] = l2;
+        a.delta[(int64_t)hq * a.rows_q + ws_row0 + iq] = dl;
       }
     }
     lse2[qb] = l2;
@@ -1562,44 +1672,11 @@ __global__ __launch_bounds__(256) void attn_bwd_prep_kernel(const AttnArgs a) {
     const int64_t used = a.rows_q * a.heads_q;
     if (used + threadIdx.x < a.delta - a.lse2) a.lse2[used + threadIdx.x] = -__builtin_inff();
   }
-  // The first block of a pack's launch writes the key tile table: running sums of the sequences'
-  // tile counts, 256 sequences at a time (a scan in each wave, the waves' totals through LDS).
-  if (a.ktile) {
-    if (blockIdx.x == 0) {
-      __shared__ int wave_sum[4];
-      const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-      const int first_n = (a.cu_k[1] - a.cu_k[0] + (1 << a.ktile_log2) - 1) >> a.ktile_log2;
-      int unlike = 0;  // some sequence has another number of tiles than the first
-      int base = 0;
-      for (int b0 = 0; b0 < a.batch; b0 += 256) {
-        const int b = b0 + (int)threadIdx.x;
-        const int len = b < a.batch ? a.cu_k[b + 1] - a.cu_k[b] : 0;
-        const int n = (len + (1 << a.ktile_log2) - 1) >> a.ktile_log2;
-        int sum = n;  // inclusive
-#pragma unroll
-        for (int m = 1; m < 64; m <<= 1) {
-          const int up = __shfl_up(sum, m, 64);
-          if (lane >= m) sum += up;
-        }
-        __syncthreads();  // (wave_sum of the previous pass has been read)
-        if (lane == 63) wave_sum[wave] = sum;
-        __syncthreads();
-        int before = base;
-        for (int w = 0; w < 4; w++) {
-          if (w < wave) before += wave_sum[w];
-          base += wave_sum[w];
-        }
-        if (b < a.batch) a.ktile[b] = before + sum - n;
-        // (the last sequence may be a remainder)
-        unlike |= b < a.batch - 1 && n != first_n;
-      }
-      unlike = __syncthreads_or(unlike);
-      if (threadIdx.x == 0) {
-        a.ktile[a.batch] = base;
-        a.ktile[a.batch + 1] = !unlike && first_n << a.ktile_log2 <= kSnakeKeys;
-      }
-      return;
-    }
+  // the first block of a pack's launch writes the key tile table
+  if (a.ktile && blockIdx.x == 0) {
+    __shared__ int wave_sum[4];
+    write_ktile<256>(a, wave_sum);
+    return;
   }
   const unsigned blk = blockIdx.x - (a.ktile ? 1 : 0);
   const int h = (int)(blk % (unsigned)a.heads_q);
@@ -1658,10 +1735,12 @@ __global__ __launch_bounds__(256) void attn_bwd_prep_kernel(const AttnArgs a) {
   template __global__ void attn_bwd_dkdv_kernel<T, D, false, true, false>(const AttnArgs); \
   template __global__ void attn_bwd_dkdv_kernel<T, D, false, true, true>(const AttnArgs); \
   template __global__ void attn_bwd_dq_ds_kernel<T, D>(const AttnArgs);                     \
-  template __global__ void attn_bwd_dq_kernel<T, D, false, 8>(const AttnArgs);       \
-  template __global__ void attn_bwd_dq_kernel<T, D, true, 8>(const AttnArgs);        \
-  template __global__ void attn_bwd_dq_kernel<T, D, false, 4>(const AttnArgs);       \
-  template __global__ void attn_bwd_dq_kernel<T, D, true, 4>(const AttnArgs);        \
+  template __global__ void attn_bwd_dq_kernel<T, D, false, 8, false>(const AttnArgs); \
+  template __global__ void attn_bwd_dq_kernel<T, D, false, 8, true>(const AttnArgs); \
+  template __global__ void attn_bwd_dq_kernel<T, D, true, 8, false>(const AttnArgs); \
+  template __global__ void attn_bwd_dq_kernel<T, D, false, 4, false>(const AttnArgs); \
+  template __global__ void attn_bwd_dq_kernel<T, D, false, 4, true>(const AttnArgs); \
+  template __global__ void attn_bwd_dq_kernel<T, D, true, 4, false>(const AttnArgs); \
   template __global__ void attn_bwd_sink_kernel<T, D>(const AttnArgs);                  \
   template __global__ void attn_bwd_prep_kernel<T, D>(const AttnArgs);
 RSWA_INSTANTIATE(__bf16, 128)
@@ -1728,7 +1807,47 @@ int launch_bwd(AttnArgs& a, hipStream_t stream, int phases) {
   const int64_t units = a.rows_q * a.heads_q;
   const bool walk4 = dkv_walk4(a, D);
   a.ktile_log2 = walk4 ? 6 : 8;
-  if (units > 0 && (phases & RSWA_BWD_PREP)) {
+  auto launch_dq = [&](auto stats) {
+    constexpr bool STATS = decltype(stats)::value;
+    const bool pair = (a.group & 1) == 0;
+    const bool small = a.avg_keys <= RSWA_DQ_SMALL_AVG_KEYS;
+    const int bm = (pair ? 16 : 32) * (small ? 4 : 8);
+    const int units_q = (pair ? a.group / 2 : a.group) * a.heads_kv;  // blocks per q tile
+    if (a.cu_q) {
+      a.n_tile = (int)(ceil_div(a.rows_q, bm) + a.batch);
+      a.n_work = a.n_tile * units_q;
+    } else {
+      a.n_tile = (int)ceil_div(a.seqlen_q, bm);
+      a.n_work = a.n_tile * units_q * a.batch;
+    }
+    if (a.n_work == 0) return (int)RSWA_OK;
+    clear_launch_error();
+    const dim3 grid(padded_grid(a.n_work)), block(small ? 256 : 512);
+    if constexpr (!STATS) {
+      if (a.far) {
+        if (small) hipLaunchKernelGGL((attn_bwd_dq_kernel<T, D, true, 4, false>), grid, block, 0, stream, a);
+        else hipLaunchKernelGGL((attn_bwd_dq_kernel<T, D, true, 8, false>), grid, block, 0, stream, a);
+        return check_launch("attn_bwd dq");
+      }
+    }
+    if (small) hipLaunchKernelGGL((attn_bwd_dq_kernel<T, D, false, 4, STATS>), grid, block, 0, stream, a);
+    else hipLaunchKernelGGL((attn_bwd_dq_kernel<T, D, false, 8, STATS>), grid, block, 0, stream, a);
+    return check_launch("attn_bwd dq");
+  };
+  // Statistics and dQ asked for in one call: the dQ kernel goes first and makes the statistics.
+  // (dS hand-off: dQ needs the dK/dV kernel's tiles, so the statistics have a kernel of their own;
+  // so they have where the dQ kernel would spill, in the second addressing form.)
+  const bool fused = units > 0 && (phases & RSWA_BWD_PREP) && (phases & RSWA_BWD_DQ) && !a.ds && !a.far;
+  if (fused) {
+    if (a.cu_q || a.n_count > 0) {
+      clear_launch_error();
+      hipLaunchKernelGGL(attn_bwd_rest_kernel, dim3(1), dim3(256), 0, stream, a);
+      int rc = check_launch("attn_bwd rest");
+      if (rc != RSWA_OK) return rc;
+    }
+    int rc = launch_dq(std::true_type{});
+    if (rc != RSWA_OK) return rc;
+  } else if (units > 0 && (phases & RSWA_BWD_PREP)) {
     const int64_t blocks = ceil_div(a.rows_q, PrepCfg<D>::ROWS) * a.heads_q + (a.ktile ? 1 : 0);
     RSWA_REQUIRE(blocks < (1ll << 31), RSWA_ERR_UNSUPPORTED, "attn_bwd: too many (row, head) pairs");
     clear_launch_error();
@@ -1788,31 +1907,8 @@ int launch_bwd(AttnArgs& a, hipStream_t stream, int phases) {
       int rc = check_launch("attn_bwd dq (dS hand-off)");
       if (rc != RSWA_OK) return rc;
     }
-  } else if (phases & RSWA_BWD_DQ) {
-    const bool pair = (a.group & 1) == 0;
-    const bool small = a.avg_keys <= RSWA_DQ_SMALL_AVG_KEYS;
-    const int bm = (pair ? 16 : 32) * (small ? 4 : 8);
-    const int units_q = (pair ? a.group / 2 : a.group) * a.heads_kv;  // blocks per q tile
-    if (a.cu_q) {
-      a.n_tile = (int)(ceil_div(a.rows_q, bm) + a.batch);
-      a.n_work = a.n_tile * units_q;
-    } else {
-      a.n_tile = (int)ceil_div(a.seqlen_q, bm);
-      a.n_work = a.n_tile * units_q * a.batch;
-    }
-    if (a.n_work > 0) {
-      clear_launch_error();
-      const dim3 grid(padded_grid(a.n_work)), block(small ? 256 : 512);
-      if (small) {
-        if (a.far) hipLaunchKernelGGL((attn_bwd_dq_kernel<T, D, true, 4>), grid, block, 0, stream, a);
-        else hipLaunchKernelGGL((attn_bwd_dq_kernel<T, D, false, 4>), grid, block, 0, stream, a);
-      } else {
-        if (a.far) hipLaunchKernelGGL((attn_bwd_dq_kernel<T, D, true, 8>), grid, block, 0, stream, a);
-        else hipLaunchKernelGGL((attn_bwd_dq_kernel<T, D, false, 8>), grid, block, 0, stream, a);
-      }
-      int rc = check_launch("attn_bwd dq");
-      if (rc != RSWA_OK) return rc;
-    }
+  } else if ((phases & RSWA_BWD_DQ) && !fused) {
+    return launch_dq(std::false_type{});
   }
   return RSWA_OK;
 }

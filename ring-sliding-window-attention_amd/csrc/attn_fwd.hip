@@ -41,7 +41,7 @@ struct FwdCfg {
   // Blocks per compute unit (a block has one wave per SIMD).  head_dim 128 needs 214 registers, so
   // two.  head_dim 64 has half the MFMAs per score and is bound by the softmax's vector work and
   // its latencies; it fits three (148 registers; four would spill): 8000 rows in four sequences,
-  // 28 / 4 heads, window 1000, fp16: 83.6 -> 79.0 us.
+  // 28 / 4 heads, window 1000, fp16: 79-84 -> 77-79 us (by box; the two alternating on one).
   static constexpr int WAVES_PER_SIMD = D == 64 ? 3 : 2;
   static_assert(TILE >= 32 * O_STRIDE, "one wave's epilogue staging fits one tile buffer");
 };

@@ -478,8 +478,9 @@ def _backward_one_pass(q, k, v, prev_kv, out, lse, do, one, scale):
     ws = torch.empty(bwd_workspace_bytes(q, kk, second_rows=s, window_size=(w, 0), causal=True,
                                          handoff=None), dtype=torch.uint8, device=q.device)
     handed = bwd_handoff_active(q, kk, second_rows=s, window_size=(w, 0), causal=True)
-    # the dQ kernel of the hand-off route reads what the dK/dV kernel stored
-    for phases in ((PREP, DKDV, DQ) if handed else (PREP, DQ, DKDV)):
+    # the dQ kernel of the hand-off route reads what the dK/dV kernel stored; otherwise it makes
+    # the statistics itself
+    for phases in ((PREP, DKDV, DQ) if handed else (PREP | DQ, DKDV)):
         attn_bwd(q, kk, vv, out, lse, do, dq, dkk, dvv, scale, (w, 0), True, workspace=ws,
                  phases=phases, second=(k, v, dk, dv))
     return (dq, dk, dv, *dprev)
