@@ -238,6 +238,11 @@ typedef struct rswa_attn_params {
    * accumulators before the backward, ring_swa/sliding_window/nonvarlen.py:156-157). */
   int32_t wide;
   int32_t dkv_accumulate; /* only with RSWA_WIDE_DKV */
+  /* Backward only.  Blocks of the dK/dV kernel: RSWA_DKDV_AUTO (0) picks by an estimate of both
+   * forms' times; RSWA_DKDV_WIDE (1) blocks of 256 keys, RSWA_DKDV_SHORT (2) blocks of 64 keys whose
+   * four waves share the walk over the query rows, whatever the sizes (the same sums in another
+   * order): for tests of either form and measurements of one against the other. */
+  int32_t dkdv_form;
 } rswa_attn_params;
 
 #define RSWA_WIDE_OUT 1
@@ -246,6 +251,10 @@ typedef struct rswa_attn_params {
 
 #define RSWA_ADDR_AUTO 0
 #define RSWA_ADDR_FAR 1
+
+#define RSWA_DKDV_AUTO 0
+#define RSWA_DKDV_WIDE 1
+#define RSWA_DKDV_SHORT 2
 
 int rswa_attn_fwd(const rswa_attn_params* p, void* stream);
 int rswa_attn_bwd(const rswa_attn_params* p, void* stream);
@@ -298,6 +307,11 @@ uint64_t rswa_attn_bwd_workspace_bytes(const rswa_attn_params* p);
 /* 1 when a backward with these parameters takes the dS hand-off route (ds_handoff != 0 and the
  * shape is eligible), 0 otherwise. */
 int rswa_attn_bwd_handoff_active(const rswa_attn_params* p);
+
+/* Keys per block of the dK/dV launch of a backward with these parameters (p->workspace and
+ * p->workspace_bytes are ignored): 256 or 64 (see dkdv_form); a negative status if the call would
+ * be refused. */
+int rswa_attn_bwd_dkdv_keys(const rswa_attn_params* p);
 
 /* Message of the calling thread's last failed call ("" if none). */
 const char* rswa_last_error(void);

@@ -181,6 +181,7 @@ int fill_args(const rswa_attn_params* p, bool backward, AttnArgs& a, bool allow_
   a.n_count = 0;
   a.ktile = nullptr;
   a.ktile_log2 = 0;
+  a.dkdv_form = p->dkdv_form;
   a.snake = 0;
   a.sink_part = nullptr;
   a.sink_count = nullptr;

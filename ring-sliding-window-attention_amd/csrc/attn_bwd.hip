@@ -1765,6 +1765,7 @@ RSWA_INSTANTIATE(_Float16, 64)
 // 262 / 173, 64-256 193 / 175, 16-1024 260 / 216; all of 512 198 / 204, 32 / 32 heads 16-1024 348 / 475.
 // The 0.9 leans to the wide form where lengths are alike (65536 tokens of 512: 715 / 784).
 bool dkv_walk4(const AttnArgs& a, int head_dim) {
+  if (a.dkdv_form == RSWA_DKDV_WIDE || a.dkdv_form == RSWA_DKDV_SHORT) return a.dkdv_form == RSWA_DKDV_SHORT;
   const bool pack = a.cu_q != nullptr;
   const int64_t lk1 = pack ? std::max<int64_t>(1, a.rows_k / a.batch) : a.seqlen_k;
   const int64_t lq1 = pack ? std::max<int64_t>(1, a.rows_q / a.batch) : a.seqlen_q;
@@ -1936,6 +1937,18 @@ int bwd_entry(const rswa_attn_params* p, void* stream, int phases, bool allow_ha
 
 extern "C" int rswa_attn_bwd_phases(const rswa_attn_params* p, void* stream, int phases) {
   return rswa::bwd_entry(p, stream, phases, true);
+}
+
+extern "C" int rswa_attn_bwd_dkdv_keys(const rswa_attn_params* p) {
+  using namespace rswa;
+  RSWA_REQUIRE(p != nullptr, RSWA_ERR_INVALID, "attn_bwd: null params");
+  rswa_attn_params q = *p;
+  q.workspace = (void*)(uintptr_t)256;  // (any aligned address: nothing is launched)
+  q.workspace_bytes = ~0ull;
+  AttnArgs a;
+  const int rc = fill_args(&q, true, a, true);
+  if (rc != RSWA_OK) return rc;
+  return dkv_walk4(a, p->head_dim) ? kDkvKeysPerBlock / 4 : kDkvKeysPerBlock;
 }
 
 extern "C" int rswa_attn_bwd(const rswa_attn_params* p, void* stream) {

@@ -40,6 +40,7 @@ struct AttnArgs {
   // kernel; a tile has 2^ktile_log2 keys
   int32_t* ktile;
   int32_t ktile_log2;
+  int32_t dkdv_form;  // RSWA_DKDV_*: the caller's choice of the dK/dV kernel's blocks
   int32_t snake;    // dK/dV: see the kernel (dense; of a pack the device decides)
   const int32_t* cu_q;
   const int32_t* cu_k;

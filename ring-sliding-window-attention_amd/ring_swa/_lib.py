@@ -81,9 +81,11 @@ class AttnParams(Structure):
         ("ds_handoff", c_int32),
         ("wide", c_int32),
         ("dkv_accumulate", c_int32),
+        ("dkdv_form", c_int32),
     ]
 
 WIDE_OUT, WIDE_DQ, WIDE_DKV = 1, 2, 4
+DKDV_FORMS = {"wide": 1, "short": 2}
 
 
 class RswaError(RuntimeError):
@@ -136,6 +138,8 @@ def load(path: str) -> ctypes.CDLL:
     L.rswa_attn_bwd_workspace_bytes.argtypes = [POINTER(AttnParams)]
     L.rswa_attn_bwd_handoff_active.restype = c_int
     L.rswa_attn_bwd_handoff_active.argtypes = [POINTER(AttnParams)]
+    L.rswa_attn_bwd_dkdv_keys.restype = c_int
+    L.rswa_attn_bwd_dkdv_keys.argtypes = [POINTER(AttnParams)]
     if L.rswa_sizeof_attn_params() != ctypes.sizeof(AttnParams):
         raise ImportError(
             "rswa_attn_params layout mismatch between librswa.so "

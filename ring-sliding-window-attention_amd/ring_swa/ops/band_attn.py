@@ -287,6 +287,10 @@ def attn_bwd(
         )
         p.dk2, p.dv2 = dk2.data_ptr(), dv2.data_ptr()
     p.dq_accumulate = int(bool(dq_accumulate))
+    # RSWA_DKDV_FORM=wide / short: the dK/dV kernel's blocks of 256 / of 64 keys whatever the sizes
+    form = os.environ.get("RSWA_DKDV_FORM", "")
+    if form:
+        p.dkdv_form = _lib.DKDV_FORMS[form]
     p.dkv_accumulate = int(bool(dkv_accumulate))
     p.wide = (_lib.WIDE_DQ if wide_dq else 0) | (_lib.WIDE_DKV if wide_dkv else 0)
     p.out = o.data_ptr()

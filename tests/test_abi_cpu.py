@@ -208,3 +208,20 @@ def test_two_key_ranges_are_checked_before_any_launch():
     p.workspace_bytes = 0
     assert L.rswa_attn_bwd(p, None) == -1
     assert b"workspace" in L.rswa_last_error()
+
+
+def test_form_of_the_dkdv_blocks_can_be_chosen():
+    """dkdv_form picks blocks of 256 or of 64 keys whatever the sizes; by itself a launch that fills
+    the chip with 256-key blocks takes those, a small one the others."""
+    _ensure_built()
+    from ring_swa import _lib
+
+    L = _lib.lib()
+    for tokens, auto in ((1024, 64), (65536, 256)):
+        p = _fake_params(tokens)
+        assert L.rswa_attn_bwd_dkdv_keys(p) == auto
+        for form, keys in (("wide", 256), ("short", 64)):
+            p.dkdv_form = _lib.DKDV_FORMS[form]
+            assert L.rswa_attn_bwd_dkdv_keys(p) == keys
+    p.head_dim = 96
+    assert L.rswa_attn_bwd_dkdv_keys(p) < 0
