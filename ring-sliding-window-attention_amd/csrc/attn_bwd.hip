@@ -89,7 +89,8 @@ __device__ __forceinline__ void put_grad8(void* buf, int64_t at, typename Mma<T>
   }
 }
 
-constexpr int kSnakeKeys = 4096;  // longest sequence whose dK/dV blocks take the snake order
+// Sequences of at most this many keys whose dK/dV blocks take the snake order (see the kernel)
+constexpr int kSnakeKeys = 4096;
 
 // ============================================================================
 // dK / dV
@@ -147,9 +148,13 @@ __global__ __launch_bounds__(256) void attn_bwd_dkdv_kernel(const AttnArgs a) {
   // pack's tiles numbered by slots, one of them unused per sequence, as in the other kernels, 64
   // sequences of 256 tokens (32 / 8 heads, head_dim 128) took 242 us, every other block being empty;
   // numbered exactly, 129 us.  `snake` reverses every other group of four blocks where the walks
-  // of a short sequence's few tiles, one sequence like the other, are the pattern: 64 sequences of
-  // 1024 tokens 1368 -> 1141 us, dense causal 4096 rows x 32 heads 300 -> 277 us.  (Sequences
-  // longer than 4096 keys keep the plain order: four of 16384 tokens lose 3 % by it.)
+  // of a sequence's few tiles are such a pattern: of 256-key tiles only a number that is a multiple
+  // of four repeats in step with the engines (us, plain / snake, all alike: 64 sequences of 1024
+  // tokens, 32 / 32 heads, 1720 / 1400; dense causal, head_dim 64, 4016 rows x 32 heads 188 / 170; but
+  // 1954 rows against 2466 keys, ten tiles, 59 / 67, 2 x 1110 rows, five, 54 / 61), of the 64-key
+  // form's tiles any (422 shapes, mean 1.2 % faster, 10 % slower to 20 % faster).  Sequences of
+  // more than 4096 keys keep the plain order: four of 16384 tokens lose 3 % by it, 10240 keys under
+  // 8192 rows in 40 wide tiles 447 / 550.
   int n_tile = a.n_tile, n_work = a.n_work, per_xcd = (int)gridDim.x >> 3, snake = a.snake;
   if (a.ktile) {
     n_tile = a.ktile[a.batch];
@@ -992,7 +997,7 @@ template <int THREADS>
 __device__ __forceinline__ void write_ktile(const AttnArgs& a, int* wave_sum) {
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int first_n = (a.cu_k[1] - a.cu_k[0] + (1 << a.ktile_log2) - 1) >> a.ktile_log2;
-  int unlike = 0;  // some sequence has another number of tiles than the first
+  int period = 0;  // tiles (of this thread's sequences) for which the snake order is
   int base = 0;
   for (int b0 = 0; b0 < a.batch; b0 += THREADS) {
     const int b = b0 + (int)threadIdx.x;
@@ -1013,13 +1018,19 @@ __device__ __forceinline__ void write_ktile(const AttnArgs& a, int* wave_sum) {
       base += wave_sum[w];
     }
     if (b < a.batch) a.ktile[b] = before + sum - n;
-    // (the last sequence may be a remainder)
-    unlike |= b < a.batch - 1 && n != first_n;
+    const bool in_step = a.ktile_log2 == 8 ? (n & 3) == 0 : n == first_n;
+    if (in_step && n << a.ktile_log2 <= kSnakeKeys) period += n;
   }
-  unlike = __syncthreads_or(unlike);
+  __syncthreads();
+  if (threadIdx.x == 0) wave_sum[0] = 0;
+  __syncthreads();
+  if (period) atomicAdd(wave_sum, period);
+  __syncthreads();
   if (threadIdx.x == 0) {
     a.ktile[a.batch] = base;
-    a.ktile[a.batch + 1] = !unlike && first_n << a.ktile_log2 <= kSnakeKeys;
+    // (28 sequences of 900 to 1083 tokens, 0.77 of the 256-key tiles in fours: 625 us plain, 538 snake;
+    // drawn packs of which less than that are: 0.8 % slower by it on average, up to 32 %)
+    a.ktile[a.batch + 1] = base > 0 && (int64_t)wave_sum[0] * 10 >= (int64_t)base * 7;
   }
 }
 
@@ -1866,7 +1877,7 @@ int launch_bwd(AttnArgs& a, hipStream_t stream, int phases) {
       a.n_tile = (int)ceil_div(a.seqlen_k, bn);
       a.n_work = a.n_tile * a.heads_kv * a.batch;
     }
-    a.snake = !a.cu_q && a.seqlen_k <= kSnakeKeys;
+    a.snake = !a.cu_q && a.seqlen_k <= kSnakeKeys && (walk4 || a.n_tile % 4 == 0);
     if (a.n_work > 0) {
       clear_launch_error();
       const dim3 grid(padded_grid(a.n_work)), block(C::THREADS);

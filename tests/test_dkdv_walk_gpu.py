@@ -51,6 +51,8 @@ PACKS = [
     ([0, 64, 0, 1, 700, 0, 129, 0], 4, 1, 128, 50),   # empty sequences everywhere
     ([1 + i % 3 for i in range(300)], 2, 1, 64, 8),   # more than 256 sequences: two passes of the scan
     ([40] * 64 + [41], 2, 2, 128, 64),                # 65 sequences: two levels of the search
+    ([1024, 1000, 970, 300], 4, 4, 64, 2000),         # most tiles in fours: wide blocks in snake order
+    ([1024, 300, 700], 4, 2, 128, 150),               # fewer: plain order
 ]
 
 
