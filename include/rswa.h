@@ -264,8 +264,11 @@ int rswa_attn_bwd(const rswa_attn_params* p, void* stream);
  * (dk, dv written; reads the statistics) and DQ (dq written; reads the statistics).
  * This variant enqueues only the phases named in the bit mask, on the same
  * workspace: it lets a profiler or benchmark bracket one kernel alone, and lets a
- * caller that needs only some of the gradients skip the rest.  Same interface
- * replaced as rswa_attn_bwd (ring_swa/ops/wrap_flash.py:276-429).
+ * caller that needs only some of the gradients skip the rest.  What DKDV and DQ take from an
+ * earlier call is the row statistics (of the same q heads, rows, out, lse and dout); with sink
+ * keys under a bounded window DKDV also needs PREP of the same num_sink and window_left, which
+ * clears its counters.  Everything else a phase needs it makes itself, whatever the mask of the
+ * call that ran PREP.  Same interface replaced as rswa_attn_bwd (ring_swa/ops/wrap_flash.py:276-429).
  */
 #define RSWA_BWD_PREP 1
 #define RSWA_BWD_DKDV 2

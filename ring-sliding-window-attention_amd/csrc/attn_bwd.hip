@@ -141,8 +141,8 @@ __global__ __launch_bounds__(256) void attn_bwd_dkdv_kernel(const AttnArgs a) {
   __shared__ __attribute__((aligned(1024))) float st_s0[(WALK4 ? 8 : 2) * C::BM];  // -lse2[BM], -delta[BM]
   __shared__ __attribute__((aligned(1024))) float st_s1[(WALK4 ? 8 : 2) * C::BM];
 
-  // A pack's exact number of key tiles is known on the device only (ktile, see the statistics
-  // kernel): the tiles come first in the launch, dealt evenly to the XCDs, and the blocks beyond
+  // A pack's exact number of key tiles is known on the device only (ktile, see
+  // write_ktile): the tiles come first in the launch, dealt evenly to the XCDs, and the blocks beyond
   // them end here.  Consecutive blocks of an XCD go to its shader engines in turn and wait for the
   // engine whose turn it is, so lengths that repeat with an even period leave engines idle: with a
   // pack's tiles numbered by slots, one of them unused per sequence, as in the other kernels, 64
@@ -1034,6 +1034,13 @@ __device__ __forceinline__ void write_ktile(const AttnArgs& a, int* wave_sum) {
   }
 }
 
+// The table alone, for a dK/dV launch whose statistics came with another call: that call's table may
+// be of another tile size or lie elsewhere, and the kernel takes its block count and rows from it.
+__global__ __launch_bounds__(256) void attn_bwd_ktile_kernel(const AttnArgs a) {
+  __shared__ int wave_sum[4];
+  write_ktile<256>(a, wave_sum);
+}
+
 // What the statistics kernel leaves in the workspace of a pack or a call with sink keys beside the
 // statistics of the rows, by one block: the sink kernel's arrival counters at zero, the neutral
 // value behind a pack's lse2 array, the neutral pair for the rows after a pack's last that the
@@ -1819,6 +1826,7 @@ int launch_bwd(AttnArgs& a, hipStream_t stream, int phases) {
   const int64_t units = a.rows_q * a.heads_q;
   const bool walk4 = dkv_walk4(a, D);
   a.ktile_log2 = walk4 ? 6 : 8;
+  if (!(phases & RSWA_BWD_DKDV)) a.ktile = nullptr;  // the table serves the dK/dV launch of its own call
   auto launch_dq = [&](auto stats) {
     constexpr bool STATS = decltype(stats)::value;
     const bool pair = (a.group & 1) == 0;
@@ -1876,6 +1884,12 @@ int launch_bwd(AttnArgs& a, hipStream_t stream, int phases) {
     } else {
       a.n_tile = (int)ceil_div(a.seqlen_k, bn);
       a.n_work = a.n_tile * a.heads_kv * a.batch;
+    }
+    if (a.ktile && !(phases & RSWA_BWD_PREP)) {
+      clear_launch_error();
+      hipLaunchKernelGGL(attn_bwd_ktile_kernel, dim3(1), dim3(256), 0, stream, a);
+      int rc = check_launch("attn_bwd key tile table");
+      if (rc != RSWA_OK) return rc;
     }
     a.snake = !a.cu_q && a.seqlen_k <= kSnakeKeys && (walk4 || a.n_tile % 4 == 0);
     if (a.n_work > 0) {

@@ -36,8 +36,8 @@ struct AttnArgs {
   float* lse2;    // fp32 [heads_q, rows_q] packed: -lse * log2(e); empty rows -inf (workspace)
   int32_t n_count;    // arrival counters in the workspace (sink kernel)
   // backward of a pack (workspace; null: no table): number of dK/dV key tiles before sequence b, for
-  // b = 0 .. batch, then whether all sequences have the same number; written by the statistics
-  // kernel; a tile has 2^ktile_log2 keys
+  // b = 0 .. batch, then whether the blocks take the snake order; written ahead of the dK/dV launch
+  // by a kernel of the same call; a tile has 2^ktile_log2 keys
   int32_t* ktile;
   int32_t ktile_log2;
   int32_t dkdv_form;  // RSWA_DKDV_*: the caller's choice of the dK/dV kernel's blocks

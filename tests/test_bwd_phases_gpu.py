@@ -1,0 +1,44 @@
+"""Phases of a pack's backward spread over calls with different masks: the dK/dV launch takes the row
+statistics from the earlier call and nothing else.  Its table of key tiles in particular is of its own
+call's tile size and place -- the earlier call may have had another (other blocks, sink keys ahead of
+it in the workspace, or what was there overwritten since)."""
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("form", ["wide", "short"])
+@pytest.mark.parametrize("prep", ["other form", "sinks", "overwritten"])
+def test_dkdv_launch_makes_its_own_key_tile_table(monkeypatch, form, prep):
+    from ring_swa.ops.band_attn import attn_bwd, attn_fwd, bwd_workspace_bytes
+
+    cu = [0, 700, 700, 1300, 1301, 1900]
+    hq, hk, d, w = 4, 2, 64, 200
+    gen = torch.Generator(device="cuda").manual_seed(3)
+    q, do = (torch.randn(cu[-1], hq, d, device="cuda", dtype=torch.bfloat16, generator=gen) for _ in range(2))
+    k, v = (torch.randn(cu[-1], hk, d, device="cuda", dtype=torch.bfloat16, generator=gen) for _ in range(2))
+    cu_t = torch.tensor(cu, dtype=torch.int32, device="cuda")
+    out, lse = attn_fwd(q, k, v, None, (w, 0), True, cu_t, cu_t)
+    sinks = 3 if prep == "sinks" else 0
+    need = max(bwd_workspace_bytes(q, k, cu_t, cu_t, window_size=(w, 0), causal=True, num_sink=n) for n in (0, sinks))
+    results = []
+    for split in (False, True):
+        ws = torch.zeros(need, dtype=torch.uint8, device="cuda")
+        grads = [torch.zeros_like(t) for t in (q, k, v)]
+
+        def run(phases, n_sink=0):
+            attn_bwd(q, k, v, out, lse, do, *grads, None, (w, 0), True, cu_t, cu_t, num_sink=n_sink,
+                     workspace=ws, phases=phases, handoff=False)
+
+        if split:
+            other = {"wide": "short", "short": "wide"}[form]
+            monkeypatch.setenv("RSWA_DKDV_FORM", other if prep == "other form" else form)
+            run(1, sinks)
+            if prep == "overwritten":  # all behind the statistics (two arrays, each to a multiple of 256 bytes)
+                ws[2 * (-(-cu[-1] * hq * 4 // 256) * 256):] = 0x11
+        monkeypatch.setenv("RSWA_DKDV_FORM", form)
+        run(2 if split else 7)
+        results.append(grads[1:])
+    for one, two in zip(*results):
+        assert torch.equal(one, two)
