@@ -154,7 +154,7 @@ class RankShareVarlenFunc(torch.autograd.Function):
         q4, k4, v4 = q.unsqueeze(0), k.unsqueeze(0), v.unsqueeze(0)
         prev4 = [p.unsqueeze(1) for p in prev_kv]
         ctx.plan, ctx.scale, ctx.ring_dtypes = plan, softmax_scale, ring_dtypes
-        ctx.joined = len(plan) > 1 and not ring_dtypes
+        ctx.joined = not ring_dtypes and _joinable(q4, k4, v4, prev4, plan)
         if ctx.joined:
             # keys of the pack's first sequence that lie before the chunk
             start = rank * s
@@ -325,6 +325,24 @@ def _one_pass(q, k, v, prev_kv, plan, local_cu):
     return w, kk, vv, tail
 
 
+def _joinable(q, k, v, prev_kv, plan):
+    """May the plan's blocks run as one band over joined keys (``_Joined``)?  The copies into its
+    buffer would convert and broadcast: tensors that do not all have the own chunk's shape, type and
+    device, or that the kernels would refuse for their layout, go to the block route, which refuses
+    them or takes them as they are."""
+    hops = plan[-1][0]
+    if hops == 0 or k.dim() != 4 or len(prev_kv) < hops:
+        return False
+    dtype, device, own = q.dtype, q.device, q.shape[:2] + k.shape[2:]
+    for t, shape in ((k, own), (v, own), *((p, (2,) + own) for p in prev_kv[:hops])):
+        if t.shape != shape or t.dtype != dtype or t.device != device or t.data_ptr() % 16:
+            return False
+        *outer, last = t.stride()
+        if last != 1 or any([x % 8 for x in outer]):
+            return False
+    return True
+
+
 class _Joined:
     """The rank's visible keys as one row range: the rows of earlier ranks' chunks that the window
     reaches, then its own chunk, copied into one buffer, so that every block of the plan is part of
@@ -396,7 +414,7 @@ def _forward_blocks(q, k, v, prev_kv, plan, scale, local_cu, ring_dtypes, one_pa
         # 4096; two launches and a merge remain for every other shape and for ring_dtypes).
         w, kk, vv, _ = one
         return (*attn_fwd(q, kk, vv, scale, (w, 0), True, second=(k, v)), None)
-    if one_pass and not ring_dtypes and len(plan) > 1:
+    if one_pass and not ring_dtypes and _joinable(q, k, v, prev_kv, plan):
         joined = _join_keys(k, v, prev_kv, plan, plan[0][3][0])
         return (*attn_fwd(q, joined.kv[0], joined.kv[1], scale, plan[0][3], True), joined)
     if ring_dtypes or len(plan) > 2:

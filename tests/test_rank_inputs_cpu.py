@@ -1,0 +1,54 @@
+"""What a rank step accepts: the joined-keys route copies keys and values, which would convert types
+and broadcast shapes on the way, so only tensors that need neither take it.  Everything else goes to
+the block route, whose checks refuse it (or which takes it as it is)."""
+import pytest
+import torch
+
+import ring_swa
+from ring_swa import rank_share as RS
+
+S, HQ, HK, D = 64, 4, 2, 64
+
+
+def _inputs(b=2):
+    q = torch.randn(b, S, HQ, D).bfloat16()
+    k, v = (torch.randn(b, S, HK, D).bfloat16() for _ in range(2))
+    return q, k, v, [torch.randn(2, b, S, HK, D).bfloat16() for _ in range(2)]
+
+
+def _joinable(q, k, v, prev, window=S + 30):
+    return RS._joinable(q, k, v, prev, RS.plan_nonvarlen(S, window, 4, 2))
+
+
+def test_tensors_alike_are_joined():
+    q, k, v, prev = _inputs()
+    assert _joinable(q, k, v, prev)
+    fused = torch.randn(2, S, HQ + 2 * HK, D).bfloat16()
+    assert _joinable(fused[:, :, :HQ], fused[:, :, HQ:HQ + HK], fused[:, :, HQ + HK:], prev)
+    # a chunk beyond the window's reach is not looked at
+    assert not _joinable(q, k, v, prev[:1]) and _joinable(q, k, v, [prev[0], prev[1], prev[1].float()])
+
+
+def test_what_the_copies_would_change_is_not_joined():
+    q, k, v, prev = _inputs()
+    shifted = torch.empty(prev[0].numel() + 4).bfloat16()[4:].view_as(prev[0])  # rows not 16-byte aligned
+    for bad in (prev[1].float(), prev[1].half(), prev[1].to("meta"), prev[1][:, :1], prev[1][:, :, :, :1],
+                prev[1][:, :, :S // 2], prev[1][..., :1], prev[1].transpose(3, 4).contiguous().transpose(3, 4),
+                shifted):
+        assert not _joinable(q, k, v, [prev[0], bad])
+    for bad in (v.float(), v[:, :, :1], v[:1], v.transpose(2, 3).contiguous().transpose(2, 3)):
+        assert not _joinable(q, k, bad, prev) and not _joinable(q, bad, bad if bad.shape != v.shape else v, prev)
+
+
+@pytest.mark.parametrize("packed", [False, True], ids=["dense", "packed"])
+def test_the_entry_points_refuse_values_of_another_kind(packed):
+    """(The first block's checks come before the one for a GPU, so this runs without.)"""
+    q, k, v, prev = _inputs(1)
+    if packed:
+        q, k, v, prev = q[0], k[0], v[0], [p[:, 0] for p in prev]
+    for bad in (v.float(), v[..., :1, :]):
+        with pytest.raises(AssertionError):
+            if packed:
+                ring_swa.ring_rank_share_attn_varlen(q, k, bad, prev, S + 30, [0, 4 * S], 4, 2)
+            else:
+                ring_swa.ring_rank_share_attn(q, k, bad, prev, S + 30, 4, 2)
