@@ -107,8 +107,7 @@ class RankShareFunc(torch.autograd.Function):
         ctx.plan, ctx.scale, ctx.ring_dtypes, ctx.one_pass = plan, softmax_scale, ring_dtypes, one_pass
         ctx.joined = joined is not None
         if ctx.joined:
-            ctx.save_for_backward(q, out, lse, joined.kv)
-            ctx.prev_shapes = [p.shape for p in prev_kv]
+            ctx.save_for_backward(q, out, lse, joined.kv, *prev_kv[plan[-1][0]:])
         else:
             ctx.save_for_backward(q, k, v, out, lse, *prev_kv)
         return out
@@ -116,8 +115,8 @@ class RankShareFunc(torch.autograd.Function):
     @staticmethod
     def backward(ctx, do):
         if ctx.joined:
-            q, out, lse, kv = ctx.saved_tensors
-            grads = _backward_joined(q, kv, out, lse, do, ctx.plan, ctx.scale, ctx.prev_shapes)
+            q, out, lse, kv, *unreached = ctx.saved_tensors
+            grads = _backward_joined(q, kv, out, lse, do, ctx.plan, ctx.scale, unreached)
             return (grads[0], grads[1], grads[2], None, None, None, None, None, None, *grads[3:])
         q, k, v, out, lse, *prev_kv = ctx.saved_tensors
         grads = _backward_blocks(q, k, v, prev_kv, out, lse, do, ctx.plan, ctx.scale, None,
@@ -162,8 +161,8 @@ class RankShareVarlenFunc(torch.autograd.Function):
             joined = _join_keys(k4, v4, prev4, plan, window_size, local_cu, before)
             out, lse = attn_fwd(q, joined.kv[0, 0], joined.kv[1, 0], softmax_scale, plan[0][3], True,
                                 joined.cu_q, joined.cu_k)
-            ctx.save_for_backward(q, out, lse, joined.kv, joined.cu_q, joined.cu_k)
-            ctx.prev_shapes = [p.shape for p in prev4]
+            ctx.save_for_backward(q, out, lse, joined.kv, joined.cu_q, joined.cu_k,
+                                  *prev_kv[plan[-1][0]:])
             return out
         cu_dev = _device_cu(local_cu, q.device)
         out, lse, _ = _forward_blocks(q4, k4, v4, prev4, plan, softmax_scale, cu_dev, ring_dtypes)
@@ -174,9 +173,10 @@ class RankShareVarlenFunc(torch.autograd.Function):
     @staticmethod
     def backward(ctx, do):
         if ctx.joined:
-            q, out, lse, kv, cu_q, cu_k = ctx.saved_tensors
+            q, out, lse, kv, cu_q, cu_k, *unreached = ctx.saved_tensors
             grads = _backward_joined(q.unsqueeze(0), kv, out.unsqueeze(0), lse.unsqueeze(0),
-                                     do.unsqueeze(0), ctx.plan, ctx.scale, ctx.prev_shapes, cu_q, cu_k)
+                                     do.unsqueeze(0), ctx.plan, ctx.scale,
+                                     [p.unsqueeze(1) for p in unreached], cu_q, cu_k)
             dprev = [g.squeeze(1) for g in grads[3:]]
             return (grads[0].squeeze(0), grads[1].squeeze(0), grads[2].squeeze(0), None, None, None,
                     None, None, None, *dprev)
@@ -378,27 +378,32 @@ def _join_keys(k, v, prev_kv, plan, window, local_cu=None, first_kv_len=0):
     return _Joined(k, v, prev_kv, hops, reach, cu_q, cu_k)
 
 
-def _backward_joined(q, kv, out, lse, do, plan, scale, prev_shapes, cu_q=None, cu_k=None):
-    """Backward on joined keys.  The gradients of all reached chunks are views of one buffer of
-    whole chunks, zero in the rows that no query sees; chunks beyond get zeros of their own."""
+def _backward_joined(q, kv, out, lse, do, plan, scale, unreached, cu_q=None, cu_k=None):
+    """Backward on joined keys.  The kernel writes the gradients of all joined rows into one buffer;
+    a reached chunk's are copied into a tensor of its own, zero in the rows that no query sees; the
+    own chunk's stay where they are (copied, too, for batch > 1, where they would not be
+    contiguous).  ``unreached``: the chunks beyond the plan's."""
     if do.stride(-1) != 1:
         do = do.contiguous()
     (_, _, _, window, _), hops, s = plan[0], plan[-1][0], q.shape[1]
-    dq = torch.empty_like(q)
-    whole = torch.empty((2, kv.shape[1], (hops + 1) * s) + tuple(kv.shape[3:]), dtype=kv.dtype,
-                        device=kv.device)
-    unseen = whole.shape[2] - kv.shape[2]
-    if unseen:
-        whole[:, :, :unseen].zero_()
-    dk, dv = whole[0, :, unseen:], whole[1, :, unseen:]
+    reach = kv.shape[2] - s
+    dq, dkv = torch.empty_like(q), torch.empty_like(kv)
     if cu_q is None:
-        attn_bwd(q, kv[0], kv[1], out, lse, do, dq, dk, dv, scale, window, True)
+        attn_bwd(q, kv[0], kv[1], out, lse, do, dq, dkv[0], dkv[1], scale, window, True)
     else:
-        attn_bwd(q[0], kv[0, 0], kv[1, 0], out[0], lse[0], do[0], dq[0], dk[0], dv[0], scale, window,
-                 True, cu_q, cu_k)
-    dprev = [whole[:, :, (hops - 1 - i) * s:(hops - i) * s] if i < hops else
-             torch.zeros(shape, dtype=kv.dtype, device=kv.device) for i, shape in enumerate(prev_shapes)]
-    return (dq, whole[0, :, hops * s:], whole[1, :, hops * s:], *dprev)
+        attn_bwd(q[0], kv[0, 0], kv[1, 0], out[0], lse[0], do[0], dq[0], dkv[0, 0], dkv[1, 0], scale,
+                 window, True, cu_q, cu_k)
+    dprev = []
+    for i in range(1, hops + 1):
+        end = reach - (i - 1) * s
+        n = min(end, s)
+        g = kv.new_empty(kv.shape[:2] + (s,) + kv.shape[3:])
+        if n < s:
+            g[:, :, :s - n].zero_()
+        g[:, :, s - n:].copy_(dkv[:, :, end - n:end])
+        dprev.append(g)
+    dprev += [torch.zeros_like(p) for p in unreached]
+    return (dq, dkv[0, :, reach:].contiguous(), dkv[1, :, reach:].contiguous(), *dprev)
 
 
 def _forward_blocks(q, k, v, prev_kv, plan, scale, local_cu, ring_dtypes, one_pass=True):

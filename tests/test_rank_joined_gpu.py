@@ -64,3 +64,27 @@ def test_shares_on_joined_keys_match_the_oracle(s, w, packed):
     assert (torch.cat(outs, 1) - ro).abs().max().item() <= 2e-2
     errs = [_rel(torch.cat(dqs, 1), rq), _rel(dk, rk), _rel(dv, rv)]
     assert max(errs) <= 1e-2, f"dq / dk / dv relative norm {errs}"
+
+
+@pytest.mark.parametrize("packed", [False, True], ids=["dense", "packed"])
+def test_gradients_are_contiguous_tensors_of_their_inputs_type(packed):
+    """Also the chunks': each a tensor of its own (a ring sends it on its way back), a chunk beyond the
+    reach whatever its type."""
+    import ring_swa
+
+    s, w, hq, hk, d, b = 100, 130, 4, 2, 64, 1 if packed else 2
+    g = torch.Generator().manual_seed(1)
+    q, k, v, do = (torch.randn(b, s, h, d, generator=g).bfloat16().cuda() for h in (hq, hk, hk, hq))
+    prev = [torch.randn(2, b, s, hk, d, generator=g).to(t).cuda() for t in (torch.bfloat16, torch.bfloat16, torch.float32)]
+    if packed:
+        q, k, v, do, prev = q[0], k[0], v[0], do[0], [p[:, 0] for p in prev]
+    leaves = [t.contiguous().requires_grad_() for t in (q, k, v, *prev)]
+    if packed:
+        out = ring_swa.ring_rank_share_attn_varlen(*leaves[:3], leaves[3:], w, [0, 4 * s], 4, 3)
+    else:
+        out = ring_swa.ring_rank_share_attn(*leaves[:3], leaves[3:], w, 4, 3)
+    grads = torch.autograd.grad(out, leaves, do)
+    for t, x in zip(leaves, grads):
+        assert x.is_contiguous() and x.dtype == t.dtype and x.shape == t.shape
+    chunks = [x.untyped_storage().data_ptr() for x in grads[3:]]
+    assert len(set(chunks)) == 3 and not set(chunks) & {x.untyped_storage().data_ptr() for x in grads[:3]}
