@@ -107,7 +107,7 @@ class RankShareFunc(torch.autograd.Function):
         ctx.plan, ctx.scale, ctx.ring_dtypes, ctx.one_pass = plan, softmax_scale, ring_dtypes, one_pass
         ctx.joined = joined is not None
         if ctx.joined:
-            ctx.save_for_backward(q, out, lse, joined.kv, *prev_kv[plan[-1][0]:])
+            ctx.save_for_backward(q, out, lse, *joined, *prev_kv[plan[-1][0]:])
         else:
             ctx.save_for_backward(q, k, v, out, lse, *prev_kv)
         return out
@@ -115,8 +115,8 @@ class RankShareFunc(torch.autograd.Function):
     @staticmethod
     def backward(ctx, do):
         if ctx.joined:
-            q, out, lse, kv, *unreached = ctx.saved_tensors
-            grads = _backward_joined(q, kv, out, lse, do, ctx.plan, ctx.scale, unreached)
+            q, out, lse, kk, vv, *unreached = ctx.saved_tensors
+            grads = _backward_joined(q, kk, vv, out, lse, do, ctx.plan, ctx.scale, unreached)
             return (grads[0], grads[1], grads[2], None, None, None, None, None, None, *grads[3:])
         q, k, v, out, lse, *prev_kv = ctx.saved_tensors
         grads = _backward_blocks(q, k, v, prev_kv, out, lse, do, ctx.plan, ctx.scale, None,
@@ -153,16 +153,16 @@ class RankShareVarlenFunc(torch.autograd.Function):
         q4, k4, v4 = q.unsqueeze(0), k.unsqueeze(0), v.unsqueeze(0)
         prev4 = [p.unsqueeze(1) for p in prev_kv]
         ctx.plan, ctx.scale, ctx.ring_dtypes = plan, softmax_scale, ring_dtypes
-        ctx.joined = not ring_dtypes and _joinable(q4, k4, v4, prev4, plan)
-        if ctx.joined:
-            # keys of the pack's first sequence that lie before the chunk
+        ctx.joined = False
+        if len(plan) > 1 and not ring_dtypes:
             start = rank * s
-            before = start - max(c for c in cu_host if c <= start)
-            joined = _join_keys(k4, v4, prev4, plan, window_size, local_cu, before)
-            out, lse = attn_fwd(q, joined.kv[0, 0], joined.kv[1, 0], softmax_scale, plan[0][3], True,
-                                joined.cu_q, joined.cu_k)
-            ctx.save_for_backward(q, out, lse, joined.kv, joined.cu_q, joined.cu_k,
-                                  *prev_kv[plan[-1][0]:])
+            reach = _reach(plan, s, window_size, start - max(c for c in cu_host if c <= start))
+            ctx.joined = _joinable(q4, k4, v4, prev4, plan, window_size, reach)
+        if ctx.joined:
+            kk, vv = _join_keys(k4, v4, prev4, plan, reach)
+            cu_q, cu_k = _packed_cu(local_cu, reach, q.device)
+            out, lse = attn_fwd(q, kk[0], vv[0], softmax_scale, plan[0][3], True, cu_q, cu_k)
+            ctx.save_for_backward(q, out, lse, kk, vv, cu_q, cu_k, *prev_kv[plan[-1][0]:])
             return out
         cu_dev = _device_cu(local_cu, q.device)
         out, lse, _ = _forward_blocks(q4, k4, v4, prev4, plan, softmax_scale, cu_dev, ring_dtypes)
@@ -173,8 +173,8 @@ class RankShareVarlenFunc(torch.autograd.Function):
     @staticmethod
     def backward(ctx, do):
         if ctx.joined:
-            q, out, lse, kv, cu_q, cu_k, *unreached = ctx.saved_tensors
-            grads = _backward_joined(q.unsqueeze(0), kv, out.unsqueeze(0), lse.unsqueeze(0),
+            q, out, lse, kk, vv, cu_q, cu_k, *unreached = ctx.saved_tensors
+            grads = _backward_joined(q.unsqueeze(0), kk, vv, out.unsqueeze(0), lse.unsqueeze(0),
                                      do.unsqueeze(0), ctx.plan, ctx.scale,
                                      [p.unsqueeze(1) for p in unreached], cu_q, cu_k)
             dprev = [g.squeeze(1) for g in grads[3:]]
@@ -325,15 +325,43 @@ def _one_pass(q, k, v, prev_kv, plan, local_cu):
     return w, kk, vv, tail
 
 
-def _joinable(q, k, v, prev_kv, plan):
-    """May the plan's blocks run as one band over joined keys (``_Joined``)?  The copies into its
-    buffer would convert and broadcast: tensors that do not all have the own chunk's shape, type and
-    device, or that the kernels would refuse for their layout, go to the block route, which refuses
-    them or takes them as they are."""
+# Two blocks run as one band up to this much work (visible pairs x q heads x head_dim); see _joinable.
+_JOIN_TWO_WORK = 128e6 * 128
+
+
+def _reach(plan, s, window, first_kv_len=None):
+    """Rows of earlier chunks that the plan's blocks see: of a packed chunk only its first sequence
+    has keys before it, ``first_kv_len`` of them."""
+    reach = min(window, plan[-1][0] * s)
+    return reach if first_kv_len is None else min(reach, first_kv_len)
+
+
+def _joinable(q, k, v, prev_kv, plan, window, reach):
+    """May the plan's blocks run as one band over joined keys (``_join_keys``), and is that the faster
+    way?
+
+    The copies would convert and broadcast: tensors that do not all have the own chunk's shape, type
+    and device, or that the kernels would refuse for their layout, go to the block route, which
+    refuses them or takes them as they are.
+
+    Three and more blocks are always joined (forward 0.66 to 1.01 of the blocks' time, forward and
+    backward 0.65 to 0.94, over 17 shapes).  Two only where the host bounds their many launches and
+    the copies are small (forward and backward of 28 / 4 heads, 1607 tokens, window 556: 444 -> 256 us).
+    Beyond that two launches side by side fill the chip better than one of half as many, longer
+    blocks, and the copies show (us, blocks / joined, forward and backward: 8 / 2 heads, 8192 tokens of a
+    pack, window 8192, 585 / 724; 28 / 4 heads 1326 / 1627; forward alone, 32 / 32 heads, 447 / 514)."""
     hops = plan[-1][0]
     if hops == 0 or k.dim() != 4 or len(prev_kv) < hops:
         return False
-    dtype, device, own = q.dtype, q.device, q.shape[:2] + k.shape[2:]
+    (b, s, hq, d), hk = q.shape, k.shape[2]
+    if hops == 1:
+        # rows see min(window, reach + row) + 1 keys (a pack's no more than that)
+        m = min(max(window - reach, 0), s)
+        pairs = b * (m * reach + m * (m + 1) // 2 + (s - m) * (window + 1))
+        copied = 4 * b * (reach + s) * hk * d  # bytes
+        if pairs * hq * d > _JOIN_TWO_WORK or copied > max(8 << 20, pairs * hq // 4):
+            return False
+    dtype, device, own = q.dtype, q.device, (b, s, hk, d)
     for t, shape in ((k, own), (v, own), *((p, (2,) + own) for p in prev_kv[:hops])):
         if t.shape != shape or t.dtype != dtype or t.device != device or t.data_ptr() % 16:
             return False
@@ -343,42 +371,39 @@ def _joinable(q, k, v, prev_kv, plan):
     return True
 
 
-class _Joined:
-    """The rank's visible keys as one row range: the rows of earlier ranks' chunks that the window
-    reaches, then its own chunk, copied into one buffer, so that every block of the plan is part of
-    one causal band over them.  ``kv``: ``[2, batch, reach + seq, kv_heads, dim]``, ``reach`` rows of it from
-    the ``hops`` chunks before the own one; ``cu_q`` / ``cu_k``: packed chunks.
+def _join_keys(k, v, prev_kv, plan, reach):
+    """The rank's visible keys and values as one row range each: ``reach`` rows of the earlier ranks'
+    chunks, then its own chunk, copied side by side (``[batch, reach + seq, kv_heads, dim]``), so that
+    every block of the plan is part of one causal band over them.
 
-    Against the blocks one after the other, with merges and fp32 accumulators in between: 2.90 -> 2.45
-    ms for a step on 4096-token chunks, window 10000, 32 / 8 heads (the copies are 35 us of it); against
-    two blocks on two streams, a packed 8192-token chunk, window 2048: 845 -> 834 us."""
-
-    def __init__(self, k, v, prev_kv, hops, reach, cu_q=None, cu_k=None):
-        b, s, hk, d = k.shape
-        self.kv = kv = torch.empty((2, b, reach + s, hk, d), dtype=k.dtype, device=k.device)
-        self.hops, self.cu_q, self.cu_k = hops, cu_q, cu_k
-        for i in range(1, hops + 1):
-            end = reach - (i - 1) * s
-            n = min(end, s)
-            kv[:, :, end - n:end].copy_(prev_kv[i - 1][:, :, s - n:])
-        kv[0, :, reach:].copy_(k)
-        kv[1, :, reach:].copy_(v)
-
-
-def _join_keys(k, v, prev_kv, plan, window, local_cu=None, first_kv_len=0):
-    """``_Joined`` for a plan of two and more blocks.  Of a packed chunk only the first sequence
-    has keys before it, ``first_kv_len`` of them."""
-    hops = plan[-1][0]
-    reach = min(window, hops * k.shape[1])
-    if local_cu is None:
-        return _Joined(k, v, prev_kv, hops, reach)
-    reach = min(reach, first_kv_len)
-    cu_q = _device_cu(local_cu, k.device)
-    cu_k = _device_cu([0] + [reach + c for c in local_cu[1:]], k.device)
-    return _Joined(k, v, prev_kv, hops, reach, cu_q, cu_k)
+    Against the blocks one after the other, with merges and fp32 accumulators in between: 2.87 -> 2.43
+    ms for a step on 4096-token chunks, window 10000, 32 / 8 heads (copies and zero fills are 60 us
+    of it)."""
+    b, s, hk, d = k.shape
+    if b * (reach + s) * hk * d <= 3 << 19:
+        # two calls instead of three and fewer views: 14 against 19 us where the host bounds them; on
+        # many bytes cat reaches half the copies' rate (134 MB: 50 against 25 us; a forward of 2048
+        # tokens, 32 / 8 heads, reach 2048: 74 against 69)
+        rows = [(prev_kv[i - 1], s - min(reach - (i - 1) * s, s)) for i in range(plan[-1][0], 0, -1)]
+        return (torch.cat([p[0][:, first:] for p, first in rows] + [k], 1),
+                torch.cat([p[1][:, first:] for p, first in rows] + [v], 1))
+    kv = torch.empty((2, b, reach + s, hk, d), dtype=k.dtype, device=k.device)
+    for i in range(1, plan[-1][0] + 1):
+        end = reach - (i - 1) * s
+        n = min(end, s)
+        kv[:, :, end - n:end].copy_(prev_kv[i - 1][:, :, s - n:])
+    kv[0, :, reach:].copy_(k)
+    kv[1, :, reach:].copy_(v)
+    return kv[0], kv[1]
 
 
-def _backward_joined(q, kv, out, lse, do, plan, scale, unreached, cu_q=None, cu_k=None):
+def _packed_cu(local_cu, reach, device):
+    """Device ``cu_seqlens`` of the queries and of the joined keys of a packed chunk."""
+    return (_device_cu(local_cu, device),
+            _device_cu([0] + [reach + c for c in local_cu[1:]], device))
+
+
+def _backward_joined(q, kk, vv, out, lse, do, plan, scale, unreached, cu_q=None, cu_k=None):
     """Backward on joined keys.  The kernel writes the gradients of all joined rows into one buffer;
     a reached chunk's are copied into a tensor of its own, zero in the rows that no query sees; the
     own chunk's stay where they are (copied, too, for batch > 1, where they would not be
@@ -386,18 +411,18 @@ def _backward_joined(q, kv, out, lse, do, plan, scale, unreached, cu_q=None, cu_
     if do.stride(-1) != 1:
         do = do.contiguous()
     (_, _, _, window, _), hops, s = plan[0], plan[-1][0], q.shape[1]
-    reach = kv.shape[2] - s
-    dq, dkv = torch.empty_like(q), torch.empty_like(kv)
+    reach = kk.shape[1] - s
+    dq, dkv = torch.empty_like(q), kk.new_empty((2,) + kk.shape)
     if cu_q is None:
-        attn_bwd(q, kv[0], kv[1], out, lse, do, dq, dkv[0], dkv[1], scale, window, True)
+        attn_bwd(q, kk, vv, out, lse, do, dq, dkv[0], dkv[1], scale, window, True)
     else:
-        attn_bwd(q[0], kv[0, 0], kv[1, 0], out[0], lse[0], do[0], dq[0], dkv[0, 0], dkv[1, 0], scale,
-                 window, True, cu_q, cu_k)
+        attn_bwd(q[0], kk[0], vv[0], out[0], lse[0], do[0], dq[0], dkv[0, 0], dkv[1, 0], scale, window,
+                 True, cu_q, cu_k)
     dprev = []
     for i in range(1, hops + 1):
         end = reach - (i - 1) * s
         n = min(end, s)
-        g = kv.new_empty(kv.shape[:2] + (s,) + kv.shape[3:])
+        g = kk.new_empty((2, kk.shape[0], s) + kk.shape[2:])
         if n < s:
             g[:, :, :s - n].zero_()
         g[:, :, s - n:].copy_(dkv[:, :, end - n:end])
@@ -408,7 +433,7 @@ def _backward_joined(q, kv, out, lse, do, plan, scale, unreached, cu_q=None, cu_
 
 def _forward_blocks(q, k, v, prev_kv, plan, scale, local_cu, ring_dtypes, one_pass=True):
     """Run the planned blocks and merge them.  Dense 4-d tensors (batch 1 when packed).  Returns
-    ``(out, lse, joined)``, ``joined`` being the ``_Joined`` keys when that route was taken."""
+    ``(out, lse, joined)``, ``joined`` being the joined keys and values when that route was taken."""
     assert plan and plan[0][0] == 0, "the diagonal block comes first: it covers every row"
     one = _one_pass(q, k, v, prev_kv, plan, local_cu) if one_pass and not ring_dtypes else None
     if one is not None:
@@ -419,9 +444,12 @@ def _forward_blocks(q, k, v, prev_kv, plan, scale, local_cu, ring_dtypes, one_pa
         # 4096; two launches and a merge remain for every other shape and for ring_dtypes).
         w, kk, vv, _ = one
         return (*attn_fwd(q, kk, vv, scale, (w, 0), True, second=(k, v)), None)
-    if one_pass and not ring_dtypes and _joinable(q, k, v, prev_kv, plan):
-        joined = _join_keys(k, v, prev_kv, plan, plan[0][3][0])
-        return (*attn_fwd(q, joined.kv[0], joined.kv[1], scale, plan[0][3], True), joined)
+    if one_pass and not ring_dtypes and local_cu is None and len(plan) > 1:
+        window = plan[0][3][0]
+        reach = _reach(plan, q.shape[1], window)
+        if _joinable(q, k, v, prev_kv, plan, window, reach):
+            joined = _join_keys(k, v, prev_kv, plan, reach)
+            return (*attn_fwd(q, *joined, scale, plan[0][3], True), joined)
     if ring_dtypes or len(plan) > 2:
         # With two blocks the 16-bit running output is merged once and rounded once, the same
         # bits as the fp32 accumulator gives; from three blocks on every further merge would
@@ -598,8 +626,9 @@ def ring_rank_share_attn(
     running output in fp32 and the running LSE in fp64 as upstream does.  ``one_pass=False``
     keeps upstream's block structure -- own-chunk block, previous-chunk block, LSE merge
     (``ring_swa/sliding_window/nonvarlen.py:95-154``) -- where the default computes the blocks as
-    one band: over both key ranges where they lie (window shorter than a chunk), or over one
-    buffer that the reached chunks are copied into."""
+    one band where that is faster: over both key ranges where they lie (window shorter than a
+    chunk), or over a copy of the reached rows and the own chunk side by side, which is then what
+    the backward holds on to instead of ``k``, ``v`` and the reached chunks."""
     assert q.shape[1] == k.shape[1] == v.shape[1], "Sequence length must be the same"
     return RankShareFunc.apply(q, k, v, int(window_size), int(cp_size), int(cp_local_rank),
                                softmax_scale, bool(ring_dtypes), bool(one_pass), *prev_kv)

@@ -16,8 +16,10 @@ def _inputs(b=2):
     return q, k, v, [torch.randn(2, b, S, HK, D).bfloat16() for _ in range(2)]
 
 
-def _joinable(q, k, v, prev, window=S + 30):
-    return RS._joinable(q, k, v, prev, RS.plan_nonvarlen(S, window, 4, 2))
+def _joinable(q, k, v, prev, window=S + 30, rank=2):
+    s = q.shape[1]
+    plan = RS.plan_nonvarlen(s, window, 4, rank)
+    return RS._joinable(q, k, v, prev, plan, window, RS._reach(plan, s, window))
 
 
 def test_tensors_alike_are_joined():
@@ -52,3 +54,32 @@ def test_the_entry_points_refuse_values_of_another_kind(packed):
                 ring_swa.ring_rank_share_attn_varlen(q, k, bad, prev, S + 30, [0, 4 * S], 4, 2)
             else:
                 ring_swa.ring_rank_share_attn(q, k, bad, prev, S + 30, 4, 2)
+
+
+@pytest.mark.parametrize("s,hq,hk,d,window,rank,joined", [
+    (1000, 16, 4, 128, 1500, 1, True),      # two blocks, the host's launches are most of it
+    (2048, 32, 8, 128, 1536, 1, True),
+    (1000, 32, 32, 64, 250, 1, False),      # the copies are as large as the work
+    (8192, 8, 2, 128, 12288, 1, False),     # two launches fill the chip better than one
+    (7379, 4, 4, 128, 10877, 1, False),
+    (4096, 32, 8, 128, 10000, 3, True),     # four blocks, whatever the work
+    (6000, 32, 32, 128, 15600, 3, True),
+])
+def test_two_blocks_are_joined_only_where_launches_are_the_time(s, hq, hk, d, window, rank, joined):
+    q, k = torch.empty(1, s, hq, d, device="meta", dtype=torch.bfloat16), torch.empty(1, s, hk, d, device="meta", dtype=torch.bfloat16)
+    prev = [torch.empty(2, 1, s, hk, d, device="meta", dtype=torch.bfloat16) for _ in range(rank)]
+    assert _joinable(q, k, k, prev, window, rank) == joined
+
+
+@pytest.mark.parametrize("s,window,hops", [(64, 40, 1), (64, 128, 2), (1500, 2000, 2), (1500, 4500, 3)])
+def test_joined_rows_are_the_reached_rows_in_order(s, window, hops):
+    """Both ways of copying (one call per tensor for few elements, one per chunk for many)."""
+    b, hk, d = 2, 4, 64
+    rows = torch.randn(2, b, (hops + 1) * s, hk, d).bfloat16()
+    prev = [rows[:, :, (hops - i) * s:(hops - i + 1) * s] for i in range(1, hops + 1)]
+    k, v = rows[:, :, hops * s:]
+    plan = RS.plan_nonvarlen(s, window, hops + 2, hops)
+    reach = RS._reach(plan, s, window)
+    kk, vv = RS._join_keys(k, v, prev, plan, reach)
+    assert kk.shape[1] == reach + s == min(window, hops * s) + s
+    assert torch.equal(kk, rows[0, :, -kk.shape[1]:]) and torch.equal(vv, rows[1, :, -kk.shape[1]:])

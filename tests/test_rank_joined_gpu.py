@@ -1,5 +1,6 @@
 """A rank step whose window reaches over several earlier chunks, or over one whose size the two-range
-pass does not take, runs as one band over the joined keys.  All ranks' shares against the oracle on
+pass does not take, runs as one band over the joined keys (large steps of two blocks: block by block, so
+that route runs here, too).  All ranks' shares against the oracle on
 the whole sequence (out <= 2e-2 max-abs, gradients <= 1e-2 relative norm), odd chunk sizes, windows at
 and around multiples of a chunk, batch 2, a pack whose sequences start anywhere, and held chunks
 beyond the window's reach, whose gradient is zero."""
@@ -18,9 +19,15 @@ def _rel(x, ref):
 
 @pytest.mark.parametrize("s,w", [(100, 30), (100, 100), (100, 101), (193, 400), (64, 1000), (256, 511)])
 @pytest.mark.parametrize("packed", [False, True], ids=["dense", "packed"])
-def test_shares_on_joined_keys_match_the_oracle(s, w, packed):
+@pytest.mark.parametrize("route", ["joined", "blocks"])
+def test_shares_on_joined_keys_match_the_oracle(monkeypatch, s, w, packed, route):
     import ring_swa
+    from ring_swa import rank_share
 
+    joined, real = [], rank_share._join_keys
+    monkeypatch.setattr(rank_share, "_join_keys", lambda *a: joined.append(1) or real(*a))
+    if route == "blocks":
+        monkeypatch.setattr(rank_share, "_joinable", lambda *a: False)
     hq, hk, d, total = 4, 2, 64, s * CP
     b = 1 if packed else 2
     cu = [0, s // 2, s // 2 + 1, 2 * s + 7, total]
@@ -62,6 +69,7 @@ def test_shares_on_joined_keys_match_the_oracle(s, w, packed):
             if (i - 1) * s >= w:
                 assert not p.any()
     assert (torch.cat(outs, 1) - ro).abs().max().item() <= 2e-2
+    assert bool(joined) == (route == "joined")
     errs = [_rel(torch.cat(dqs, 1), rq), _rel(dk, rk), _rel(dv, rv)]
     assert max(errs) <= 1e-2, f"dq / dk / dv relative norm {errs}"
 
