@@ -225,3 +225,22 @@ def test_form_of_the_dkdv_blocks_can_be_chosen():
             assert L.rswa_attn_bwd_dkdv_keys(p) == keys
     p.head_dim = 96
     assert L.rswa_attn_bwd_dkdv_keys(p) < 0
+
+
+@pytest.mark.parametrize("tokens,heads,d,window,sequences,keys", [
+    (7428, 12, 128, 64, 1, 256), (20873, 4, 128, 211, 1, 256), (31427, 4, 128, 715, 11, 256),
+    (3010, 32, 128, 2028, 15, 256),             # more than a round of 256-key blocks
+    (4070, 4, 128, 925, 1, 64), (4091, 8, 128, 4096, 3, 64), (1402, 32, 128, 810, 1, 64),   # less
+])
+def test_without_grouped_heads_short_blocks_stay_below_one_round(tokens, heads, d, window, sequences, keys):
+    """With as many kv heads as q heads the 64-key form has only query tiles to share out, and a launch of
+    more than 256 blocks of 256 keys loses by it (these shapes were timed in both forms)."""
+    _ensure_built()
+    from ring_swa import _lib
+
+    p = _fake_params(tokens, heads, heads, d)
+    p.window_left = window
+    if sequences > 1:
+        p.batch, p.total_q, p.total_k = sequences, tokens, tokens
+        p.cu_seqlens_q = p.cu_seqlens_k = 4096
+    assert _lib.lib().rswa_attn_bwd_dkdv_keys(p) == keys
