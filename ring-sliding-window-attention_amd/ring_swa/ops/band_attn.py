@@ -217,6 +217,7 @@ def attn_bwd(
     second: Optional[Tuple[torch.Tensor, torch.Tensor, torch.Tensor, torch.Tensor]] = None,
     handoff=None,
     dkv_accumulate: bool = False,
+    dkdv_form: Optional[str] = None,
 ) -> None:
     """Masked attention backward; overwrites ``dq, dk, dv`` (views are fine).
 
@@ -245,7 +246,11 @@ def attn_bwd(
     (shapes the library does not accept still take the recomputing route); ``False`` never.  With
     ``phases`` spread over several calls the same value must be passed to each, on the same
     workspace, and the dK/dV phase must run before the dQ phase.  A ``workspace`` the caller
-    supplies without room for the dS tiles makes the automatic choice (``None``) recompute."""
+    supplies without room for the dS tiles makes the automatic choice (``None``) recompute.
+
+    ``dkdv_form``: ``"wide"`` or ``"short"`` blocks (256 or 64 keys) of the dK/dV kernel whatever the
+    sizes; ``None`` picks by an estimate that takes the launch to have the chip to itself.  The
+    environment's ``RSWA_DKDV_FORM`` comes first."""
     packed = cu_seqlens_q is not None
     _check_qkv(q, k, v, packed)
     assert second is None or k.numel() > 0, "two key ranges: the first must not be empty"
@@ -288,7 +293,7 @@ def attn_bwd(
         p.dk2, p.dv2 = dk2.data_ptr(), dv2.data_ptr()
     p.dq_accumulate = int(bool(dq_accumulate))
     # RSWA_DKDV_FORM=wide / short: the dK/dV kernel's blocks of 256 / of 64 keys whatever the sizes
-    form = os.environ.get("RSWA_DKDV_FORM", "")
+    form = os.environ.get("RSWA_DKDV_FORM", "") or dkdv_form
     if form:
         p.dkdv_form = _lib.DKDV_FORMS[form]
     p.dkv_accumulate = int(bool(dkv_accumulate))

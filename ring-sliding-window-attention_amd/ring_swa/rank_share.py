@@ -537,6 +537,22 @@ def _backward_one_pass(q, k, v, prev_kv, out, lse, do, one, scale):
     return (dq, dk, dv, *dprev)
 
 
+def _two_block_forms(s, prev_rows, batch, heads_q, heads_kv, window):
+    """Blocks of the two dK/dV launches of ``_backward_two_blocks`` (``dkdv_form`` of ``attn_bwd``): the
+    own chunk's, the other's.  The library's estimate takes a launch to be alone and splits blocks
+    that would leave compute units idle; here the other launch fills them, and the 256-key blocks'
+    cheaper steps win (us, estimate's choice / this one, backward of 32 / 8 heads: 8192 tokens, window
+    4096, 1635 / 1564; 7000, 5000, 1784 / 1719; 10000, 5000, 2552 / 2393; without grouped heads, where
+    a wide walk is a quarter as long, also with fewer own blocks: 8 / 8 heads, 7379 tokens, window 6641,
+    751 / 672).  Launches of even blocks beyond one round stay with the estimate: 12000 tokens,
+    window 3000, 1869 / 1973."""
+    own = batch * heads_kv * -(-s // 256)
+    if heads_q == heads_kv:
+        wide = own + batch * heads_kv * -(-prev_rows // 256) >= 200
+        return ("wide", "wide") if wide else (None, None)
+    return "wide" if own >= 200 and (own <= 256 or window >= 0.4 * s) else None, None
+
+
 def _backward_two_blocks(q, k, v, kv1, dkv1, out, lse, do, plan, scale, local_cu, wide=False,
                          after_rest=None):
     """Own-chunk block + one block on another rank's key range ``kv1`` (stacked, already sliced;
@@ -576,20 +592,24 @@ def _backward_two_blocks(q, k, v, kv1, dkv1, out, lse, do, plan, scale, local_cu
         need = bwd_workspace_bytes(q, k)
     ws = torch.empty(need, dtype=torch.uint8, device=q.device)
     ws_prev = torch.empty(bwd_workspace_bytes(q[:, qs], kv1[0]), dtype=torch.uint8, device=q.device)
+    form_own = form_prev = None
+    if local_cu is None or local_cu.numel() == 2:  # one sequence: its tiles are known here
+        form_own, form_prev = _two_block_forms(q.shape[1], kv1[0].shape[1], q.shape[0], q.shape[2], k.shape[2],
+                                               window0[0])
 
     def own(phases, accumulate):
         if local_cu is not None:
             attn_bwd(q[0], k[0], v[0], out[0], lse[0], do[0], dq[0], dk[0], dv[0], scale, window0,
                      causal0, local_cu, local_cu, workspace=ws, phases=phases,
-                     dq_accumulate=accumulate, handoff=False)
+                     dq_accumulate=accumulate, handoff=False, dkdv_form=form_own)
         else:
             attn_bwd(q, k, v, out, lse, do, dq, dk, dv, scale, window0, causal0, workspace=ws,
-                     phases=phases, dq_accumulate=accumulate, handoff=False)
+                     phases=phases, dq_accumulate=accumulate, handoff=False, dkdv_form=form_own)
 
     def prev(phases):
         attn_bwd(q[:, qs], kv1[0], kv1[1], out[:, qs], lse[:, :, qs], do[:, qs], dq[:, qs],
                  dkv1[0], dkv1[1], scale, window1, causal1, workspace=ws_prev,
-                 phases=phases, dq_accumulate=False, handoff=False)
+                 phases=phases, dq_accumulate=False, handoff=False, dkdv_form=form_prev)
 
     side = _fork(q.device)
     with torch.cuda.stream(side):

@@ -101,3 +101,16 @@ def test_signatures_match_upstream_order():
         params = [n for n, p in inspect.signature(fn).parameters.items()
                   if p.kind is p.POSITIONAL_OR_KEYWORD]
         assert params == base + extra + cp, fn.__name__
+
+
+def test_forms_of_the_two_dkdv_launches_of_a_step():
+    """Side by side: 256-key blocks once the own chunk has about a round of them (beyond it, where
+    their lengths vary), without grouped heads once both have; shapes timed in all forms."""
+    for (s, prev, hq, hk, w), forms in (((8192, 4096, 32, 8, 4096), ("wide", None)),
+                                        ((10000, 5000, 32, 8, 5000), ("wide", None)),
+                                        ((12000, 3000, 32, 8, 3000), (None, None)),
+                                        ((4096, 2048, 32, 8, 2048), (None, None)),
+                                        ((8192, 4096, 28, 4, 4096), (None, None)),
+                                        ((7379, 7379, 4, 4, 11068), ("wide", "wide")),
+                                        ((5000, 4500, 4, 4, 4500), (None, None))):
+        assert RS._two_block_forms(s, prev, 1, hq, hk, w) == forms
