@@ -26,7 +26,7 @@ static bool handoff_eligible(const rswa_attn_params* p) {
   return true;
 }
 
-BwdLayout bwd_layout(const rswa_attn_params* p, bool allow_handoff, uint64_t max_bytes) {
+static BwdLayout layout_of(const rswa_attn_params* p, bool allow_handoff, bool ktile_table) {
   BwdLayout L{};
   if (!p || p->batch <= 0 || p->heads_q <= 0 || p->heads_kv <= 0 || p->head_dim <= 0) return L;
   L.stats_bytes = delta_bytes(p);
@@ -47,13 +47,9 @@ BwdLayout bwd_layout(const rswa_attn_params* p, bool allow_handoff, uint64_t max
   L.sink_off = L.count_off + align_up((uint64_t)L.n_count * sizeof(int32_t), 256);
   L.total_bytes = L.sink_off + (uint64_t)sink_units * L.sink_chunks * p->num_sink * 2 * p->head_dim *
                                    sizeof(float);
-  if (packed) {
-    const uint64_t off = align_up(L.total_bytes, 256);
-    const uint64_t end = off + ((uint64_t)p->batch + 2) * sizeof(int32_t);
-    if (end <= max_bytes) {
-      L.ktile_off = off;
-      L.total_bytes = end;
-    }
+  if (packed && ktile_table) {
+    L.ktile_off = align_up(L.total_bytes, 256);
+    L.total_bytes = L.ktile_off + ((uint64_t)p->batch + 2) * sizeof(int32_t);
   }
   // dS hand-off: one 4 KiB unit per (q head, 32-row tile slot, 256-key block modulo nkb, 64-key
   // group).  A row tile sees keys [i0 + shift - left, i0 + 31 + shift + right]: left + right + 32
@@ -81,6 +77,11 @@ BwdLayout bwd_layout(const rswa_attn_params* p, bool allow_handoff, uint64_t max
     }
   }
   return L;
+}
+
+BwdLayout bwd_layout(const rswa_attn_params* p, bool allow_handoff, uint64_t max_bytes) {
+  const BwdLayout L = layout_of(p, allow_handoff, true);
+  return L.total_bytes <= max_bytes ? L : layout_of(p, allow_handoff, false);
 }
 
 uint64_t bwd_workspace_bytes(const rswa_attn_params* p) { return bwd_layout(p, true).total_bytes; }
@@ -311,6 +312,10 @@ int fill_args(const rswa_attn_params* p, bool backward, AttnArgs& a, bool allow_
 
 extern "C" uint64_t rswa_attn_bwd_workspace_bytes(const rswa_attn_params* p) {
   return rswa::bwd_workspace_bytes(p);
+}
+
+extern "C" uint64_t rswa_attn_bwd_workspace_min_bytes(const rswa_attn_params* p) {
+  return rswa::bwd_layout(p, true, 0).total_bytes;
 }
 
 extern "C" int rswa_attn_bwd_handoff_active(const rswa_attn_params* p) {

@@ -1952,7 +1952,7 @@ int launch_bwd(AttnArgs& a, hipStream_t stream, int phases) {
 namespace rswa {
 namespace {
 int bwd_entry(const rswa_attn_params* p, void* stream, int phases, bool allow_handoff,
-              uint64_t max_bytes = ~0ull) {
+              uint64_t max_bytes) {
   AttnArgs a;
   int rc = fill_args(p, true, a, allow_handoff, max_bytes);
   if (rc != RSWA_OK) return rc;
@@ -1968,7 +1968,7 @@ int bwd_entry(const rswa_attn_params* p, void* stream, int phases, bool allow_ha
 }  // namespace rswa
 
 extern "C" int rswa_attn_bwd_phases(const rswa_attn_params* p, void* stream, int phases) {
-  return rswa::bwd_entry(p, stream, phases, true);
+  return rswa::bwd_entry(p, stream, phases, true, p ? p->workspace_bytes : 0);
 }
 
 extern "C" int rswa_attn_bwd_dkdv_keys(const rswa_attn_params* p) {

@@ -136,6 +136,8 @@ def load(path: str) -> ctypes.CDLL:
     L.rswa_attn_bwd_phases.argtypes = [POINTER(AttnParams), c_void_p, c_int]
     L.rswa_attn_bwd_workspace_bytes.restype = c_uint64
     L.rswa_attn_bwd_workspace_bytes.argtypes = [POINTER(AttnParams)]
+    L.rswa_attn_bwd_workspace_min_bytes.restype = c_uint64
+    L.rswa_attn_bwd_workspace_min_bytes.argtypes = [POINTER(AttnParams)]
     L.rswa_attn_bwd_handoff_active.restype = c_int
     L.rswa_attn_bwd_handoff_active.argtypes = [POINTER(AttnParams)]
     L.rswa_attn_bwd_dkdv_keys.restype = c_int

@@ -224,10 +224,10 @@ def attn_bwd(
     ``second=(k2, v2, dk2, dv2)``: keys in two row ranges as in ``attn_fwd``; the gradients of
     the second range's rows go to ``dk2, dv2`` (shapes and strides of ``k2, v2``).
 
-    ``workspace`` (uint8, at least ``bwd_workspace_bytes(q, k, ...)``) may be supplied to avoid the
-    per-call scratch allocation, and must be when the phases of one backward are spread
-    over several calls; ``phases`` is the bit mask of ``rswa_attn_bwd_phases`` (1 prep,
-    2 dk/dv kernel, 4 dq kernel).  ``dq_accumulate`` adds this call's dQ to the values
+    ``workspace`` (uint8, ``bwd_workspace_bytes(q, k, ...)`` of it; packs also take one without room
+    for the key tile table) may be supplied to avoid the per-call scratch allocation, and must be
+    when the phases of one backward are spread over several calls; ``phases`` is the bit mask of
+    ``rswa_attn_bwd_phases`` (1 prep, 2 dk/dv kernel, 4 dq kernel).  ``dq_accumulate`` adds this call's dQ to the values
     already in ``dq`` (fp32 add of the two 16-bit values, one rounding).
     ``static_workspace=True`` runs the whole backward on the library's built-in statistics
     buffer (``rswa_attn_bwd_static``): no device memory is allocated by the call; sizes
@@ -314,18 +314,19 @@ def attn_bwd(
         _lib.launch(dev, L.rswa_attn_bwd_static, p)
         return
     _set_handoff(p, handoff)
-    need = int(L.rswa_attn_bwd_workspace_bytes(p))
-    if workspace is not None and handoff is None and p.ds_handoff and workspace.numel() < need:
-        # a caller's workspace without room for the dS tiles: the automatic choice recomputes
-        p.ds_handoff = 0
-        need = int(L.rswa_attn_bwd_workspace_bytes(p))
     if workspace is None:
-        workspace = q.new_empty(need, dtype=torch.uint8)  # 512-B aligned by torch
-    assert workspace.dtype == torch.uint8 and workspace.device == dev
-    assert workspace.numel() >= need, (
-        f"workspace of {workspace.numel()} bytes, {need} needed: size it with bwd_workspace_bytes "
-        "and the mask / num_sink / handoff of this call"
-    )
+        workspace = q.new_empty(int(L.rswa_attn_bwd_workspace_bytes(p)), dtype=torch.uint8)  # 512-B aligned by torch
+    else:
+        least = int(L.rswa_attn_bwd_workspace_min_bytes(p))
+        if handoff is None and p.ds_handoff and workspace.numel() < least:
+            # a caller's workspace without room for the dS tiles: the automatic choice recomputes
+            p.ds_handoff = 0
+            least = int(L.rswa_attn_bwd_workspace_min_bytes(p))
+        assert workspace.dtype == torch.uint8 and workspace.device == dev
+        assert workspace.numel() >= least, (
+            f"workspace of {workspace.numel()} bytes, {least} needed: size it with bwd_workspace_bytes "
+            "and the mask / num_sink / handoff of this call"
+        )
     p.workspace = workspace.data_ptr()
     p.workspace_bytes = workspace.numel()
     _lib.launch(dev, L.rswa_attn_bwd_phases, p, int(phases))

@@ -244,3 +244,28 @@ def test_without_grouped_heads_short_blocks_stay_below_one_round(tokens, heads, 
         p.batch, p.total_q, p.total_k = sequences, tokens, tokens
         p.cu_seqlens_q = p.cu_seqlens_k = 4096
     assert _lib.lib().rswa_attn_bwd_dkdv_keys(p) == keys
+
+
+def test_workspace_without_the_key_tile_table_is_accepted():
+    """A pack's table only saves time: a workspace of the two statistics arrays is enough (phases = 0:
+    all checks, no launch), one byte less is not."""
+    _ensure_built()
+    from ring_swa import _lib
+
+    L = _lib.lib()
+    p = _fake_params(1000)
+    p.batch, p.total_q, p.total_k = 7, 1000, 1000
+    p.cu_seqlens_q = p.cu_seqlens_k = 4096
+    stats = 2 * (-(-1000 * 32 * 4 // 256) * 256)
+    assert L.rswa_attn_bwd_workspace_min_bytes(p) == stats < L.rswa_attn_bwd_workspace_bytes(p)
+    p.workspace_bytes = stats
+    assert L.rswa_attn_bwd_phases(p, None, 0) == 0
+    p.workspace_bytes = stats - 1
+    assert L.rswa_attn_bwd_phases(p, None, 0) == -1 and b"workspace" in L.rswa_last_error()
+    # with the dS tiles behind: room for them alone is enough, too
+    p.ds_handoff = 1
+    least = L.rswa_attn_bwd_workspace_min_bytes(p)
+    assert stats < least <= L.rswa_attn_bwd_workspace_bytes(p)
+    for room, rc in ((least, 0), (least - 1, -1)):
+        p.workspace_bytes = room
+        assert L.rswa_attn_bwd_phases(p, None, 0) == rc

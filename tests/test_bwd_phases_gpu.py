@@ -42,3 +42,28 @@ def test_dkdv_launch_makes_its_own_key_tile_table(monkeypatch, form, prep):
         results.append(grads[1:])
     for one, two in zip(*results):
         assert torch.equal(one, two)
+
+
+@pytest.mark.parametrize("form", ["wide", "short"])
+@pytest.mark.parametrize("sinks", [0, 2])
+def test_pack_without_room_for_the_table_gets_the_same_bits(monkeypatch, form, sinks):
+    from ring_swa.ops.band_attn import attn_bwd, attn_fwd, bwd_workspace_bytes
+
+    cu = [0, 300, 300, 301, 901, 1500]
+    hq, hk, d, w = 4, 2, 128, 100
+    gen = torch.Generator(device="cuda").manual_seed(4)
+    q, do = (torch.randn(cu[-1], hq, d, device="cuda", dtype=torch.bfloat16, generator=gen) for _ in range(2))
+    k, v = (torch.randn(cu[-1], hk, d, device="cuda", dtype=torch.bfloat16, generator=gen) for _ in range(2))
+    cu_t = torch.tensor(cu, dtype=torch.int32, device="cuda")
+    out, lse = attn_fwd(q, k, v, None, (w, 0), True, cu_t, cu_t, num_sink=sinks)
+    monkeypatch.setenv("RSWA_DKDV_FORM", form)
+    need = bwd_workspace_bytes(q, k, cu_t, cu_t, window_size=(w, 0), causal=True, num_sink=sinks)
+    table = (len(cu) + 1) * 4  # the last thing in it
+    results = []
+    for room in (need, need - table):
+        ws = torch.full((room,), 0xff, dtype=torch.uint8, device="cuda")
+        grads = [torch.zeros_like(t) for t in (q, k, v)]
+        attn_bwd(q, k, v, out, lse, do, *grads, None, (w, 0), True, cu_t, cu_t, num_sink=sinks, workspace=ws)
+        results.append(grads)
+    for one, two in zip(*results):
+        assert torch.equal(one, two)
