@@ -257,6 +257,8 @@ typedef struct rswa_attn_params {
 #define RSWA_DKDV_SHORT 2
 
 int rswa_attn_fwd(const rswa_attn_params* p, void* stream);
+/* Outputs must not share memory with inputs or with each other, except that dq may lie over q, out or
+ * dout, with that tensor's strides. */
 int rswa_attn_bwd(const rswa_attn_params* p, void* stream);
 
 /*

@@ -86,6 +86,42 @@ BwdLayout bwd_layout(const rswa_attn_params* p, bool allow_handoff, uint64_t max
 
 uint64_t bwd_workspace_bytes(const rswa_attn_params* p) { return bwd_layout(p, true).total_bytes; }
 
+// Bytes from the first to behind the last element of a strided [batch, rows, heads, width] tensor
+// (strides in elements, of any sign).  Nothing in an empty one.
+struct Span {
+  const char *lo, *hi;
+};
+static Span span_of(const void* ptr, const int64_t* st, int64_t batch, int64_t rows, int64_t heads, int64_t width,
+                    int elem_bytes) {
+  const char* base = (const char*)ptr;
+  if (!ptr || batch <= 0 || rows <= 0 || heads <= 0) return {base, base};
+  int64_t lo = 0, hi = width;
+  const int64_t ext[3] = {(batch - 1) * st[0], (rows - 1) * st[1], (heads - 1) * st[2]};
+  for (int64_t e : ext) (e < 0 ? lo : hi) += e;
+  return {base + lo * elem_bytes, base + hi * elem_bytes};
+}
+
+// Does dq share memory with anything that the dK/dV kernel or another row's statistics read?
+static bool dq_overlays_inputs(const rswa_attn_params* p, const AttnArgs& a) {
+  const bool packed = a.cu_q != nullptr;
+  const int64_t nb = packed ? 1 : a.batch, rq = packed ? a.rows_q : a.seqlen_q, rk = packed ? a.rows_k : a.seqlen_k;
+  const int64_t rk1 = std::min<int64_t>(rk, a.seg), rk2 = rk - rk1;
+  const int d = p->head_dim;
+  const Span dq = span_of(p->dq, a.dq_st, nb, rq, a.heads_q, d, a.wide_dq ? 4 : 2);
+  const int64_t lse_st[3] = {a.lse_st[0], a.lse_st[2], a.lse_st[1]};
+  const Span in[] = {span_of(p->q, a.q_st, nb, rq, a.heads_q, d, 2),
+                     span_of(p->out, a.o_st, nb, rq, a.heads_q, d, 2),
+                     span_of(p->dout, a.do_st, nb, rq, a.heads_q, d, 2),
+                     span_of(p->lse, lse_st, nb, rq, a.heads_q, 1, 4),
+                     span_of(p->k, a.k_st, nb, rk1, a.heads_kv, d, 2),
+                     span_of(p->v, a.v_st, nb, rk1, a.heads_kv, d, 2),
+                     span_of(a.k2, a.k_st, nb, rk2, a.heads_kv, d, 2),
+                     span_of(a.v2, a.v_st, nb, rk2, a.heads_kv, d, 2)};
+  for (const Span& x : in)
+    if (x.lo < dq.hi && dq.lo < x.hi) return true;
+  return false;
+}
+
 static bool rows_aligned(const void* ptr, const int64_t* st, int elem_bytes = 2) {
   if (((uintptr_t)ptr) % 16) return false;
   for (int i = 0; i < 3; i++)
@@ -187,6 +223,7 @@ int fill_args(const rswa_attn_params* p, bool backward, AttnArgs& a, bool allow_
   a.sink_part = nullptr;
   a.sink_count = nullptr;
   a.sink_chunks = 0;
+  a.dq_last = 0;
   a.ds = nullptr;
   a.ds_nkb = 0;
   a.ds_slots = 0;
@@ -299,6 +336,7 @@ int fill_args(const rswa_attn_params* p, bool backward, AttnArgs& a, bool allow_
       a.ds_nkb = L.ds_nkb;
       a.ds_slots = L.ds_slots;
     }
+    a.dq_last = dq_overlays_inputs(p, a);
     // one load reaches from a row's lse2 to its delta, one array further on
     RSWA_REQUIRE(delta_bytes(p) < (1ull << 31) - 65536, RSWA_ERR_UNSUPPORTED,
                  "attn_bwd: rows * heads_q = %lld: each statistics array must stay below 2 GiB "

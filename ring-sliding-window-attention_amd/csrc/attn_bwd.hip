@@ -1863,8 +1863,9 @@ int launch_bwd(AttnArgs& a, hipStream_t stream, int phases) {
   };
   // Statistics and dQ asked for in one call: the dQ kernel goes first and makes the statistics.
   // (dS hand-off: dQ needs the dK/dV kernel's tiles, so the statistics have a kernel of their own;
-  // so they have where the dQ kernel would spill, in the second addressing form.)
-  const bool fused = units > 0 && (phases & RSWA_BWD_PREP) && (phases & RSWA_BWD_DQ) && !a.ds && !a.far;
+  // so they have where the dQ kernel would spill, in the second addressing form, and where dq lies
+  // over an input, which dK/dV have to read before it is written.)
+  const bool fused = units > 0 && (phases & RSWA_BWD_PREP) && (phases & RSWA_BWD_DQ) && !a.ds && !a.far && !a.dq_last;
   if (fused) {
     if (a.cu_q || a.n_count > 0) {
       clear_launch_error();

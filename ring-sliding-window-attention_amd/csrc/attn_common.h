@@ -41,6 +41,7 @@ struct AttnArgs {
   int32_t* ktile;
   int32_t ktile_log2;
   int32_t dkdv_form;  // RSWA_DKDV_*: the caller's choice of the dK/dV kernel's blocks
+  int32_t dq_last;  // dq lies over an input: the dQ kernel must not run before dK/dV (host only)
   int32_t snake;    // dK/dV: see the kernel (dense; of a pack the device decides)
   const int32_t* cu_q;
   const int32_t* cu_k;

@@ -67,3 +67,25 @@ def test_pack_without_room_for_the_table_gets_the_same_bits(monkeypatch, form, s
         results.append(grads)
     for one, two in zip(*results):
         assert torch.equal(one, two)
+
+
+@pytest.mark.parametrize("over", ["q", "out", "dout"])
+@pytest.mark.parametrize("hq,hk,d,cu", [(4, 4, 64, None), (6, 2, 128, None), (4, 2, 128, [0, 130, 200, 700])])
+def test_dq_over_an_input_gets_the_same_bits(over, hq, hk, d, cu):
+    """The dQ kernel, which otherwise goes first, then runs behind the dK/dV kernel."""
+    from ring_swa.ops.band_attn import attn_bwd, attn_fwd
+
+    s, w = 700, 150
+    lead = (s,) if cu else (2, s)
+    gen = torch.Generator(device="cuda").manual_seed(6)
+    q, do = (torch.randn(*lead, hq, d, device="cuda", dtype=torch.bfloat16, generator=gen) for _ in range(2))
+    k, v = (torch.randn(*lead, hk, d, device="cuda", dtype=torch.bfloat16, generator=gen) for _ in range(2))
+    cu_t = torch.tensor(cu, dtype=torch.int32, device="cuda") if cu else None
+    out, lse = attn_fwd(q, k, v, None, (w, 0), True, cu_t, cu_t)
+    apart = [torch.empty_like(t) for t in (q, k, v)]
+    attn_bwd(q, k, v, out, lse, do, *apart, None, (w, 0), True, cu_t, cu_t)
+    dq = {"q": q, "out": out, "dout": do}[over]
+    dk, dv = torch.empty_like(k), torch.empty_like(v)
+    attn_bwd(q, k, v, out, lse, do, dq, dk, dv, None, (w, 0), True, cu_t, cu_t)
+    for one, two in zip(apart, (dq, dk, dv)):
+        assert torch.equal(one, two)
