@@ -10,8 +10,10 @@ import concurrent.futures as cf
 import os
 import re
 import shutil
+import struct
 import subprocess
 import sys
+import tempfile
 from typing import List
 
 HERE = os.path.dirname(os.path.abspath(__file__))
@@ -22,7 +24,7 @@ LIB = os.path.join(LIBDIR, "librswa.so")
 # the same library with every MFMA issued through the compiler builtin (hazards padded by the
 # compiler): the cross-check of the hand-kept hazard distance of the inline-assembly MFMAs
 LIB_BUILTIN_MFMA = os.path.join(LIBDIR, "librswa_builtin_mfma.so")
-ASM_MFMA_SOURCES = ("attn_bwd.hip",)  # sources that issue MFMAs as inline assembly
+ASM_MFMA_SOURCES = ("attn_bwd.hip",)  # sources that issue MFMAs, and loads into LDS, as inline assembly
 
 ARCH = "gfx950"
 FLAGS = [
@@ -116,6 +118,93 @@ def _check_no_scratch(src: str, stderr: str) -> None:
         raise RuntimeError(f"{src}: kernels spill registers to scratch memory:\n  " + "\n  ".join(bad))
 
 
+def _code_objects(fat: bytes):
+    """The code objects for ARCH in a fatbin section (bundles one behind the other)."""
+    magic = b"__CLANG_OFFLOAD_BUNDLE__"
+    at = fat.find(magic)
+    while at >= 0:
+        (count,) = struct.unpack_from("<Q", fat, at + 24)
+        p = at + 32
+        for _ in range(count):
+            off, size, n = struct.unpack_from("<QQQ", fat, p)
+            if ARCH.encode() in fat[p + 24:p + 24 + n] and size:
+                yield fat[at + off:at + off + size]
+            p += 24 + n
+        at = fat.find(magic, at + 24)
+
+
+_LDS_LOAD_WAIT = 5  # wait states from a vector instruction's write of an SGPR to its use by a memory instruction
+
+
+def _sgprs(operand: str) -> set:
+    m = re.fullmatch(r"s\[(\d+):(\d+)\]|s(\d+)", operand)
+    if not m:
+        return {operand} & {"m0"}
+    return set(range(int(m[1]), int(m[2]) + 1)) if m[1] else {int(m[3])}
+
+
+def close_sgpr_writes(listing: List[str]) -> List[str]:
+    """Loads into LDS of one kernel (disassembled, branch targets as ``<L0>:`` lines) that a vector
+    instruction's write of one of their scalar registers comes too close to, along any path: the
+    hand-written ones are invisible to the compiler's hazard pass."""
+    code = [line.split("//")[0].split(";")[0].strip() for line in listing]
+    jumps = {}
+    for i, x in enumerate(code):
+        m = re.match(r"s_c?branch\S* (\S+)$", x)
+        if m:
+            jumps.setdefault(m[1].strip("<>"), []).append(i)
+    bad = []
+
+    def writer(i: int, left: int, used: set, load: str):
+        """Walk back from line i (not included) with ``left`` wait states to go."""
+        while left > 0 and i > 0:
+            i -= 1
+            x = code[i]
+            label = re.fullmatch(r"(?:[0-9a-f]+ )?<(L\d+)>:", x)
+            if label:
+                for j in jumps.get(label[1], ()):
+                    writer(j, left - 1, used, load)
+                continue
+            if not x:
+                continue
+            if x.startswith(("s_branch", "s_endpgm", "s_setpc")):
+                return  # not reached from here
+            name, _, rest = x.partition(" ")
+            if name.startswith("v_"):
+                ops = [o.strip() for o in rest.split(",")]
+                out = ops[:2] if "_co_" in name or "div_scale" in name else ops[:1]
+                if any(_sgprs(o) & used for o in out):
+                    bad.append(f"{x}  ...  {load}")
+                    return
+            left -= int(rest) + 1 if name == "s_nop" else 1
+
+    for i, x in enumerate(code):
+        if x.startswith("buffer_load") and x.endswith(" lds"):
+            ops = [o.strip() for o in x.partition(" ")[2].replace(" offen", ",").split(",")]
+            writer(i, _LDS_LOAD_WAIT, set().union({"m0"}, *(_sgprs(o) for o in ops)), x)
+    return bad
+
+
+def _check_lds_loads(obj: str) -> None:
+    """No load into LDS may follow a vector instruction's write of its scalar registers too closely."""
+    llvm = os.path.join(os.path.dirname(os.path.realpath(_hipcc())), "..", "llvm", "bin")
+    with tempfile.TemporaryDirectory() as tmp:
+        fat = os.path.join(tmp, "fat")
+        subprocess.run([os.path.join(llvm, "llvm-objcopy"), "--dump-section", ".hip_fatbin=" + fat, obj, os.devnull],
+                       check=True)
+        for i, code in enumerate(_code_objects(open(fat, "rb").read())):
+            path = os.path.join(tmp, f"{i}.co")
+            with open(path, "wb") as f:
+                f.write(code)
+            text = subprocess.run([os.path.join(llvm, "llvm-objdump"), "-d", "--no-show-raw-insn",
+                                   "--symbolize-operands", path], check=True, capture_output=True, text=True).stdout
+            for name, body in re.findall(r"^[0-9a-f]+ <(_Z\w+)>:\n(.*?)(?=^[0-9a-f]+ <_Z|\Z)", text, re.M | re.S):
+                bad = close_sgpr_writes(body.splitlines())
+                if bad:
+                    raise RuntimeError(f"{name}: scalar registers written too close to a load into LDS:\n  "
+                                       + "\n  ".join(bad))
+
+
 def build(force: bool = False, jobs: int = 8) -> str:
     os.makedirs(OBJ, exist_ok=True)
     os.makedirs(LIBDIR, exist_ok=True)
@@ -126,6 +215,9 @@ def build(force: bool = False, jobs: int = 8) -> str:
         alt_futs = {s: ex.submit(_compile, s, force, True) for s in asm_srcs}
         objs = [f.result() for f in futs]
         alt = {s: f.result() for s, f in alt_futs.items()}
+    for o in objs:
+        if os.path.basename(o)[:-2] + ".hip" in ASM_MFMA_SOURCES and (force or _stale(LIB, [o])):
+            _check_lds_loads(o)
     alt_objs = [alt.get(s, o) for s, o in zip(srcs, objs)]
     for lib, members in ((LIB, objs), (LIB_BUILTIN_MFMA, alt_objs)):
         if force or _stale(lib, members):

@@ -450,16 +450,19 @@ __device__ __forceinline__ u32x4 tile_words(const void* base, int row0, int rows
 // compiler does not see it write LDS and so never waits for it on its own -- the caller waits
 // (wait_dma) before it reads what was loaded.  For tile buffers picked at run time, which the
 // compiler cannot tell apart: with the builtin it would wait for the load in flight before every
-// LDS read.  (One wait state between the write of m0 and its use.)
+// LDS read.  The compiler sets m0 and knows of it; its hazard pass does not look inside.  The wait
+// state behind the write of m0 is here; the five between a vector instruction's write of a scalar
+// register (what a spilled one comes back by) and its use by the load are not (they cost the short
+// dK/dV form 2.8 % over 119 shapes): the build fails where one comes closer (build.py).
 template <int BYTES>
 __device__ __forceinline__ void lds_load_asm(u32x4 rsrc, int voff, int soff, uint32_t lds) {
   static_assert(BYTES == 4 || BYTES == 16, "one dword or four per lane");
   if constexpr (BYTES == 16) {
-    asm volatile("s_mov_b32 m0, %3\n\ts_nop 0\n\tbuffer_load_dwordx4 %0, %1, %2 offen lds"
-                 :: "v"(voff), "s"(rsrc), "s"(soff), "s"(lds) : "memory");
+    asm volatile("s_nop 0\n\tbuffer_load_dwordx4 %0, %1, %2 offen lds"
+                 :: "v"(voff), "s"(rsrc), "s"(soff), "{m0}"(lds) : "memory");
   } else {
-    asm volatile("s_mov_b32 m0, %3\n\ts_nop 0\n\tbuffer_load_dword %0, %1, %2 offen lds"
-                 :: "v"(voff), "s"(rsrc), "s"(soff), "s"(lds) : "memory");
+    asm volatile("s_nop 0\n\tbuffer_load_dword %0, %1, %2 offen lds"
+                 :: "v"(voff), "s"(rsrc), "s"(soff), "{m0}"(lds) : "memory");
   }
 }
 
