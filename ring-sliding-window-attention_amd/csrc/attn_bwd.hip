@@ -794,8 +794,8 @@ __global__ __launch_bounds__(256) void attn_bwd_dkdv_kernel(const AttnArgs a) {
 // sink keys; a lane owns 8 consecutive d of one row at a time (D / 8 lanes per row), the dot
 // products are summed across those lanes, and the block's sums -- added in a fixed order -- go
 // to the workspace as fp32 [unit][chunk][sink][dK, dV][D].  The block of a unit that arrives
-// last adds the chunks in chunk order and writes the rows (same protocol as the split dK/dV
-// blocks: deterministic, nobody waits).
+// last adds the chunks in chunk order and writes the rows (the same order whichever block that is, so
+// the result does not depend on timing, and nobody waits).
 constexpr int kSinkPass = 4;
 
 // sum over the aligned group of W = 8 or 16 lanes, in every lane of the group

@@ -75,16 +75,13 @@ def test_handoff_dense_matches_oracle_and_recompute(case, dtype):
         lambda q, k, v: O.window_attention(q, k, v, scale, window, causal, 0), q, k, v, do)
     qc, kc, vc, dc = q.cuda(), k.cuda(), v.cuda(), do.cuda()
     out, lse = attn_fwd(qc, kc, vc, scale, window, causal)
-    # ("force": these launches are small enough for the dK/dV kernel to split their key tiles
-    # over several blocks, which keeps the recomputing route unless the hand-off is preferred)
     (hq_, hk_, hv_), active = _bwd(qc, kc, vc, out, lse, dc, scale, window, causal, "force")
     assert active, "the route was expected to be taken"
     (bq, bk, bv), _ = _bwd(qc, kc, vc, out, lse, dc, scale, window, causal, False)
     errs = [relnorm(g, r) for g, r in ((hq_, rq), (hk_, rk), (hv_, rv))]
     assert max(errs) <= GRAD_TOL, f"rel-norm errors dq/dk/dv = {errs}"
-    # dK / dV: the same sums in the same order wherever the recomputing route did not split
-    if (sk + 255) // 256 * hk * b >= 129 or hq == hk:
-        assert torch.equal(hk_, bk) and torch.equal(hv_, bv), "dK / dV differ between the routes"
+    # dK / dV: the same sums in the same order
+    assert torch.equal(hk_, bk) and torch.equal(hv_, bv), "dK / dV differ between the routes"
     assert relnorm(hq_, bq.float().cpu()) <= 6e-3, "dQ of the two routes"
 
 
@@ -200,7 +197,7 @@ def test_automatic_choice_follows_the_workspace_it_is_given(monkeypatch):
     from ring_swa.ops import attn_fwd
     from ring_swa.ops.band_attn import attn_bwd, bwd_workspace_bytes
 
-    b, s, hq, hk, d, w = 1, 70000, 8, 8, 128, 300   # 274 key blocks x 8 heads: no split launch
+    b, s, hq, hk, d, w = 1, 70000, 8, 8, 128, 300   # 274 key blocks x 8 heads: 256-key blocks
     q, do = _rand((b, s, hq, d), torch.bfloat16, 1).cuda(), _rand((b, s, hq, d), torch.bfloat16, 4).cuda()
     k, v = _rand((b, s, hk, d), torch.bfloat16, 2).cuda(), _rand((b, s, hk, d), torch.bfloat16, 3).cuda()
     out, lse = attn_fwd(q, k, v, None, (w, 0), True)

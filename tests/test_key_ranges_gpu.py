@@ -17,7 +17,7 @@ CASES = [
     (1, 512, 256, 512, 4, 2, 128, (256, 0), True, torch.bfloat16),     # tail + own chunk, band
     (2, 300, 512, 300, 4, 4, 64, (200, 0), True, torch.bfloat16),      # ragged second range
     (1, 700, 256, 700, 8, 2, 128, (-1, -1), False, torch.float16),     # full attention
-    (1, 1024, 768, 1024, 8, 2, 128, (768, 0), True, torch.bfloat16),   # few key tiles: split dK/dV
+    (1, 1024, 768, 1024, 8, 2, 128, (768, 0), True, torch.bfloat16),   # few key tiles: 64-key blocks
     (1, 130, 256, 77, 2, 1, 64, (100, 30), False, torch.bfloat16),     # two-sided window
 ]
 

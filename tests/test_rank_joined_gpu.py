@@ -1,6 +1,6 @@
 """A rank step whose window reaches over several earlier chunks, or over one whose size the two-range
-pass does not take, runs as one band over the joined keys (large steps of two blocks: block by block, so
-that route runs here, too).  All ranks' shares against the oracle on
+pass does not take, runs as one band over the joined keys; large steps of two blocks run block by block,
+ring_dtypes in the ring's accumulators: those routes run here, too.  All ranks' shares against the oracle on
 the whole sequence (out <= 2e-2 max-abs, gradients <= 1e-2 relative norm), odd chunk sizes, windows at
 and around multiples of a chunk, batch 2, a pack whose sequences start anywhere, and held chunks
 beyond the window's reach, whose gradient is zero."""
@@ -19,7 +19,7 @@ def _rel(x, ref):
 
 @pytest.mark.parametrize("s,w", [(100, 30), (100, 100), (100, 101), (193, 400), (64, 1000), (256, 511)])
 @pytest.mark.parametrize("packed", [False, True], ids=["dense", "packed"])
-@pytest.mark.parametrize("route", ["joined", "blocks"])
+@pytest.mark.parametrize("route", ["joined", "blocks", "ring_dtypes"])
 def test_shares_on_joined_keys_match_the_oracle(monkeypatch, s, w, packed, route):
     import ring_swa
     from ring_swa import rank_share
@@ -50,10 +50,11 @@ def test_shares_on_joined_keys_match_the_oracle(monkeypatch, s, w, packed, route
         if packed:
             own, prev = [t[0] for t in own], [t[:, 0] for t in prev]
         own, prev = [t.requires_grad_() for t in own], [t.requires_grad_() for t in prev]
+        kw = dict(ring_dtypes=route == "ring_dtypes")
         if packed:
-            out = ring_swa.ring_rank_share_attn_varlen(*own, prev, w, cu, CP, r)
+            out = ring_swa.ring_rank_share_attn_varlen(*own, prev, w, cu, CP, r, **kw)
         else:
-            out = ring_swa.ring_rank_share_attn(*own, prev, w, CP, r)
+            out = ring_swa.ring_rank_share_attn(*own, prev, w, CP, r, **kw)
         grads = torch.autograd.grad(out, own + prev, do[:, sl].cuda() if not packed else do[0, sl].cuda())
         cpu = [x.float().cpu() for x in (out.detach(), *grads)]
         if packed:

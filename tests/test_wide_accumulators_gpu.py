@@ -20,7 +20,7 @@ CASES = [
     (1, 513, 700, 4, 4, 64, (64, 0), True, torch.float16),
     (1, 200, 456, 6, 2, 128, (0, 456), False, torch.bfloat16),   # a corner block of the ring
     (1, 333, 200, 4, 2, 128, (40, 0), True, torch.bfloat16),     # leading rows see nothing
-    (1, 2048, 40000, 2, 2, 128, (4000, 0), True, torch.bfloat16),  # 157 key tiles x 2 heads: no split
+    (1, 2048, 40000, 2, 2, 128, (4000, 0), True, torch.bfloat16),  # 157 key tiles x 2 heads: 256-key blocks
 ]
 
 
