@@ -182,7 +182,7 @@ def clock_probe(dev, qd, kd, vd, prev, do, S, W, seconds=4.0):
         band(7)
         kernels = [("attn_fwd_kernel", lambda: attn_fwd(qd, tk, tv, None, (W, 0), True, second=(kd, vd))),
                    ("attn_bwd_dkdv_kernel", lambda: band(2)),
-                   ("attn_bwd_dq_kernel", lambda: band(4)),
+                   ("attn_bwd_dq_kernel with the row statistics", lambda: band(1 | 4)),
                    ("device copy of 1 GiB", lambda: big2.copy_(big))]
         out = {}
         for name, fn in kernels:
@@ -328,9 +328,9 @@ def main():
     ap.add_argument("--clock-probe", action="store_true",
                     help="loop each kernel of the step's band for a few seconds and print the shader "
                          "clock rocm-smi reads meanwhile (one JSON line; no timing claims)")
-    ap.add_argument("--trace", choices=["c2", "c4", "c5"],
-                    help="kernel-trace pass: run only that configuration's step a few times "
-                         "(under rocprofv3 --kernel-trace --stats) and exit")
+    ap.add_argument("--trace",
+                    help="profiling pass: run only that configuration's step (c2, c4, c5, or the name of a "
+                         "case of perf/cases.py) a few times (under rocprofv3) and exit")
     args = ap.parse_args()
     if args.gpus != 1 or int(os.environ.get("WORLD_SIZE", "1")) != 1:
         sys.exit("bench.py: this build covers the single-GPU path only; run with --gpus 1 "
@@ -375,8 +375,13 @@ def main():
             steps = [lambda: (f2(), b2())]
         elif args.trace == "c4":
             steps = list(case_c4(dev)[:2])
-        else:
+        elif args.trace == "c5":
             steps = [case_c5(dev, "fused", 4)[0]]
+        else:
+            from perf import cases
+
+            state = cases.prepare(next(c for c in cases.listed() if c["name"] == args.trace), 0)
+            steps = [lambda: cases.run(state)]
         for fn in steps:
             for _ in range(args.steps):
                 fn()
@@ -494,8 +499,8 @@ def main():
         o_d, lse_d = attn_fwd(qd, kd, vd, None, (W, 0), True)
         dq, dk, dv = torch.empty_like(qd), torch.empty_like(kd), torch.empty_like(vd)
         ws = torch.empty(bwd_workspace_bytes(qd, kd), dtype=torch.uint8, device=dev)
-        bwd = lambda ph: attn_bwd(qd, kd, vd, o_d, lse_d, do, dq, dk, dv, None, (W, 0), True,  # noqa: E731
-                                  workspace=ws, phases=ph)
+        bwd = lambda ph, form=None: attn_bwd(qd, kd, vd, o_d, lse_d, do, dq, dk, dv, None, (W, 0), True,  # noqa: E731
+                                             workspace=ws, phases=ph, dkdv_form=form)
         bwd(7)
         n = 5 if args.no_extras else 20
         PREP, DKDV, DQ = 1, 2, 4
@@ -525,12 +530,14 @@ def main():
         if not args.no_extras:
             band_fwd, _ = event_ms(lambda: attn_fwd(qd, tk, tv, None, (W, 0), True,
                                                     second=(kd, vd)), 20)
-            band_dq, _ = event_ms(lambda: band(DQ), 20)
+            # (the step's dQ launch makes the row statistics; a kernel of their own they have where the
+            # phases are asked for one by one)
+            band_dq, _ = event_ms(lambda: band(PREP | DQ), 20)
+            band_dq_alone, _ = event_ms(lambda: band(DQ), 20)
             band_prep, _ = event_ms(lambda: band(PREP), 20)
             dkdv_med, dkdv_avg = event_ms(lambda: bwd(DKDV), n)
             fwd_med, _ = event_ms(lambda: attn_fwd(qd, kd, vd, None, (W, 0), True), 20)
-            dq_med, _ = event_ms(lambda: bwd(DQ), 20)
-            prep_med, _ = event_ms(lambda: bwd(PREP), 20)
+            dq_med, _ = event_ms(lambda: bwd(PREP | DQ), 20)
             bwd_med, _ = event_ms(lambda: bwd(7), 20)
             tf = lambda fl, ms_: fl / ms_ / 1e9  # noqa: E731
             rec["kernels"] = {
@@ -540,15 +547,15 @@ def main():
                                        "TFLOP/s": tf(8 * fl_band, rec["roofline"]["median_launch_ms"]),
                                        "flops_per_pair": "8 D"},
                 "bwd_dq_step_band": {"ms": band_dq, "TFLOP/s": tf(6 * fl_band, band_dq),
-                                     "flops_per_pair": "6 D"},
-                "bwd_prep_step_band": {"ms": band_prep},
+                                     "flops_per_pair": "6 D", "note": "makes the row statistics, too"},
+                "bwd_dq_step_band_phases_apart": {"dq_ms": band_dq_alone, "statistics_ms": band_prep,
+                                                  "note": "two kernels; not launched by the step"},
                 "fwd_own_chunk": {"ms": fwd_med, "TFLOP/s": tf(4 * fl_pair, fwd_med),
                                   "flops_per_pair": "4 D"},
                 "bwd_dkdv_own_chunk": {"ms": dkdv_med, "TFLOP/s": tf(8 * fl_pair, dkdv_med),
                                        "flops_per_pair": "8 D"},
                 "bwd_dq_own_chunk": {"ms": dq_med, "TFLOP/s": tf(6 * fl_pair, dq_med),
-                                     "flops_per_pair": "6 D"},
-                "bwd_prep_own_chunk": {"ms": prep_med},
+                                     "flops_per_pair": "6 D", "note": "makes the row statistics, too"},
                 "bwd_own_chunk_all_kernels": {"ms": bwd_med, "TFLOP/s": tf(10 * fl_pair, bwd_med),
                                               "flops_per_pair": "10 D (window-effective)"},
             }
@@ -586,7 +593,7 @@ def main():
                 with torch.cuda.stream(side):
                     attn_bwd(qd[:, :W], pk, pv_, o_p, lse_p, do[:, :W], dqp, dkp, dvp, None,
                              (0, S), False, workspace=ws_p, phases=DKDV)
-                bwd(DKDV)
+                bwd(DKDV, "wide")  # (as the two-block schedule asks for it)
                 torch.cuda.current_stream(dev).wait_stream(side)
 
             pair_med, _ = event_ms(dkdv_pair, 20)
