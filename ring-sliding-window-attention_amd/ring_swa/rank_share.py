@@ -95,7 +95,7 @@ class RankShareFunc(torch.autograd.Function):
 
     @staticmethod
     def forward(ctx, q, k, v, window_size, cp_size, rank, softmax_scale, ring_dtypes, one_pass,
-                *prev_kv):
+                training, *prev_kv):
         b, s, hq, d = q.shape
         if softmax_scale is None:
             softmax_scale = d ** (-0.5)
@@ -103,7 +103,7 @@ class RankShareFunc(torch.autograd.Function):
         for (i, _, _, _, _) in plan:
             assert i == 0 or i <= len(prev_kv), f"step {i} needs the chunk of rank {rank - i}"
         out, lse, joined = _forward_blocks(q, k, v, prev_kv, plan, softmax_scale, None, ring_dtypes,
-                                           one_pass)
+                                           one_pass, training)
         ctx.plan, ctx.scale, ctx.ring_dtypes, ctx.one_pass = plan, softmax_scale, ring_dtypes, one_pass
         ctx.joined = joined is not None
         if ctx.joined:
@@ -117,11 +117,11 @@ class RankShareFunc(torch.autograd.Function):
         if ctx.joined:
             q, out, lse, kk, vv, *unreached = ctx.saved_tensors
             grads = _backward_joined(q, kk, vv, out, lse, do, ctx.plan, ctx.scale, unreached)
-            return (grads[0], grads[1], grads[2], None, None, None, None, None, None, *grads[3:])
+            return (*grads[:3], *[None] * 7, *grads[3:])
         q, k, v, out, lse, *prev_kv = ctx.saved_tensors
         grads = _backward_blocks(q, k, v, prev_kv, out, lse, do, ctx.plan, ctx.scale, None,
                                  ctx.ring_dtypes, ctx.one_pass)
-        return (grads[0], grads[1], grads[2], None, None, None, None, None, None, *grads[3:])
+        return (*grads[:3], *[None] * 7, *grads[3:])
 
 
 _CU_CACHE = {}
@@ -145,7 +145,7 @@ class RankShareVarlenFunc(torch.autograd.Function):
 
     @staticmethod
     def forward(ctx, q, k, v, window_size, cu_host, cp_size, rank, softmax_scale, ring_dtypes,
-                *prev_kv):
+                training, *prev_kv):
         s, hq, d = q.shape
         if softmax_scale is None:
             softmax_scale = d ** (-0.5)
@@ -157,7 +157,7 @@ class RankShareVarlenFunc(torch.autograd.Function):
         if len(plan) > 1 and not ring_dtypes:
             start = rank * s
             reach = _reach(plan, s, window_size, start - max(c for c in cu_host if c <= start))
-            ctx.joined = _joinable(q4, k4, v4, prev4, plan, window_size, reach)
+            ctx.joined = _joinable(q4, k4, v4, prev4, plan, window_size, reach, training, True)
         if ctx.joined:
             kk, vv = _join_keys(k4, v4, prev4, plan, reach)
             cu_q, cu_k = _packed_cu(local_cu, reach, q.device)
@@ -177,17 +177,13 @@ class RankShareVarlenFunc(torch.autograd.Function):
             grads = _backward_joined(q.unsqueeze(0), kk, vv, out.unsqueeze(0), lse.unsqueeze(0),
                                      do.unsqueeze(0), ctx.plan, ctx.scale,
                                      [p.unsqueeze(1) for p in unreached], cu_q, cu_k)
-            dprev = [g.squeeze(1) for g in grads[3:]]
-            return (grads[0].squeeze(0), grads[1].squeeze(0), grads[2].squeeze(0), None, None, None,
-                    None, None, None, *dprev)
+            return (*[g.squeeze(0) for g in grads[:3]], *[None] * 7, *[g.squeeze(1) for g in grads[3:]])
         q, k, v, out, lse, cu_dev, *prev_kv = ctx.saved_tensors
         prev4 = [p.unsqueeze(1) for p in prev_kv]
         grads = _backward_blocks(q.unsqueeze(0), k.unsqueeze(0), v.unsqueeze(0), prev4,
                                  out.unsqueeze(0), lse.unsqueeze(0), do.unsqueeze(0), ctx.plan,
                                  ctx.scale, cu_dev, ctx.ring_dtypes)
-        dprev = [g.squeeze(1) for g in grads[3:]]
-        return (grads[0].squeeze(0), grads[1].squeeze(0), grads[2].squeeze(0), None, None, None,
-                None, None, None, *dprev)
+        return (*[g.squeeze(0) for g in grads[:3]], *[None] * 7, *[g.squeeze(1) for g in grads[3:]])
 
 
 _SIDE_STREAMS = threading.local()  # .by_device: {device index: stream}; gone with its thread
@@ -336,7 +332,7 @@ def _reach(plan, s, window, first_kv_len=None):
     return reach if first_kv_len is None else min(reach, first_kv_len)
 
 
-def _joinable(q, k, v, prev_kv, plan, window, reach):
+def _joinable(q, k, v, prev_kv, plan, window, reach, training, packed=False):
     """May the plan's blocks run as one band over joined keys (``_join_keys``), and is that the faster
     way?
 
@@ -345,11 +341,14 @@ def _joinable(q, k, v, prev_kv, plan, window, reach):
     refuses them or takes them as they are.
 
     Three and more blocks are always joined (forward 0.66 to 1.01 of the blocks' time, forward and
-    backward 0.65 to 0.94, over 17 shapes).  Two only where the host bounds their many launches and
-    the copies are small (forward and backward of 28 / 4 heads, 1607 tokens, window 556: 444 -> 256 us).
-    Beyond that two launches side by side fill the chip better than one of half as many, longer
-    blocks, and the copies show (us, blocks / joined, forward and backward: 8 / 2 heads, 8192 tokens of a
-    pack, window 8192, 585 / 724; 28 / 4 heads 1326 / 1627; forward alone, 32 / 32 heads, 447 / 514)."""
+    backward 0.65 to 0.94, over 17 shapes; against 64 bits ``out`` and ``dq`` are closer, 2.4e-3
+    instead of 2.9e-3 in bf16, ``dk`` and ``dv`` the same).  Two only where the host bounds their many
+    launches (forward and backward of 28 / 4 heads, 1607 tokens, window 556: 444 -> 256 us); with more
+    work two launches side by side fill the chip better than one of half as many, longer blocks
+    (8192 tokens of a pack, window 8192, 8 / 2 heads, 585 -> 724 us; 28 / 4 heads 1326 -> 1627).  A
+    forward alone is two launches block by block, so there the copies have to be small beside the
+    work (2048 tokens, 28 / 4 heads, window 1536, 84 -> 69 us; but of a pack, 32 / 32 heads, window 2048,
+    72 -> 90); of a pack, whose block route costs the host more, a few MB are always."""
     hops = plan[-1][0]
     if hops == 0 or k.dim() != 4 or len(prev_kv) < hops:
         return False
@@ -359,7 +358,9 @@ def _joinable(q, k, v, prev_kv, plan, window, reach):
         m = min(max(window - reach, 0), s)
         pairs = b * (m * reach + m * (m + 1) // 2 + (s - m) * (window + 1))
         copied = 4 * b * (reach + s) * hk * d  # bytes
-        if pairs * hq * d > _JOIN_TWO_WORK or copied > max(8 << 20, pairs * hq // 4):
+        if pairs * hq * d > _JOIN_TWO_WORK:
+            return False
+        if not training and copied * 10 > pairs * hq and not (packed and copied <= 5e6):
             return False
     dtype, device, own = q.dtype, q.device, (b, s, hk, d)
     for t, shape in ((k, own), (v, own), *((p, (2,) + own) for p in prev_kv[:hops])):
@@ -431,7 +432,8 @@ def _backward_joined(q, kk, vv, out, lse, do, plan, scale, unreached, cu_q=None,
     return (dq, dkv[0, :, reach:].contiguous(), dkv[1, :, reach:].contiguous(), *dprev)
 
 
-def _forward_blocks(q, k, v, prev_kv, plan, scale, local_cu, ring_dtypes, one_pass=True):
+def _forward_blocks(q, k, v, prev_kv, plan, scale, local_cu, ring_dtypes, one_pass=True,
+                    training=False):
     """Run the planned blocks and merge them.  Dense 4-d tensors (batch 1 when packed).  Returns
     ``(out, lse, joined)``, ``joined`` being the joined keys and values when that route was taken."""
     assert plan and plan[0][0] == 0, "the diagonal block comes first: it covers every row"
@@ -447,7 +449,7 @@ def _forward_blocks(q, k, v, prev_kv, plan, scale, local_cu, ring_dtypes, one_pa
     if one_pass and not ring_dtypes and local_cu is None and len(plan) > 1:
         window = plan[0][3][0]
         reach = _reach(plan, q.shape[1], window)
-        if _joinable(q, k, v, prev_kv, plan, window, reach):
+        if _joinable(q, k, v, prev_kv, plan, window, reach, training):
             joined = _join_keys(k, v, prev_kv, plan, reach)
             return (*attn_fwd(q, *joined, scale, plan[0][3], True), joined)
     if ring_dtypes or len(plan) > 2:
@@ -626,6 +628,10 @@ def _backward_two_blocks(q, k, v, kv1, dkv1, out, lse, do, plan, scale, local_cu
     return dq, dkv
 
 
+def _backward_follows(*tensors) -> bool:
+    return torch.is_grad_enabled() and any([t.requires_grad for t in tensors])
+
+
 def ring_rank_share_attn(
     q: torch.Tensor,
     k: torch.Tensor,
@@ -651,7 +657,8 @@ def ring_rank_share_attn(
     the backward holds on to instead of ``k``, ``v`` and the reached chunks."""
     assert q.shape[1] == k.shape[1] == v.shape[1], "Sequence length must be the same"
     return RankShareFunc.apply(q, k, v, int(window_size), int(cp_size), int(cp_local_rank),
-                               softmax_scale, bool(ring_dtypes), bool(one_pass), *prev_kv)
+                               softmax_scale, bool(ring_dtypes), bool(one_pass),
+                               _backward_follows(q, k, v, *prev_kv), *prev_kv)
 
 
 def ring_rank_share_attn_varlen(
@@ -675,4 +682,5 @@ def ring_rank_share_attn_varlen(
         "cu_seqlens does not match with sequence length per rank"
     )
     return RankShareVarlenFunc.apply(q, k, v, int(window_size), cu_host, int(cp_size),
-                                     int(cp_local_rank), softmax_scale, bool(ring_dtypes), *prev_kv)
+                                     int(cp_local_rank), softmax_scale, bool(ring_dtypes),
+                                     _backward_follows(q, k, v, *prev_kv), *prev_kv)

@@ -16,10 +16,10 @@ def _inputs(b=2):
     return q, k, v, [torch.randn(2, b, S, HK, D).bfloat16() for _ in range(2)]
 
 
-def _joinable(q, k, v, prev, window=S + 30, rank=2):
+def _joinable(q, k, v, prev, window=S + 30, rank=2, training=True, packed=False):
     s = q.shape[1]
     plan = RS.plan_nonvarlen(s, window, 4, rank)
-    return RS._joinable(q, k, v, prev, plan, window, RS._reach(plan, s, window))
+    return RS._joinable(q, k, v, prev, plan, window, RS._reach(plan, s, window), training, packed)
 
 
 def test_tensors_alike_are_joined():
@@ -59,7 +59,7 @@ def test_the_entry_points_refuse_values_of_another_kind(packed):
 @pytest.mark.parametrize("s,hq,hk,d,window,rank,joined", [
     (1000, 16, 4, 128, 1500, 1, True),      # two blocks, the host's launches are most of it
     (2048, 32, 8, 128, 1536, 1, True),
-    (1000, 32, 32, 64, 250, 1, False),      # the copies are as large as the work
+    (1000, 32, 32, 64, 250, 1, True),
     (8192, 8, 2, 128, 12288, 1, False),     # two launches fill the chip better than one
     (7379, 4, 4, 128, 10877, 1, False),
     (4096, 32, 8, 128, 10000, 3, True),     # four blocks, whatever the work
@@ -69,6 +69,16 @@ def test_two_blocks_are_joined_only_where_launches_are_the_time(s, hq, hk, d, wi
     q, k = torch.empty(1, s, hq, d, device="meta", dtype=torch.bfloat16), torch.empty(1, s, hk, d, device="meta", dtype=torch.bfloat16)
     prev = [torch.empty(2, 1, s, hk, d, device="meta", dtype=torch.bfloat16) for _ in range(rank)]
     assert _joinable(q, k, k, prev, window, rank) == joined
+
+
+@pytest.mark.parametrize("s,hq,hk,window,dense,packed", [
+    (2048, 28, 4, 1536, True, True), (2048, 32, 32, 2048, False, False), (1000, 8, 2, 250, False, True),
+])
+def test_a_forward_alone_joins_two_blocks_only_with_small_copies(s, hq, hk, window, dense, packed):
+    q, k = (torch.empty(1, s, h, 128, device="meta", dtype=torch.bfloat16) for h in (hq, hk))
+    prev = [torch.empty(2, 1, s, hk, 128, device="meta", dtype=torch.bfloat16)]
+    assert _joinable(q, k, k, prev, window, 1, training=False) == dense
+    assert _joinable(q, k, k, prev, window, 1, training=False, packed=True) == packed
 
 
 @pytest.mark.parametrize("s,window,hops", [(64, 40, 1), (64, 128, 2), (1500, 2000, 2), (1500, 4500, 3)])

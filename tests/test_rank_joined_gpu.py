@@ -55,6 +55,13 @@ def test_shares_on_joined_keys_match_the_oracle(monkeypatch, s, w, packed, route
             out = ring_swa.ring_rank_share_attn_varlen(*own, prev, w, cu, CP, r, **kw)
         else:
             out = ring_swa.ring_rank_share_attn(*own, prev, w, CP, r, **kw)
+        with torch.no_grad():  # (joins two blocks more seldom)
+            if packed:
+                alone = ring_swa.ring_rank_share_attn_varlen(*own, prev, w, cu, CP, r, **kw)
+            else:
+                alone = ring_swa.ring_rank_share_attn(*own, prev, w, CP, r, **kw)
+        want = ro[:, sl] if not packed else ro[0, sl]
+        assert (alone.float().cpu() - want).abs().max().item() <= 2e-2
         grads = torch.autograd.grad(out, own + prev, do[:, sl].cuda() if not packed else do[0, sl].cuda())
         cpu = [x.float().cpu() for x in (out.detach(), *grads)]
         if packed:
