@@ -287,8 +287,7 @@ int rswa_attn_bwd_phases(const rswa_attn_params* p, void* stream, int phases);
  * (8 bytes per (row, q head) pair) exceed the buffer -- more than 4 194 304 pairs -- are
  * refused with RSWA_ERR_UNSUPPORTED.  The buffer's address is looked up on the
  * first call on each device (the device must be current, as for every other call); nothing
- * in it has to be cleared between calls, the statistics kernel rewrites what the others
- * read.  All calls on one GPU share the one buffer: calls that may overlap in time on the
+ * in it has to be cleared between calls, each writes what it reads of it.  All calls on one GPU share the one buffer: calls that may overlap in time on the
  * same GPU (different streams, different threads) race and must be serialised by the caller.
  */
 #define RSWA_BWD_STATIC_MAX_BYTES (32u << 20)

@@ -1078,9 +1078,9 @@ __global__ __launch_bounds__(256) void attn_bwd_rest_kernel(const AttnArgs a) {
 //
 // STATS: the kernel also makes the row statistics of the backward, which it has to read dO for
 // anyway, and writes them for the dK/dV kernel, launched after it.  Same bits as the statistics
-// kernel's (same order of sums).  Both kernels are at memory speed there, so what falls away is the
-// second read of dO and a launch; us, statistics + dQ, bf16, head_dim 128: 2 x 8192 rows, 32 / 32 heads,
-// window 1000 461 -> 422; a pack of 16384 tokens in sequences of 16 to 1024, 32 / 8 heads, 217 -> 203.
+// kernel's (same order of sums).  What falls away is the second read of dO and a launch; us, statistics +
+// dQ, bf16, head_dim 128, two kernels / one: 2 x 8192 rows, 32 / 32 heads, window 1000 457 / 444; a pack of
+// 16384 tokens in sequences of 16 to 1024, 32 / 8 heads, 213 / 206; 4001 rows, window 1024, 105 / 99.
 template <typename T, int D, bool FAR, int NW, bool STATS>
 __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(2, 2)))
 void attn_bwd_dq_kernel(const AttnArgs a) {
@@ -1775,8 +1775,9 @@ RSWA_INSTANTIATE(_Float16, 64)
 // head_dim 64, 0.77 + 18 and 0.93 + 7.  Measured on both sides of the line (us, wide / WALK4, bf16,
 // head_dim 128): 32 / 8 heads, window 1024, 4096 rows 217 / 128, 6000 rows 218 / 190, 8192 rows (256
 // wide blocks, one full round) 229 / 255, 9000 rows 368 / 303, 16384 rows 477 / 523; 32 / 32 heads,
-// window 1000, 2 x 8192 rows 545 / 700; full attention over 4096 rows, 32 / 8 heads, 615 / 238.  Of the
-// 78 dense shapes timed the rule is 1 % behind the better form on average.
+// window 1000, 2 x 8192 rows 545 / 700; 4096 rows, 32 / 8 heads, causal without a window 623 / 252, without
+// a mask 620 / 454.  Of 258 dense and packed shapes drawn the rule is 0.5 % behind the better form on
+// average.
 // A pack is judged on its average length L, the only one the host knows, as if of sequences of
 // 1.5 L (what a token sees when lengths vary), the longest as long as the pack or the window, with
 // half a key tile per sequence wasted.  Packs of 16384 tokens, 32 / 8 heads, window 1024, lengths log-uniform: 16-64

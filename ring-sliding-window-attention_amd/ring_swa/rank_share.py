@@ -4,10 +4,15 @@ The compute body of upstream's ring loops
 (``ring_swa/sliding_window/nonvarlen.py:46-150`` forward, ``:182-333`` backward;
 ``ring_swa/sliding_window/varlen.py:56-172`` and ``:194-359``) with the P2P
 exchange replaced by KV chunks the caller already holds in HBM: the rank's own
-chunk plus the chunks of the ranks before it.  Per step: one band-attention
-kernel on the block the window selects, LSE-merged into the running output;
-backward runs one kernel call per block with the final merged ``(o, lse)`` and
-accumulates ``dq`` / per-chunk ``dkv`` in fp32, as upstream does.
+chunk plus the chunks of the ranks before it.
+
+Because the chunks are at hand, the default computes a plan's blocks as one band where that is
+faster: over the previous chunk's tail and the own chunk where they lie, or over the reached rows
+copied side by side.  Upstream's own structure -- one band-attention kernel per block, LSE-merged
+into the running output; backward one kernel call per block with the final merged ``(o, lse)``,
+``dq`` / per-chunk ``dkv`` accumulated in fp32 -- is ``blocks_forward`` / ``blocks_backward`` and
+``_backward_two_blocks``: what ``ring_dtypes=True``, ``one_pass=False``, the larger packed steps of two
+blocks and the ring over a ``cp_group`` (whose chunks arrive while it computes) run.
 
 What is left out is exactly what needs a second GPU: moving KV forward and
 KV + dKV backward around the ring.
