@@ -322,6 +322,10 @@ int rswa_attn_bwd_handoff_active(const rswa_attn_params* p);
  * be refused. */
 int rswa_attn_bwd_dkdv_keys(const rswa_attn_params* p);
 
+/* Blocks per compute unit that the forward kernel of these parameters is built for, 2 or 3 (the same
+ * bits either way); a negative status if the call would be refused. */
+int rswa_attn_fwd_blocks_per_cu(const rswa_attn_params* p);
+
 /* Message of the calling thread's last failed call ("" if none). */
 const char* rswa_last_error(void);
 

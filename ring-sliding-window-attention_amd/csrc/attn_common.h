@@ -40,8 +40,6 @@ struct AttnArgs {
   // by a kernel of the same call; a tile has 2^ktile_log2 keys
   int32_t* ktile;
   int32_t ktile_log2;
-  int32_t dkdv_form;  // RSWA_DKDV_*: the caller's choice of the dK/dV kernel's blocks
-  int32_t dq_last;  // dq lies over an input: the dQ kernel must not run before dK/dV (host only)
   int32_t snake;    // dK/dV: see the kernel (dense; of a pack the device decides)
   const int32_t* cu_q;
   const int32_t* cu_k;
@@ -87,6 +85,10 @@ struct AttnArgs {
   int32_t ds_nkb;
   int32_t ds_slots;  // 32-row tile slots per q head (dense: batch * tiles; packed: rows / 32 + batch)
   float scale, scale_log2;
+  // ---- for the host's choices only; behind the rest, so that the kernels' argument loads stay put
+  int32_t max_keys;   // keys a query row sees at most (of the rows avg_keys samples)
+  int32_t dkdv_form;  // RSWA_DKDV_*: the caller's choice of the dK/dV kernel's blocks
+  int32_t dq_last;    // dq lies over an input: the dQ kernel must not run before dK/dV
 };
 
 struct SeqInfo {

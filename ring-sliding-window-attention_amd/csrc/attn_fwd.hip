@@ -38,16 +38,12 @@ struct FwdCfg {
   static constexpr int ROWB = D * 2;  // bytes per row
   static constexpr int TILE = BN * ROWB;
   static constexpr int O_STRIDE = D * 2 + 16;
-  // Blocks per compute unit (a block has one wave per SIMD).  head_dim 128 needs 214 registers, so
-  // two.  head_dim 64 has half the MFMAs per score and is bound by the softmax's vector work and
-  // its latencies; it fits three (148 registers; four would spill): 8000 rows in four sequences,
-  // 28 / 4 heads, window 1000, fp16: 79-84 -> 77-79 us (by box; the two alternating on one).
-  static constexpr int WAVES_PER_SIMD = D == 64 ? 3 : 2;
   static_assert(TILE >= 32 * O_STRIDE, "one wave's epilogue staging fits one tile buffer");
 };
 
-template <typename T, int D, bool SKIP, bool FAR>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(FwdCfg<D>::WAVES_PER_SIMD, FwdCfg<D>::WAVES_PER_SIMD)))
+// WAVES: blocks per compute unit (a block has one wave per SIMD), see fwd_three_blocks.
+template <typename T, int D, bool SKIP, bool FAR, int WAVES>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(WAVES, WAVES)))
 void attn_fwd_kernel(const AttnArgs a) {
   using C = FwdCfg<D>;
   constexpr int NW = C::THREADS / 64;
@@ -434,23 +430,45 @@ void attn_fwd_kernel(const AttnArgs a) {
 
 // Explicit instantiations: with implicit instantiation alone this hipcc emits the host
 // launch stubs of only some of the four variants.
-#define RSWA_INSTANTIATE(T, D)                                                   \
-  template __global__ void attn_fwd_kernel<T, D, false, false>(const AttnArgs); \
-  template __global__ void attn_fwd_kernel<T, D, true, false>(const AttnArgs);  \
-  template __global__ void attn_fwd_kernel<T, D, false, true>(const AttnArgs);  \
-  template __global__ void attn_fwd_kernel<T, D, true, true>(const AttnArgs);
-RSWA_INSTANTIATE(__bf16, 128)
-RSWA_INSTANTIATE(__bf16, 64)
-RSWA_INSTANTIATE(_Float16, 128)
-RSWA_INSTANTIATE(_Float16, 64)
+#define RSWA_INSTANTIATE(T, D, W)                                                   \
+  template __global__ void attn_fwd_kernel<T, D, false, false, W>(const AttnArgs); \
+  template __global__ void attn_fwd_kernel<T, D, true, false, W>(const AttnArgs);  \
+  template __global__ void attn_fwd_kernel<T, D, false, true, W>(const AttnArgs);  \
+  template __global__ void attn_fwd_kernel<T, D, true, true, W>(const AttnArgs);
+RSWA_INSTANTIATE(__bf16, 128, 2)
+RSWA_INSTANTIATE(__bf16, 64, 2)
+RSWA_INSTANTIATE(__bf16, 64, 3)
+RSWA_INSTANTIATE(_Float16, 128, 2)
+RSWA_INSTANTIATE(_Float16, 64, 2)
+RSWA_INSTANTIATE(_Float16, 64, 3)
 #undef RSWA_INSTANTIATE
 
-template <typename T, int D>
+int rows_per_block(const AttnArgs& a) { return (a.group & 1) == 0 ? 64 : 128; }
+int blocks_per_tile(const AttnArgs& a) { return ((a.group & 1) == 0 ? a.group / 2 : a.group) * a.heads_kv; }
+
+// Three blocks per compute unit instead of two?  head_dim 128 needs 214 registers, so two.  head_dim 64
+// has half the MFMAs per score and is bound by the softmax's vector work and its latencies; it fits
+// three (148 registers; four would spill), but built for that a block is 3 to 12 % slower by itself.
+// So three where the launch has more blocks than fit at two per compute unit (us, two / three: 504
+// blocks of 2241 rows, 28 / 4 heads, window 4232, 55 / 61; 552 blocks of 5855 rows, 12 heads, window
+// 236, 27 / 22; 4 x 2000 rows, 28 / 4 heads, window 1000, 1792 blocks, 79 / 78), and where blocks are
+// long and of unlike length, so that the longest decide, several rounds of them (causal without a
+// window, 8 heads, 13513 tokens in three sequences, 864 blocks, 147 / 178; 12 heads, 20738 tokens in
+// four, 1980 blocks, 300 / 299).  Of 438 shapes drawn the rule is 0.3 % behind the better build on
+// average (more than 3 % slower than two blocks on 8 of them, 11 % at most), three alone 4 %, two alone 5 %.
+bool fwd_three_blocks(const AttnArgs& a, int head_dim) {
+  if (head_dim != 64) return false;
+  const double tiles = a.cu_q ? (double)a.rows_q / rows_per_block(a) + 0.5 * a.batch
+                              : (double)ceil_div(a.seqlen_q, rows_per_block(a)) * a.batch;
+  const bool even = a.avg_keys >= 0.7 * a.max_keys || a.avg_keys <= 250;
+  return tiles * blocks_per_tile(a) > (even ? 2 * kComputeUnits : 1500);
+}
+
+template <typename T, int D, int WAVES>
 int launch_fwd(AttnArgs& a, hipStream_t stream) {
   using C = FwdCfg<D>;
-  const bool pair = (a.group & 1) == 0;
-  const int bm = pair ? 64 : 128;
-  const int units = (pair ? a.group / 2 : a.group) * a.heads_kv;  // blocks per q tile
+  const int bm = rows_per_block(a);
+  const int units = blocks_per_tile(a);
   if (a.cu_q) {
     a.n_tile = (int)(ceil_div(a.rows_q, bm) + a.batch);
     a.n_work = a.n_tile * units;
@@ -468,11 +486,11 @@ int launch_fwd(AttnArgs& a, hipStream_t stream) {
   clear_launch_error();
   const dim3 grid(padded_grid(a.n_work)), block(C::THREADS);
   if (skip) {
-    if (a.far) hipLaunchKernelGGL((attn_fwd_kernel<T, D, true, true>), grid, block, 0, stream, a);
-    else hipLaunchKernelGGL((attn_fwd_kernel<T, D, true, false>), grid, block, 0, stream, a);
+    if (a.far) hipLaunchKernelGGL((attn_fwd_kernel<T, D, true, true, WAVES>), grid, block, 0, stream, a);
+    else hipLaunchKernelGGL((attn_fwd_kernel<T, D, true, false, WAVES>), grid, block, 0, stream, a);
   } else {
-    if (a.far) hipLaunchKernelGGL((attn_fwd_kernel<T, D, false, true>), grid, block, 0, stream, a);
-    else hipLaunchKernelGGL((attn_fwd_kernel<T, D, false, false>), grid, block, 0, stream, a);
+    if (a.far) hipLaunchKernelGGL((attn_fwd_kernel<T, D, false, true, WAVES>), grid, block, 0, stream, a);
+    else hipLaunchKernelGGL((attn_fwd_kernel<T, D, false, false, WAVES>), grid, block, 0, stream, a);
   }
   return check_launch("attn_fwd");
 }
@@ -487,8 +505,16 @@ extern "C" int rswa_attn_fwd(const rswa_attn_params* p, void* stream) {
   if (rc != RSWA_OK) return rc;
   if (a.rows_q == 0) return RSWA_OK;
   hipStream_t st = (hipStream_t)stream;
-  if (p->dtype == RSWA_BF16) {
-    return p->head_dim == 128 ? launch_fwd<__bf16, 128>(a, st) : launch_fwd<__bf16, 64>(a, st);
-  }
-  return p->head_dim == 128 ? launch_fwd<_Float16, 128>(a, st) : launch_fwd<_Float16, 64>(a, st);
+  const bool bf16 = p->dtype == RSWA_BF16;
+  if (p->head_dim == 128) return bf16 ? launch_fwd<__bf16, 128, 2>(a, st) : launch_fwd<_Float16, 128, 2>(a, st);
+  if (fwd_three_blocks(a, 64)) return bf16 ? launch_fwd<__bf16, 64, 3>(a, st) : launch_fwd<_Float16, 64, 3>(a, st);
+  return bf16 ? launch_fwd<__bf16, 64, 2>(a, st) : launch_fwd<_Float16, 64, 2>(a, st);
+}
+
+extern "C" int rswa_attn_fwd_blocks_per_cu(const rswa_attn_params* p) {
+  using namespace rswa;
+  AttnArgs a;
+  const int rc = fill_args(p, false, a);
+  if (rc != RSWA_OK) return rc;
+  return fwd_three_blocks(a, p->head_dim) ? 3 : 2;
 }

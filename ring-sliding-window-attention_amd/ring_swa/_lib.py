@@ -140,6 +140,8 @@ def load(path: str) -> ctypes.CDLL:
     L.rswa_attn_bwd_workspace_min_bytes.argtypes = [POINTER(AttnParams)]
     L.rswa_attn_bwd_handoff_active.restype = c_int
     L.rswa_attn_bwd_handoff_active.argtypes = [POINTER(AttnParams)]
+    L.rswa_attn_fwd_blocks_per_cu.restype = c_int
+    L.rswa_attn_fwd_blocks_per_cu.argtypes = [POINTER(AttnParams)]
     L.rswa_attn_bwd_dkdv_keys.restype = c_int
     L.rswa_attn_bwd_dkdv_keys.argtypes = [POINTER(AttnParams)]
     if L.rswa_sizeof_attn_params() != ctypes.sizeof(AttnParams):

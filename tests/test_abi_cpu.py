@@ -269,3 +269,25 @@ def test_workspace_without_the_key_tile_table_is_accepted():
     for room, rc in ((least, 0), (least - 1, -1)):
         p.workspace_bytes = room
         assert L.rswa_attn_bwd_phases(p, None, 0) == rc
+
+
+@pytest.mark.parametrize("tokens,heads_q,heads_kv,window,sequences,blocks", [
+    (2241, 28, 4, 4232, 1, 2), (10505, 4, 4, 3221, 3, 2), (1461, 32, 32, 960, 1, 2),  # fit two per unit
+    (5855, 12, 12, 236, 1, 3), (29004, 32, 8, 171, 25, 3), (8000, 28, 4, 1000, 4, 3),
+    (13513, 8, 8, -1, 3, 2), (4382, 32, 8, 2466, 5, 2),  # more, but long ones of unlike length
+    (11207, 28, 4, -1, 1, 3),
+])
+def test_head_dim_64_forward_takes_three_blocks_per_unit_where_two_do_not_hold_them(tokens, heads_q, heads_kv, window,
+                                                                                    sequences, blocks):
+    """(These shapes were timed in both builds.)"""
+    _ensure_built()
+    from ring_swa import _lib
+
+    p = _fake_params(tokens, heads_q, heads_kv, 64)
+    p.window_left = window
+    if sequences > 1:
+        p.batch, p.total_q, p.total_k = sequences, tokens, tokens
+        p.cu_seqlens_q = p.cu_seqlens_k = 4096
+    assert _lib.lib().rswa_attn_fwd_blocks_per_cu(p) == blocks
+    p.head_dim = 128
+    assert _lib.lib().rswa_attn_fwd_blocks_per_cu(p) == 2

@@ -228,3 +228,35 @@ def test_fwd_accumulate_into_equals_forward_plus_merge(case):
              accumulate_into=(big_out[:, :n], big_lse[:, :, :n]))
     assert torch.equal(big_out[:, n:], out0[:, n:]) and torch.equal(big_lse[:, :, n:], lse0[:, :, n:])
     assert torch.equal(big_out[:, :n], ref_out[:, :n]) and torch.equal(big_lse[:, :, :n], ref_lse[:, :, :n])
+
+
+@pytest.mark.parametrize("addressing", ["near", "far"])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16], ids=["bf16", "fp16"])
+@pytest.mark.parametrize("s,hq,hk,window,n_sink,copies", [
+    (300, 8, 2, 100, 0, 28), (300, 8, 2, 100, 0, 30),    # 560 and 600 blocks of 64 rows, per-wave tile skip
+    (257, 3, 1, 30, 4, 70), (640, 4, 2, 500, 0, 80),     # 128-row blocks with sinks; no skip, unlike lengths
+    (129, 28, 4, 64, 1, 15),
+])
+def test_head_dim_64_builds_for_two_and_three_blocks_agree(monkeypatch, s, hq, hk, window, n_sink, copies, dtype,
+                                                           addressing):
+    """One batch entry (few blocks: two per compute unit) against the oracle, and many copies of it (more
+    blocks than two per unit hold: three) bit for bit against that."""
+    from ring_swa import _lib
+    from ring_swa.ops import attn_fwd
+
+    if addressing == "far":
+        monkeypatch.setenv("RSWA_ADDRESSING", "far")
+    builds, real = [], _lib.launch
+
+    def launch(dev, entry, p, *rest):
+        builds.append(_lib.lib().rswa_attn_fwd_blocks_per_cu(p))
+        real(dev, entry, p, *rest)
+
+    monkeypatch.setattr(_lib, "launch", launch)
+    q, k, v = (_rand((1, s, h, 64), dtype, i) for i, h in enumerate((hq, hk, hk)))
+    out, lse = attn_fwd(q.cuda(), k.cuda(), v.cuda(), None, (window, 0), True, num_sink=n_sink)
+    _check(out, lse, *O.window_attention(q, k, v, 0.125, (window, 0), True, n_sink))
+    many = [t.cuda().expand(copies, -1, -1, -1) for t in (q, k, v)]
+    outs, lses = attn_fwd(*many, None, (window, 0), True, num_sink=n_sink)
+    assert builds == [2, 3]
+    assert torch.equal(outs, out.expand_as(outs)) and torch.equal(lses, lse.expand_as(lses))
