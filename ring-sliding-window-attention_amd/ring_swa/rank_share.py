@@ -326,7 +326,8 @@ def _one_pass(q, k, v, prev_kv, plan, local_cu):
     return w, kk, vv, tail
 
 
-# Two blocks run as one band up to this much work (visible pairs x q heads x head_dim); see _joinable.
+# Two blocks run as one band up to this much work (visible pairs x q heads x head_dim), and beyond it
+# where the blocks of the band are even; see _joinable.
 _JOIN_TWO_WORK = 128e6 * 128
 
 
@@ -350,10 +351,15 @@ def _joinable(q, k, v, prev_kv, plan, window, reach, training, packed=False):
     instead of 2.9e-3 in bf16, ``dk`` and ``dv`` the same).  Two only where the host bounds their many
     launches (forward and backward of 28 / 4 heads, 1607 tokens, window 556: 444 -> 256 us); with more
     work two launches side by side fill the chip better than one of half as many, longer blocks
-    (8192 tokens of a pack, window 8192, 8 / 2 heads, 585 -> 724 us; 28 / 4 heads 1326 -> 1627).  A
-    forward alone is two launches block by block, so there the copies have to be small beside the
-    work (2048 tokens, 28 / 4 heads, window 1536, 84 -> 69 us; but of a pack, 32 / 32 heads, window 2048,
-    72 -> 90); of a pack, whose block route costs the host more, a few MB are always."""
+    (8192 tokens of a pack, window 8192, 8 / 2 heads, 585 -> 724 us; 28 / 4 heads 1326 -> 1627), unless
+    the joined rows see about as many keys each (a window shorter than the chunk, no pack) and the
+    heads are grouped, which makes the copies small: over 51 such shapes forward and backward takes
+    0.60 to 1.04 of the blocks' time (8000 tokens, window 7999, 32 / 8 heads, 3970 -> 3794 us; 8 / 2
+    heads 1426 -> 1270), a forward alone 0.68 to 1.08 (335 -> 257; worst 8191 tokens, window 4000,
+    32 / 8 heads, 529 -> 569).  A forward alone is two launches block by block, so there the copies
+    have to be small beside the work (2048 tokens, 28 / 4 heads, window 1536, 84 -> 69 us; but of a
+    pack, 32 / 32 heads, window 2048, 72 -> 90); of a pack, whose block route costs the host more, a
+    few MB are always."""
     hops = plan[-1][0]
     if hops == 0 or k.dim() != 4 or len(prev_kv) < hops:
         return False
@@ -363,7 +369,8 @@ def _joinable(q, k, v, prev_kv, plan, window, reach, training, packed=False):
         m = min(max(window - reach, 0), s)
         pairs = b * (m * reach + m * (m + 1) // 2 + (s - m) * (window + 1))
         copied = 4 * b * (reach + s) * hk * d  # bytes
-        if pairs * hq * d > _JOIN_TWO_WORK:
+        even = not packed and window < s and hq > hk
+        if pairs * hq * d > _JOIN_TWO_WORK and not even:
             return False
         if not training and copied * 10 > pairs * hq and not (packed and copied <= 5e6):
             return False

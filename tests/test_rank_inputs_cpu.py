@@ -62,6 +62,8 @@ def test_the_entry_points_refuse_values_of_another_kind(packed):
     (1000, 32, 32, 64, 250, 1, True),
     (8192, 8, 2, 128, 12288, 1, False),     # two launches fill the chip better than one
     (7379, 4, 4, 128, 10877, 1, False),
+    (8000, 32, 8, 128, 7999, 1, True),      # even blocks, grouped heads
+    (8000, 32, 32, 128, 7999, 1, False),
     (4096, 32, 8, 128, 10000, 3, True),     # four blocks, whatever the work
     (6000, 32, 32, 128, 15600, 3, True),
 ])
