@@ -4,8 +4,8 @@
 // Replaces flash-attn's forward as wrapped at ring_swa/ops/wrap_flash.py:168-273.
 //
 // One block = 4 waves x 32 query rows sharing every K/V tile it loads: either 64 rows of
-// TWO q heads of one GQA group (group size even) or 128 rows of one q head; two blocks (three at
-// head_dim 64) fit a compute unit (waves of a SIMD are from independent blocks).  Per 64-key
+// TWO q heads of one GQA group (group size even) or 128 rows of one q head; two blocks (at
+// head_dim 64 also three, fwd_three_blocks) fit a compute unit (waves of a SIMD are from independent blocks).  Per 64-key
 // tile a wave computes S^T = K Q^T (keys x queries) with v_mfma_f32_32x32x16, so each
 // lane owns ONE query column: the row max / sum of the online softmax are in-lane
 // reductions plus a single half-wave exchange, and P^T is already laid out as the B
