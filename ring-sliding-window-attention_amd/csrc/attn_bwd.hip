@@ -89,6 +89,31 @@ __device__ __forceinline__ void put_grad8(void* buf, int64_t at, typename Mma<T>
   }
 }
 
+// N times a wave's rows of a gradient tile, RPI rows each: get(n) is the lane's 8 values of its row
+// n RPI, at element offset `at` + n RPI row_st of the buffer; of its rows the lane owns those with
+// n RPI < left (all of them where `all`, a uniform condition, says so).
+template <typename T, int RPI, int N, typename Get>
+__device__ __forceinline__ void put_rows(void* buf, int64_t at, int64_t row_st, int left, bool all, bool wide,
+                                         bool accumulate, Get&& get) {
+  using V8 = typename Mma<T>::V8;
+  const int64_t step = RPI * row_st;
+  if (!(wide | accumulate)) {
+    T* dst = (T*)buf + at;
+    if (all) {
+#pragma unroll
+      for (int n = 0; n < N; n++) *(V8*)(dst + n * step) = get(n);
+    } else {
+#pragma unroll
+      for (int n = 0; n < N; n++)
+        if (n * RPI < left) *(V8*)(dst + n * step) = get(n);
+    }
+  } else {
+#pragma unroll 1
+    for (int n = 0; n < N; n++)
+      if (n * RPI < left) put_grad8<T>(buf, at + n * step, get(n), wide, accumulate);
+  }
+}
+
 // Sequences of at most this many keys whose dK/dV blocks take the snake order (see the kernel)
 constexpr int kSnakeKeys = 4096;
 
@@ -244,34 +269,19 @@ __global__ __launch_bounds__(256) void attn_bwd_dkdv_kernel(const AttnArgs a) {
   const int t_row1 = w_lds + (rl + 8) * C::ROWB + ((lp ^ swz_f<C::CPR>(rl + 8)) << 4) + (i16 & 1) * 8;
 
   // ---- this wave's K fragments stay in registers for the whole walk (B operand of
-  // S = Q K^T: lane = key column, 8 consecutive d per k-step); keys past the end are zero
-  V8 kf[KB][KS];
+  // S = Q K^T: lane = key column, 8 consecutive d per k-step)
+  // (keys past the end read the last one's values: their columns are masked in every tile and never
+  // stored)
+  V8 kf[KB][KS], vf[KB][KS];  // (the V fragments: B operand of dP = dO V^T, same layout)
 #pragma unroll
   for (int kb = 0; kb < KB; kb++) {
-    const int jc = jw0 + kb * 32 + l32;
+    const int jc = min(jw0 + kb * 32 + l32, len_k - 1);
+    const T* k_row = k_ptr + (int64_t)jc * a.k_st[1] + g * 8;
+    const T* v_row = v_ptr + (int64_t)jc * a.v_st[1] + g * 8;
 #pragma unroll
-    for (int ks = 0; ks < KS; ks++) {
-      if (jc < len_k) {
-        kf[kb][ks] = *(const V8*)(k_ptr + (int64_t)jc * a.k_st[1] + ks * 16 + g * 8);
-      } else {
-        kf[kb][ks] = V8{0, 0, 0, 0, 0, 0, 0, 0};
-      }
-    }
-  }
-
-  // ... and so do its V fragments (B operand of dP = dO V^T, same layout)
-  V8 vf[KB][KS];
+    for (int ks = 0; ks < KS; ks++) kf[kb][ks] = *(const V8*)(k_row + ks * 16);
 #pragma unroll
-  for (int kb = 0; kb < KB; kb++) {
-    const int jc = jw0 + kb * 32 + l32;
-#pragma unroll
-    for (int ks = 0; ks < KS; ks++) {
-      if (jc < len_k) {
-        vf[kb][ks] = *(const V8*)(v_ptr + (int64_t)jc * a.v_st[1] + ks * 16 + g * 8);
-      } else {
-        vf[kb][ks] = V8{0, 0, 0, 0, 0, 0, 0, 0};
-      }
-    }
+    for (int ks = 0; ks < KS; ks++) vf[kb][ks] = *(const V8*)(v_row + ks * 16);
   }
   f32x16 dk_acc[KB][DB], dv_acc[KB][DB];
 #pragma unroll
@@ -715,23 +725,24 @@ __global__ __launch_bounds__(256) void attn_bwd_dkdv_kernel(const AttnArgs a) {
       void* const dst = mtx == 0 ? dk_buf : dv_buf;
       const int64_t dst_off = mtx == 0 ? dk_off : dv_off;
       const int64_t dst_st = mtx == 0 ? a.dk_st[1] : a.dv_st[1];
+      constexpr int RPI = 256 / C::CPR;
+      const int row0 = (wave * 64 + lane_e) / C::CPR, c = (lane_e % C::CPR) * 2;
+      put_rows<T, RPI, 64 / RPI>(
+          dst, dst_off + (int64_t)(j0 + row0) * dst_st + c * 4, dst_st, len_k - j0 - row0, j0 + 63 < len_k, a.wide_dkv,
+          a.dkv_accumulate, [&](int n) {
+            const int row = row0 + n * RPI;
+            const char* src = q_s0 + row * (D * 4);
+            const int at0 = (c ^ (row & (FPR - 1))) << 4, at1 = ((c + 1) ^ (row & (FPR - 1))) << 4;
+            f32x4 lo = *(const f32x4*)(src + at0), hi = *(const f32x4*)(src + at1);
 #pragma unroll
-      for (int n = 0; n < 64 * C::CPR / 256; n++) {
-        const int idx = n * 256 + wave * 64 + lane_e;
-        const int row = idx / C::CPR, c = (idx % C::CPR) * 2;
-        const char* src = q_s0 + row * (D * 4);
-        const int at0 = (c ^ (row & (FPR - 1))) << 4, at1 = ((c + 1) ^ (row & (FPR - 1))) << 4;
-        f32x4 lo = *(const f32x4*)(src + at0), hi = *(const f32x4*)(src + at1);
-#pragma unroll
-        for (int w = 1; w < 4; w++) {
-          lo += *(const f32x4*)(src + w * W_LDS + at0);
-          hi += *(const f32x4*)(src + w * W_LDS + at1);
-        }
-        const float x[8] = {lo[0] * sc, lo[1] * sc, lo[2] * sc, lo[3] * sc,
-                            hi[0] * sc, hi[1] * sc, hi[2] * sc, hi[3] * sc};
-        if (j0 + row < len_k)
-          put_grad8<T>(dst, dst_off + (int64_t)(j0 + row) * dst_st + c * 4, M::pack(x), a.wide_dkv, a.dkv_accumulate);
-      }
+            for (int w = 1; w < 4; w++) {
+              lo += *(const f32x4*)(src + w * W_LDS + at0);
+              hi += *(const f32x4*)(src + w * W_LDS + at1);
+            }
+            const float x[8] = {lo[0] * sc, lo[1] * sc, lo[2] * sc, lo[3] * sc,
+                                hi[0] * sc, hi[1] * sc, hi[2] * sc, hi[3] * sc};
+            return M::pack(x);
+          });
       __syncthreads();
     }
     return;
@@ -764,15 +775,14 @@ __global__ __launch_bounds__(256) void attn_bwd_dkdv_kernel(const AttnArgs a) {
       void* const dst = mtx == 0 ? dk_buf : dv_buf;
       const int64_t dst_off = mtx == 0 ? dk_off : dv_off;
       const int64_t dst_st = mtx == 0 ? a.dk_st[1] : a.dv_st[1];
-#pragma unroll
-      for (int n = 0; n < 32 * C::CPR / 64; n++) {
-        const int idx = n * 64 + lane_e;
-        const int row = idx / C::CPR, c = idx % C::CPR;
-        const V8 val = *(const V8*)(stage + row * C::ROWB + ((c ^ (row & (C::CPR - 1))) << 4));
-        const int jc = jw0 + kb * 32 + row;
-        if (jc < len_k)
-          put_grad8<T>(dst, dst_off + (int64_t)jc * dst_st + c * 8, val, a.wide_dkv, a.dkv_accumulate);
-      }
+      constexpr int RPI = 64 / C::CPR;
+      const int row0 = lane_e / C::CPR, c = lane_e % C::CPR;
+      const int64_t at = dst_off + (int64_t)(jw0 + kb * 32 + row0) * dst_st + c * 8;
+      put_rows<T, RPI, 32 / RPI>(dst, at, dst_st, len_k - jw0 - kb * 32 - row0, jw0 + kb * 32 + 31 < len_k,
+                                 a.wide_dkv, a.dkv_accumulate, [&](int n) {
+                                   const int row = row0 + n * RPI;
+                                   return *(const V8*)(stage + row * C::ROWB + ((c ^ (row & (C::CPR - 1))) << 4));
+                                 });
       asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // read before the next block overwrites
     }
 }
@@ -1109,18 +1119,20 @@ void attn_bwd_dq_kernel(const AttnArgs a) {
   const bool pair = (a.group & 1) == 0;
   const int units = pair ? a.group >> 1 : a.group;
   const int bm = pair ? 16 * NW : 32 * NW;
-  const int hu = wid % units;
-  int rest = wid / units;
-  const int slot = a.rev_q ? a.n_tile - 1 - rest % a.n_tile : rest % a.n_tile;
-  rest /= a.n_tile;
-  const int hk = rest % a.heads_kv;
+  int rest = quotient(wid, a.by_units);
+  const int hu = wid - rest * units;
+  const int tiles_before = quotient(rest, a.by_tile);
+  const int tile = rest - tiles_before * a.n_tile;
+  const int slot = a.rev_q ? a.n_tile - 1 - tile : tile;
+  rest = quotient(tiles_before, a.by_heads);  // batch entry (dense)
+  const int hk = tiles_before - rest * a.heads_kv;
   const int hq = hk * a.group + (pair ? 2 * hu + (wave >> HSH) : hu);
   SeqInfo s;
   int qt;
   if (a.cu_q) {
     if (!locate_packed(a, slot, (pair ? 4 : 5) + (NW == 8 ? 3 : 2), false, s, qt)) return;
   } else {
-    s.batch_idx = rest / a.heads_kv;
+    s.batch_idx = rest;
     s.q_row0 = s.k_row0 = 0;
     s.len_q = a.seqlen_q;
     s.len_k = a.seqlen_k;
@@ -1156,60 +1168,79 @@ void attn_bwd_dq_kernel(const AttnArgs a) {
   const RowBounds wb_first = row_bounds(a, r0, len_q, len_k);
   const RowBounds wb_last = row_bounds(a, min(r0 + 31, len_q - 1), len_q, len_k);
 
+  TileDma<D, C::BN, NW * 64, true> k_dma, v_dma;
+  k_dma.init(a.k_st[1], tid);
+  v_dma.init(a.v_st[1], tid);
+  const int k_row_bytes = (int)(a.k_st[1] * 2), v_row_bytes = (int)(a.v_st[1] * 2);
+  // (keys in two row ranges: the second range's tensors, at this batch entry and kv head)
+  const T* k2_ptr = a.k2 ? (const T*)a.k2 + b * a.k_st[0] + hk * a.k_st[2] : k_ptr;
+  const T* v2_ptr = a.v2 ? (const T*)a.v2 + b * a.v_st[0] + hk * a.v_st[2] : v_ptr;
+  auto load_tile = [&](int it, char* kd, char* vd) __attribute__((always_inline)) {
+    const int j = tile_of(it) * C::BN;
+    const KeySeg<T> gk = key_seg(k_ptr, k2_ptr, a.seg, j, len_k);
+    const KeySeg<T> gv = key_seg(v_ptr, v2_ptr, a.seg, j, len_k);
+    k_dma.load(tile_src<C::BN, FAR>(gk.base, gk.row0, gk.rows, k_row_bytes, C::ROWB), kd);
+    v_dma.load(tile_src<C::BN, FAR>(gv.base, gv.row0, gv.rows, v_row_bytes, C::ROWB), vd);
+  };
+
+  // The first tiles are asked for ahead of the rows' own data, and of that everything before the first
+  // use: one 16-row half after the other with its statistics, then the tiles, were three round trips to
+  // memory, 8 us of a block's start (of 53 at window 1000, of 18 in a pack of short sequences), now 7.
+  // us, before / after: a pack of 16384 tokens in sequences of 16 to 1024 189 / 183; rows 8192 with the
+  // statistics, window 4096, 664 / 655; 4001 rows, window 1024, 93.7 / 93.1.
+  if (n_tiles > 0) load_tile(0, k_s0, v_s0);
+
   // Q / dO fragments (B operands) and the (negated) statistics of the lane's two query rows.  The
   // dP^T accumulator chains start from -delta: the MFMAs then deliver dP - delta, and the vector ALU
   // is left with a multiply-add, an exponential, a product and the 16-bit conversion per score.
+  // All loads are issued before the first use.  (Rows past the end read the last row's values:
+  // their columns are masked in every tile and never stored.)
   V8 qf[2][KS], dof[2][KS];
+  float lse2[2];   // -lse2 of the lane's two queries
+  f32x4 delta[2];  // -delta of the same, in all four elements (start value of the dP^T chains)
+  [[maybe_unused]] V8 of[2][KS];
+#pragma unroll
+  for (int qb = 0; qb < 2; qb++) {
+    const int iq = r0 + 16 * qb + r, row = min(iq, len_q - 1);
+    const T* q_row = q_ptr + (int64_t)row * a.q_st[1] + u * 8;
+    const T* do_row = do_ptr + (int64_t)row * a.do_st[1] + u * 8;
+#pragma unroll
+    for (int ks = 0; ks < KS; ks++) dof[qb][ks] = *(const V8*)(do_row + ks * 32);
+    if constexpr (STATS) {
+      const T* o_row = (const T*)a.out + b * a.o_st[0] + (s.q_row0 + row) * a.o_st[1] + hq * a.o_st[2] + u * 8;
+#pragma unroll
+      for (int ks = 0; ks < KS; ks++) of[qb][ks] = *(const V8*)(o_row + ks * 32);
+      lse2[qb] = a.lse[b * a.lse_st[0] + hq * a.lse_st[1] + (s.q_row0 + row) * a.lse_st[2]];
+    } else {
+      lse2[qb] = a.lse2[(int64_t)hq * a.rows_q + ws_row0 + row];
+      delta[qb][0] = a.delta[(int64_t)hq * a.rows_q + ws_row0 + row];
+    }
+#pragma unroll
+    for (int ks = 0; ks < KS; ks++) qf[qb][ks] = *(const V8*)(q_row + ks * 32);
+  }
   if constexpr (STATS) {
     // the elements behind the lse2 array (see attn_bwd_prep_kernel), where block 0 surely is at
     // work; for a pack, whose first slot may stand for no tile, attn_bwd_rest_kernel writes them
     const int64_t used = a.rows_q * a.heads_q;
     if (!a.cu_q && wid == 0 && used + tid < a.delta - a.lse2) a.lse2[used + tid] = -__builtin_inff();
   }
-  float lse2[2];   // -lse2 of the lane's two queries
-  f32x4 delta[2];  // -delta of the same, in all four elements (start value of the dP^T chains)
 #pragma unroll
   for (int qb = 0; qb < 2; qb++) {
     const int iq = r0 + 16 * qb + r;
-    float l2 = -__builtin_inff(), dl = 0.f;
-    if (iq < len_q) {
-#pragma unroll
-      for (int ks = 0; ks < KS; ks++) {
-        qf[qb][ks] = *(const V8*)(q_ptr + (int64_t)iq * a.q_st[1] + ks * 32 + u * 8);
-        dof[qb][ks] = *(const V8*)(do_ptr + (int64_t)iq * a.do_st[1] + ks * 32 + u * 8);
-      }
-      if constexpr (!STATS) {
-        l2 = a.lse2[(int64_t)hq * a.rows_q + ws_row0 + iq];
-        dl = a.delta[(int64_t)hq * a.rows_q + ws_row0 + iq];
-      }
-    } else {
-#pragma unroll
-      for (int ks = 0; ks < KS; ks++) {
-        qf[qb][ks] = V8{0, 0, 0, 0, 0, 0, 0, 0};
-        dof[qb][ks] = V8{0, 0, 0, 0, 0, 0, 0, 0};
-      }
-    }
     if constexpr (STATS) {
       // delta = sum over d of dO * O: eight elements a time, then the 16 (8) parts of a row
       // pairwise from the farthest, as in the statistics kernel
       float part[KS];
 #pragma unroll
-      for (int ks = 0; ks < KS; ks++) part[ks] = 0.f;
-      if (iq < len_q) {
-        const T* o_ptr = (const T*)a.out + b * a.o_st[0] + (s.q_row0 + iq) * a.o_st[1] + hq * a.o_st[2];
-        const float l = a.lse[b * a.lse_st[0] + hq * a.lse_st[1] + (s.q_row0 + iq) * a.lse_st[2]];
+      for (int ks = 0; ks < KS; ks++) {
+        part[ks] = 0.f;
 #pragma unroll
-        for (int ks = 0; ks < KS; ks++) {
-          const V8 o8 = *(const V8*)(o_ptr + ks * 32 + u * 8);
-#pragma unroll
-          for (int j = 0; j < 8; j++) {
-            // (products of 16-bit values are exact; contracted, fp16 becomes v_dot2, which rounds
-            // otherwise than the statistics kernel)
+        for (int j = 0; j < 8; j++) {
+          // (products of 16-bit values are exact; contracted, fp16 becomes v_dot2, which rounds
+          // otherwise than the statistics kernel)
 #pragma clang fp contract(off)
-            part[ks] += (float)o8[j] * (float)dof[qb][ks][j];
-          }
+          part[ks] += (float)of[qb][ks][j] * (float)dof[qb][ks][j];
         }
-        l2 = (l == -__builtin_inff()) ? l : -l * kLog2e;
       }
 #pragma unroll
       for (int m = KS / 2; m >= 1; m >>= 1)
@@ -1218,13 +1249,14 @@ void attn_bwd_dq_kernel(const AttnArgs a) {
       float sum = part[0];
       sum += __shfl_xor(sum, 32, 64);
       sum += __shfl_xor(sum, 16, 64);
-      dl = -sum;
+      lse2[qb] = (lse2[qb] == -__builtin_inff()) ? lse2[qb] : -lse2[qb] * kLog2e;
+      delta[qb][0] = -sum;
       if (u == 0 && iq < len_q) {
-        a.lse2[(int64_t)hq * a.rows_q + ws_row0 + iq] = l2;
-        a.delta[(int64_t)hq * a.rows_q + ws_row0 + iq] = dl;
+        a.lse2[(int64_t)hq * a.rows_q + ws_row0 + iq] = lse2[qb];
+        a.delta[(int64_t)hq * a.rows_q + ws_row0 + iq] = delta[qb][0];
       }
     }
-    lse2[qb] = l2;
+    const float dl = delta[qb][0];
     delta[qb] = f32x4{dl, dl, dl, dl};
   }
 
@@ -1243,21 +1275,6 @@ void attn_bwd_dq_kernel(const AttnArgs a) {
   //   offset = (t_row ^ (db << 5)) + (32 ks2 + 16 blk) * ROWB
   const int rl = 4 * u + (r >> 2);
   const int t_row = rl * C::ROWB + ((((r & 3) >> 1) ^ swz16_f<C::CPR>(rl)) << 4) + (r & 1) * 8;
-
-  TileDma<D, C::BN, NW * 64, true> k_dma, v_dma;
-  k_dma.init(a.k_st[1], tid);
-  v_dma.init(a.v_st[1], tid);
-  const int k_row_bytes = (int)(a.k_st[1] * 2), v_row_bytes = (int)(a.v_st[1] * 2);
-  // (keys in two row ranges: the second range's tensors, at this batch entry and kv head)
-  const T* k2_ptr = a.k2 ? (const T*)a.k2 + b * a.k_st[0] + hk * a.k_st[2] : k_ptr;
-  const T* v2_ptr = a.v2 ? (const T*)a.v2 + b * a.v_st[0] + hk * a.v_st[2] : v_ptr;
-  auto load_tile = [&](int it, char* kd, char* vd) __attribute__((always_inline)) {
-    const int j = tile_of(it) * C::BN;
-    const KeySeg<T> gk = key_seg(k_ptr, k2_ptr, a.seg, j, len_k);
-    const KeySeg<T> gv = key_seg(v_ptr, v2_ptr, a.seg, j, len_k);
-    k_dma.load(tile_src<C::BN, FAR>(gk.base, gk.row0, gk.rows, k_row_bytes, C::ROWB), kd);
-    v_dma.load(tile_src<C::BN, FAR>(gv.base, gv.row0, gv.rows, v_row_bytes, C::ROWB), vd);
-  };
 
   auto step = [&](int it, const char* kc, const char* vc, char* kn,
                   char* vn) __attribute__((always_inline)) {
@@ -1373,7 +1390,6 @@ void attn_bwd_dq_kernel(const AttnArgs a) {
     __syncthreads();
   };
 
-  if (n_tiles > 0) load_tile(0, k_s0, v_s0);
   __syncthreads();
   for (int it = 0; it < n_tiles; it += 2) {
     step(it, k_s0, v_s0, k_s1, v_s1);
@@ -1396,16 +1412,12 @@ void attn_bwd_dq_kernel(const AttnArgs a) {
     }
     __syncthreads();
     if ((wave >> 2) == half) {
-#pragma unroll
-      for (int n = 0; n < 32 * C::CPR / 64; n++) {
-        const int c = lane + n * 64;
-        const int row = c / C::CPR, col = (c % C::CPR) * 8;
-        if (r0 + row < len_q) {
-          const V8 val = *(const V8*)(stage + row * C::O_STRIDE + col * 2);
-          put_grad8<T>(a.dq, dq_off + (int64_t)(r0 + row) * a.dq_st[1] + col, val, a.wide_dq,
-                       a.dq_accumulate);
-        }
-      }
+      constexpr int RPI = 64 / C::CPR;
+      const int row0 = lane / C::CPR, col = (lane % C::CPR) * 8;
+      const char* src = stage + row0 * C::O_STRIDE + col * 2;
+      put_rows<T, RPI, 32 / RPI>(a.dq, dq_off + (int64_t)(r0 + row0) * a.dq_st[1] + col, a.dq_st[1],
+                                 len_q - r0 - row0, wave_rows_full, a.wide_dq, a.dq_accumulate,
+                                 [&](int n) { return *(const V8*)(src + n * RPI * C::O_STRIDE); });
     }
     __syncthreads();
   }
@@ -1849,6 +1861,7 @@ int launch_bwd(AttnArgs& a, hipStream_t stream, int phases) {
       a.n_work = a.n_tile * units_q * a.batch;
     }
     if (a.n_work == 0) return (int)RSWA_OK;
+    set_divisors(a, units_q / a.heads_kv);
     clear_launch_error();
     const dim3 grid(padded_grid(a.n_work)), block(small ? 256 : 512);
     if constexpr (!STATS) {

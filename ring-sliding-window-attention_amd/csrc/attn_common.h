@@ -21,6 +21,21 @@ namespace rswa {
 
 constexpr float kLog2e = 1.4426950408889634f;
 
+// Division of 0 <= n < 2^31 by a launch constant as a multiplication and a shift (a division by a value
+// the compiler does not know is some 30 dependent instructions, five of them ahead of a block's first
+// load).
+struct FastDiv {
+  uint32_t d, mul, shift;
+};
+inline FastDiv fast_div(uint32_t d) {  // d >= 1
+  uint32_t s = 0;
+  while ((1ull << s) < d) s++;
+  return {d, (uint32_t)(((1ull << 32) * ((1ull << s) - d)) / d + 1), s};
+}
+__device__ __forceinline__ int quotient(int n, const FastDiv& f) {
+  return (int)((__umulhi((uint32_t)n, f.mul) + (uint32_t)n) >> f.shift);
+}
+
 // Kernel-side view of rswa_attn_params (strides in elements).
 struct AttnArgs {
   const void* q;
@@ -57,6 +72,7 @@ struct AttnArgs {
   int32_t wide_out, wide_dq, wide_dkv, dkv_accumulate;
   int32_t n_tile;          // tiles per sequence (dense) / total tile slots (packed)
   int32_t n_work;          // logical blocks
+  FastDiv by_tile, by_heads, by_units;  // n_tile, heads_kv, blocks per (kv head, tile)
   // Blocks are dispatched in logical order; these flags reverse the order of the query
   // tiles (forward, dQ) or key tiles (dK/dV) so that the tiles with the most visible
   // pairs start first and the short ones fill the tail of the launch.
@@ -107,6 +123,12 @@ __device__ __forceinline__ int logical_block_id(int n_work) {
   return id < n_work ? id : -1;
 }
 
+inline void set_divisors(AttnArgs& a, int blocks_per_tile) {
+  a.by_tile = fast_div((uint32_t)a.n_tile);
+  a.by_heads = fast_div((uint32_t)a.heads_kv);
+  a.by_units = fast_div((uint32_t)blocks_per_tile);
+}
+
 static inline unsigned padded_grid(int64_t n_work) { return (unsigned)(ceil_div(n_work, 8) * 8); }
 
 // Mask bounds of one query row i (local index): visible keys are
@@ -126,19 +148,27 @@ __device__ __forceinline__ RowBounds row_bounds(const AttnArgs& a, int i, int le
 
 // Packed mode: which sequence, and which of its tiles of `tile` = 2^tile_log2 rows, does
 // tile slot `t` along the q or k axis stand for?  Sequence b owns the slots from
-// cu[b] / tile + b on -- strictly increasing in b, so a binary search over cu finds b in
-// log2(batch) dependent loads, where a running count of tiles would have to walk every
-// sequence before it.  ceil(len_b / tile) of its slots are its tiles; at most one more, before
+// cu[b] / tile + b on -- strictly increasing in b, so a search over cu finds b, where a running
+// count of tiles would have to walk every sequence before it.  The search goes 64 ways at a time (each
+// lane tests one entry, the ballot counts those at or below t): one load deep up to 64 sequences, two up
+// to 4096, where halving took a dependent load per factor of two, 7 of them ahead of a block's first
+// load in a pack of 70 sequences.  Every lane takes part; the results are wave-uniform.
+// ceil(len_b / tile) of its slots are its tiles; at most one more, before
 // the next sequence's first, stays unused (false is returned for it), which is why a packed
 // grid has ceil(rows / tile) + batch slots.
 __device__ __forceinline__ bool locate_packed(const AttnArgs& a, int t, int tile_log2, bool along_k,
                                               SeqInfo& s, int& tile_in_seq) {
   const int32_t* cu = along_k ? a.cu_k : a.cu_q;
-  int lo = 0, hi = a.batch;  // first slot of lo <= t; hi == batch or first slot of hi > t
-  while (hi - lo > 1) {
-    const int mid = (lo + hi) >> 1;
-    if ((cu[mid] >> tile_log2) + mid <= t) lo = mid;
-    else hi = mid;
+  const int lane = (int)__builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, 0u));
+  int lo = 0, n = a.batch;  // the sequence is one of lo .. lo + n - 1
+  for (;;) {
+    const int step = (n + 63) >> 6;
+    const int i = min(lo + lane * step, lo + n - 1);
+    const int slot = (cu[i] >> tile_log2) + i;
+    const int at = max(__popcll(__builtin_amdgcn_ballot_w64(lane * step < n && slot <= t)) - 1, 0);
+    lo += at * step;
+    if (step == 1) break;
+    n = min(step, n - at * step);
   }
   const int b = lo;
   const int first = cu[b];

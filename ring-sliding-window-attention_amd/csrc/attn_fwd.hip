@@ -70,18 +70,20 @@ void attn_fwd_kernel(const AttnArgs a) {
   const bool pair = (a.group & 1) == 0;
   const int units = pair ? a.group >> 1 : a.group;  // blocks per (kv head, q tile)
   const int bm = pair ? 16 * NW : 32 * NW;          // query rows per block
-  const int hu = wid % units;
-  int rest = wid / units;
-  const int slot = a.rev_q ? a.n_tile - 1 - rest % a.n_tile : rest % a.n_tile;
-  rest /= a.n_tile;
-  const int hk = rest % a.heads_kv;
+  int rest = quotient(wid, a.by_units);
+  const int hu = wid - rest * units;
+  const int tiles_before = quotient(rest, a.by_tile);
+  const int tile = rest - tiles_before * a.n_tile;
+  const int slot = a.rev_q ? a.n_tile - 1 - tile : tile;
+  rest = quotient(tiles_before, a.by_heads);  // batch entry (dense)
+  const int hk = tiles_before - rest * a.heads_kv;
   const int hq = hk * a.group + (pair ? 2 * hu + (wave >> 1) : hu);
   SeqInfo s;
   int qt;
   if (a.cu_q) {
     if (!locate_packed(a, slot, pair ? 6 : 7, false, s, qt)) return;
   } else {
-    s.batch_idx = rest / a.heads_kv;
+    s.batch_idx = rest;
     s.q_row0 = s.k_row0 = 0;
     s.len_q = a.seqlen_q;
     s.len_k = a.seqlen_k;
@@ -119,16 +121,39 @@ void attn_fwd_kernel(const AttnArgs a) {
   const RowBounds wb_first = row_bounds(a, r0, len_q, len_k);
   const RowBounds wb_last = row_bounds(a, min(r0 + 31, len_q - 1), len_q, len_k);
 
-  // Q fragments (B operand of K Q^T): lane = query column, 8 consecutive d per k-step.
+  // ---- tile DMA: rows past len_k read as zero ---------------------------------
+  TileDma<D, C::BN, C::THREADS> k_dma, v_dma;
+  k_dma.init(a.k_st[1], tid);
+  v_dma.init(a.v_st[1], tid);
+  const int k_row_bytes = (int)(a.k_st[1] * 2), v_row_bytes = (int)(a.v_st[1] * 2);
+  // (keys in two row ranges: the second range's tensors, at this batch entry and kv head)
+  const T* k2_ptr = a.k2 ? (const T*)a.k2 + b * a.k_st[0] + hk * a.k_st[2] : k_ptr;
+  const T* v2_ptr = a.v2 ? (const T*)a.v2 + b * a.v_st[0] + hk * a.v_st[2] : v_ptr;
+  auto load_k = [&](int it, char* dst) __attribute__((always_inline)) {
+    const KeySeg<T> g = key_seg(k_ptr, k2_ptr, a.seg, tile_of(it) * C::BN, len_k);
+    k_dma.load(tile_src<C::BN, FAR>(g.base, g.row0, g.rows, k_row_bytes, C::ROWB), dst);
+  };
+  auto load_v = [&](int it, char* dst) __attribute__((always_inline)) {
+    const KeySeg<T> g = key_seg(v_ptr, v2_ptr, a.seg, tile_of(it) * C::BN, len_k);
+    v_dma.load(tile_src<C::BN, FAR>(g.base, g.row0, g.rows, v_row_bytes, C::ROWB), dst);
+  };
+
+  // The first tiles and the rows' own data are asked for before anything else is computed: K(0) and Q
+  // first, which S(0) needs.  (A block's start and end are 6 of its 31 us at window 1024, 6 of 13 in a
+  // pack of short sequences.  This, divisions by multiplication, the search of locate_packed and an
+  // epilogue without branches or a 64-bit product per row: us, before / after, 4001 rows, window 1024,
+  // 32 / 8 heads 75.4 / 73.0; a pack of 16384 tokens in sequences of 16 to 1024 149 / 144; 2 x 8192 rows,
+  // 32 heads, window 1000 358 / 351; 4 x 2000 rows, 28 / 4 heads, head_dim 64, fp16 79.0 / 76.1.)
+  if (n_tiles > 0) load_k(0, k_s0);
+  // Q fragments (B operand of K Q^T): lane = query column, 8 consecutive d per k-step.  (Rows past the
+  // end read the last row's values: their columns are masked in every tile and never stored.)
+  const T* q_row = q_ptr + (int64_t)min(iq, len_q - 1) * a.q_st[1] + g * 8;
   V8 qf[C::KSTEPS];
 #pragma unroll
-  for (int ks = 0; ks < C::KSTEPS; ks++) {
-    if (iq < len_q) {
-      qf[ks] = *(const V8*)(q_ptr + (int64_t)iq * a.q_st[1] + ks * 16 + g * 8);
-    } else {
-      qf[ks] = V8{0, 0, 0, 0, 0, 0, 0, 0};
-    }
-  }
+  for (int ks = 0; ks < C::KSTEPS; ks++) qf[ks] = *(const V8*)(q_row + ks * 16);
+
+  if (n_tiles > 0) load_v(0, v_s0);
+  if (n_tiles > 1) load_k(1, k_s1);
 
   f32x16 o_acc[C::DBLK];
 #pragma unroll
@@ -148,23 +173,6 @@ void attn_fwd_kernel(const AttnArgs a) {
   const int lp = 2 * (u & 1) + ((i16 & 3) >> 1);
   const int t_row0 = rl * C::ROWB + ((lp ^ swz_f<C::CPR>(rl)) << 4) + (i16 & 1) * 8;
   const int t_row1 = (rl + 8) * C::ROWB + ((lp ^ swz_f<C::CPR>(rl + 8)) << 4) + (i16 & 1) * 8;
-
-  // ---- tile DMA: rows past len_k read as zero ---------------------------------
-  TileDma<D, C::BN, C::THREADS> k_dma, v_dma;
-  k_dma.init(a.k_st[1], tid);
-  v_dma.init(a.v_st[1], tid);
-  const int k_row_bytes = (int)(a.k_st[1] * 2), v_row_bytes = (int)(a.v_st[1] * 2);
-  // (keys in two row ranges: the second range's tensors, at this batch entry and kv head)
-  const T* k2_ptr = a.k2 ? (const T*)a.k2 + b * a.k_st[0] + hk * a.k_st[2] : k_ptr;
-  const T* v2_ptr = a.v2 ? (const T*)a.v2 + b * a.v_st[0] + hk * a.v_st[2] : v_ptr;
-  auto load_k = [&](int it, char* dst) __attribute__((always_inline)) {
-    const KeySeg<T> g = key_seg(k_ptr, k2_ptr, a.seg, tile_of(it) * C::BN, len_k);
-    k_dma.load(tile_src<C::BN, FAR>(g.base, g.row0, g.rows, k_row_bytes, C::ROWB), dst);
-  };
-  auto load_v = [&](int it, char* dst) __attribute__((always_inline)) {
-    const KeySeg<T> g = key_seg(v_ptr, v2_ptr, a.seg, tile_of(it) * C::BN, len_k);
-    v_dma.load(tile_src<C::BN, FAR>(g.base, g.row0, g.rows, v_row_bytes, C::ROWB), dst);
-  };
 
   // ---- pieces of one tile ------------------------------------------------------
   // S^T[key, query] = K Q^T
@@ -324,11 +332,6 @@ void attn_fwd_kernel(const AttnArgs a) {
     }
   };
 
-  if (n_tiles > 0) {
-    load_k(0, k_s0);
-    load_v(0, v_s0);
-  }
-  if (n_tiles > 1) load_k(1, k_s1);
   __syncthreads();
   if (wave_needs(0)) qk(k_s0, s_cur);
   for (int it = 0; it < n_tiles; it += 2) {
@@ -381,13 +384,28 @@ void attn_fwd_kernel(const AttnArgs a) {
       wgt[2 * l32 + 1] = w_new;
     }
     asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    constexpr int RPI = 64 / C::CPR, N = 32 / RPI;  // rows per store instruction, stores
+    const int row0 = lane / C::CPR, col = (lane % C::CPR) * 8;
+    const char* src = stage + row0 * C::O_STRIDE + col * 2;
+    const int64_t at0 = o_off + (int64_t)(r0 + row0) * a.o_st[1] + col, step = RPI * a.o_st[1];
+    const int left = len_q - r0 - row0;  // rows the lane has to store: n RPI < left
+    if (!(a.wide_out | a.out_accumulate)) {
+      T* dst = (T*)a.out + at0;
+      if (wave_rows_full) {
 #pragma unroll
-    for (int n = 0; n < 32 * C::CPR / 64; n++) {
-      const int c = lane + n * 64;
-      const int row = c / C::CPR, col = (c % C::CPR) * 8;
-      if (r0 + row < len_q) {
-        V8 val = *(const V8*)(stage + row * C::O_STRIDE + col * 2);
-        const int64_t at = o_off + (int64_t)(r0 + row) * a.o_st[1] + col;
+        for (int n = 0; n < N; n++) *(V8*)(dst + n * step) = *(const V8*)(src + n * RPI * C::O_STRIDE);
+      } else {
+#pragma unroll
+        for (int n = 0; n < N; n++)
+          if (n * RPI < left) *(V8*)(dst + n * step) = *(const V8*)(src + n * RPI * C::O_STRIDE);
+      }
+      return;
+    }
+    for (int n = 0; n < N; n++) {
+      if (n * RPI < left) {
+        V8 val = *(const V8*)(src + n * RPI * C::O_STRIDE);
+        const int64_t at = at0 + n * step;
+        const int row = row0 + n * RPI;
         const float wo = a.out_accumulate ? wgt[2 * row] : 0.f;
         const float wn = a.out_accumulate ? wgt[2 * row + 1] : 1.f;
         if (a.wide_out) {
@@ -409,19 +427,16 @@ void attn_fwd_kernel(const AttnArgs a) {
           *(f32x4*)(dst + 4) = y[1];
         } else {
           T* dst = (T*)a.out + at;
-          if (a.out_accumulate) {
-            const V8 old = *(const V8*)dst;
-            float y[8];
+          const V8 old = *(const V8*)dst;
+          float y[8];
 #pragma unroll
-            for (int j = 0; j < 8; j++) {
-              // a zero weight must annihilate whatever the other side holds
-              const float t0 = (wo == 0.f) ? 0.f : (float)old[j] * wo;
-              const float t1 = (wn == 0.f) ? 0.f : (float)val[j] * wn;
-              y[j] = t0 + t1;
-            }
-            val = M::pack(y);
+          for (int j = 0; j < 8; j++) {
+            // a zero weight must annihilate whatever the other side holds
+            const float t0 = (wo == 0.f) ? 0.f : (float)old[j] * wo;
+            const float t1 = (wn == 0.f) ? 0.f : (float)val[j] * wn;
+            y[j] = t0 + t1;
           }
-          *(V8*)dst = val;
+          *(V8*)dst = M::pack(y);
         }
       }
     }
@@ -477,6 +492,7 @@ int launch_fwd(AttnArgs& a, hipStream_t stream) {
     a.n_work = a.n_tile * units * a.batch;
   }
   if (a.n_work == 0) return RSWA_OK;
+  set_divisors(a, units / a.heads_kv);
   // keys a row sees at most; the per-wave tile skip pays when the rows of a block beyond one
   // wave's 32 add a tenth or more to that span
   const int64_t span = (a.wl < 0 || a.wr < 0) ? (int64_t)1 << 40 : (int64_t)a.wl + a.wr + 1;
