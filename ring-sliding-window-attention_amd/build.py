@@ -1,7 +1,8 @@
-"""Build librswa.so (HIP, gfx950 only) in-tree with hipcc.
+"""Build librswa.so (HIP, gfx950 only) in-tree with hipcc, and the module that calls it from
+PyTorch (host code) with the C++ compiler.
 
 Usage: ``python build.py [--force]``.  Objects go to ``build/``, the shared
-library to ``lib/librswa.so`` next to this file.  hipcc cross-compiles, so no
+library to ``lib/librswa.so`` next to this file, the module to ``lib/rswa_torch.so``.  hipcc cross-compiles, so no
 GPU is needed to build.
 """
 from __future__ import annotations
@@ -205,16 +206,39 @@ def _check_lds_loads(obj: str) -> None:
                                        + "\n  ".join(bad))
 
 
+def _build_torch_calls(force: bool) -> str:
+    """The module of csrc/torch_calls.cpp, against the installed PyTorch."""
+    src, out = os.path.join(CSRC, "torch_calls.cpp"), os.path.join(LIBDIR, "rswa_torch.so")
+    if force or _stale(out, [src] + _headers()):
+        import sysconfig
+
+        import torch
+
+        root = os.path.dirname(torch.__file__)
+        inc = [os.path.join(root, "include"), os.path.join(root, "include", "torch", "csrc", "api", "include"),
+               os.path.join(os.environ.get("ROCM_PATH", "/opt/rocm"), "include"), sysconfig.get_paths()["include"]]
+        cmd = [os.environ.get("CXX", "g++"), "-O2", "-std=c++17", "-fPIC", "-shared", "-Wall", "-D__HIP_PLATFORM_AMD__=1",
+               "-DUSE_ROCM=1", f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}",
+               *[x for i in inc for x in ("-isystem", i)], src, "-o", out, "-L" + os.path.join(root, "lib"),
+               *["-l" + n for n in ("c10", "c10_hip", "torch_cpu", "torch_hip", "torch", "torch_python")]]
+        r = subprocess.run(cmd, capture_output=True, text=True)
+        if r.returncode != 0:
+            raise RuntimeError(f"C++ compiler failed for {src}:\n{r.stdout}\n{r.stderr}")
+    return out
+
+
 def build(force: bool = False, jobs: int = 8) -> str:
     os.makedirs(OBJ, exist_ok=True)
     os.makedirs(LIBDIR, exist_ok=True)
     srcs = sources()
     asm_srcs = [s for s in srcs if os.path.basename(s) in ASM_MFMA_SOURCES]
-    with cf.ThreadPoolExecutor(max_workers=min(jobs, len(srcs) + len(asm_srcs))) as ex:
+    with cf.ThreadPoolExecutor(max_workers=min(jobs, len(srcs) + len(asm_srcs) + 1)) as ex:
+        calls = ex.submit(_build_torch_calls, force)
         futs = [ex.submit(_compile, s, force) for s in srcs]
         alt_futs = {s: ex.submit(_compile, s, force, True) for s in asm_srcs}
         objs = [f.result() for f in futs]
         alt = {s: f.result() for s, f in alt_futs.items()}
+        calls.result()
     for o in objs:
         if os.path.basename(o)[:-2] + ".hip" in ASM_MFMA_SOURCES and (force or _stale(LIB, [o])):
             _check_lds_loads(o)

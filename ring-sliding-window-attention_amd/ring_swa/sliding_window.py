@@ -12,7 +12,26 @@ from typing import Optional
 
 import torch
 
+from . import _lib
 from .ops.band_attn import attn_bwd, attn_fwd
+
+
+def band_backward(q, k, v, out, lse, do, dq, dk, dv, softmax_scale, window_size, cu_seqlens, num_sink):
+    attn_bwd(q, k, v, out, lse, do, dq, dk, dv, softmax_scale, (window_size, 0), True, cu_seqlens,
+             cu_seqlens, num_sink=num_sink)
+
+
+def band_attn(q, k, v, window_size, softmax_scale, cu_seqlens, num_sink):
+    """One band over a sequence or a pack, differentiable.  The native node takes every call that it can
+    answer (tensors on the GPU in the kernels' layout, nothing tracing or transforming the call);
+    :class:`BandAttnFunc` takes or refuses the rest."""
+    if q.is_cuda and not torch.compiler.is_compiling():
+        calls = _lib.torch_calls()
+        if calls is not None:
+            out = calls.band_attn(q, k, v, window_size, softmax_scale, cu_seqlens, num_sink)
+            if out is not None:
+                return out
+    return BandAttnFunc.apply(q, k, v, window_size, softmax_scale, cu_seqlens, num_sink)
 
 
 class BandAttnFunc(torch.autograd.Function):
@@ -40,8 +59,7 @@ class BandAttnFunc(torch.autograd.Function):
         if do.stride(-1) != 1:
             do = do.contiguous()
         dq, dk, dv = torch.empty_like(q), torch.empty_like(k), torch.empty_like(v)
-        attn_bwd(q, k, v, out, lse, do, dq, dk, dv, softmax_scale, (window_size, 0), True,
-                 ctx.cu_seqlens, ctx.cu_seqlens, num_sink=num_sink)
+        band_backward(q, k, v, out, lse, do, dq, dk, dv, softmax_scale, window_size, ctx.cu_seqlens, num_sink)
         return dq, dk, dv, None, None, None, None
 
 
@@ -114,7 +132,7 @@ def ring_sliding_window_attn(
         cp_size, cp_local_rank = _ring_ranks(cp_group, cp_size, cp_local_rank,
                                              cp_prev_global_rank, cp_next_global_rank)
         return ring_attn(q, k, v, window_size, cp_group, cp_size, cp_local_rank, softmax_scale)
-    return BandAttnFunc.apply(q, k, v, int(window_size), softmax_scale, None, 0)
+    return band_attn(q, k, v, int(window_size), softmax_scale, None, 0)
 
 
 def ring_sliding_window_attn_varlen(
@@ -144,4 +162,4 @@ def ring_sliding_window_attn_varlen(
         return ring_attn(q, k, v, window_size, cp_group, cp_size, cp_local_rank, softmax_scale,
                          cu_seqlens)
     _check_packed(q, k, v, cu_seqlens, cp_size)
-    return BandAttnFunc.apply(q, k, v, int(window_size), softmax_scale, cu_seqlens.contiguous(), 0)
+    return band_attn(q, k, v, int(window_size), softmax_scale, cu_seqlens.contiguous(), 0)

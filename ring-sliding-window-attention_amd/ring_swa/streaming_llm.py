@@ -33,7 +33,7 @@ import torch
 
 from .ops.band_attn import attn_bwd, attn_fwd
 from .ops.lse_merge import merge_attn_out
-from .sliding_window import BandAttnFunc, _check_dense, _check_packed, _ring_ranks
+from .sliding_window import band_attn, _check_dense, _check_packed, _ring_ranks
 
 
 class SinkWindowSplitFunc(torch.autograd.Function):
@@ -150,8 +150,7 @@ def ring_streaming_llm_attn(
         return ring_slm_attn(q, k, v, window_size, cp_group, cp_size, cp_local_rank,
                              softmax_scale, num_sink_tokens=num_sink_tokens)
     if _impl(impl) or num_sink_tokens == 0:
-        return BandAttnFunc.apply(q, k, v, int(window_size), softmax_scale, None,
-                                  int(num_sink_tokens))
+        return band_attn(q, k, v, int(window_size), softmax_scale, None, int(num_sink_tokens))
     return SinkWindowSplitFunc.apply(q, k, v, int(window_size), softmax_scale,
                                      int(num_sink_tokens))
 
@@ -187,7 +186,6 @@ def ring_streaming_llm_attn_varlen(
     _check_packed(q, k, v, cu_seqlens, cp_size)
     cu = cu_seqlens.contiguous()
     if _impl(impl) or num_sink_tokens == 0:
-        return BandAttnFunc.apply(q, k, v, int(window_size), softmax_scale, cu,
-                                  int(num_sink_tokens))
+        return band_attn(q, k, v, int(window_size), softmax_scale, cu, int(num_sink_tokens))
     return SinkWindowSplitVarlenFunc.apply(q, k, v, int(window_size), cu, softmax_scale,
                                            int(num_sink_tokens))
