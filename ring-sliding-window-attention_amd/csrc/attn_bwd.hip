@@ -1321,50 +1321,60 @@ void attn_bwd_dq_kernel(const AttnArgs a) {
       }
       // P = exp2(S c - lse2), dS^T = P (dP^T - delta), packed slab by slab (32 keys) as the B
       // operands of dQ^T += K^T dS^T
-      V8 dsb[2][2];
-      auto body = [&](auto full_c) __attribute__((always_inline)) {
-        constexpr bool FULL = decltype(full_c)::value;
-        int hi_rel[2], lo_rel[2], sink_rel = 0, u_m = 0;
-        if constexpr (!FULL) {
-          // edge tile: the lane's own mask bounds are recomputed here (only a few tiles per
-          // block take this path; kept across the loop they would cost registers)
-          int lane_m = (int)__builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, 0u));
-          asm volatile("" : "+v"(lane_m));
-          u_m = lane_m >> 4;
-          sink_rel = a.n_sink - j0;
 #pragma unroll
-          for (int qb = 0; qb < 2; qb++) {
-            const RowBounds rb = row_bounds(a, r0 + 16 * qb + (lane_m & 15), len_q, len_k);
-            hi_rel[qb] = rb.hi - j0;
-            lo_rel[qb] = rb.lo - j0;
+      for (int kb = 0; kb < KBLK; kb++)
+#pragma unroll
+        for (int qb = 0; qb < 2; qb++)
+#pragma unroll
+          for (int i = 0; i < 4; i++)
+            sacc[kb][qb][i] = __builtin_amdgcn_exp2f(__builtin_fmaf(sacc[kb][qb][i], a.scale_log2, lse2[qb])) *
+                              pacc[kb][qb][i];
+      if (!full) {
+        // edge tile: key j = j0 + 16 kb + i + 4 u is visible iff j <= hi and (j >= lo or j < n_sink); a
+        // comparison with a constant and a select per score for the bound that cuts the tile (us, dQ with
+        // statistics, before / after: 4001 rows, window 1024 91.5 / 89.3; the pack of short sequences
+        // 180 / 176).  The lane's own bounds are recomputed here: kept across the loop they would cost
+        // registers.
+        int lane_m = (int)__builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, 0u));
+        asm volatile("" : "+v"(lane_m));
+        const int at = j0 + 4 * (lane_m >> 4);
+        int hi_rel[2], lo_rel[2];
+#pragma unroll
+        for (int qb = 0; qb < 2; qb++) {
+          const RowBounds rb = row_bounds(a, r0 + 16 * qb + (lane_m & 15), len_q, len_k);
+          hi_rel[qb] = rb.hi - at;
+          lo_rel[qb] = rb.lo - at;
+        }
+        auto keep = [&](auto visible) __attribute__((always_inline)) {
+#pragma unroll
+          for (int kb = 0; kb < KBLK; kb++)
+#pragma unroll
+            for (int qb = 0; qb < 2; qb++)
+#pragma unroll
+              for (int i = 0; i < 4; i++)
+                sacc[kb][qb][i] = visible(16 * kb + i, qb) ? sacc[kb][qb][i] : 0.f;
+        };
+        if (!(wave_rows_full && j1 <= wb_first.hi)) keep([&](int c, int qb) { return c <= hi_rel[qb]; });
+        if (j0 < wb_last.lo && j1 >= a.n_sink) {
+          if (j0 < a.n_sink) {  // some of the tile's keys are sinks
+            const int sink_rel = a.n_sink - at;
+            keep([&](int c, int qb) { return (c >= lo_rel[qb]) | (c < sink_rel); });
+          } else {
+            keep([&](int c, int qb) { return c >= lo_rel[qb]; });
           }
         }
-#pragma unroll
-        for (int ks2 = 0; ks2 < 2; ks2++)
-#pragma unroll
-          for (int qb = 0; qb < 2; qb++) {
-            float dsv[8];
-#pragma unroll
-            for (int e = 0; e < 8; e++) {
-              const int kb = 2 * ks2 + (e >> 2), i = e & 3;
-              float ds = __builtin_amdgcn_exp2f(__builtin_fmaf(sacc[kb][qb][i], a.scale_log2, lse2[qb])) *
-                         pacc[kb][qb][i];
-              if constexpr (!FULL) {
-                const int j = 16 * kb + 4 * u_m + i;
-                const bool ok = (j <= hi_rel[qb]) & ((j >= lo_rel[qb]) | (j < sink_rel));
-                ds = ok ? ds : 0.f;
-              }
-              dsv[e] = ds;
-            }
-            dsb[ks2][qb] = M::pack(dsv);
-            asm volatile("" : "+v"(dsb[ks2][qb]));
-          }
-      };
-      if (full) {
-        body(std::true_type{});
-      } else {
-        body(std::false_type{});
       }
+      V8 dsb[2][2];
+#pragma unroll
+      for (int ks2 = 0; ks2 < 2; ks2++)
+#pragma unroll
+        for (int qb = 0; qb < 2; qb++) {
+          float dsv[8];
+#pragma unroll
+          for (int e = 0; e < 8; e++) dsv[e] = sacc[2 * ks2 + (e >> 2)][qb][e & 3];
+          dsb[ks2][qb] = M::pack(dsv);
+          asm volatile("" : "+v"(dsb[ks2][qb]));
+        }
       int t_off = t_row;
       asm volatile("" : "+v"(t_off));
 #pragma unroll

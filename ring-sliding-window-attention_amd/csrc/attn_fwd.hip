@@ -58,7 +58,9 @@ void attn_fwd_kernel(const AttnArgs a) {
   if (wid < 0) return;
   const int tid = threadIdx.x;
   const int lane = tid & 63;
-  const int wave = tid >> 6;
+  // (known to be uniform: the rows' bounds are scalars, 20 registers less; with SKIP, whose branches then
+  // are scalar ones, the compiler would keep both sides' fragments and spill)
+  const int wave = SKIP ? tid >> 6 : __builtin_amdgcn_readfirstlane(tid >> 6);
   const int l32 = lane & 31;
   const int g = lane >> 5;
   const int i16 = lane & 15;
@@ -191,24 +193,42 @@ void attn_fwd_kernel(const AttnArgs a) {
       }
     }
   };
-  // mask of an edge tile: visible iff j <= hi and (j >= lo or j < n_sink)
+  // mask of an edge tile: visible iff j <= hi and (j >= lo or j < n_sink).  Key j = j0 + c + 4 g, c known
+  // per register: either bound is one comparison with a constant and one select per score, and a tile
+  // pays for the bound that cuts it.  (As logic on three comparisons for all of it an edge tile had 190
+  // instructions more than another, half as many again as the softmax.  us, before / after, with the wave's
+  // bounds as scalars: 4001 rows, window 1024, 32 / 8 heads 68.9 / 65.9; a pack of 16384 tokens in
+  // sequences of 16 to 1024 140 / 132; 4 x 2000 rows, 28 / 4 heads, head_dim 64, 4 sinks 74.0 / 68.9.)
   auto mask = [&](int it, f32x16(&sacc)[2]) __attribute__((always_inline)) {
     const int j0 = tile_of(it) * C::BN;
     const int j1 = j0 + C::BN - 1;
-    const bool full =
-        wave_rows_full && j1 <= wb_first.hi && (j0 >= wb_last.lo || j1 < a.n_sink);
-    if (!full) {
-      const int hi_rel = rb.hi - j0;
-      const int lo_rel = rb.lo - j0;
-      const int sink_rel = a.n_sink - j0;
+    if (!(wave_rows_full && j1 <= wb_first.hi)) {
+      const int hi_rel = rb.hi - j0 - 4 * g;
 #pragma unroll
       for (int t = 0; t < 2; t++)
 #pragma unroll
-        for (int i = 0; i < 16; i++) {
-          const int j = t * 32 + 8 * (i >> 2) + 4 * g + (i & 3);
-          const bool ok = (j <= hi_rel) & ((j >= lo_rel) | (j < sink_rel));
-          sacc[t][i] = ok ? sacc[t][i] : -__builtin_inff();
-        }
+        for (int i = 0; i < 16; i++)
+          sacc[t][i] = t * 32 + 8 * (i >> 2) + (i & 3) <= hi_rel ? sacc[t][i] : -__builtin_inff();
+    }
+    if (j0 < wb_last.lo && j1 >= a.n_sink) {
+      int lo_rel = rb.lo - j0 - 4 * g;
+      if (j0 < a.n_sink) {  // some of the tile's keys are sinks
+        const int sink_rel = a.n_sink - j0 - 4 * g;
+        asm volatile("" : "+v"(lo_rel));  // (or both branches' comparisons are made ahead of them, in 64 SGPRs)
+#pragma unroll
+        for (int t = 0; t < 2; t++)
+#pragma unroll
+          for (int i = 0; i < 16; i++) {
+            const int c = t * 32 + 8 * (i >> 2) + (i & 3);
+            sacc[t][i] = ((c >= lo_rel) | (c < sink_rel)) ? sacc[t][i] : -__builtin_inff();
+          }
+      } else {
+#pragma unroll
+        for (int t = 0; t < 2; t++)
+#pragma unroll
+          for (int i = 0; i < 16; i++)
+            sacc[t][i] = t * 32 + 8 * (i >> 2) + (i & 3) >= lo_rel ? sacc[t][i] : -__builtin_inff();
+      }
     }
   };
   // online softmax of one tile (raw-score max, exponent in base 2); P^T packed for the
@@ -227,7 +247,9 @@ void attn_fwd_kernel(const AttnArgs a) {
     const bool bump = (m_new - m_run) * a.scale_log2 > 8.f;  // true from -inf, false for NaN
     const float m_keep = bump ? m_new : m_run;
     const float m_use = (m_keep == -__builtin_inff()) ? 0.f : m_keep;
-    const float alpha = __builtin_amdgcn_exp2f((m_run - m_use) * a.scale_log2);
+    // (1 also where the row has seen no key yet: O is zero then, and the first tile needs no rescale)
+    const float alpha =
+        m_run == -__builtin_inff() ? 1.f : __builtin_amdgcn_exp2f((m_run - m_use) * a.scale_log2);
     const float mc = m_use * a.scale_log2;
     m_run = m_keep;
     float psum[4] = {0.f, 0.f, 0.f, 0.f};
@@ -461,22 +483,18 @@ RSWA_INSTANTIATE(_Float16, 64, 3)
 int rows_per_block(const AttnArgs& a) { return (a.group & 1) == 0 ? 64 : 128; }
 int blocks_per_tile(const AttnArgs& a) { return ((a.group & 1) == 0 ? a.group / 2 : a.group) * a.heads_kv; }
 
-// Three blocks per compute unit instead of two?  head_dim 128 needs 214 registers, so two.  head_dim 64
-// has half the MFMAs per score and is bound by the softmax's vector work and its latencies; it fits
-// three (148 registers; four would spill), but built for that a block is 3 to 12 % slower by itself.
-// So three where the launch has more blocks than fit at two per compute unit (us, two / three: 504
-// blocks of 2241 rows, 28 / 4 heads, window 4232, 55 / 61; 552 blocks of 5855 rows, 12 heads, window
-// 236, 27 / 22; 4 x 2000 rows, 28 / 4 heads, window 1000, 1792 blocks, 79 / 78), and where blocks are
-// long and of unlike length, so that the longest decide, several rounds of them (causal without a
-// window, 8 heads, 13513 tokens in three sequences, 864 blocks, 147 / 178; 12 heads, 20738 tokens in
-// four, 1980 blocks, 300 / 299).  Of 438 shapes drawn the rule is 0.3 % behind the better build on
-// average (more than 3 % slower than two blocks on 8 of them, 11 % at most), three alone 4 %, two alone 5 %.
+// Three blocks per compute unit instead of two?  head_dim 128 needs 191 registers and 64 KiB of LDS, so two.
+// head_dim 64 has half the MFMAs per score and is bound by the softmax's vector work and its latencies;
+// it fits three (135 registers, 158 with SKIP; built for four it fits without SKIP and is up to 17 %
+// slower).  Three wherever the launch has more blocks than fit at two per unit (us, two / three: 4 x 2000
+// rows, 28 / 4 heads, window 1000, 1792 blocks, 68 / 67; 8192 rows, 32 / 8 heads, window 1024, 91 / 83;
+// 2 x 6000 rows, 8 / 2 heads, window 3000, 100 / 81; of 49 shapes 21 equal, 26 faster by 4 to 29 %, and 2 x
+// 4000 rows, 12 heads, 768 blocks, 60 / 64); where they all fit anyway the two are equal.
 bool fwd_three_blocks(const AttnArgs& a, int head_dim) {
   if (head_dim != 64) return false;
   const double tiles = a.cu_q ? (double)a.rows_q / rows_per_block(a) + 0.5 * a.batch
                               : (double)ceil_div(a.seqlen_q, rows_per_block(a)) * a.batch;
-  const bool even = a.avg_keys >= 0.7 * a.max_keys || a.avg_keys <= 250;
-  return tiles * blocks_per_tile(a) > (even ? 2 * kComputeUnits : 1500);
+  return tiles * blocks_per_tile(a) > 2 * kComputeUnits;
 }
 
 template <typename T, int D, int WAVES>
