@@ -299,7 +299,12 @@ int fill_args(const rswa_attn_params* p, bool backward, AttnArgs& a, bool allow_
     a.rev_k = rows_of(lk - 1) > rows_of(0);
     // keys a query row sees on average (keys_of is piecewise linear: 17 samples)
     int64_t sum = 0;
-    for (int t = 0; t <= 16; t++) sum += keys_of((lq - 1) * t / 16);
+    a.max_keys = 0;
+    for (int t = 0; t <= 16; t++) {
+      const int64_t n = keys_of((lq - 1) * t / 16);
+      sum += n;
+      a.max_keys = (int32_t)std::max<int64_t>(a.max_keys, std::min<int64_t>(n, INT32_MAX));
+    }
     a.avg_keys = (int32_t)std::min<int64_t>(sum / 17, INT32_MAX);
   }
   a.scale = p->softmax_scale;

@@ -102,6 +102,7 @@ struct AttnArgs {
   int32_t ds_slots;  // 32-row tile slots per q head (dense: batch * tiles; packed: rows / 32 + batch)
   float scale, scale_log2;
   // ---- for the host's choices only; behind the rest, so that the kernels' argument loads stay put
+  int32_t max_keys;   // keys a query row sees at most (of the rows avg_keys samples)
   int32_t dkdv_form;  // RSWA_DKDV_*: the caller's choice of the dK/dV kernel's blocks
   int32_t dq_last;    // dq lies over an input: the dQ kernel must not run before dK/dV
 };

@@ -486,15 +486,19 @@ int blocks_per_tile(const AttnArgs& a) { return ((a.group & 1) == 0 ? a.group / 
 // Three blocks per compute unit instead of two?  head_dim 128 needs 191 registers and 64 KiB of LDS, so two.
 // head_dim 64 has half the MFMAs per score and is bound by the softmax's vector work and its latencies;
 // it fits three (135 registers, 158 with SKIP; built for four it fits without SKIP and is up to 17 %
-// slower).  Three wherever the launch has more blocks than fit at two per unit (us, two / three: 4 x 2000
+// slower).  Three where the launch has more blocks than fit at two per unit (us, two / three: 4 x 2000
 // rows, 28 / 4 heads, window 1000, 1792 blocks, 68 / 67; 8192 rows, 32 / 8 heads, window 1024, 91 / 83;
-// 2 x 6000 rows, 8 / 2 heads, window 3000, 100 / 81; of 49 shapes 21 equal, 26 faster by 4 to 29 %, and 2 x
-// 4000 rows, 12 heads, 768 blocks, 60 / 64); where they all fit anyway the two are equal.
+// 2 x 6000 rows, 8 / 2 heads, window 3000, 100 / 81; 2 x 4000 rows, 12 heads, 768 blocks, 60 / 64; where
+// they all fit anyway the two are equal), and where blocks are long and of unlike length, so that the
+// longest decide, a little over two rounds (causal without a window: 8 heads, 13513 tokens in three
+// sequences, 864 blocks, 105 / 121; 32 heads, 2 x 1250 tokens, 640 blocks, 34 / 36; 28 / 4 heads, 3000
+// tokens, 672 blocks, 69 / 61; 12 heads, 20738 tokens in four, 1968 blocks, 249 / 236).
 bool fwd_three_blocks(const AttnArgs& a, int head_dim) {
   if (head_dim != 64) return false;
   const double tiles = a.cu_q ? (double)a.rows_q / rows_per_block(a) + 0.5 * a.batch
                               : (double)ceil_div(a.seqlen_q, rows_per_block(a)) * a.batch;
-  return tiles * blocks_per_tile(a) > 2 * kComputeUnits;
+  const bool even = a.avg_keys >= 0.7 * a.max_keys || a.avg_keys <= 250;
+  return tiles * blocks_per_tile(a) > (even ? 2 * kComputeUnits : 1150);
 }
 
 template <typename T, int D, int WAVES>
