@@ -791,50 +791,64 @@ __global__ __launch_bounds__(256) void attn_bwd_dkdv_kernel(const AttnArgs a) {
 // dK / dV of sink keys
 // ============================================================================
 // With sink keys and a bounded window, key j < n_sink is seen by every later row of its
-// sequence: a few keys against all the rows, far too thin for MFMA tiles.  Left to the dK/dV
+// sequence: a few keys against all the rows, far too thin for the dK/dV kernel's tiles.  Left to that
 // kernel, the first key tile of every sequence walked every query tile with one wave of four
 // at work and took several times as long as any other block (a pack of 65536 tokens in four
 // sequences: 10.8 ms, a third of it that tail).  So the dK/dV kernel treats sink keys like any
 // other key (band pairs only), and this kernel, which runs after it, computes the sink keys'
-// complete dK / dV -- all the rows that see them, inside the window and beyond -- as plain
-// fp32 vector work at memory speed, and overwrites those few rows of dk / dv:
+// complete dK / dV -- all the rows that see them, inside the window and beyond -- and overwrites those
+// few rows of dk / dv:
 //   s = q . k_j, P = exp2(s c - lse2), dP = dO . v_j, dS = P (dP - delta)
 //   dV_j = sum P dO, dK_j = scale sum dS q
-// One block per (sequence, kv head, chunk of rows); Q and dO are read once per pass of kSinkPass
-// sink keys; a lane owns 8 consecutive d of one row at a time (D / 8 lanes per row), the dot
-// products are summed across those lanes, and the block's sums -- added in a fixed order -- go
-// to the workspace as fp32 [unit][chunk][sink][dK, dV][D].  The block of a unit that arrives
+// A wave takes 16 rows of one q head at a time, fetched one tile ahead: Q and dO as B operands (lane =
+// row l % 16, 8 consecutive d at 32 ks + 8 (l / 16)), four sinks repeated four times as the A operand, so
+// that after KS MFMAs each lane holds s and dP - delta of its own row for all four of them, and
+// multiplies them in fp32 into its own 2 x D / 4 sums per sink.  (P and dS stay fp32: as MFMA operands they
+// would be 16 bits.)  256 registers hold the sums of two sinks: with more than one, pairs of waves share the
+// rows and take two sinks each.  The sums of a block, over the 16 rows of a tile and its waves,
+// leave through LDS in a fixed order.
+// A unit (sequence, kv head) of up to sink_chunks chunks of tiles; with more than one, their sums go to the
+// workspace as fp32 [unit][chunk][sink][dK, dV][D], and the block of a unit that arrives
 // last adds the chunks in chunk order and writes the rows (the same order whichever block that is, so
 // the result does not depend on timing, and nobody waits).
-constexpr int kSinkPass = 4;
+// Bound by reading Q and dO once where there are many rows, by latencies where there are few.
+// The earlier form, whose lanes held 8 d of a row and summed every dot product across 16 lanes, walked 512
+// rows of each head of the group in one block without fetching ahead: us, before / now, dK/dV and sink
+// launch: 2 x 300 rows, 32 / 8 heads, 1 sink 68 / 42; 12053 rows, 8 / 2 heads, window 67, 142 / 73; 2 x 31793
+// rows, 16 / 4 heads, 4 sinks 638 / 601; 550 sequences of 20 tokens, 12 heads, 570 / 276; the sink launch
+// alone on 65536 tokens, 32 / 8 heads, 4 sinks 458 / 390.
 
-// sum over the aligned group of W = 8 or 16 lanes, in every lane of the group
-template <int W>
-__device__ __forceinline__ float lane_group_sum(float x) {
+// sum over the aligned group of 16 lanes, in every lane of the group
+__device__ __forceinline__ float lane_group_sum16(float x) {
   auto dpp = [](float v, auto ctrl) __attribute__((always_inline)) {
     return __uint_as_float(__builtin_amdgcn_update_dpp(0u, __float_as_uint(v), decltype(ctrl)::value,
                                                        0xf, 0xf, true));
   };
-  if constexpr (W == 16) x += dpp(x, std::integral_constant<int, 0x140>{});  // row_mirror
-  x += dpp(x, std::integral_constant<int, 0x141>{});                          // row_half_mirror
-  x += dpp(x, std::integral_constant<int, 0x1b>{});                           // quad_perm 3 2 1 0
-  x += dpp(x, std::integral_constant<int, 0xb1>{});                           // quad_perm 1 0 3 2
+  x += dpp(x, std::integral_constant<int, 0x140>{});  // row_mirror
+  x += dpp(x, std::integral_constant<int, 0x141>{});  // row_half_mirror
+  x += dpp(x, std::integral_constant<int, 0x1b>{});   // quad_perm 3 2 1 0
+  x += dpp(x, std::integral_constant<int, 0xb1>{});   // quad_perm 1 0 3 2
   return x;
 }
 
-template <typename T, int D>
-__global__ __launch_bounds__(256) void attn_bwd_sink_kernel(const AttnArgs a) {
-  using V8 = typename Mma<T>::V8;
-  constexpr int LPR = D / 8;     // lanes per row
-  constexpr int RPW = 64 / LPR;  // rows per wave pass
-  constexpr int NS = kSinkPass;
-  constexpr int NSRC = 4 * RPW;  // (wave, row group) sources of the block's sums
-  __shared__ float red_s[NSRC][NS * 2 * D];
-  static_assert(sizeof(red_s) <= 65536, "staging buffer");
+// NS: sinks of a wave, 1 (the waves of a block share out the tiles) or 2 (pairs of waves do, and the
+// waves of a pair take sinks 0, 1 and 2, 3 of every four)
+template <typename T, int D, int NS>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2)))
+void attn_bwd_sink_kernel(const AttnArgs a) {
+  using M = Mma<T>;
+  using V8 = typename M::V8;
+  constexpr int KS = D / 32;
+  constexpr int SG = NS;        // groups of sinks in the block (waves of a pair)
+  constexpr int RW = 4 / SG;    // waves that share out the tiles
+  constexpr int NB = NS * SG;   // sinks of a pass
+  __shared__ float red_s[4][NS * 2 * D];
+  __shared__ __attribute__((aligned(16))) T k_s[SG * 4 * D], v_s[SG * 4 * D];  // the pass's sinks, NS of every four rows
 
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int sub = lane % LPR, rg = lane / LPR;
+  const int r = lane & 15, u = lane >> 4;
+  const int sg = wave & (SG - 1), rw = wave / SG;
   const int c = blockIdx.x % a.sink_chunks;
   const int unit = blockIdx.x / a.sink_chunks;  // (sequence, kv head)
   const int hk = unit % a.heads_kv, b = unit / a.heads_kv;
@@ -847,101 +861,132 @@ __global__ __launch_bounds__(256) void attn_bwd_sink_kernel(const AttnArgs a) {
     len_k = a.cu_k[b + 1] - a.cu_k[b];
   }
   const int ns_all = min(a.n_sink, len_k);
-  // rows of the sequence in n_chunks chunks (at most a.sink_chunks)
-  const int rows_per = (len_q + a.sink_chunks - 1) / a.sink_chunks;
-  const int n_chunks = rows_per > 0 ? (len_q + rows_per - 1) / rows_per : 0;
+  // the unit's tiles in n_chunks chunks (at most a.sink_chunks, of two tiles per wave or
+  // more)
+  const int n_rt = (len_q + 15) >> 4, total = n_rt * a.group;
+  const int per = max((total + a.sink_chunks - 1) / a.sink_chunks, 2 * RW);
+  const int n_chunks = (total + per - 1) / per;
   if (c >= n_chunks || ns_all == 0) return;
   const int shift = a.shift_explicit ? a.shift_val : len_k - len_q;
-  const int r_begin = c * rows_per, r_end = min(len_q, r_begin + rows_per);
+  const int t_end = min(total, (c + 1) * per);
 
-  const T* q_ptr = (const T*)a.q + b * a.q_st[0] + q_row0 * a.q_st[1];
-  const T* do_ptr = (const T*)a.dout + b * a.do_st[0] + q_row0 * a.do_st[1];
+  const T* q_ptr = (const T*)a.q + b * a.q_st[0] + q_row0 * a.q_st[1] + hk * a.group * a.q_st[2] + u * 8;
+  const T* do_ptr = (const T*)a.dout + b * a.do_st[0] + q_row0 * a.do_st[1] + hk * a.group * a.do_st[2] + u * 8;
   const T* k_ptr = (const T*)a.k + b * a.k_st[0] + k_row0 * a.k_st[1] + hk * a.k_st[2];
   const T* v_ptr = (const T*)a.v + b * a.v_st[0] + k_row0 * a.v_st[1] + hk * a.v_st[2];
-  const int64_t ws_row0 = a.cu_q ? q_row0 : (int64_t)b * a.seqlen_q;
-  float* out = a.sink_part + ((int64_t)unit * a.sink_chunks + c) * (a.n_sink * 2 * D);
+  const int64_t ws_row0 = (int64_t)hk * a.group * a.rows_q + (a.cu_q ? q_row0 : (int64_t)b * a.seqlen_q);
+  T* dk_ptr = (T*)a.dk + b * a.dk_st[0] + k_row0 * a.dk_st[1] + hk * a.dk_st[2];
+  T* dv_ptr = (T*)a.dv + b * a.dv_st[0] + k_row0 * a.dv_st[1] + hk * a.dv_st[2];
+  auto put = [&](int j, int at, float sum) __attribute__((always_inline)) {  // at: d of dK, then of dV
+    if (at < D) dk_ptr[(int64_t)j * a.dk_st[1] + at] = (T)(sum * a.scale);
+    else dv_ptr[(int64_t)j * a.dv_st[1] + at - D] = (T)sum;
+  };
 
-  for (int j0 = 0; j0 < ns_all; j0 += NS) {
-    float kf[NS][8], vf[NS][8], acck[NS][8], accv[NS][8];
+  struct Tile {
+    V8 q[KS], d[KS];
+    float nl, nd;  // the row's statistics, stored negated
+    int row;
+  };
+  for (int j0 = 0; j0 < ns_all; j0 += NB) {
+    const int jb = j0 + sg * NS;  // the wave's sinks: jb .. jb + NS - 1
+    if (j0 > 0) __syncthreads();  // the previous pass's readers are done
+    for (int idx = tid; idx < SG * 4 * D; idx += 256) {
+      const int row = idx / D, j = j0 + (row >> 2) * NS + (row & 3);
+      const bool real = (row & 3) < NS && j < ns_all;
+      k_s[idx] = real ? k_ptr[(int64_t)j * a.k_st[1] + idx % D] : (T)0.f;
+      v_s[idx] = real ? v_ptr[(int64_t)j * a.v_st[1] + idx % D] : (T)0.f;
+    }
+    float acck[NS][KS * 8], accv[NS][KS * 8];
 #pragma unroll
-    for (int jj = 0; jj < NS; jj++) {
-      V8 k8 = V8{0, 0, 0, 0, 0, 0, 0, 0}, v8 = k8;
-      if (j0 + jj < ns_all) {
-        k8 = *(const V8*)(k_ptr + (int64_t)(j0 + jj) * a.k_st[1] + sub * 8);
-        v8 = *(const V8*)(v_ptr + (int64_t)(j0 + jj) * a.v_st[1] + sub * 8);
-      }
+    for (int i = 0; i < NS; i++)
 #pragma unroll
-      for (int e = 0; e < 8; e++) {
-        kf[jj][e] = (float)k8[e];
-        vf[jj][e] = (float)v8[e];
-        acck[jj][e] = 0.f;
-        accv[jj][e] = 0.f;
+      for (int e = 0; e < KS * 8; e++) acck[i][e] = accv[i][e] = 0.f;
+    int t = c * per + rw;
+    __syncthreads();
+    if (jb < ns_all && t < t_end) {
+      // cursor: tile rt of the unit's q head h, the heads of a tile's rows one after the other, which lie side
+      // by side in memory (the loads of a tile behind the chunk's last are those of the last, and not used)
+      int rt = t / a.group, h = t - rt * a.group;
+      auto fetch = [&](Tile& x) __attribute__((always_inline)) {
+        x.row = rt * 16 + r;
+        const int row = min(x.row, len_q - 1);
+        const T* q_row = q_ptr + h * a.q_st[2] + (int64_t)row * a.q_st[1];
+        const T* do_row = do_ptr + h * a.do_st[2] + (int64_t)row * a.do_st[1];
+#pragma unroll
+        for (int ks = 0; ks < KS; ks++) {
+          x.q[ks] = *(const V8*)(q_row + ks * 32);
+          x.d[ks] = *(const V8*)(do_row + ks * 32);
+        }
+        x.nl = a.lse2[ws_row0 + h * a.rows_q + row];
+        x.nd = a.delta[ws_row0 + h * a.rows_q + row];
+      };
+      Tile cur, nxt;
+      fetch(cur);
+      for (; t < t_end; t += RW) {
+        if (t + RW < t_end) {
+          h += RW;
+          while (h >= a.group) {
+            h -= a.group;
+            rt++;
+          }
+        }
+        fetch(nxt);
+        f32x4 s = {0.f, 0.f, 0.f, 0.f}, dp = {cur.nd, cur.nd, cur.nd, cur.nd};
+        int a_row = (sg * 4 + (r & 3)) * D + u * 8;  // row r of the A operand: sink r % 4
+        asm volatile("" : "+v"(a_row));              // (read here: kept in registers the operands would spill)
+#pragma unroll
+        for (int ks = 0; ks < KS; ks++) {
+          s = M::mfma16(*(const V8*)(k_s + a_row + ks * 32), cur.q[ks], s);
+          dp = M::mfma16(*(const V8*)(v_s + a_row + ks * 32), cur.d[ks], dp);
+        }
+        const int hi = (a.wr >= 0) ? min(len_k - 1, cur.row + shift + a.wr) : len_k - 1;
+        float p[NS], ds[NS];
+#pragma unroll
+        for (int i = 0; i < NS; i++) {
+          const int j = jb + i;
+          const bool vis = cur.row < len_q && j < ns_all && j <= hi;  // a sink key: no lower bound
+          p[i] = vis ? __builtin_amdgcn_exp2f(__builtin_fmaf(s[i], a.scale_log2, cur.nl)) : 0.f;
+          ds[i] = vis ? p[i] * dp[i] : 0.f;
+        }
+#pragma unroll
+        for (int ks = 0; ks < KS; ks++)
+#pragma unroll
+          for (int e = 0; e < 8; e++) {
+            const float qe = (float)cur.q[ks][e], de = (float)cur.d[ks][e];
+#pragma unroll
+            for (int i = 0; i < NS; i++) {
+              acck[i][ks * 8 + e] = __builtin_fmaf(ds[i], qe, acck[i][ks * 8 + e]);
+              accv[i][ks * 8 + e] = __builtin_fmaf(p[i], de, accv[i][ks * 8 + e]);
+            }
+          }
+        cur = nxt;
       }
     }
-    for (int h = 0; h < a.group; h++) {
-      const int hq = hk * a.group + h;
-      const T* qh = q_ptr + (int64_t)hq * a.q_st[2] + sub * 8;
-      const T* doh = do_ptr + (int64_t)hq * a.do_st[2] + sub * 8;
-      const float* lse_h = a.lse2 + (int64_t)hq * a.rows_q + ws_row0;
-      const float* delta_h = a.delta + (int64_t)hq * a.rows_q + ws_row0;
-      for (int base = r_begin + wave * RPW; base < r_end; base += 4 * RPW) {
-        const int row = base + rg;
-        const bool valid = row < r_end;
-        V8 q8 = V8{0, 0, 0, 0, 0, 0, 0, 0}, d8 = q8;
-        float nl = -__builtin_inff(), nd = 0.f;  // the statistics are stored negated
-        if (valid) {
-          q8 = *(const V8*)(qh + (int64_t)row * a.q_st[1]);
-          d8 = *(const V8*)(doh + (int64_t)row * a.do_st[1]);
-          nl = lse_h[row];
-          nd = delta_h[row];
-        }
-        float qf[8], df[8];
+    // the wave's sums over its 16 rows, then the block's over its waves, in wave order
+#pragma unroll
+    for (int i = 0; i < NS; i++)
+#pragma unroll
+      for (int ks = 0; ks < KS; ks++)
 #pragma unroll
         for (int e = 0; e < 8; e++) {
-          qf[e] = (float)q8[e];
-          df[e] = (float)d8[e];
-        }
-        const int hi = (a.wr >= 0) ? min(len_k - 1, row + shift + a.wr) : len_k - 1;
-#pragma unroll
-        for (int jj = 0; jj < NS; jj++) {
-          float sdot = 0.f, pdot = 0.f;
-#pragma unroll
-          for (int e = 0; e < 8; e++) {
-            sdot = __builtin_fmaf(qf[e], kf[jj][e], sdot);
-            pdot = __builtin_fmaf(df[e], vf[jj][e], pdot);
-          }
-          sdot = lane_group_sum<LPR>(sdot);
-          pdot = lane_group_sum<LPR>(pdot);
-          const int j = j0 + jj;
-          const bool vis = valid && j < ns_all && j <= hi;  // a sink key: no lower bound
-          const float p = vis ? __builtin_amdgcn_exp2f(__builtin_fmaf(sdot, a.scale_log2, nl)) : 0.f;
-          const float ds = vis ? p * (pdot + nd) : 0.f;
-#pragma unroll
-          for (int e = 0; e < 8; e++) {
-            accv[jj][e] = __builtin_fmaf(p, df[e], accv[jj][e]);
-            acck[jj][e] = __builtin_fmaf(ds, qf[e], acck[jj][e]);
+          const float k_sum = lane_group_sum16(acck[i][ks * 8 + e]), v_sum = lane_group_sum16(accv[i][ks * 8 + e]);
+          if (r == 0) {
+            red_s[wave][(i * 2 + 0) * D + ks * 32 + u * 8 + e] = k_sum;
+            red_s[wave][(i * 2 + 1) * D + ks * 32 + u * 8 + e] = v_sum;
           }
         }
-      }
-    }
-    // the block's sums: every (wave, row group) source staged, then added in source order
-    __syncthreads();  // the previous pass's readers are done
-#pragma unroll
-    for (int jj = 0; jj < NS; jj++)
-#pragma unroll
-      for (int e = 0; e < 8; e++) {
-        red_s[wave * RPW + rg][(jj * 2 + 0) * D + sub * 8 + e] = acck[jj][e];
-        red_s[wave * RPW + rg][(jj * 2 + 1) * D + sub * 8 + e] = accv[jj][e];
-      }
     __syncthreads();
-    for (int idx = tid; idx < NS * 2 * D; idx += 256) {
+    for (int idx = tid; idx < NB * 2 * D; idx += 256) {
+      const int jj = idx / (2 * D), at = idx % (2 * D);
+      if (j0 + jj >= ns_all) break;
       float sum = 0.f;
 #pragma unroll
-      for (int src = 0; src < NSRC; src++) sum += red_s[src][idx];
-      const int jj = idx / (2 * D);
-      if (j0 + jj < ns_all) out[(int64_t)(j0 + jj) * (2 * D) + idx % (2 * D)] = sum;
+      for (int w = 0; w < RW; w++) sum += red_s[w * SG + jj / NS][(jj % NS) * 2 * D + at];
+      if (n_chunks == 1) put(j0 + jj, at, sum);
+      else a.sink_part[((int64_t)unit * a.sink_chunks + c) * (a.n_sink * 2 * D) + (j0 + jj) * (2 * D) + at] = sum;
     }
   }
+  if (n_chunks == 1) return;
   // count this chunk in; the last one of the unit adds them all up
   __shared__ int arrived_s;
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
@@ -954,18 +999,12 @@ __global__ __launch_bounds__(256) void attn_bwd_sink_kernel(const AttnArgs a) {
   if (arrived_s != n_chunks - 1) return;
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
   if (tid == 0) a.sink_count[unit] = 0;  // the next launch on this workspace starts from zero
-  T* dk_ptr = (T*)a.dk + b * a.dk_st[0] + k_row0 * a.dk_st[1] + hk * a.dk_st[2];
-  T* dv_ptr = (T*)a.dv + b * a.dv_st[0] + k_row0 * a.dv_st[1] + hk * a.dv_st[2];
   const float* parts = a.sink_part + (int64_t)unit * a.sink_chunks * (a.n_sink * 2 * D);
   for (int idx = tid; idx < ns_all * 2 * D; idx += 256) {
     float sum = 0.f;
+#pragma unroll 8
     for (int cc = 0; cc < n_chunks; cc++) sum += parts[(int64_t)cc * (a.n_sink * 2 * D) + idx];
-    const int j = idx / (2 * D), dd = idx % D;
-    if ((idx / D) & 1) {
-      dv_ptr[(int64_t)j * a.dv_st[1] + dd] = (T)sum;
-    } else {
-      dk_ptr[(int64_t)j * a.dk_st[1] + dd] = (T)(sum * a.scale);
-    }
+    put(idx / (2 * D), idx % (2 * D), sum);
   }
 }
 
@@ -1781,7 +1820,8 @@ __global__ __launch_bounds__(256) void attn_bwd_prep_kernel(const AttnArgs a) {
   template __global__ void attn_bwd_dq_kernel<T, D, false, 4, false>(const AttnArgs); \
   template __global__ void attn_bwd_dq_kernel<T, D, false, 4, true>(const AttnArgs); \
   template __global__ void attn_bwd_dq_kernel<T, D, true, 4, false>(const AttnArgs); \
-  template __global__ void attn_bwd_sink_kernel<T, D>(const AttnArgs);                  \
+  template __global__ void attn_bwd_sink_kernel<T, D, 1>(const AttnArgs);               \
+  template __global__ void attn_bwd_sink_kernel<T, D, 2>(const AttnArgs);               \
   template __global__ void attn_bwd_prep_kernel<T, D>(const AttnArgs);
 RSWA_INSTANTIATE(__bf16, 128)
 RSWA_INSTANTIATE(__bf16, 64)
@@ -1941,8 +1981,9 @@ int launch_bwd(AttnArgs& a, hipStream_t stream, int phases) {
     }
     if (a.n_work > 0 && a.sink_part && a.rows_q > 0) {
       clear_launch_error();
-      hipLaunchKernelGGL((attn_bwd_sink_kernel<T, D>), dim3(a.batch * a.heads_kv * a.sink_chunks),
-                         dim3(256), 0, stream, a);
+      const dim3 grid(a.batch * a.heads_kv * a.sink_chunks), block(256);
+      if (a.n_sink == 1) hipLaunchKernelGGL((attn_bwd_sink_kernel<T, D, 1>), grid, block, 0, stream, a);
+      else hipLaunchKernelGGL((attn_bwd_sink_kernel<T, D, 2>), grid, block, 0, stream, a);
       int rc = check_launch("attn_bwd sink");
       if (rc != RSWA_OK) return rc;
     }

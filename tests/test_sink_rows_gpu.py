@@ -1,0 +1,44 @@
+"""Gradients of sink keys, whose rows a kernel of its own computes in tiles of 16 rows: sequences of a
+tile, one row more and less, one chunk and several, one sink per wave and two, more sinks than a pass."""
+import pytest
+import torch
+
+from oracle import attention_oracle as O
+from tests.gradcheck_util import GRAD_TOL, relnorm
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("d", [64, 128])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16], ids=["bf16", "fp16"])
+@pytest.mark.parametrize("lens,hq,hk,window,sinks", [
+    ([1, 15, 16, 17, 0, 33], 3, 1, 4, 1), ([1, 2, 3, 40], 4, 4, 0, 2), ([130, 64, 5], 8, 2, 10, 3),
+    ([700], 4, 1, 50, 4), ([515, 520], 2, 2, 30, 5), ([900, 20], 6, 2, 100, 9), ([2100], 4, 2, 64, 1),
+])
+def test_sink_rows(lens, hq, hk, window, sinks, d, dtype):
+    from ring_swa.ops import attn_bwd, attn_fwd
+    from ring_swa.ops.band_attn import bwd_workspace_bytes
+
+    cu = [0]
+    for n in lens:
+        cu.append(cu[-1] + n)
+    torch.manual_seed(sum(lens))
+    q, do = (torch.randn(cu[-1], hq, d, device="cuda", dtype=dtype) for _ in range(2))
+    k, v = (torch.randn(cu[-1], hk, d, device="cuda", dtype=dtype) for _ in range(2))
+    cud = torch.tensor(cu, dtype=torch.int32, device="cuda")
+    out, lse = attn_fwd(q, k, v, None, (window, 0), True, cud, cud, num_sink=sinks)
+    ws = torch.full((bwd_workspace_bytes(q, k, cud, cud, window_size=(window, 0), causal=True, num_sink=sinks),), 255,
+                    dtype=torch.uint8, device="cuda")
+    got = []
+    for _ in range(2):  # (twice on one workspace: the arrival counters are left at zero)
+        g = [torch.full_like(x, float("nan")) for x in (q, k, v)]
+        attn_bwd(q, k, v, out, lse, do, *g, None, (window, 0), True, cud, cud, num_sink=sinks, workspace=ws)
+        got.append(g)
+    _, _, rq, rk, rv = O.attention_fwd_bwd(
+        lambda q, k, v: O.streaming_llm_attn_varlen(q, k, v, window, cu, n_sink=sinks), q, k, v, do)
+    for x, again, r in zip(*got, (rq, rk, rv)):
+        assert torch.equal(x, again)
+        assert relnorm(x, r) <= GRAD_TOL
+    at = torch.tensor([c + j for c, n in zip(cu, lens) for j in range(min(sinks, n))])
+    for x, r in ((got[0][1], rk), (got[0][2], rv)):  # (and by themselves, so that no other row hides one)
+        assert relnorm(x[at.cuda()], r[at]) <= GRAD_TOL
