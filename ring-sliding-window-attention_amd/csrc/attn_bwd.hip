@@ -273,15 +273,31 @@ __global__ __launch_bounds__(256) void attn_bwd_dkdv_kernel(const AttnArgs a) {
   // (keys past the end read the last one's values: their columns are masked in every tile and never
   // stored)
   V8 kf[KB][KS], vf[KB][KS];  // (the V fragments: B operand of dP = dO V^T, same layout)
+  // WALK4: all four waves want the same 64 rows, which come through LDS, where the tiles of odd steps will
+  // be: a wave's direct loads touch 32 rows with 32 bytes each, and a block's 128 of them took its vector
+  // memory unit 2 of the block's first 5 us (us, dK/dV, direct / staged: 4001 rows, window 1024, 32 / 8 heads
+  // 125 / 121; a pack of 16384 tokens in sequences of 16 to 1024 220 / 208)
+  [[maybe_unused]] char *const k_stage = q_s0 + 2 * C::Q_TILE, *const v_stage = q_s0 + (WALK4 ? W_LDS : 0) + 2 * C::Q_TILE;
+  if constexpr (WALK4) {
+    const int rows = min(len_k - j0, 64);
+    const auto stage_rows = [&](const T* base, int64_t st, char* dst) __attribute__((always_inline)) {
+      TileDma<D, 64, 256> dma;
+      dma.init(st, tid);
+      dma.load(make_rows_rsrc(base + (int64_t)j0 * st, rows, st * 2, C::ROWB), 0, dst);  // (rows past the end: zero)
+    };
+    stage_rows(k_ptr, a.k_st[1], k_stage);
+    stage_rows(v_ptr, a.v_st[1], v_stage);
+  } else {
 #pragma unroll
-  for (int kb = 0; kb < KB; kb++) {
-    const int jc = min(jw0 + kb * 32 + l32, len_k - 1);
-    const T* k_row = k_ptr + (int64_t)jc * a.k_st[1] + g * 8;
-    const T* v_row = v_ptr + (int64_t)jc * a.v_st[1] + g * 8;
+    for (int kb = 0; kb < KB; kb++) {
+      const int jc = min(jw0 + kb * 32 + l32, len_k - 1);
+      const T* k_row = k_ptr + (int64_t)jc * a.k_st[1] + g * 8;
+      const T* v_row = v_ptr + (int64_t)jc * a.v_st[1] + g * 8;
 #pragma unroll
-    for (int ks = 0; ks < KS; ks++) kf[kb][ks] = *(const V8*)(k_row + ks * 16);
+      for (int ks = 0; ks < KS; ks++) kf[kb][ks] = *(const V8*)(k_row + ks * 16);
 #pragma unroll
-    for (int ks = 0; ks < KS; ks++) vf[kb][ks] = *(const V8*)(v_row + ks * 16);
+      for (int ks = 0; ks < KS; ks++) vf[kb][ks] = *(const V8*)(v_row + ks * 16);
+    }
   }
   f32x16 dk_acc[KB][DB], dv_acc[KB][DB];
 #pragma unroll
@@ -448,8 +464,21 @@ __global__ __launch_bounds__(256) void attn_bwd_dkdv_kernel(const AttnArgs a) {
     static_for<NPART>([&](auto pc) __attribute__((always_inline)) { load_part(pc, qb0, dob0, stb0); });
     if (n_iter > 1) advance();
   }
-  if constexpr (WALK4) wait_vmem_but<0>();
-  else __syncthreads();
+  if constexpr (WALK4) {
+    wait_vmem_but<0>();
+    lds_barrier();
+#pragma unroll
+    for (int kb = 0; kb < KB; kb++)
+#pragma unroll
+      for (int ks = 0; ks < KS; ks++) {
+        const int at = ((a_row - w_lds) ^ (ks << 5)) + kb * 32 * C::ROWB;
+        kf[kb][ks] = *(const V8*)(k_stage + at);
+        vf[kb][ks] = *(const V8*)(v_stage + at);
+      }
+    lds_barrier();  // (every wave has read before a first step's loads overwrite)
+  } else {
+    __syncthreads();
+  }
 
   // byte of a lane's 16 in a 1 KiB piece of a dS unit: [key l32][query group g]
   const int ds_lane = l32 * 32 + g * 16;
