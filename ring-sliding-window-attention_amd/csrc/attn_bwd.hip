@@ -1049,8 +1049,10 @@ void attn_bwd_sink_kernel(const AttnArgs a) {
 #ifndef RSWA_DQ_AH2
 #define RSWA_DQ_AH2 4
 #endif
-// dQ launches whose rows see at most this many keys on average use blocks of 4 waves, two per
-// compute unit (measured, 32 / 8 heads, head_dim 128: window 256 -22 %, window 1000 -8 %, the rank
+// dQ launches of head_dim 128 whose rows see at most this many keys on average, and all of head_dim 64, use
+// blocks of 4 waves, two per compute unit (three at head_dim 64, against which a block of 8 is slower at any
+// length: us, 8 / 4 waves, 32768 rows, 32 / 8 heads, window 4096, 1546 / 1301; 12000 rows, 28 / 4 heads, causal
+// without a window, 1082 / 834; 20000 rows, 8 heads, window 4096, 272 / 219; head_dim 128, 32 / 8 heads: window 256 -22 %, window 1000 -8 %, the rank
 // step with its half-empty previous-chunk block -1.4 %; sequences of 16384 and more rows at
 // window 4096 +1 %; 32 = 32 heads, window 1000: -2 %)
 #ifndef RSWA_DQ_SMALL_AVG_KEYS
@@ -1068,6 +1070,14 @@ struct DqCfg {
   static constexpr int O_STRIDE = D * 2 + 16;
   static_assert(TILE >= 32 * O_STRIDE, "one wave's epilogue staging fits one tile buffer");
 };
+
+// Waves per SIMD that the dQ kernel is built for.  At head_dim 64 blocks of 4 waves fit three times into
+// a compute unit, with 164 registers and a shorter read-ahead (3 / 2; 7 / 4 would spill): half the MFMAs
+// per score leave the vector work and its latencies as the bound, which a third wave fills (us, dQ with
+// statistics, two / three: 2 x 31654 rows, 28 / 4 heads, window 100, 308 / 245; 2 x 7078, window 570, 120 /
+// 104; 15510 rows, 16 / 4 heads, window 990, 112 / 106; launches that two blocks per unit hold +-1 %).
+template <int D, int NW>
+constexpr int dq_waves = D == 64 && NW == 4 ? 3 : 2;
 
 // The key tile table of a pack, by one block: running sums of the sequences' tile counts, THREADS
 // sequences at a time (a scan in each wave, the waves' totals through LDS).
@@ -1160,9 +1170,10 @@ __global__ __launch_bounds__(256) void attn_bwd_rest_kernel(const AttnArgs a) {
 // dQ, bf16, head_dim 128, two kernels / one: 2 x 8192 rows, 32 / 32 heads, window 1000 457 / 444; a pack of
 // 16384 tokens in sequences of 16 to 1024, 32 / 8 heads, 213 / 206; 4001 rows, window 1024, 105 / 99.
 template <typename T, int D, bool FAR, int NW, bool STATS>
-__global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(2, 2)))
+__global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(dq_waves<D, NW>, dq_waves<D, NW>)))
 void attn_bwd_dq_kernel(const AttnArgs a) {
   using C = DqCfg<D>;
+  constexpr bool THREE = dq_waves<D, NW> == 3;
   static_assert(NW == 8 || NW == 4, "waves per block");
   static_assert(!(FAR && STATS), "statistics in the first addressing form only");
   constexpr int HSH = NW == 8 ? 2 : 1;  // waves per q head in pair mode: 1 << HSH
@@ -1378,7 +1389,7 @@ void attn_bwd_dq_kernel(const AttnArgs a) {
           }
         }
       {
-        constexpr int NRD = 2 * KBLK * KS, AH = RSWA_DQ_AH1;  // LDS reads AH ahead, 2 MFMAs each
+        constexpr int NRD = 2 * KBLK * KS, AH = THREE ? 3 : RSWA_DQ_AH1;  // LDS reads AH ahead, 2 MFMAs each
         __builtin_amdgcn_sched_group_barrier(0x100, AH, 0);
 #pragma unroll
         for (int i = 0; i < NRD - AH; i++) {
@@ -1455,7 +1466,7 @@ void attn_bwd_dq_kernel(const AttnArgs a) {
           for (int qb = 0; qb < 2; qb++) dq_acc[d][qb] = M::mfma16(kt, dsb[ks2][qb], dq_acc[d][qb]);
         }
       {
-        constexpr int NFR = 2 * DB, AH = RSWA_DQ_AH2;  // transposed fragments (2 reads, 2 MFMAs each)
+        constexpr int NFR = 2 * DB, AH = THREE ? 2 : RSWA_DQ_AH2;  // transposed fragments (2 reads, 2 MFMAs each)
         __builtin_amdgcn_sched_group_barrier(0x100, 2 * AH, 0);
 #pragma unroll
         for (int i = 0; i < NFR - AH; i++) {
@@ -1843,9 +1854,6 @@ __global__ __launch_bounds__(256) void attn_bwd_prep_kernel(const AttnArgs a) {
   template __global__ void attn_bwd_dkdv_kernel<T, D, false, true, false>(const AttnArgs); \
   template __global__ void attn_bwd_dkdv_kernel<T, D, false, true, true>(const AttnArgs); \
   template __global__ void attn_bwd_dq_ds_kernel<T, D>(const AttnArgs);                     \
-  template __global__ void attn_bwd_dq_kernel<T, D, false, 8, false>(const AttnArgs); \
-  template __global__ void attn_bwd_dq_kernel<T, D, false, 8, true>(const AttnArgs); \
-  template __global__ void attn_bwd_dq_kernel<T, D, true, 8, false>(const AttnArgs); \
   template __global__ void attn_bwd_dq_kernel<T, D, false, 4, false>(const AttnArgs); \
   template __global__ void attn_bwd_dq_kernel<T, D, false, 4, true>(const AttnArgs); \
   template __global__ void attn_bwd_dq_kernel<T, D, true, 4, false>(const AttnArgs); \
@@ -1856,6 +1864,13 @@ RSWA_INSTANTIATE(__bf16, 128)
 RSWA_INSTANTIATE(__bf16, 64)
 RSWA_INSTANTIATE(_Float16, 128)
 RSWA_INSTANTIATE(_Float16, 64)
+#undef RSWA_INSTANTIATE
+#define RSWA_INSTANTIATE(T)                                                           \
+  template __global__ void attn_bwd_dq_kernel<T, 128, false, 8, false>(const AttnArgs); \
+  template __global__ void attn_bwd_dq_kernel<T, 128, false, 8, true>(const AttnArgs); \
+  template __global__ void attn_bwd_dq_kernel<T, 128, true, 8, false>(const AttnArgs);
+RSWA_INSTANTIATE(__bf16)
+RSWA_INSTANTIATE(_Float16)
 #undef RSWA_INSTANTIATE
 
 // Does the dK/dV launch take blocks of 64 keys whose waves share out the walk (WALK4) instead of
@@ -1929,7 +1944,7 @@ int launch_bwd(AttnArgs& a, hipStream_t stream, int phases) {
   auto launch_dq = [&](auto stats) {
     constexpr bool STATS = decltype(stats)::value;
     const bool pair = (a.group & 1) == 0;
-    const bool small = a.avg_keys <= RSWA_DQ_SMALL_AVG_KEYS;
+    const bool small = D == 64 || a.avg_keys <= RSWA_DQ_SMALL_AVG_KEYS;
     const int bm = (pair ? 16 : 32) * (small ? 4 : 8);
     const int units_q = (pair ? a.group / 2 : a.group) * a.heads_kv;  // blocks per q tile
     if (a.cu_q) {
@@ -1945,13 +1960,19 @@ int launch_bwd(AttnArgs& a, hipStream_t stream, int phases) {
     const dim3 grid(padded_grid(a.n_work)), block(small ? 256 : 512);
     if constexpr (!STATS) {
       if (a.far) {
-        if (small) hipLaunchKernelGGL((attn_bwd_dq_kernel<T, D, true, 4, false>), grid, block, 0, stream, a);
-        else hipLaunchKernelGGL((attn_bwd_dq_kernel<T, D, true, 8, false>), grid, block, 0, stream, a);
+        if (small) {
+          hipLaunchKernelGGL((attn_bwd_dq_kernel<T, D, true, 4, false>), grid, block, 0, stream, a);
+        } else {
+          if constexpr (D == 128) hipLaunchKernelGGL((attn_bwd_dq_kernel<T, D, true, 8, false>), grid, block, 0, stream, a);
+        }
         return check_launch("attn_bwd dq");
       }
     }
-    if (small) hipLaunchKernelGGL((attn_bwd_dq_kernel<T, D, false, 4, STATS>), grid, block, 0, stream, a);
-    else hipLaunchKernelGGL((attn_bwd_dq_kernel<T, D, false, 8, STATS>), grid, block, 0, stream, a);
+    if (small) {
+      hipLaunchKernelGGL((attn_bwd_dq_kernel<T, D, false, 4, STATS>), grid, block, 0, stream, a);
+    } else {
+      if constexpr (D == 128) hipLaunchKernelGGL((attn_bwd_dq_kernel<T, D, false, 8, STATS>), grid, block, 0, stream, a);
+    }
     return check_launch("attn_bwd dq");
   };
   // Statistics and dQ asked for in one call: the dQ kernel goes first and makes the statistics.
