@@ -1893,13 +1893,15 @@ bool dkv_walk4(const AttnArgs& a, int head_dim) {
   if (a.dkdv_form == RSWA_DKDV_WIDE || a.dkdv_form == RSWA_DKDV_SHORT) return a.dkdv_form == RSWA_DKDV_SHORT;
   const bool pack = a.cu_q != nullptr;
   const int64_t lk1 = pack ? std::max<int64_t>(1, a.rows_k / a.batch) : a.seqlen_k;
-  // As many kv heads as q heads: a walk has no heads to deal, only query tiles, and with more than a
-  // round of 256-key blocks the short form loses by its longer fetches (us, wide / short, bf16, head_dim
+  // As many kv heads as q heads: a walk has no heads to deal, only query tiles, and with clearly more than
+  // a round of 256-key blocks the short form loses by its longer fetches (us, wide / short, bf16, head_dim
   // 128: a pack of 3010 tokens, 32 heads, window 2028, 54 / 96; 31427 tokens, 4 heads, 715, 133 / 164;
-  // dense 7428 rows, 12 heads, 64, 58 / 70; of 59 shapes drawn it was 13 % faster to 78 % slower, 16 %
-  // slower on average).
+  // dense 7428 rows, 12 heads, 64, 58 / 70).  Of 60 shapes drawn with 1 to 4 rounds it was 27 % faster to 7 %
+  // slower up to 1.25 rounds, 8 % faster on average (a pack of 7408 tokens, 8 heads, window 1374, 83 / 62;
+  // 3 x 2018 rows, 12 heads, window 323, 75 / 61), which are left to the estimate, and beyond that 13 %
+  // faster to 32 % slower, 6 % slower on average.
   const double wide_tiles = pack ? (double)lk1 / kDkvKeysPerBlock + 0.5 : (double)ceil_div(lk1, kDkvKeysPerBlock);
-  if (a.group == 1 && wide_tiles * a.heads_kv * a.batch > kComputeUnits) return false;
+  if (a.group == 1 && wide_tiles * a.heads_kv * a.batch > 1.25 * kComputeUnits) return false;
   const int64_t lq1 = pack ? std::max<int64_t>(1, a.rows_q / a.batch) : a.seqlen_q;
   const int64_t lq = pack ? std::min(a.rows_q, lq1 * 3 / 2) : lq1, lk = pack ? std::min(a.rows_k, lk1 * 3 / 2) : lk1;
   // query rows that see a key, of the first the band kernel owns to the last: on average, at most
