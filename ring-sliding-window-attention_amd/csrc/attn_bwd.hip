@@ -845,7 +845,7 @@ __global__ __launch_bounds__(256) void attn_bwd_dkdv_kernel(const AttnArgs a) {
 // rows of each head of the group in one block without fetching ahead: us, before / now, dK/dV and sink
 // launch: 2 x 300 rows, 32 / 8 heads, 1 sink 68 / 42; 12053 rows, 8 / 2 heads, window 67, 142 / 73; 2 x 31793
 // rows, 16 / 4 heads, 4 sinks 638 / 601; 550 sequences of 20 tokens, 12 heads, 570 / 276; the sink launch
-// alone on 65536 tokens, 32 / 8 heads, 4 sinks 458 / 390.
+// alone on 65536 tokens, 32 / 8 heads, 4 sinks 458 / 316.
 
 // sum over the aligned group of 16 lanes, in every lane of the group
 __device__ __forceinline__ float lane_group_sum16(float x) {
@@ -909,6 +909,10 @@ void attn_bwd_sink_kernel(const AttnArgs a) {
   auto put = [&](int j, int at, float sum) __attribute__((always_inline)) {  // at: d of dK, then of dV
     if (at < D) dk_ptr[(int64_t)j * a.dk_st[1] + at] = (T)(sum * a.scale);
     else dv_ptr[(int64_t)j * a.dv_st[1] + at - D] = (T)sum;
+  };
+
+  auto publish = [](float* at, float x) __attribute__((always_inline)) {
+    __hip_atomic_store(at, x, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   };
 
   struct Tile {
@@ -1012,27 +1016,29 @@ void attn_bwd_sink_kernel(const AttnArgs a) {
 #pragma unroll
       for (int w = 0; w < RW; w++) sum += red_s[w * SG + jj / NS][(jj % NS) * 2 * D + at];
       if (n_chunks == 1) put(j0 + jj, at, sum);
-      else a.sink_part[((int64_t)unit * a.sink_chunks + c) * (a.n_sink * 2 * D) + (j0 + jj) * (2 * D) + at] = sum;
+      else publish(a.sink_part + ((int64_t)unit * a.sink_chunks + c) * (a.n_sink * 2 * D) + (j0 + jj) * (2 * D) + at, sum);
     }
   }
   if (n_chunks == 1) return;
-  // count this chunk in; the last one of the unit adds them all up
+  // Count this chunk in; the last one of the unit adds them all up.  The sums are written through to where
+  // every XCD reads them and read from there, each by itself: a fence would write back and then drop
+  // the XCD's whole L2, under the feet of the blocks that are at work, for every block (us, this launch,
+  // with a fence per block / so: 51330 tokens in long sequences, 32 / 8 heads, head_dim 64, 191 / 105; 65536
+  // tokens, 4 sinks, 390 / 316; 3 x 5000 rows, 32 heads, head_dim 64, 105 / 60; with four times the blocks the
+  // fences cost 382 and 670).
   __shared__ int arrived_s;
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
   __syncthreads();
-  if (tid == 0) {
-    __threadfence();
-    arrived_s = atomicAdd(a.sink_count + unit, 1);
-  }
+  if (tid == 0) arrived_s = __hip_atomic_fetch_add(a.sink_count + unit, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   __syncthreads();
   if (arrived_s != n_chunks - 1) return;
-  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
   if (tid == 0) a.sink_count[unit] = 0;  // the next launch on this workspace starts from zero
   const float* parts = a.sink_part + (int64_t)unit * a.sink_chunks * (a.n_sink * 2 * D);
   for (int idx = tid; idx < ns_all * 2 * D; idx += 256) {
     float sum = 0.f;
 #pragma unroll 8
-    for (int cc = 0; cc < n_chunks; cc++) sum += parts[(int64_t)cc * (a.n_sink * 2 * D) + idx];
+    for (int cc = 0; cc < n_chunks; cc++)
+      sum += __hip_atomic_load(parts + (int64_t)cc * (a.n_sink * 2 * D) + idx, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     put(idx / (2 * D), idx % (2 * D), sum);
   }
 }
