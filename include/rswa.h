@@ -308,8 +308,9 @@ int rswa_attn_bwd_static_init(void);
  * key tile table), and with ds_handoff the dS tiles.  Nothing in the workspace has to be initialised by the caller. */
 uint64_t rswa_attn_bwd_workspace_bytes(const rswa_attn_params* p);
 
-/* The least workspace_bytes such a call accepts: without the key tile table, which only saves time
- * (packs run without it where the workspace has no room for it).  No counterpart in the upstream
+/* The least workspace_bytes such a call accepts: without the key tile table and with fewer sums of the
+ * sink kernel, which only cost time (a call takes that layout where the workspace has no room for the
+ * other).  No counterpart in the upstream
  * package, like the buffer itself. */
 uint64_t rswa_attn_bwd_workspace_min_bytes(const rswa_attn_params* p);
 

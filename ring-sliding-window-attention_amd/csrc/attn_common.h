@@ -586,8 +586,8 @@ struct BwdLayout {
   uint64_t ds_off, ds_bytes;
   int ds_nkb, ds_slots;
 };
-// (`max_bytes`: room there is; the key tile table of a pack, which only saves time, is left out
-// where it would not fit)
+// (`max_bytes`: room there is; where the whole would not fit, the key tile table of a pack is left out and
+// the sink kernel gets fewer chunks, which only cost time)
 BwdLayout bwd_layout(const rswa_attn_params* p, bool allow_handoff, uint64_t max_bytes = ~0ull);
 
 // Fill an AttnArgs from the public struct; validates what both directions share.

@@ -136,7 +136,9 @@ int forward(const Call& c, const Tensor& q, const Tensor& k, const Tensor& v, Te
   const auto f32 = q.options().dtype(at::kFloat);
   lse = c.packed ? at::empty({q.size(1), q.size(0)}, f32) : at::empty({q.size(0), q.size(2), q.size(1)}, f32);
   const rswa_attn_params p = params(c, q, k, v, out, lse);
-  return lib.fwd(&p, stream_of(q));
+  void* const stream = stream_of(q);
+  pybind11::gil_scoped_release others_run;  // (a launch waits where the queue is full)
+  return lib.fwd(&p, stream);
 }
 
 [[noreturn]] void throw_python() {
