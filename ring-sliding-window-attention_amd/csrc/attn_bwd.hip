@@ -964,6 +964,13 @@ void attn_bwd_sink_kernel(const AttnArgs a) {
           }
         }
         fetch(nxt);
+        // rows past the end, which hold the last row's values: their P and dS are zero, but zero times an
+        // infinity or a NaN of that row is a NaN
+        if (__builtin_amdgcn_readfirstlane(cur.row - r) + 16 > len_q) {
+#pragma unroll
+          for (int ks = 0; ks < KS; ks++)
+            if (cur.row >= len_q) cur.q[ks] = cur.d[ks] = V8{0, 0, 0, 0, 0, 0, 0, 0};
+        }
         f32x4 s = {0.f, 0.f, 0.f, 0.f}, dp = {cur.nd, cur.nd, cur.nd, cur.nd};
         int a_row = (sg * 4 + (r & 3)) * D + u * 8;  // row r of the A operand: sink r % 4
         asm volatile("" : "+v"(a_row));              // (read here: kept in registers the operands would spill)

@@ -42,3 +42,28 @@ def test_sink_rows(lens, hq, hk, window, sinks, d, dtype):
     at = torch.tensor([c + j for c, n in zip(cu, lens) for j in range(min(sinks, n))])
     for x, r in ((got[0][1], rk), (got[0][2], rv)):  # (and by themselves, so that no other row hides one)
         assert relnorm(x[at.cuda()], r[at]) <= GRAD_TOL
+
+
+@pytest.mark.parametrize("n", [15, 16, 17, 47])
+@pytest.mark.parametrize("sinks", [1, 3])
+def test_an_infinity_in_the_last_row_stays_one(n, sinks):
+    """dV of a key is sum P dO: an infinite dO of the last row makes it infinite in that column and leaves the
+    others.  (The lanes of a tile that stand for rows past the end have P = 0, which must not meet it.)"""
+    from ring_swa.ops import attn_bwd, attn_fwd
+
+    torch.manual_seed(n)
+    q, do = (torch.randn(1, n, 4, 64, device="cuda").bfloat16() for _ in range(2))
+    k, v = (torch.randn(1, n, 2, 64, device="cuda").bfloat16() for _ in range(2))
+    out, lse = attn_fwd(q, k, v, None, (4, 0), True, num_sink=sinks)
+
+    def dv_of(do):
+        g = [torch.empty_like(x) for x in (q, k, v)]
+        attn_bwd(q, k, v, out, lse, do, *g, None, (4, 0), True, num_sink=sinks)
+        return g[2]
+
+    want = dv_of(do)
+    do[0, -1, 0, 3] = float("inf")
+    got = dv_of(do)
+    assert (got[0, :sinks, 0, 3] == float("inf")).all()
+    want[0, :, 0, 3] = got[0, :, 0, 3] = 0
+    assert torch.equal(got[0, :sinks], want[0, :sinks])
