@@ -43,7 +43,7 @@ struct {
   int (*bwd)(const rswa_attn_params*, void*) = nullptr;
   uint64_t (*bwd_bytes)(const rswa_attn_params*) = nullptr;
   PyObject* raise = nullptr;         // raises what a non-zero status means
-  PyObject* python_bwd = nullptr;    // backward in Python, for the environment's switches
+  PyObject* python_bwd = nullptr;    // backward in Python, for the environment's switches and what has to be refused
 } lib;
 
 bool env_switches() {
@@ -72,6 +72,32 @@ bool plain(const Tensor& t) {
                            c10::DispatchKey::ADInplaceOrView});
   return t.defined() && t.is_cuda() && t.layout() == at::kStrided && (t.key_set().raw_repr() & ~known.raw_repr()) == 0 &&
          !t._fw_grad(0).defined();
+}
+
+// Queries, keys and values that the kernels take as they are?
+bool fits(const Tensor& q, const Tensor& k, const Tensor& v, bool packed) {
+  const int nd = packed ? 3 : 4;
+  if (!plain(q) || !plain(k) || !plain(v)) return false;
+  const auto type = q.scalar_type();
+  if ((type != at::kBFloat16 && type != at::kHalf) || k.scalar_type() != type || v.scalar_type() != type) return false;
+  if (q.dim() != nd || k.dim() != nd || v.dim() != nd || k.sizes() != v.sizes()) return false;
+  if (q.device() != k.device() || q.device() != v.device()) return false;
+  if (q.numel() == 0 || k.numel() == 0) return false;
+  for (int d = 0; d < nd - 2; d++)
+    if (q.size(d) != k.size(d) || q.size(d) >= (1 << 28)) return false;
+  if (q.size(-1) != k.size(-1) || q.size(-2) % k.size(-2) != 0 || q.size(-2) >= (1 << 28)) return false;
+  return q.stride(-1) == 1 && k.stride(-1) == 1 && v.stride(-1) == 1;
+}
+
+// ... and another tensor of q's type, shape and device
+bool like(const Tensor& t, const Tensor& q) {
+  return plain(t) && t.scalar_type() == q.scalar_type() && t.sizes() == q.sizes() && t.device() == q.device() &&
+         t.stride(-1) == 1;
+}
+
+bool lse_of(const Tensor& t, const Tensor& q, bool packed) {
+  if (!plain(t) || t.scalar_type() != at::kFloat || t.device() != q.device()) return false;
+  return packed ? t.sizes().equals({q.size(1), q.size(0)}) : t.sizes().equals({q.size(0), q.size(2), q.size(1)});
 }
 
 struct Call {
@@ -170,7 +196,10 @@ struct BandNode : torch::autograd::Function<BandNode> {
     Tensor dout = grads[0];
     if (dout.stride(-1) != 1) dout = dout.contiguous();
     const Tensor dq = at::empty_like(q), dk = at::empty_like(k), dv = at::empty_like(v);
-    if (env_switches()) {
+    // (hooks of saved tensors may give back others: what does not fit is for the Python route to refuse)
+    const bool as_saved = fits(q, k, v, c.packed) && like(out, q) && like(dout, q) && lse_of(lse, q, c.packed) &&
+                          (!c.packed || c.cu.device() == q.device());
+    if (!as_saved || env_switches()) {
       pybind11::gil_scoped_acquire gil;
       PyObject* r = PyObject_CallFunction(
           lib.python_bwd, "NNNNNNNNNdiNi", THPVariable_Wrap(q), THPVariable_Wrap(k), THPVariable_Wrap(v),
@@ -220,18 +249,7 @@ PyObject* band_attn(PyObject*, PyObject* const* args, Py_ssize_t n) {
     if (!plain(cu) || cu.scalar_type() != at::kInt || cu.dim() != 1 || !cu.is_contiguous() || cu.numel() < 2)
       Py_RETURN_NONE;
   }
-  const int nd = c.packed ? 3 : 4;
-  if (!plain(q) || !plain(k) || !plain(v) || observed() || env_switches()) Py_RETURN_NONE;
-  const auto type = q.scalar_type();
-  if ((type != at::kBFloat16 && type != at::kHalf) || k.scalar_type() != type || v.scalar_type() != type)
-    Py_RETURN_NONE;
-  if (q.dim() != nd || k.dim() != nd || v.dim() != nd || k.sizes() != v.sizes()) Py_RETURN_NONE;
-  if (q.device() != k.device() || q.device() != v.device() || (c.packed && q.device() != c.cu.device())) Py_RETURN_NONE;
-  if (q.numel() == 0 || k.numel() == 0) Py_RETURN_NONE;
-  for (int d = 0; d < nd - 2; d++)
-    if (q.size(d) != k.size(d) || q.size(d) >= (1 << 28)) Py_RETURN_NONE;
-  if (q.size(-1) != k.size(-1) || q.size(-2) % k.size(-2) != 0 || q.size(-2) >= (1 << 28)) Py_RETURN_NONE;
-  if (q.stride(-1) != 1 || k.stride(-1) != 1 || v.stride(-1) != 1) Py_RETURN_NONE;
+  if (!fits(q, k, v, c.packed) || (c.packed && q.device() != c.cu.device()) || observed() || env_switches()) Py_RETURN_NONE;
   if (!PyLong_CheckExact(args[3]) || !PyLong_CheckExact(args[6])) Py_RETURN_NONE;
   int over = 0;
   const long long window = PyLong_AsLongLongAndOverflow(args[3], &over);

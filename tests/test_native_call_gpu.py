@@ -165,3 +165,34 @@ def test_streams_and_threads():
     [t.start() for t in ts]
     [t.join() for t in ts]
     assert not bad
+
+
+@pytest.mark.parametrize("packed", [False, True])
+@pytest.mark.parametrize("which,change,error", [
+    (0, lambda t: t.cpu(), RuntimeError), (4, lambda t: t.cpu(), RuntimeError), (3, lambda t: t.cpu(), RuntimeError),
+    (4, lambda t: t.to(torch.bfloat16), AssertionError), (4, lambda t: t[..., :-8], AssertionError),
+    (1, lambda t: t.float(), AssertionError), (1, lambda t: t[..., :-1, :], AssertionError),
+    (2, lambda t: t.transpose(-1, -2).contiguous().transpose(-1, -2), AssertionError),
+    (3, lambda t: t[..., :32], AssertionError), (0, lambda t: t.flatten(-2), AssertionError),
+])
+def test_saved_tensors_that_hooks_gave_back_changed_are_refused(packed, which, change, error):
+    """What is unpacked need not be what was packed: another type, shape, device or layout is refused ahead of
+    any launch (saved are q, k, v, out and lse, in this order); the same values in another layout that the
+    kernels take are used."""
+    import ring_swa
+
+    q, k, v = _inputs(packed)
+    args = (31, torch.tensor([0, 70, 200], dtype=torch.int32, device="cuda")) if packed else (31,)
+    attn = ring_swa.ring_sliding_window_attn_varlen if packed else ring_swa.ring_sliding_window_attn
+    want = torch.autograd.grad(attn(q, k, v, *args).float().sum(), (q, k, v))
+
+    def grads(pack):
+        n = []
+        with torch.autograd.graph.saved_tensors_hooks(lambda t: (n.append(1), pack(len(n) - 1, t))[1], lambda t: t):
+            out = attn(q, k, v, *args)
+        return torch.autograd.grad(out.float().sum(), (q, k, v))
+
+    with pytest.raises(error):
+        grads(lambda i, t: change(t.detach()) if i == which else t)
+    for x, r in zip(grads(lambda i, t: torch.stack([t.detach()] * 2, -2)[..., 0, :] if i < 4 else t), want):
+        assert torch.equal(x, r)
