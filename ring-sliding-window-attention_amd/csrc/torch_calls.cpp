@@ -46,7 +46,10 @@ struct {
   PyObject* python_bwd = nullptr;    // backward in Python, for the environment's switches and what has to be refused
 } lib;
 
+// With the interpreter lock only: Python changes the environment under it, and a getenv beside such a change
+// may read the array that it has just freed.
 bool env_switches() {
+  TORCH_INTERNAL_ASSERT(PyGILState_Check());
   for (const char* name : {"RSWA_ADDRESSING", "RSWA_DKDV_FORM", "RSWA_DS_HANDOFF"}) {
     const char* v = std::getenv(name);
     if (v && *v) return true;
@@ -199,7 +202,11 @@ struct BandNode : torch::autograd::Function<BandNode> {
     // (hooks of saved tensors may give back others: what does not fit is for the Python route to refuse)
     const bool as_saved = fits(q, k, v, c.packed) && like(out, q) && like(dout, q) && lse_of(lse, q, c.packed) &&
                           (!c.packed || c.cu.device() == q.device());
-    if (!as_saved || env_switches()) {
+    const bool switched = [] {  // (the thread that waits for the engine has let go of the lock: no cost to be seen)
+      pybind11::gil_scoped_acquire gil;
+      return env_switches();
+    }();
+    if (!as_saved || switched) {
       pybind11::gil_scoped_acquire gil;
       PyObject* r = PyObject_CallFunction(
           lib.python_bwd, "NNNNNNNNNdiNi", THPVariable_Wrap(q), THPVariable_Wrap(k), THPVariable_Wrap(v),

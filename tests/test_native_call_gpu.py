@@ -196,3 +196,34 @@ def test_saved_tensors_that_hooks_gave_back_changed_are_refused(packed, which, c
         grads(lambda i, t: change(t.detach()) if i == which else t)
     for x, r in zip(grads(lambda i, t: torch.stack([t.detach()] * 2, -2)[..., 0, :] if i < 4 else t), want):
         assert torch.equal(x, r)
+
+
+def test_backward_beside_a_thread_that_changes_the_environment():
+    """The backward looks at the environment from the autograd thread, where another thread may be adding
+    variables (which moves the array that getenv walks): it does so under the interpreter's lock, and says so
+    itself where it does not."""
+    import os
+    import threading
+
+    import ring_swa
+
+    q, k, v = _inputs(False)
+    want = torch.autograd.grad(ring_swa.ring_sliding_window_attn(q, k, v, 31).float().sum(), (q, k, v))
+    stop, names = threading.Event(), [f"RSWA_TEST_{i}" for i in range(200)]
+
+    def change():
+        while not stop.is_set():
+            for n in names:
+                os.environ[n] = "x" * 50
+            for n in names:
+                del os.environ[n]
+
+    t = threading.Thread(target=change)
+    t.start()
+    try:
+        for _ in range(20):
+            got = torch.autograd.grad(ring_swa.ring_sliding_window_attn(q, k, v, 31).float().sum(), (q, k, v))
+            assert all(torch.equal(x, r) for x, r in zip(got, want))
+    finally:
+        stop.set()
+        t.join()
