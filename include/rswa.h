@@ -309,9 +309,10 @@ int rswa_attn_bwd_static_init(void);
 uint64_t rswa_attn_bwd_workspace_bytes(const rswa_attn_params* p);
 
 /* The least workspace_bytes such a call accepts: without the key tile table and with fewer sums of the
- * sink kernel, which only cost time (a call takes that layout where the workspace has no room for the
- * other).  No counterpart in the upstream
- * package, like the buffer itself. */
+ * sink kernel.  A call takes the whole where there is room for it, else leaves out the table (which only
+ * costs time: the same bits), else takes the fewer sums too: slower, and dk / dv of sink keys are the same
+ * fp32 sums added in another order, so that their last bit may differ from a call with more room.  No
+ * counterpart in the upstream package, like the buffer itself. */
 uint64_t rswa_attn_bwd_workspace_min_bytes(const rswa_attn_params* p);
 
 /* 1 when a backward with these parameters takes the dS hand-off route (ds_handoff != 0 and the

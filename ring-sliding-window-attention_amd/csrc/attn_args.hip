@@ -26,7 +26,10 @@ static bool handoff_eligible(const rswa_attn_params* p) {
   return true;
 }
 
-static BwdLayout layout_of(const rswa_attn_params* p, bool allow_handoff, bool lean) {
+// What a workspace has room for
+enum class Room { ALL, NO_TABLE, LEAST };
+
+static BwdLayout layout_of(const rswa_attn_params* p, bool allow_handoff, Room room) {
   BwdLayout L{};
   if (!p || p->batch <= 0 || p->heads_q <= 0 || p->heads_kv <= 0 || p->head_dim <= 0) return L;
   L.stats_bytes = delta_bytes(p);
@@ -35,14 +38,14 @@ static BwdLayout layout_of(const rswa_attn_params* p, bool allow_handoff, bool l
   const int group = p->heads_q / p->heads_kv;
   // Sink keys under a bounded window: the sink kernel, with one arrival counter per (sequence, kv head) and
   // chunks of the tiles of an average one: up to 64, some 2048 blocks in all, of eight tiles of 16 rows or
-  // more (lean: no more than one per 512 rows)
+  // more (LEAST: no more than one per 512 rows)
   int64_t sink_units = 0;
   if (p->num_sink > 0 && p->window_left >= 0) {
     const int64_t rows_q = packed ? p->total_q / p->batch : p->seqlen_q;
     sink_units = (int64_t)p->batch * p->heads_kv;
     const int64_t tiles = (rows_q + 15) / 16 * group;
     int64_t chunks = std::min({(int64_t)64, (2047 + sink_units) / sink_units, (tiles + 7) / 8});
-    if (lean) chunks = std::min(chunks, (rows_q + 511) / 512);
+    if (room == Room::LEAST) chunks = std::min(chunks, (rows_q + 511) / 512);
     L.sink_chunks = (int)std::max<int64_t>(1, chunks);
   }
   // workspace: statistics | arrival counters and sums of the sink kernel | key tile table | dS tiles
@@ -51,7 +54,7 @@ static BwdLayout layout_of(const rswa_attn_params* p, bool allow_handoff, bool l
   L.sink_off = L.count_off + align_up((uint64_t)L.n_count * sizeof(int32_t), 256);
   L.total_bytes = L.sink_off + (uint64_t)sink_units * L.sink_chunks * p->num_sink * 2 * p->head_dim *
                                    sizeof(float);
-  if (packed && !lean) {
+  if (packed && room == Room::ALL) {
     L.ktile_off = align_up(L.total_bytes, 256);
     L.total_bytes = L.ktile_off + ((uint64_t)p->batch + 2) * sizeof(int32_t);
   }
@@ -84,8 +87,10 @@ static BwdLayout layout_of(const rswa_attn_params* p, bool allow_handoff, bool l
 }
 
 BwdLayout bwd_layout(const rswa_attn_params* p, bool allow_handoff, uint64_t max_bytes) {
-  const BwdLayout L = layout_of(p, allow_handoff, false);
-  return L.total_bytes <= max_bytes ? L : layout_of(p, allow_handoff, true);
+  // (the table, of a few bytes, alone first: without it the results keep their bits)
+  BwdLayout L = layout_of(p, allow_handoff, Room::ALL);
+  if (L.total_bytes > max_bytes) L = layout_of(p, allow_handoff, Room::NO_TABLE);
+  return L.total_bytes <= max_bytes ? L : layout_of(p, allow_handoff, Room::LEAST);
 }
 
 uint64_t bwd_workspace_bytes(const rswa_attn_params* p) { return bwd_layout(p, true).total_bytes; }

@@ -586,8 +586,9 @@ struct BwdLayout {
   uint64_t ds_off, ds_bytes;
   int ds_nkb, ds_slots;
 };
-// (`max_bytes`: room there is; where the whole would not fit, the key tile table of a pack is left out and
-// the sink kernel gets fewer chunks, which only cost time)
+// (`max_bytes`: room there is; where the whole would not fit, the key tile table of a pack is left out, which
+// only costs time, and where that is not enough the sink kernel gets fewer chunks: the same sums in another
+// order)
 BwdLayout bwd_layout(const rswa_attn_params* p, bool allow_handoff, uint64_t max_bytes = ~0ull);
 
 // Fill an AttnArgs from the public struct; validates what both directions share.

@@ -224,8 +224,8 @@ def attn_bwd(
     ``second=(k2, v2, dk2, dv2)``: keys in two row ranges as in ``attn_fwd``; the gradients of
     the second range's rows go to ``dk2, dv2`` (shapes and strides of ``k2, v2``).
 
-    ``workspace`` (uint8, ``bwd_workspace_bytes(q, k, ...)`` of it; packs also take one without room
-    for the key tile table) may be supplied to avoid the per-call scratch allocation, and must be
+    ``workspace`` (uint8, ``bwd_workspace_bytes(q, k, ...)`` of it; one without room for a pack's key tile
+    table, which gives the same bits, or for all sums of the sink kernel is taken too) may be supplied to avoid the per-call scratch allocation, and must be
     when the phases of one backward are spread over several calls; ``phases`` is the bit mask of
     ``rswa_attn_bwd_phases`` (1 prep, 2 dk/dv kernel, 4 dq kernel).  ``dq_accumulate`` adds this call's dQ to the values
     already in ``dq`` (fp32 add of the two 16-bit values, one rounding).

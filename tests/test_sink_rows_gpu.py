@@ -67,3 +67,38 @@ def test_an_infinity_in_the_last_row_stays_one(n, sinks):
     assert (got[0, :sinks, 0, 3] == float("inf")).all()
     want[0, :, 0, 3] = got[0, :, 0, 3] = 0
     assert torch.equal(got[0, :sinks], want[0, :sinks])
+
+
+@pytest.mark.parametrize("d", [64, 128])
+def test_sink_rows_with_less_workspace(d):
+    """Without room for a pack's key tile table the sums are chunked as with it: the same bits (fp16 and many
+    sinks, so that sums in another order show: in 95 values with head_dim 128).  With the least workspace
+    they are not: held to the oracle."""
+    from ring_swa import _lib
+    from ring_swa.ops import attn_bwd, attn_fwd
+    from ring_swa.ops.band_attn import _params, bwd_workspace_bytes
+
+    cu, hq, hk, window, sinks = [0, 300, 300, 301, 901, 1500], 4, 2, 100, 64
+    torch.manual_seed(4)
+    q, do = (torch.randn(cu[-1], hq, d, device="cuda", dtype=torch.float16) for _ in range(2))
+    k, v = (torch.randn(cu[-1], hk, d, device="cuda", dtype=torch.float16) for _ in range(2))
+    cud = torch.tensor(cu, dtype=torch.int32, device="cuda")
+    out, lse = attn_fwd(q, k, v, None, (window, 0), True, cud, cud, num_sink=sinks)
+    need = bwd_workspace_bytes(q, k, cud, cud, window_size=(window, 0), causal=True, num_sink=sinks)
+    table = (len(cu) + 1) * 4  # the last thing in it
+    p = _params(q, k, v, 1., (window, 0), True, cud, cud, sinks)
+    least = _lib.lib().rswa_attn_bwd_workspace_min_bytes(p)
+    assert least < need - table
+    got = []
+    for room in (need, need - table, need - table - 256, least):
+        ws = torch.full((room,), 255, dtype=torch.uint8, device="cuda")
+        g = [torch.full_like(x, float("nan")) for x in (q, k, v)]
+        attn_bwd(q, k, v, out, lse, do, *g, None, (window, 0), True, cud, cud, num_sink=sinks, workspace=ws)
+        got.append(g)
+    for x, same in zip(*got[:2]):
+        assert torch.equal(x, same)
+    _, _, *ref = O.attention_fwd_bwd(
+        lambda q, k, v: O.streaming_llm_attn_varlen(q, k, v, window, cu, n_sink=sinks), q, k, v, do)
+    for g in got:
+        for x, r in zip(g, ref):
+            assert relnorm(x, r) <= GRAD_TOL
