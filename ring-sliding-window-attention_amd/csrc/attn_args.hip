@@ -26,6 +26,9 @@ static bool handoff_eligible(const rswa_attn_params* p) {
   return true;
 }
 
+// Bytes that the sink kernel's sums may take before there is no more than one chunk per 512 rows
+constexpr double kSinkSumBytes = 64 << 20;
+
 // What a workspace has room for
 enum class Room { ALL, NO_TABLE, LEAST };
 
@@ -38,14 +41,18 @@ static BwdLayout layout_of(const rswa_attn_params* p, bool allow_handoff, Room r
   const int group = p->heads_q / p->heads_kv;
   // Sink keys under a bounded window: the sink kernel, with one arrival counter per (sequence, kv head) and
   // chunks of the tiles of an average one: up to 64, some 2048 blocks in all, of eight tiles of 16 rows or
-  // more (LEAST: no more than one per 512 rows)
+  // more (LEAST: no more than one per 512 rows; nor beyond kSinkSumBytes, which only a hundred sinks or more
+  // reach: 128 of 4001 rows, 32 / 8 heads, take 64 MiB and 1240 us, dK/dV and sink launch, against 2077 in 8)
   int64_t sink_units = 0;
   if (p->num_sink > 0 && p->window_left >= 0) {
     const int64_t rows_q = packed ? p->total_q / p->batch : p->seqlen_q;
     sink_units = (int64_t)p->batch * p->heads_kv;
     const int64_t tiles = (rows_q + 15) / 16 * group;
     int64_t chunks = std::min({(int64_t)64, (2047 + sink_units) / sink_units, (tiles + 7) / 8});
-    if (room == Room::LEAST) chunks = std::min(chunks, (rows_q + 511) / 512);
+    const int64_t by_rows = (rows_q + 511) / 512;
+    const double chunk_bytes = (double)sink_units * p->num_sink * 2 * p->head_dim * sizeof(float);
+    if (room == Room::LEAST || chunks * chunk_bytes > kSinkSumBytes)
+      chunks = std::min(chunks, room == Room::LEAST ? by_rows : std::max(by_rows, (int64_t)(kSinkSumBytes / chunk_bytes)));
     L.sink_chunks = (int)std::max<int64_t>(1, chunks);
   }
   // workspace: statistics | arrival counters and sums of the sink kernel | key tile table | dS tiles

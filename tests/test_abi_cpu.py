@@ -291,3 +291,23 @@ def test_head_dim_64_forward_takes_three_blocks_per_unit_where_two_do_not_hold_t
     assert _lib.lib().rswa_attn_fwd_blocks_per_cu(p) == blocks
     p.head_dim = 128
     assert _lib.lib().rswa_attn_fwd_blocks_per_cu(p) == 2
+
+
+@pytest.mark.parametrize("rows,heads_q,heads_kv,batch,sinks", [
+    (4001, 32, 8, 1, 4096), (4001, 32, 8, 1, 128), (1024, 32, 32, 16, 512), (65536, 32, 8, 1, 4), (65536, 8, 2, 1, 4096),
+    (300, 4, 1, 2, 1), (20, 12, 12, 550, 1 << 20),
+])
+def test_workspace_of_many_sink_keys_is_bounded(rows, heads_q, heads_kv, batch, sinks):
+    """The sink kernel's sums take 64 MiB, or what one chunk of them per 512 rows (at most 64) takes: a few
+    thousand sinks in as many chunks as a few keys get would be gigabytes."""
+    _ensure_built()
+    from ring_swa import _lib
+
+    p = _fake_params(rows, heads_q, heads_kv)
+    p.batch, p.num_sink = batch, sinks
+    stats = 2 * (-(-batch * rows * heads_q * 4 // 256) * 256) + -(-batch * heads_kv * 4 // 256) * 256
+    per_chunk = batch * heads_kv * sinks * 2 * 128 * 4
+    sums = _lib.lib().rswa_attn_bwd_workspace_bytes(p) - stats
+    assert sums % per_chunk == 0 and 1 <= sums // per_chunk <= 64
+    assert sums <= max(64 << 20, min(64, -(-rows // 512)) * per_chunk)
+    assert _lib.lib().rswa_attn_bwd_workspace_min_bytes(p) - stats <= min(64, -(-rows // 512)) * per_chunk
