@@ -8,6 +8,7 @@ from __future__ import annotations
 import ctypes
 import importlib.util
 import os
+import warnings
 from ctypes import (POINTER, Structure, c_char_p, c_float, c_int, c_int32, c_int64, c_uint64,
                     c_void_p)
 
@@ -159,29 +160,33 @@ _torch_calls = None
 
 def torch_calls():
     """The module of ``csrc/torch_calls.cpp``: the plain attention call without Python between the
-    checks and the launch.  Built beside the library; next to a library from elsewhere
-    (``RSWA_LIBRARY``) the package also works without it, through Python (None)."""
+    checks and the launch.  Built beside the library; where it is not, the package works without it,
+    through Python (None), and says so once."""
     global _torch_calls
     if _torch_calls is None:
-        L = lib()
-        path = os.path.join(_PKG_ROOT, "lib", "rswa_torch.so")
-        if not os.path.exists(path):
-            if os.environ.get("RSWA_LIBRARY"):
-                _torch_calls = False
-                return None
-            raise ImportError(f"{path} is missing: build it with `python {os.path.join(_PKG_ROOT, 'build.py')}`")
-        spec = importlib.util.spec_from_file_location("rswa_torch", path)
-        mod = importlib.util.module_from_spec(spec)
-        spec.loader.exec_module(mod)
-        if mod.params_bytes() != ctypes.sizeof(AttnParams):
-            raise ImportError(f"{path} was built for another rswa_attn_params: rebuild it")
-        from .sliding_window import band_backward
-
-        mod.bind(*[ctypes.cast(fn, c_void_p).value
-                   for fn in (L.rswa_attn_fwd, L.rswa_attn_bwd, L.rswa_attn_bwd_workspace_bytes)],
-                 check, band_backward)
-        _torch_calls = mod
+        _torch_calls = _load_torch_calls() or False
     return _torch_calls or None
+
+
+def _load_torch_calls():
+    L = lib()
+    path = os.path.join(_PKG_ROOT, "lib", "rswa_torch.so")
+    if not os.path.exists(path):
+        if not os.environ.get("RSWA_LIBRARY"):
+            warnings.warn(f"{path} is missing: small calls take twice the host time. Build it with "
+                          f"`python {os.path.join(_PKG_ROOT, 'build.py')}`", RuntimeWarning)
+        return None
+    spec = importlib.util.spec_from_file_location("rswa_torch", path)
+    mod = importlib.util.module_from_spec(spec)
+    spec.loader.exec_module(mod)
+    if mod.params_bytes() != ctypes.sizeof(AttnParams):
+        raise ImportError(f"{path} was built for another rswa_attn_params: rebuild it")
+    from .sliding_window import band_backward
+
+    mod.bind(*[ctypes.cast(fn, c_void_p).value
+               for fn in (L.rswa_attn_fwd, L.rswa_attn_bwd, L.rswa_attn_bwd_workspace_bytes)],
+             check, band_backward)
+    return mod
 
 
 def check(status: int) -> None:
