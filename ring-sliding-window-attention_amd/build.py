@@ -206,10 +206,20 @@ def _check_lds_loads(obj: str) -> None:
                                        + "\n  ".join(bad))
 
 
+def _torch_build() -> str:
+    """The same text as ring_swa._lib.torch_build() (the build imports nothing of the package)."""
+    import torch
+
+    return (f"{torch.__version__} {torch.version.git_version} hip {torch.version.hip} "
+            f"python {sys.version_info[0]}.{sys.version_info[1]}")
+
+
 def _build_torch_calls(force: bool) -> str:
-    """The module of csrc/torch_calls.cpp, against the installed PyTorch."""
+    """The module of csrc/torch_calls.cpp, against the installed PyTorch (build/rswa_torch.for: which it was)."""
     src, out = os.path.join(CSRC, "torch_calls.cpp"), os.path.join(LIBDIR, "rswa_torch.so")
-    if force or _stale(out, [src] + _headers()):
+    made_for, now = os.path.join(OBJ, "rswa_torch.for"), _torch_build()
+    same = os.path.exists(made_for) and open(made_for).read() == now
+    if force or not same or _stale(out, [src] + _headers()):
         import sysconfig
 
         import torch
@@ -218,12 +228,14 @@ def _build_torch_calls(force: bool) -> str:
         inc = [os.path.join(root, "include"), os.path.join(root, "include", "torch", "csrc", "api", "include"),
                os.path.join(os.environ.get("ROCM_PATH", "/opt/rocm"), "include"), sysconfig.get_paths()["include"]]
         cmd = [os.environ.get("CXX", "g++"), "-O2", "-std=c++17", "-fPIC", "-shared", "-Wall", "-D__HIP_PLATFORM_AMD__=1",
-               "-DUSE_ROCM=1", f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}",
+               "-DUSE_ROCM=1", f'-DRSWA_TORCH_BUILD="{now}"', f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}",
                *[x for i in inc for x in ("-isystem", i)], src, "-o", out, "-L" + os.path.join(root, "lib"),
                *["-l" + n for n in ("c10", "c10_hip", "torch_cpu", "torch_hip", "torch", "torch_python")]]
         r = subprocess.run(cmd, capture_output=True, text=True)
         if r.returncode != 0:
             raise RuntimeError(f"C++ compiler failed for {src}:\n{r.stdout}\n{r.stderr}")
+        with open(made_for, "w") as f:
+            f.write(now)
     return out
 
 

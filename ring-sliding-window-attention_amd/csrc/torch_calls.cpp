@@ -304,12 +304,17 @@ PyObject* bind(PyObject*, PyObject* const* args, Py_ssize_t n) {
   Py_RETURN_NONE;
 }
 
+// The PyTorch whose headers this was compiled with (ring_swa._lib.torch_build): their inlined accessors read
+// tensors at its layout, so that another must not be handed any
+PyObject* torch_build(PyObject*, PyObject*) { return PyUnicode_FromString(RSWA_TORCH_BUILD); }
+
 PyObject* params_bytes(PyObject*, PyObject*) { return PyLong_FromSize_t(sizeof(rswa_attn_params)); }
 
 PyMethodDef methods[] = {
     {"band_attn", reinterpret_cast<PyCFunction>(reinterpret_cast<void*>(&band_attn)), METH_FASTCALL, nullptr},
     {"bind", reinterpret_cast<PyCFunction>(reinterpret_cast<void*>(&bind)), METH_FASTCALL, nullptr},
     {"params_bytes", &params_bytes, METH_NOARGS, nullptr},
+    {"torch_build", &torch_build, METH_NOARGS, nullptr},
     {nullptr, nullptr, 0, nullptr}};
 PyModuleDef module = {PyModuleDef_HEAD_INIT, "rswa_torch", nullptr, -1, methods, nullptr, nullptr, nullptr, nullptr};
 

@@ -8,6 +8,7 @@ from __future__ import annotations
 import ctypes
 import importlib.util
 import os
+import sys
 import warnings
 from ctypes import (POINTER, Structure, c_char_p, c_float, c_int, c_int32, c_int64, c_uint64,
                     c_void_p)
@@ -160,12 +161,18 @@ _torch_calls = None
 
 def torch_calls():
     """The module of ``csrc/torch_calls.cpp``: the plain attention call without Python between the
-    checks and the launch.  Built beside the library; where it is not, the package works without it,
-    through Python (None), and says so once."""
+    checks and the launch.  Built beside the library; where it is not, or was built for another PyTorch,
+    the package works without it, through Python (None), and says so once."""
     global _torch_calls
     if _torch_calls is None:
         _torch_calls = _load_torch_calls() or False
     return _torch_calls or None
+
+
+def torch_build() -> str:
+    """The running PyTorch, as far as code compiled against its headers depends on it."""
+    return (f"{torch.__version__} {torch.version.git_version} hip {torch.version.hip} "
+            f"python {sys.version_info[0]}.{sys.version_info[1]}")
 
 
 def _load_torch_calls():
@@ -177,8 +184,16 @@ def _load_torch_calls():
                           f"`python {os.path.join(_PKG_ROOT, 'build.py')}`", RuntimeWarning)
         return None
     spec = importlib.util.spec_from_file_location("rswa_torch", path)
-    mod = importlib.util.module_from_spec(spec)
-    spec.loader.exec_module(mod)
+    try:
+        mod = importlib.util.module_from_spec(spec)
+        spec.loader.exec_module(mod)
+        built_for = getattr(mod, "torch_build", lambda: "another PyTorch")()
+    except ImportError as e:  # (symbols that this PyTorch does not have)
+        built_for = f"another PyTorch ({e})"
+    if built_for != torch_build():
+        warnings.warn(f"{path} was built for {built_for}, this is {torch_build()}: not used, small calls take twice "
+                      f"the host time. Build it with `python {os.path.join(_PKG_ROOT, 'build.py')}`", RuntimeWarning)
+        return None
     if mod.params_bytes() != ctypes.sizeof(AttnParams):
         raise ImportError(f"{path} was built for another rswa_attn_params: rebuild it")
     from .sliding_window import band_backward
