@@ -842,10 +842,13 @@ __global__ __launch_bounds__(256) void attn_bwd_dkdv_kernel(const AttnArgs a) {
 // the result does not depend on timing, and nobody waits).
 // Bound by reading Q and dO once where there are many rows, by latencies where there are few.
 // The earlier form, whose lanes held 8 d of a row and summed every dot product across 16 lanes, walked 512
-// rows of each head of the group in one block without fetching ahead: us, before / now, dK/dV and sink
-// launch: 2 x 300 rows, 32 / 8 heads, 1 sink 68 / 42; 12053 rows, 8 / 2 heads, window 67, 142 / 73; 2 x 31793
-// rows, 16 / 4 heads, 4 sinks 638 / 601; 550 sequences of 20 tokens, 12 heads, 570 / 276; the sink launch
-// alone on 65536 tokens, 32 / 8 heads, 4 sinks 458 / 316.
+// rows of each head of the group in one block without fetching ahead.  us, before / now (traced), this launch
+// and the dK/dV launch ahead of it: 2 x 300 rows, 32 / 8 heads, window 100, 1 sink 75 / 29; 12053 rows, 8 / 2
+// heads, window 67, 1 sink 142 / 57; 2 x 31793 rows, 16 / 4 heads, window 1000, 4 sinks 1168 / 1102; 550
+// sequences of 20 tokens, 12 heads, 1 sink 565 / 269; this launch alone: 65536 tokens in four sequences, 32 / 8
+// heads, 4 sinks 389 / 304 (3.6 TB/s); packs of one long sequence among 63 of 16 tokens, 4 sinks, window 256:
+// 32000 tokens, 32 = 32 heads (2048 units of one chunk, so that 32 blocks have the long sequence) 1086 / 920,
+// 16000 tokens, 8 / 2 heads 2924 / 206.
 
 // sum over the aligned group of 16 lanes, in every lane of the group
 __device__ __forceinline__ float lane_group_sum16(float x) {
@@ -1029,7 +1032,10 @@ void attn_bwd_sink_kernel(const AttnArgs a) {
   if (n_chunks == 1) return;
   // Count this chunk in; the last one of the unit adds them all up.  The sums are written through to where
   // every XCD reads them and read from there, each by itself: a fence would write back and then drop
-  // the XCD's whole L2, under the feet of the blocks that are at work, for every block (us, this launch,
+  // the XCD's whole L2, under the feet of the blocks that are at work, for every block.  That rests on the
+  // hardware, not on the language, in which relaxed operations order nothing: on gfx950 a store of device
+  // scope is written through, s_waitcnt vmcnt(0) waits until it has arrived there, and the barrier
+  // puts every wave's wait ahead of the count (us, this launch,
   // with a fence per block / so: 51330 tokens in long sequences, 32 / 8 heads, head_dim 64, 191 / 105; 65536
   // tokens, 4 sinks, 390 / 316; 3 x 5000 rows, 32 heads, head_dim 64, 105 / 60; with four times the blocks the
   // fences cost 382 and 670).
@@ -1065,9 +1071,9 @@ void attn_bwd_sink_kernel(const AttnArgs a) {
 // dQ launches of head_dim 128 whose rows see at most this many keys on average, and all of head_dim 64, use
 // blocks of 4 waves, two per compute unit (three at head_dim 64, against which a block of 8 is slower at any
 // length: us, 8 / 4 waves, 32768 rows, 32 / 8 heads, window 4096, 1546 / 1301; 12000 rows, 28 / 4 heads, causal
-// without a window, 1082 / 834; 20000 rows, 8 heads, window 4096, 272 / 219; head_dim 128, 32 / 8 heads: window 256 -22 %, window 1000 -8 %, the rank
-// step with its half-empty previous-chunk block -1.4 %; sequences of 16384 and more rows at
-// window 4096 +1 %; 32 = 32 heads, window 1000: -2 %)
+// without a window, 1082 / 834; 20000 rows, 8 heads, window 4096, 272 / 219; head_dim 128, 32 / 8 heads:
+// window 256 -22 %, window 1000 -8 %, the rank step with its half-empty previous-chunk block -1.4 %;
+// sequences of 16384 and more rows at window 4096 +1 %; 32 = 32 heads, window 1000: -2 %)
 #ifndef RSWA_DQ_SMALL_AVG_KEYS
 #define RSWA_DQ_SMALL_AVG_KEYS 3200
 #endif
@@ -1172,10 +1178,11 @@ __global__ __launch_bounds__(256) void attn_bwd_rest_kernel(const AttnArgs a) {
 // (k order: four keys of the first block, then four of the second); the A operand follows the
 // same order: two transposing reads, one per key block.
 //
-// NW = 8: one block of 8 waves per compute unit (two waves per SIMD).  NW = 4: blocks of 4 waves,
-// two of them per compute unit -- the same two waves per SIMD, but from independent blocks, so
-// that one block's prologue (three dependent round trips to memory) and epilogue run under the
-// other's tiles; the price is that a K / V tile serves half as many rows.
+// NW = 8: one block of 8 waves per compute unit (two waves per SIMD).  NW = 4: blocks of 4 waves, two of
+// them per compute unit at head_dim 128, three at 64 (dq_waves) -- a SIMD's waves are from independent
+// blocks, so that one block's prologue (kernel arguments, a pack's sequence, then the first tiles and the
+// rows' own data at once: two or three round trips to memory) and epilogue run under the others' tiles; the
+// price is that a K / V tile serves half as many rows.
 //
 // STATS: the kernel also makes the row statistics of the backward, which it has to read dO for
 // anyway, and writes them for the dK/dV kernel, launched after it.  Same bits as the statistics
@@ -1890,13 +1897,15 @@ RSWA_INSTANTIATE(_Float16)
 // blocks of 256 keys?  Both forms keep every compute unit busy with one block; what decides is how
 // evenly the launch's blocks fill the chip.  Estimated time of a form = the larger of its longest
 // block and of rounds x average block, a block being steps x (time of a step) + (prologue and
-// epilogue), with the times measured here (us): head_dim 128, 1.2 + 20 wide, 1.5 + 10 WALK4;
-// head_dim 64, 0.77 + 18 and 0.93 + 7.  Measured on both sides of the line (us, wide / WALK4, bf16,
+// epilogue), with times fitted to launches of all kinds (us): head_dim 128, 1.2 + 20 wide, 1.5 + 10 WALK4;
+// head_dim 64, 0.77 + 18 and 0.93 + 7.  (A round of equal blocks on every compute unit, whose clock is
+// lower, measures 1.58 + 15 and 1.77 + 8.5, 0.91 + 9 and 0.98 + 7.4, which choose no better: 0.4 % behind
+// the better form where these are 0.35 %, see below.)  Measured on both sides of the line (us, wide / WALK4, bf16,
 // head_dim 128): 32 / 8 heads, window 1024, 4096 rows 217 / 128, 6000 rows 218 / 190, 8192 rows (256
 // wide blocks, one full round) 229 / 255, 9000 rows 368 / 303, 16384 rows 477 / 523; 32 / 32 heads,
 // window 1000, 2 x 8192 rows 545 / 700; 4096 rows, 32 / 8 heads, causal without a window 623 / 252, without
-// a mask 620 / 454.  Of 258 dense and packed shapes drawn the rule is 0.5 % behind the better form on
-// average.
+// a mask 620 / 454.  Of 178 dense and packed shapes drawn, with grouped heads or with at most a round of wide
+// blocks, the rule is 0.35 % behind the better form on average (more than 3 % on 6 of them, 14 % at most).
 // A pack is judged on its average length L, the only one the host knows, as if of sequences of
 // 1.5 L (what a token sees when lengths vary), the longest as long as the pack or the window, with
 // half a key tile per sequence wasted.  Packs of 16384 tokens, 32 / 8 heads, window 1024, lengths log-uniform: 16-64
@@ -1909,10 +1918,14 @@ bool dkv_walk4(const AttnArgs& a, int head_dim) {
   // As many kv heads as q heads: a walk has no heads to deal, only query tiles, and with clearly more than
   // a round of 256-key blocks the short form loses by its longer fetches (us, wide / short, bf16, head_dim
   // 128: a pack of 3010 tokens, 32 heads, window 2028, 54 / 96; 31427 tokens, 4 heads, 715, 133 / 164;
-  // dense 7428 rows, 12 heads, 64, 58 / 70).  Of 60 shapes drawn with 1 to 4 rounds it was 27 % faster to 7 %
-  // slower up to 1.25 rounds, 8 % faster on average (a pack of 7408 tokens, 8 heads, window 1374, 83 / 62;
-  // 3 x 2018 rows, 12 heads, window 323, 75 / 61), which are left to the estimate, and beyond that 13 %
-  // faster to 32 % slower, 6 % slower on average.
+  // dense 7428 rows, 12 heads, 64, 58 / 70).  Up to 1.25 rounds the estimate decides.  Of 335 such shapes drawn
+  // its choice is 2 % behind the better form on average, wide blocks alone 12 % (a pack of 7408 tokens, 8 heads,
+  // window 1374, 83 / 62; 8061 tokens, 8 heads, causal, 137 / 88); but it misses where a second round is hardly
+  // filled, which a pack's average length does not show: on 43 of them it is 3 % slower than wide blocks or more,
+  // by 41 % at most (18 sequences of 213 tokens, 12 heads, head_dim 64, 21.5 / 29.5; 4 of 1991, 8 heads, window
+  // 174, 39 / 51).  Staying wide where ceil(average / 256) tiles per sequence fit one round cured those and
+  // lost as much elsewhere (2.7 % behind on 260 fresh shapes, 1.8 % without).  Beyond 1.25 rounds WALK4 took 25 %
+  // less to 35 % more, 2 % less on average of 67 shapes.
   const double wide_tiles = pack ? (double)lk1 / kDkvKeysPerBlock + 0.5 : (double)ceil_div(lk1, kDkvKeysPerBlock);
   if (a.group == 1 && wide_tiles * a.heads_kv * a.batch > 1.25 * kComputeUnits) return false;
   const int64_t lq1 = pack ? std::max<int64_t>(1, a.rows_q / a.batch) : a.seqlen_q;

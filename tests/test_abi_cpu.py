@@ -234,7 +234,7 @@ def test_form_of_the_dkdv_blocks_can_be_chosen():
 ])
 def test_without_grouped_heads_short_blocks_stay_below_one_round(tokens, heads, d, window, sequences, keys):
     """With as many kv heads as q heads the 64-key form has only query tiles to share out, and a launch of
-    more than 256 blocks of 256 keys loses by it (these shapes were timed in both forms)."""
+    clearly more than 256 blocks of 256 keys (1.25 rounds) stays with those (shapes timed in both forms)."""
     _ensure_built()
     from ring_swa import _lib
 
@@ -279,7 +279,7 @@ def test_workspace_without_the_key_tile_table_is_accepted():
 ])
 def test_head_dim_64_forward_takes_three_blocks_per_unit_where_two_do_not_hold_them(tokens, heads_q, heads_kv, window,
                                                                                     sequences, blocks):
-    """(These shapes were timed in both builds.)"""
+    """(Shapes timed in both builds; between 512 and 1150 blocks of unlike length either can be the faster.)"""
     _ensure_built()
     from ring_swa import _lib
 
