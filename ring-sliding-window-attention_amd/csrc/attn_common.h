@@ -25,13 +25,15 @@ constexpr float kLog2e = 1.4426950408889634f;
 // the compiler does not know is some 30 dependent instructions, five of them ahead of a block's first
 // load).  The method is Granlund and Montgomery's ("Division by Invariant Integers using Multiplication",
 // 1994): multiplier 2^32 + mul with mul = floor(2^32 (2^shift - d) / d) + 1, shift = ceil(log2 d).
+// (`d` is not read: it keeps the kernel arguments behind where they load best -- without it a forward of
+// 2 x 333 rows, 8 / 2 heads, fp16, takes 9.44 us instead of 9.33.)
 struct FastDiv {
-  uint32_t mul, shift;
+  uint32_t d, mul, shift;
 };
 inline FastDiv fast_div(uint32_t d) {  // d >= 1
   uint32_t s = 0;
   while ((1ull << s) < d) s++;
-  return {(uint32_t)(((1ull << 32) * ((1ull << s) - d)) / d + 1), s};
+  return {d, (uint32_t)(((1ull << 32) * ((1ull << s) - d)) / d + 1), s};
 }
 __device__ __forceinline__ int quotient(int n, const FastDiv& f) {
   return (int)((__umulhi((uint32_t)n, f.mul) + (uint32_t)n) >> f.shift);
