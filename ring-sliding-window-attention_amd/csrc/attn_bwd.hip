@@ -1259,7 +1259,7 @@ void attn_bwd_dq_kernel(const AttnArgs a) {
   const int sink_keys = max(0, min(min(a.n_sink, hi_blk + 1), lo_blk));
   const int n_sink_t = min((sink_keys + C::BN - 1) / C::BN, t_lo);
   const int n_tiles = n_sink_t + n_band;
-  auto tile_of = [&](int it) { return it < n_sink_t ? it : t_lo + (it - n_sink_t); };
+  KeyWalk walk(a, n_sink_t, t_lo, n_band);
 
   const int r0 = i0 + (pair ? wave & ((1 << HSH) - 1) : wave) * 32;
   const bool wave_valid = r0 < len_q;
@@ -1274,8 +1274,8 @@ void attn_bwd_dq_kernel(const AttnArgs a) {
   // (keys in two row ranges: the second range's tensors, at this batch entry and kv head)
   const T* k2_ptr = a.k2 ? (const T*)a.k2 + b * a.k_st[0] + hk * a.k_st[2] : k_ptr;
   const T* v2_ptr = a.v2 ? (const T*)a.v2 + b * a.v_st[0] + hk * a.v_st[2] : v_ptr;
-  auto load_tile = [&](int it, char* kd, char* vd) __attribute__((always_inline)) {
-    const int j = tile_of(it) * C::BN;
+  auto load_tile = [&](int tile, char* kd, char* vd) __attribute__((always_inline)) {
+    const int j = tile * C::BN;
     const KeySeg<T> gk = key_seg(k_ptr, k2_ptr, a.seg, j, len_k);
     const KeySeg<T> gv = key_seg(v_ptr, v2_ptr, a.seg, j, len_k);
     k_dma.load(tile_src<C::BN, FAR>(gk.base, gk.row0, gk.rows, k_row_bytes, C::ROWB), kd);
@@ -1287,7 +1287,7 @@ void attn_bwd_dq_kernel(const AttnArgs a) {
   // memory, 8 us of a block's start (of 53 at window 1000, of 18 in a pack of short sequences), now 7.
   // us, before / after: a pack of 16384 tokens in sequences of 16 to 1024 189 / 183; rows 8192 with the
   // statistics, window 4096, 664 / 655; 4001 rows, window 1024, 93.7 / 93.1.
-  if (n_tiles > 0) load_tile(0, k_s0, v_s0);
+  if (n_tiles > 0) load_tile(walk.tile, k_s0, v_s0);
 
   // Q / dO fragments (B operands) and the (negated) statistics of the lane's two query rows.  The
   // dP^T accumulator chains start from -delta: the MFMAs then deliver dP - delta, and the vector ALU
@@ -1377,9 +1377,10 @@ void attn_bwd_dq_kernel(const AttnArgs a) {
 
   auto step = [&](int it, const char* kc, const char* vc, char* kn,
                   char* vn) __attribute__((always_inline)) {
-    const int j0 = tile_of(it) * C::BN;
+    const int j0 = walk.tile * C::BN;
     const int j1 = j0 + C::BN - 1;
-    if (it + 1 < n_tiles) load_tile(it + 1, kn, vn);
+    walk.next();
+    if (it + 1 < n_tiles) load_tile(walk.tile, kn, vn);
     const bool needed =
         wave_valid && j0 <= wb_last.hi && (j1 >= wb_first.lo || j0 < a.n_sink);
     if (needed) {
@@ -1984,6 +1985,7 @@ int launch_bwd(AttnArgs& a, hipStream_t stream, int phases) {
     }
     if (a.n_work == 0) return (int)RSWA_OK;
     set_divisors(a, units_q / a.heads_kv);
+    a.walk_mask = walk_mask(a, bm, DqCfg<D>::BN);
     clear_launch_error();
     const dim3 grid(padded_grid(a.n_work)), block(small ? 256 : 512);
     if constexpr (!STATS) {

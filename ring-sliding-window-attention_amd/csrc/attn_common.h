@@ -14,6 +14,7 @@
 
 #include "rswa_common.h"
 
+#include <algorithm>
 #include <type_traits>
 #include <utility>
 
@@ -80,6 +81,7 @@ struct AttnArgs {
   // tiles (forward, dQ) or key tiles (dK/dV) so that the tiles with the most visible
   // pairs start first and the short ones fill the tail of the launch.
   int32_t rev_q, rev_k;
+  int32_t walk_mask;  // see walk_start
   // backward with sink keys and a bounded window: workspace of the sink kernel -- fp32 sums
   // [sequence x kv head][chunk of rows][sink][dK, dV][D] and one arrival counter per
   // (sequence, kv head); null when that kernel does not run
@@ -147,6 +149,54 @@ __device__ __forceinline__ RowBounds row_bounds(const AttnArgs& a, int i, int le
   r.lo = (a.wl >= 0) ? max(0, i + shift - a.wl) : 0;
   if (i >= len_q) r.hi = -1;  // rows past the end see nothing
   return r;
+}
+
+// Offset, in a block's walk over the `n` key tiles from tile t_lo on, of the tile it starts with (the walk
+// wraps around behind the last): the first one whose number is a multiple of walk_mask + 1, the largest power
+// of two among the tiles that such blocks visit.  Blocks that start together are then on few tiles at a time
+// instead of one tile each: with as many kv heads as q heads the 64 blocks that an XCD runs at once cover
+// 8192 rows, whose K and V are as large as its L2, and every block of a window found its tiles gone again.
+// 2 x 8192 rows, 32 = 32 heads, head_dim 128, window 1000, walks from the first tile / from here: fetched beyond
+// L2 in the forward 1.89 / 0.43 GB, in dQ 1.98 / 0.72 GB; a training call 1299 / 1243 us.  Where several q heads
+// share a kv head the tiles of a window stay in L2 either way (32 / 8 heads, window 4096, 32768 rows: 0.78 /
+// 0.58 GB, 1809 / 1796 us).  A power of two, not the walk's own length (the same traffic): a block's first load
+// waits for this.  And of the mask, not of n: tiles that none of a row's keys lie in change nothing, so a
+// row's sums have the same order however many rows its block has.
+__device__ __forceinline__ int walk_start(const AttnArgs& a, int t_lo, int n) {
+  const int at = -t_lo & a.walk_mask;
+  return at < n ? at : 0;
+}
+// A walk's tiles in order: n_sink tiles from tile 0 on, then `n_band` from tile t_lo on, the first of these
+// being walk_start's; a cursor that is advanced beyond the last is on one of them still.  (A comparison and
+// three selects a tile; computing a tile from its place in the walk, three times per tile in the forward, cost
+// the launches that gain nothing from the order 1 % (24 drawn calls with equal heads: forward 0.4 % slower than
+// with walks from the first tile that way, 1.8 % faster with the cursor; dQ 0.1 and 2.2 % faster).)
+struct KeyWalk {
+  int tile;        // where the cursor is
+  int stop, jump;  // reaching tile `stop` it goes to tile `jump` ...
+  int end, back;   // ... after which these take their place
+  __device__ __forceinline__ KeyWalk(const AttnArgs& a, int n_sink, int t_lo, int n_band) {
+    const int first = n_band > 0 ? t_lo + walk_start(a, t_lo, n_band) : 0;
+    end = n_band > 0 ? t_lo + n_band : n_sink;
+    back = n_band > 0 ? t_lo : 0;
+    tile = n_sink > 0 ? 0 : first;
+    stop = n_sink > 0 ? n_sink : end;
+    jump = n_sink > 0 ? first : back;
+  }
+  __device__ __forceinline__ void next() {
+    tile++;
+    const bool at = tile == stop;
+    tile = at ? jump : tile;
+    stop = at ? end : stop;
+    jump = at ? back : jump;
+  }
+};
+inline int walk_mask(const AttnArgs& a, int block_rows, int tile_keys) {
+  if (a.wl < 0 || a.wr < 0) return 0;
+  const int64_t tiles = std::min<int64_t>(((int64_t)a.wl + a.wr + block_rows) / tile_keys, 1 << 20);
+  int mask = 0;
+  while (2 * mask + 2 <= tiles) mask = 2 * mask + 1;
+  return mask;
 }
 
 // Packed mode: which sequence, and which of its tiles of `tile` = 2^tile_log2 rows, does

@@ -113,7 +113,9 @@ void attn_fwd_kernel(const AttnArgs a) {
   const int sink_keys = max(0, min(min(a.n_sink, hi_blk + 1), lo_blk));
   const int n_sink_t = min((sink_keys + C::BN - 1) / C::BN, t_lo);
   const int n_tiles = n_sink_t + n_band;
-  auto tile_of = [&](int it) { return it < n_sink_t ? it : t_lo + (it - n_sink_t); };
+  KeyWalk walk(a, n_sink_t, t_lo, n_band);
+  const int t_first = walk.tile;
+  walk.next();
 
   // ---- this wave's rows ----------------------------------------------------
   const int r0 = i0 + (pair ? wave & 1 : wave) * 32;
@@ -131,12 +133,12 @@ void attn_fwd_kernel(const AttnArgs a) {
   // (keys in two row ranges: the second range's tensors, at this batch entry and kv head)
   const T* k2_ptr = a.k2 ? (const T*)a.k2 + b * a.k_st[0] + hk * a.k_st[2] : k_ptr;
   const T* v2_ptr = a.v2 ? (const T*)a.v2 + b * a.v_st[0] + hk * a.v_st[2] : v_ptr;
-  auto load_k = [&](int it, char* dst) __attribute__((always_inline)) {
-    const KeySeg<T> g = key_seg(k_ptr, k2_ptr, a.seg, tile_of(it) * C::BN, len_k);
+  auto load_k = [&](int tile, char* dst) __attribute__((always_inline)) {
+    const KeySeg<T> g = key_seg(k_ptr, k2_ptr, a.seg, tile * C::BN, len_k);
     k_dma.load(tile_src<C::BN, FAR>(g.base, g.row0, g.rows, k_row_bytes, C::ROWB), dst);
   };
-  auto load_v = [&](int it, char* dst) __attribute__((always_inline)) {
-    const KeySeg<T> g = key_seg(v_ptr, v2_ptr, a.seg, tile_of(it) * C::BN, len_k);
+  auto load_v = [&](int tile, char* dst) __attribute__((always_inline)) {
+    const KeySeg<T> g = key_seg(v_ptr, v2_ptr, a.seg, tile * C::BN, len_k);
     v_dma.load(tile_src<C::BN, FAR>(g.base, g.row0, g.rows, v_row_bytes, C::ROWB), dst);
   };
 
@@ -146,7 +148,7 @@ void attn_fwd_kernel(const AttnArgs a) {
   // epilogue without branches or a 64-bit product per row: us, before / after, 4001 rows, window 1024,
   // 32 / 8 heads 75.4 / 73.0; a pack of 16384 tokens in sequences of 16 to 1024 149 / 144; 2 x 8192 rows,
   // 32 heads, window 1000 358 / 351; 4 x 2000 rows, 28 / 4 heads, head_dim 64, fp16 79.0 / 76.1.)
-  if (n_tiles > 0) load_k(0, k_s0);
+  if (n_tiles > 0) load_k(t_first, k_s0);
   // Q fragments (B operand of K Q^T): lane = query column, 8 consecutive d per k-step.  (Rows past the
   // end read the last row's values: their columns are masked in every tile and never stored.)
   const T* q_row = q_ptr + (int64_t)min(iq, len_q - 1) * a.q_st[1] + g * 8;
@@ -154,8 +156,8 @@ void attn_fwd_kernel(const AttnArgs a) {
 #pragma unroll
   for (int ks = 0; ks < C::KSTEPS; ks++) qf[ks] = *(const V8*)(q_row + ks * 16);
 
-  if (n_tiles > 0) load_v(0, v_s0);
-  if (n_tiles > 1) load_k(1, k_s1);
+  if (n_tiles > 0) load_v(t_first, v_s0);
+  if (n_tiles > 1) load_k(walk.tile, k_s1);
 
   f32x16 o_acc[C::DBLK];
 #pragma unroll
@@ -199,8 +201,8 @@ void attn_fwd_kernel(const AttnArgs a) {
   // instructions more than another, half as many again as the softmax.  us, before / after, with the wave's
   // bounds as scalars: 4001 rows, window 1024, 32 / 8 heads 68.9 / 65.9; a pack of 16384 tokens in
   // sequences of 16 to 1024 140 / 132; 4 x 2000 rows, 28 / 4 heads, head_dim 64, 4 sinks 74.0 / 68.9.)
-  auto mask = [&](int it, f32x16(&sacc)[2]) __attribute__((always_inline)) {
-    const int j0 = tile_of(it) * C::BN;
+  auto mask = [&](int tile, f32x16(&sacc)[2]) __attribute__((always_inline)) {
+    const int j0 = tile * C::BN;
     const int j1 = j0 + C::BN - 1;
     if (!(wave_rows_full && j1 <= wb_first.hi)) {
       const int hi_rel = rb.hi - j0 - 4 * g;
@@ -298,9 +300,11 @@ void attn_fwd_kernel(const AttnArgs a) {
   // V(t), loaded during the previous matrix section, and releases the buffers of K(t) and
   // V(t-1), last read before it: the loads of K(t+2) and V(t+1) into them follow it.
   f32x16 s_cur[2];
+  int t_cur = t_first, t_next = walk.tile;  // tiles t and t + 1; the cursor: t + 2
+  walk.next();
   auto prefetch = [&](int it, char* kfree, char* vn) __attribute__((always_inline)) {
-    if (it + 2 < n_tiles) load_k(it + 2, kfree);
-    if (it + 1 < n_tiles) load_v(it + 1, vn);
+    if (it + 2 < n_tiles) load_k(walk.tile, kfree);
+    if (it + 1 < n_tiles) load_v(t_next, vn);
   };
   // A tile the block visits may hold no key that this wave's 32 rows can see (the block's
   // key range is as wide as the window plus all its rows): the wave then skips the tile's
@@ -308,9 +312,9 @@ void attn_fwd_kernel(const AttnArgs a) {
   // window 256 and 128 rows per block a wave needs 5 of the block's 7 tiles.
   // (SKIP is chosen by the host for short windows only: with a long window the test costs
   // more than the rare skipped tile saves.)
-  auto wave_needs = [&](int it) __attribute__((always_inline)) -> bool {
+  auto wave_needs = [&](int it, int tile) __attribute__((always_inline)) -> bool {
     if constexpr (!SKIP) return it < n_tiles;
-    const int j0 = tile_of(it) * C::BN;
+    const int j0 = tile * C::BN;
     return it < n_tiles && r0 < len_q && j0 <= wb_last.hi &&
            (j0 + C::BN - 1 >= wb_first.lo || j0 < a.n_sink);
   };
@@ -318,11 +322,11 @@ void attn_fwd_kernel(const AttnArgs a) {
                   char* vn) __attribute__((always_inline)) {
     // without SKIP both are compile-time true: one path, and after the last tile S(t+1) is
     // computed from stale LDS contents and never used
-    const bool need_cur = SKIP ? wave_needs(it) : true;
-    const bool need_next = SKIP ? wave_needs(it + 1) : true;
+    const bool need_cur = SKIP ? wave_needs(it, t_cur) : true;
+    const bool need_next = SKIP ? wave_needs(it + 1, t_next) : true;
     V8 pb[4];
     if (need_cur) {
-      mask(it, s_cur);
+      mask(t_cur, s_cur);
       const float alpha = softmax(s_cur, pb);
       rescale(alpha);
     }
@@ -333,10 +337,9 @@ void attn_fwd_kernel(const AttnArgs a) {
       // matrix section as ONE basic block, LDS reads scheduled four fragments ahead of their
       // MFMA.  The tile loads ride between the MFMAs, one every fourth: issued in a row they
       // hold the wave for about 50 cycles apiece before its first MFMA.  No branch may split
-      // the block, so past the last tile the last one is fetched again, into a buffer nobody
-      // reads.
-      load_k(min(it + 2, n_tiles - 1), kfree);
-      load_v(min(it + 1, n_tiles - 1), vn);
+      // the block, so past the last tile some are fetched again, into buffers nobody reads.
+      load_k(walk.tile, kfree);
+      load_v(t_next, vn);
       pv_acc(vc, pb);
       qk(kn, s_cur);
       __builtin_amdgcn_sched_group_barrier(0x100, 8, 0);
@@ -352,10 +355,13 @@ void attn_fwd_kernel(const AttnArgs a) {
     } else if (need_next) {
       qk(kn, s_cur);
     }
+    t_cur = t_next;
+    t_next = walk.tile;
+    walk.next();
   };
 
   __syncthreads();
-  if (wave_needs(0)) qk(k_s0, s_cur);
+  if (wave_needs(0, t_first)) qk(k_s0, s_cur);
   for (int it = 0; it < n_tiles; it += 2) {
     iter(it, k_s1, k_s0, v_s0, v_s1);
     if (it + 1 < n_tiles) iter(it + 1, k_s0, k_s1, v_s1, v_s0);
@@ -518,6 +524,7 @@ int launch_fwd(AttnArgs& a, hipStream_t stream) {
   }
   if (a.n_work == 0) return RSWA_OK;
   set_divisors(a, units / a.heads_kv);
+  a.walk_mask = walk_mask(a, bm, C::BN);
   // keys a row sees at most; the per-wave tile skip pays when the rows of a block beyond one
   // wave's 32 add a tenth or more to that span
   const int64_t span = (a.wl < 0 || a.wr < 0) ? (int64_t)1 << 40 : (int64_t)a.wl + a.wr + 1;
