@@ -325,15 +325,19 @@ __global__ __launch_bounds__(256) void attn_bwd_dkdv_kernel(const AttnArgs a) {
   const T* q_base = (const T*)a.q + b * a.q_st[0] + s.q_row0 * a.q_st[1];
   const T* do_base = (const T*)a.dout + b * a.do_st[0] + s.q_row0 * a.do_st[1];
   // statistics: one load covers both workspace arrays (lse2, then delta `stat_elems` further
-  // on) through a resource based at the tile's first row; rows past the sequence end read a
-  // neighbour's finite values, which the row mask / zero Q, dO rows void
+  // on) through one resource, the tile's first row in the scalar offset; rows past the sequence end read
+  // a neighbour's finite values, which the row mask / zero Q, dO rows void
   // (element counts below 2^30: the host refuses larger statistics arrays)
   const int stat_elems = (int)(a.delta - a.lse2);  // elements between the two arrays
   const int stat_end = stat_elems + a.heads_q * (int)a.rows_q;  // end of delta
   const int q_row_bytes = (int)(a.q_st[1] * 2), do_row_bytes = (int)(a.do_st[1] * 2);
   // Cursor over the (q head of the group, query tile) pairs, advanced incrementally so
   // that a step costs a handful of scalar instructions: the tile's first row, the head's
-  // Q / dO base pointers and the offset of its statistics.
+  // Q / dO base pointers and the offset of its statistics.  (A lone wave per SIMD pays for each: without a
+  // resource of the statistics for every tile (ten, in the wave that the others wait for), a tile count beside
+  // the row, a test for the last tile and pairs of comparisons where one will do, 66 scalar instructions a
+  // step became 48; dK/dV of 65536 tokens, window 4092, 6664 / 6527 us, of 2 x 8192 rows, 32 heads, window
+  // 1000, 620 / 607, the rank step with 14336 keys 1194 / 1162.)
   struct Cursor {
     int qt, i0;
     const T *q_head, *do_head;
@@ -347,17 +351,21 @@ __global__ __launch_bounds__(256) void attn_bwd_dkdv_kernel(const AttnArgs a) {
   // rows, and walking them in step lets one L2 fill serve all of them.
   const int qt_start = n_qt > 0 ? (n_qt - qt_lo % n_qt) % n_qt : 0;
   Cursor nxt;  // the tile that the load parts fetch
-  nxt.qt = WALK4 ? w_tile : qt_start;  // WALK4: position in the walk, counted from qt_start
+  nxt.qt = w_tile;  // WALK4: position in the walk, counted from qt_start
   auto row_of = [&](int pos) __attribute__((always_inline)) {
     const int at = qt_start + pos;
     return i_first + (at >= n_qt ? at - n_qt : at) * C::BM;
   };
   nxt.i0 = row_of(w_tile);
-  int nxt_left = n_qt;  // tiles left in the walk of nxt's head, nxt included
+  // (not WALK4: a head's walk ends behind the last tile at i_end and is through when it is back at i_start)
+  const int i_end = i_first + n_qt * C::BM, i_start = nxt.i0;
+  int heads_left = a.group - 1;  // heads of the walk after nxt's
   const int h_first = hk * a.group + (WALK4 ? wave & ((1 << hw_log2) - 1) : 0);
   nxt.q_head = q_base + (int64_t)h_first * a.q_st[2];
   nxt.do_head = do_base + (int64_t)h_first * a.do_st[2];
   nxt.stat_row = (int)(h_first * a.rows_q + ws_row0);
+  const __amdgpu_buffer_rsrc_t st_rsrc =
+      __builtin_amdgcn_make_buffer_rsrc((void*)a.lse2, 0, (int)((uint32_t)stat_end * 4u), 0x00020000);
   // dS hand-off: unit of (q head h, row tile qt of the sequence, this block's keys, this wave) at
   //   ds + (((h ds_slots + slot0 + qt) ds_nkb + kt % ds_nkb) 4 + wave) 4 KiB
   // -- per step one row of ds_nkb blocks further, per head ds_slots rows further.  The units
@@ -391,16 +399,14 @@ __global__ __launch_bounds__(256) void attn_bwd_dkdv_kernel(const AttnArgs a) {
     if constexpr (part == 0) {
       if (WALK4 || wave == 0) {  // lanes 0-31: lse2 of the 32 rows, lanes 32-63: their delta
         const int first = nxt.stat_row + nxt.i0;
-        const __amdgpu_buffer_rsrc_t st_rsrc = __builtin_amdgcn_make_buffer_rsrc(
-            (void*)(a.lse2 + first), 0, min(stat_end - first, stat_elems + C::BM) * 4, 0x00020000);
         // the per-lane offset is recomputed here (opaque to the optimiser): kept in a
         // register across the walk it could be spilled, and its reload would wait for
         // every tile load issued before it
         if constexpr (WALK4) {
-          lds_load_asm<4>(rsrc_words(a.lse2 + first, min(stat_end - first, stat_elems + C::BM) * 4), st_voff,
-                          0, (uint32_t)(uintptr_t)(lds_void_t*)std_);
+          lds_load_asm<4>(rsrc_words(a.lse2, (int)((uint32_t)stat_end * 4u)), st_voff, first * 4,
+                          (uint32_t)(uintptr_t)(lds_void_t*)std_);
         } else {
-          __builtin_amdgcn_raw_ptr_buffer_load_lds(st_rsrc, (lds_void_t*)std_, 4, st_voff, 0, 0, 0);
+          __builtin_amdgcn_raw_ptr_buffer_load_lds(st_rsrc, (lds_void_t*)std_, 4, st_voff, first * 4, 0, 0);
         }
       }
     } else if constexpr (WALK4) {
@@ -419,6 +425,8 @@ __global__ __launch_bounds__(256) void attn_bwd_dkdv_kernel(const AttnArgs a) {
       do_dma.load_one(t.rsrc, t.soff, dod, part - 1 - NQD);
     }
   };
+  // may the cursor be advanced beyond the last tile?  (with the dS hand-off the kernel spills without the test)
+  constexpr bool FREE_RUN = !WALK4 && !HAND;
   auto advance = [&]() __attribute__((always_inline)) {
     if constexpr (WALK4) {
       nxt.qt += 1 << tw_log2;
@@ -433,24 +441,19 @@ __global__ __launch_bounds__(256) void attn_bwd_dkdv_kernel(const AttnArgs a) {
       if constexpr (HAND) nxt.ds = ds_head_off + ((nxt.i0 - i_first) >> 5) * ds_row_bytes;
       return;
     }
-    nxt.qt++;
+    // (past the last head's walk the cursor stays on that head: its tiles are fetched again, into buffers
+    // nobody reads)
     nxt.i0 += C::BM;
-    if constexpr (HAND) nxt.ds += ds_row_bytes;
-    if (nxt.qt == n_qt) {
-      nxt.qt = 0;
-      nxt.i0 = i_first;
-      if constexpr (HAND) nxt.ds = ds_head_off;
-    }
-    if (--nxt_left == 0) {
-      nxt_left = n_qt;
-      nxt.qt = qt_start;
-      nxt.i0 = i_first + qt_start * C::BM;
+    if constexpr (HAND) nxt.ds = nxt.i0 == i_end ? ds_head_off : nxt.ds + ds_row_bytes;
+    nxt.i0 = nxt.i0 == i_end ? i_first : nxt.i0;
+    if (nxt.i0 == i_start && heads_left > 0) {
+      heads_left--;
       nxt.q_head += a.q_st[2];
       nxt.do_head += a.do_st[2];
       nxt.stat_row += (int)a.rows_q;
       if constexpr (HAND) {
         ds_head_off += ds_head_bytes;
-        nxt.ds = ds_head_off + qt_start * ds_row_bytes;
+        nxt.ds += ds_head_bytes;
       }
     }
   };
@@ -462,7 +465,7 @@ __global__ __launch_bounds__(256) void attn_bwd_dkdv_kernel(const AttnArgs a) {
   int cur_i0 = nxt.i0;  // first row of the tile being computed
   if (n_iter > 0) {
     static_for<NPART>([&](auto pc) __attribute__((always_inline)) { load_part(pc, qb0, dob0, stb0); });
-    if (n_iter > 1) advance();
+    if (FREE_RUN || n_iter > 1) advance();
   }
   if constexpr (WALK4) {
     wait_vmem_but<0>();
@@ -514,12 +517,13 @@ __global__ __launch_bounds__(256) void attn_bwd_dkdv_kernel(const AttnArgs a) {
   //   full:   i0 + 31 < len_q, jw1 < len_k, jw1 <= i0 + shift + wr, jw0 >= i0 + 31 + shift - wl
   // are intervals of i0 whose ends depend on the wave only: a step tests two of them.
   constexpr int kInf = 1 << 30;
-  int need_lo = (a.wr < 0) ? -kInf : jw0 - shift - a.wr - 31;
+  const int need_lo = (a.wr < 0) ? -kInf : jw0 - shift - a.wr - 31;
   int need_hi = min(len_q - 1, (a.wl < 0) ? kInf : jw1 - shift + a.wl);
   if (jw0 >= len_k || (a.wr >= 0 && len_q - 1 < jw0 - shift - a.wr)) need_hi = -kInf - 1;
-  int full_lo = (a.wr < 0) ? -kInf : jw1 - shift - a.wr;
+  const int full_lo = (a.wr < 0) ? -kInf : jw1 - shift - a.wr;
   int full_hi = min(len_q - 32, (a.wl < 0) ? kInf : jw0 - 31 - shift + a.wl);
   if (jw1 >= len_k) full_hi = -kInf - 1;
+  const unsigned need_n = (unsigned)max(need_hi - need_lo + 1, 0), full_n = (unsigned)max(full_hi - full_lo + 1, 0);
 
   // one query tile: prefetch the next one into (qn, don, stn), compute on (qc, doc, stc)
   auto step = [&](int it, const char* qc, const char* doc, const float* stc, char* qn, char* don,
@@ -533,10 +537,10 @@ __global__ __launch_bounds__(256) void attn_bwd_dkdv_kernel(const AttnArgs a) {
     const float* delta_lds = stc + C::BM;
     // (opaque: the XOR forms of the lane offsets are made where they are used, not kept)
     if constexpr (WALK4) asm volatile("" : "+v"(dma_chunk));
-    const bool needed = WALK4 || (i0 >= need_lo && i0 <= need_hi);
+    const bool needed = WALK4 || (HAND ? i0 >= need_lo && i0 <= need_hi : (unsigned)(i0 - need_lo) < need_n);
     if (!needed && has_next) {
       static_for<NPART>([&](auto pc) __attribute__((always_inline)) { load_part(pc, qn, don, stn); });
-      if (it + 2 < n_iter) advance();
+      if (FREE_RUN || it + 2 < n_iter) advance();
     }
     if constexpr (CARRY) {
       if (!needed) {
@@ -547,7 +551,7 @@ __global__ __launch_bounds__(256) void attn_bwd_dkdv_kernel(const AttnArgs a) {
       }
     }
     if (needed) {
-      const bool full = i0 >= full_lo && i0 <= full_hi;
+      const bool full = HAND ? i0 >= full_lo && i0 <= full_hi : (unsigned)(i0 - full_lo) < full_n;
       // The four GEMMs of the (32 queries x 64 keys) sub-tile -- S = Q K^T, dP = dO V^T,
       // dV^T += dO^T P, dK^T += Q^T dS; KB KS MFMAs each, rows = queries, lane = key column
       // -- their LDS reads and the vector work are written out in issue order, one group
@@ -707,7 +711,7 @@ __global__ __launch_bounds__(256) void attn_bwd_dkdv_kernel(const AttnArgs a) {
         }
         fence();
       });
-      if (it + 2 < n_iter) advance();
+      if (FREE_RUN || it + 2 < n_iter) advance();
     }
     if constexpr (WALK4) wait_vmem_but<0>();  // the wave's own tiles: nobody else reads them
     else __syncthreads();
@@ -1270,16 +1274,13 @@ void attn_bwd_dq_kernel(const AttnArgs a) {
   TileDma<D, C::BN, NW * 64, true> k_dma, v_dma;
   k_dma.init(a.k_st[1], tid);
   v_dma.init(a.v_st[1], tid);
-  const int k_row_bytes = (int)(a.k_st[1] * 2), v_row_bytes = (int)(a.v_st[1] * 2);
   // (keys in two row ranges: the second range's tensors, at this batch entry and kv head)
   const T* k2_ptr = a.k2 ? (const T*)a.k2 + b * a.k_st[0] + hk * a.k_st[2] : k_ptr;
   const T* v2_ptr = a.v2 ? (const T*)a.v2 + b * a.v_st[0] + hk * a.v_st[2] : v_ptr;
+  const KeyRows<T, C::ROWB, FAR> k_rows(k_ptr, k2_ptr, a.seg, len_k, a.k_st[1]), v_rows(v_ptr, v2_ptr, a.seg, len_k, a.v_st[1]);
   auto load_tile = [&](int tile, char* kd, char* vd) __attribute__((always_inline)) {
-    const int j = tile * C::BN;
-    const KeySeg<T> gk = key_seg(k_ptr, k2_ptr, a.seg, j, len_k);
-    const KeySeg<T> gv = key_seg(v_ptr, v2_ptr, a.seg, j, len_k);
-    k_dma.load(tile_src<C::BN, FAR>(gk.base, gk.row0, gk.rows, k_row_bytes, C::ROWB), kd);
-    v_dma.load(tile_src<C::BN, FAR>(gv.base, gv.row0, gv.rows, v_row_bytes, C::ROWB), vd);
+    k_dma.load(k_rows.template tile<C::BN>(tile * C::BN), kd);
+    v_dma.load(v_rows.template tile<C::BN>(tile * C::BN), vd);
   };
 
   // The first tiles are asked for ahead of the rows' own data, and of that everything before the first
@@ -1658,14 +1659,13 @@ __global__ __launch_bounds__(256) void attn_bwd_dq_ds_kernel(const AttnArgs a) {
 
   TileDma<D, C::BN, 256> k_dma;
   k_dma.init(a.k_st[1], tid);
-  const int k_row_bytes = (int)(a.k_st[1] * 2);
+  const KeyRows<T, C::ROWB, false> k_rows(k_ptr, k2_ptr, a.seg, len_k, a.k_st[1]);
 
   // load cursor: the stage fetched next
   int ld_j = t_lo * C::BN;
   int ld_kb = (ld_j >> 8) % a.ds_nkb;
   auto load_stage = [&](char* kd, char* dsd) __attribute__((always_inline)) {
-    const KeySeg<T> gk = key_seg(k_ptr, k2_ptr, a.seg, ld_j, len_k);
-    k_dma.load(tile_src<C::BN, false>(gk.base, gk.row0, gk.rows, k_row_bytes, C::ROWB), kd);
+    k_dma.load(k_rows.template tile<C::BN>(ld_j), kd);
     const int soff = ld_kb * kDsBlockBytes + ((ld_j >> 6) & 3) * kDsUnitBytes;
     char* dst = dsd + wave * C::WAVE_LDS;
 #pragma unroll

@@ -459,19 +459,34 @@ __device__ __forceinline__ TileSrc tile_src(const void* base, int row0, int rows
   }
 }
 
-// Key rows in two ranges (AttnArgs::seg): where the tile of key rows starting at `row0` (never
-// straddling the boundary: seg is a multiple of every tile size) is fetched from.
-template <typename T>
-struct KeySeg {
-  const T* base;
-  int row0, rows;  // first row of the tile inside its range, rows of the range
+// Key rows in two ranges (AttnArgs::seg): where the tile of key rows starting at `row0` (never straddling the
+// boundary: seg is a multiple of every tile size) is fetched from.  What does not depend on the tile is made
+// once, 12 scalar instructions a tile less (29 calls: dQ 0.4 % faster, the forward 0.2 %).
+template <typename T, int ROW_BYTES, bool FAR>
+struct KeyRows {
+  const T *first, *second;
+  int seg, rows1, rows2;  // boundary; rows of the ranges
+  int bytes1, bytes2;     // that they span
+  int stride_bytes;
+  __device__ __forceinline__ KeyRows(const T* p1, const T* p2, int seg_, int len_k, int64_t stride_elems)
+      : first(p1), second(p2), seg(seg_), rows1(min(len_k, seg_)), rows2(len_k - seg_),
+        stride_bytes((int)(stride_elems * 2)) {
+    bytes1 = rows1 > 0 ? (rows1 - 1) * stride_bytes + ROW_BYTES : 0;
+    bytes2 = rows2 > 0 ? (rows2 - 1) * stride_bytes + ROW_BYTES : 0;
+  }
+  template <int ROWS>
+  __device__ __forceinline__ TileSrc tile(int row0) const {
+    const bool s2 = row0 >= seg;
+    const T* base = s2 ? second : first;
+    const int row = row0 - (s2 ? seg : 0);
+    if constexpr (FAR) {
+      return tile_src<ROWS, true>(base, row, s2 ? rows2 : rows1, stride_bytes, ROW_BYTES);
+    } else {
+      return {__builtin_amdgcn_make_buffer_rsrc((void*)base, 0, s2 ? bytes2 : bytes1, 0x00020000),
+              row * stride_bytes};
+    }
+  }
 };
-template <typename T>
-__device__ __forceinline__ KeySeg<T> key_seg(const T* first, const T* second, int seg, int row0,
-                                             int len_k) {
-  const bool s2 = row0 >= seg;
-  return {s2 ? second : first, s2 ? row0 - seg : row0, s2 ? len_k - seg : min(len_k, seg)};
-}
 
 // Cooperative copy of a [ROWS x D] tile into a swizzled LDS tile with buffer loads that
 // land directly in LDS (buffer_load_dwordx4 ... lds: lane L of a wave writes

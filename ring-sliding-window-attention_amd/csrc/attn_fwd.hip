@@ -129,17 +129,15 @@ void attn_fwd_kernel(const AttnArgs a) {
   TileDma<D, C::BN, C::THREADS> k_dma, v_dma;
   k_dma.init(a.k_st[1], tid);
   v_dma.init(a.v_st[1], tid);
-  const int k_row_bytes = (int)(a.k_st[1] * 2), v_row_bytes = (int)(a.v_st[1] * 2);
   // (keys in two row ranges: the second range's tensors, at this batch entry and kv head)
   const T* k2_ptr = a.k2 ? (const T*)a.k2 + b * a.k_st[0] + hk * a.k_st[2] : k_ptr;
   const T* v2_ptr = a.v2 ? (const T*)a.v2 + b * a.v_st[0] + hk * a.v_st[2] : v_ptr;
+  const KeyRows<T, C::ROWB, FAR> k_rows(k_ptr, k2_ptr, a.seg, len_k, a.k_st[1]), v_rows(v_ptr, v2_ptr, a.seg, len_k, a.v_st[1]);
   auto load_k = [&](int tile, char* dst) __attribute__((always_inline)) {
-    const KeySeg<T> g = key_seg(k_ptr, k2_ptr, a.seg, tile * C::BN, len_k);
-    k_dma.load(tile_src<C::BN, FAR>(g.base, g.row0, g.rows, k_row_bytes, C::ROWB), dst);
+    k_dma.load(k_rows.template tile<C::BN>(tile * C::BN), dst);
   };
   auto load_v = [&](int tile, char* dst) __attribute__((always_inline)) {
-    const KeySeg<T> g = key_seg(v_ptr, v2_ptr, a.seg, tile * C::BN, len_k);
-    v_dma.load(tile_src<C::BN, FAR>(g.base, g.row0, g.rows, v_row_bytes, C::ROWB), dst);
+    v_dma.load(v_rows.template tile<C::BN>(tile * C::BN), dst);
   };
 
   // The first tiles and the rows' own data are asked for before anything else is computed: K(0) and Q
