@@ -186,8 +186,17 @@ def close_sgpr_writes(listing: List[str]) -> List[str]:
     return bad
 
 
+def close_m0_writes(listing: List[str]) -> List[str]:
+    """Loads into LDS with no instruction between a scalar write of m0 and them (one wait state is needed; the
+    hand-written loads that carry an offset take m0 as an earlier one left it, and have no ``s_nop`` of their own)."""
+    code = [line.split("//")[0].split(";")[0].strip() for line in listing]
+    code = [x for x in code if x and not x.endswith(">:")]
+    return [f"{w}  ...  {x}" for w, x in zip(code, code[1:])
+            if x.startswith("buffer_load") and x.endswith(" lds") and re.match(r"s_\w+ m0,", w)]
+
+
 def _check_lds_loads(obj: str) -> None:
-    """No load into LDS may follow a vector instruction's write of its scalar registers too closely."""
+    """No load into LDS may follow a write of its scalar registers too closely."""
     llvm = os.path.join(os.path.dirname(os.path.realpath(_hipcc())), "..", "llvm", "bin")
     with tempfile.TemporaryDirectory() as tmp:
         fat = os.path.join(tmp, "fat")
@@ -200,7 +209,7 @@ def _check_lds_loads(obj: str) -> None:
             text = subprocess.run([os.path.join(llvm, "llvm-objdump"), "-d", "--no-show-raw-insn",
                                    "--symbolize-operands", path], check=True, capture_output=True, text=True).stdout
             for name, body in re.findall(r"^[0-9a-f]+ <(_Z\w+)>:\n(.*?)(?=^[0-9a-f]+ <_Z|\Z)", text, re.M | re.S):
-                bad = close_sgpr_writes(body.splitlines())
+                bad = close_sgpr_writes(body.splitlines()) + close_m0_writes(body.splitlines())
                 if bad:
                     raise RuntimeError(f"{name}: scalar registers written too close to a load into LDS:\n  "
                                        + "\n  ".join(bad))

@@ -551,15 +551,22 @@ __device__ __forceinline__ u32x4 tile_words(const void* base, int row0, int rows
 // (wait_dma) before it reads what was loaded.  For tile buffers picked at run time, which the
 // compiler cannot tell apart: with the builtin it would wait for the load in flight before every
 // LDS read.  The compiler sets m0 and knows of it; its hazard pass does not look inside.  The wait
-// state behind the write of m0 is here; the five between a vector instruction's write of a scalar
+// state behind the write of m0 is here, but for loads with an OFFSET (bytes, in LDS and in memory alike), for
+// which m0 stays as the load without one left it: the build fails where it is written right ahead of one, too.
+// (One write of m0 and one wait state for four loads instead of one each: 40 of the short dK/dV form's 630
+// instructions a step; us, dK/dV: a pack of 16384 tokens in sequences of 16 to 1024 224 / 217, 4001 rows, window
+// 1024, 154 / 150, 14 drawn calls 2.7 % on average.)  The five between a vector instruction's write of a scalar
 // register (what a spilled one comes back by) and its use by the load are not (they cost the short
 // dK/dV form 2.8 % over 119 shapes): the build fails where one comes closer (build.py).
-template <int BYTES>
+template <int BYTES, int OFFSET = 0>
 __device__ __forceinline__ void lds_load_asm(u32x4 rsrc, int voff, int soff, uint32_t lds) {
   static_assert(BYTES == 4 || BYTES == 16, "one dword or four per lane");
-  if constexpr (BYTES == 16) {
+  if constexpr (BYTES == 16 && OFFSET == 0) {
     asm volatile("s_nop 0\n\tbuffer_load_dwordx4 %0, %1, %2 offen lds"
                  :: "v"(voff), "s"(rsrc), "s"(soff), "{m0}"(lds) : "memory");
+  } else if constexpr (BYTES == 16) {
+    asm volatile("buffer_load_dwordx4 %0, %1, %2 offen offset:%4 lds"
+                 :: "v"(voff), "s"(rsrc), "s"(soff), "{m0}"(lds), "n"(OFFSET) : "memory");
   } else {
     asm volatile("s_nop 0\n\tbuffer_load_dword %0, %1, %2 offen lds"
                  :: "v"(voff), "s"(rsrc), "s"(soff), "{m0}"(lds) : "memory");
@@ -588,7 +595,8 @@ struct WaveTileDma {
   __device__ __forceinline__ void load_one(u32x4 rsrc, int soff, uint32_t lds_tile, int chunk0) const {
     // rows n RPI + r, r < RPI: swz_f(n RPI + r) = swz_f(r) ^ swz_f(n RPI)
     constexpr int x = (CPR == 16 ? NTH & 3 : (NTH & 1) << 1) << 4;
-    lds_load_asm<16>(rsrc, (chunk0 ^ x) + row_off, soff + NTH * step_bytes, lds_tile + NTH * 1024);
+    constexpr int at = (NTH & 3) * 1024;  // (the instruction's offset counts in LDS and in memory)
+    lds_load_asm<16, at>(rsrc, (chunk0 ^ x) + row_off, soff + NTH * step_bytes - at, lds_tile + NTH * 1024 - at);
   }
 };
 

@@ -36,3 +36,12 @@ def test_other_registers_are_let_be():
     for other in ("v_readlane_b32 s4, v210, 7", "v_readlane_b32 s10, v210, 7", "v_mul_f32_e32 v4, s2, v4",
                   "s_mov_b32 s2, s20", "v_add_co_u32_e64 v1, s[4:5], v1, v2"):
         assert not build.close_sgpr_writes([other, *LOAD])
+
+
+def test_a_load_right_behind_a_write_of_m0_is_found():
+    load = "buffer_load_dwordx4 v4, s[0:3], s9 offen offset:1024 lds"
+    assert build.close_m0_writes(["s_mov_b32 m0, s5", load])
+    assert build.close_m0_writes(["s_add_i32 m0, s5, 64", "<L0>:", load])
+    assert not build.close_m0_writes(["s_mov_b32 m0, s5", "s_nop 0", load])
+    assert not build.close_m0_writes(["s_mov_b32 m0, s5", "v_add_u32_e32 v1, v2, v3", load])
+    assert not build.close_m0_writes(["s_mov_b32 s50, m0", load])
