@@ -672,11 +672,14 @@ __global__ __launch_bounds__(256) void attn_bwd_dkdv_kernel(const AttnArgs a) {
               const int rmax = min(t - rel_lo, rows_ok - 1);
               const unsigned width = (unsigned)max(rmax - rmin + 1, 0);
               const int base = 4 * (lane_m >> 5) - rmin;
-#pragma unroll
-              for (int i = 0; i < 16; i++) {
-                const int c = 8 * (i >> 2) + (i & 3);
-                sacc[kb][i] = ((unsigned)(base + c) < width) ? 0.f : -__builtin_inff();
-              }
+              select_lanes<16>(
+                  [&](auto nc) __attribute__((always_inline)) {
+                    constexpr int i = decltype(nc)::value;
+                    return lanes((unsigned)(base + 8 * (i >> 2) + (i & 3)) < width);
+                  },
+                  [&](auto nc, bool v) __attribute__((always_inline)) {
+                    sacc[kb][decltype(nc)::value] = v ? 0.f : -__builtin_inff();
+                  });
               M::mfma32_vec(fa[f], kf[kb][f], sacc[kb]);
             }
           } else {

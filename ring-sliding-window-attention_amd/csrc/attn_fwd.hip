@@ -202,32 +202,30 @@ void attn_fwd_kernel(const AttnArgs a) {
   auto mask = [&](int tile, f32x16(&sacc)[2]) __attribute__((always_inline)) {
     const int j0 = tile * C::BN;
     const int j1 = j0 + C::BN - 1;
+    // score n of the lane: register n % 16 of the tile's 32-key half n / 16
+    auto keep = [&](auto visible) __attribute__((always_inline)) {
+      select_lanes<32>(
+          [&](auto nc) __attribute__((always_inline)) {
+            constexpr int n = decltype(nc)::value;
+            return visible(n / 16 * 32 + 8 * (n % 16 >> 2) + (n & 3));
+          },
+          [&](auto nc, bool v) __attribute__((always_inline)) {
+            constexpr int t = decltype(nc)::value / 16, i = decltype(nc)::value % 16;
+            sacc[t][i] = v ? sacc[t][i] : -__builtin_inff();
+          });
+    };
     if (!(wave_rows_full && j1 <= wb_first.hi)) {
       const int hi_rel = rb.hi - j0 - 4 * g;
-#pragma unroll
-      for (int t = 0; t < 2; t++)
-#pragma unroll
-        for (int i = 0; i < 16; i++)
-          sacc[t][i] = t * 32 + 8 * (i >> 2) + (i & 3) <= hi_rel ? sacc[t][i] : -__builtin_inff();
+      keep([&](int c) { return lanes(c <= hi_rel); });
     }
     if (j0 < wb_last.lo && j1 >= a.n_sink) {
       int lo_rel = rb.lo - j0 - 4 * g;
       if (j0 < a.n_sink) {  // some of the tile's keys are sinks
         const int sink_rel = a.n_sink - j0 - 4 * g;
         asm volatile("" : "+v"(lo_rel));  // (or both branches' comparisons are made ahead of them, in 64 SGPRs)
-#pragma unroll
-        for (int t = 0; t < 2; t++)
-#pragma unroll
-          for (int i = 0; i < 16; i++) {
-            const int c = t * 32 + 8 * (i >> 2) + (i & 3);
-            sacc[t][i] = ((c >= lo_rel) | (c < sink_rel)) ? sacc[t][i] : -__builtin_inff();
-          }
+        keep([&](int c) { return lanes(c >= lo_rel) | lanes(c < sink_rel); });
       } else {
-#pragma unroll
-        for (int t = 0; t < 2; t++)
-#pragma unroll
-          for (int i = 0; i < 16; i++)
-            sacc[t][i] = t * 32 + 8 * (i >> 2) + (i & 3) >= lo_rel ? sacc[t][i] : -__builtin_inff();
+        keep([&](int c) { return lanes(c >= lo_rel); });
       }
     }
   };
