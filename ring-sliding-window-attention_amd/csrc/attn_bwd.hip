@@ -1273,6 +1273,18 @@ void attn_bwd_dq_kernel(const AttnArgs a) {
   const bool wave_rows_full = r0 + 31 < len_q;
   const RowBounds wb_first = row_bounds(a, r0, len_q, len_k);
   const RowBounds wb_last = row_bounds(a, min(r0 + 31, len_q - 1), len_q, len_k);
+  // Tiles, by their first key, that hold keys of the wave's rows, and that all its rows see whole: an interval
+  // of the band and one of the sinks each, so that a tile costs a comparison or two.
+  // (With this, resources kept instead of selected per tile and the walk's branch: 45 scalar instructions a tile
+  // instead of 75, 60 of which both waves of a SIMD issued ahead of their first MFMA.  us, dQ with statistics: the rank
+  // step, window 4096, 677 / 667; 2 x 8192 rows, 32 heads, window 1000, 414 / 411; 4001 rows 107 / 102 to 110 / 109.6;
+  // 22 drawn and listed calls 1.0 % on average.)
+  const int need_lo = wb_first.lo - (C::BN - 1);
+  const unsigned need_n = wave_valid ? (unsigned)max(wb_last.hi - need_lo + 1, 0) : 0u;
+  const int need_sink = wave_valid ? min(a.n_sink, wb_last.hi + 1) : 0;
+  const int full_end = wave_rows_full ? wb_first.hi - (C::BN - 1) + 1 : 0;  // behind the last not cut by the upper bound
+  const unsigned full_n = (unsigned)max(full_end - wb_last.lo, 0);
+  const int full_sink = min(a.n_sink - (C::BN - 1), full_end);
 
   TileDma<D, C::BN, NW * 64, true> k_dma, v_dma;
   k_dma.init(a.k_st[1], tid);
@@ -1282,8 +1294,19 @@ void attn_bwd_dq_kernel(const AttnArgs a) {
   const T* v2_ptr = a.v2 ? (const T*)a.v2 + b * a.v_st[0] + hk * a.v_st[2] : v_ptr;
   const KeyRows<T, C::ROWB, FAR> k_rows(k_ptr, k2_ptr, a.seg, len_k, a.k_st[1]), v_rows(v_ptr, v2_ptr, a.seg, len_k, a.v_st[1]);
   auto load_tile = [&](int tile, char* kd, char* vd) __attribute__((always_inline)) {
-    k_dma.load(k_rows.template tile<C::BN>(tile * C::BN), kd);
-    v_dma.load(v_rows.template tile<C::BN>(tile * C::BN), vd);
+    const int row = tile * C::BN;
+    if constexpr (FAR || THREE) {  // (THREE: the resources would spill)
+      k_dma.load(k_rows.template tile<C::BN>(row), kd);
+      v_dma.load(v_rows.template tile<C::BN>(row), vd);
+    } else if (__builtin_expect(row < a.seg, 1)) {
+      k_dma.load(k_rows.first_range(), row * k_rows.stride_bytes, kd);
+      v_dma.load(v_rows.first_range(), row * v_rows.stride_bytes, vd);
+    } else {  // (code of its own: the first range's resources stay as they are, in registers)
+      asm volatile("");
+      k_dma.load(k_rows.template tile<C::BN>(row), kd);
+      v_dma.load(v_rows.template tile<C::BN>(row), vd);
+      asm volatile("");
+    }
   };
 
   // The first tiles are asked for ahead of the rows' own data, and of that everything before the first
@@ -1383,13 +1406,14 @@ void attn_bwd_dq_kernel(const AttnArgs a) {
                   char* vn) __attribute__((always_inline)) {
     const int j0 = walk.tile * C::BN;
     const int j1 = j0 + C::BN - 1;
-    walk.next();
+    walk.next<!THREE>();
     if (it + 1 < n_tiles) load_tile(walk.tile, kn, vn);
-    const bool needed =
-        wave_valid && j0 <= wb_last.hi && (j1 >= wb_first.lo || j0 < a.n_sink);
+    // (THREE has no scalar registers for the intervals)
+    const bool needed = THREE ? wave_valid && j0 <= wb_last.hi && (j1 >= wb_first.lo || j0 < a.n_sink)
+                              : (unsigned)(j0 - need_lo) < need_n || j0 < need_sink;
     if (needed) {
-      const bool full = wave_rows_full && j1 <= wb_first.hi &&
-                        (j0 >= wb_last.lo || j1 < a.n_sink);
+      const bool full = THREE ? wave_rows_full && j1 <= wb_first.hi && (j0 >= wb_last.lo || j1 < a.n_sink)
+                              : (unsigned)(j0 - wb_last.lo) < full_n || j0 < full_sink;
       // S^T and dP^T (element i of tile [kb][qb]: key 16 kb + 4 u + i, query 16 qb + r); every
       // K / V fragment read feeds the MFMAs of both query blocks; the chains start from the
       // row statistics.  The two waves of a SIMD overlap best when each keeps its matrix and
@@ -1458,7 +1482,7 @@ void attn_bwd_dq_kernel(const AttnArgs a) {
               for (int i = 0; i < 4; i++)
                 sacc[kb][qb][i] = visible(16 * kb + i, qb) ? sacc[kb][qb][i] : 0.f;
         };
-        if (!(wave_rows_full && j1 <= wb_first.hi)) keep([&](int c, int qb) { return c <= hi_rel[qb]; });
+        if (THREE ? !(wave_rows_full && j1 <= wb_first.hi) : j0 >= full_end) keep([&](int c, int qb) { return c <= hi_rel[qb]; });
         if (j0 < wb_last.lo && j1 >= a.n_sink) {
           if (j0 < a.n_sink) {  // some of the tile's keys are sinks
             const int sink_rel = a.n_sink - at;

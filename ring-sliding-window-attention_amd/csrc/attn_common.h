@@ -183,12 +183,24 @@ struct KeyWalk {
     stop = n_sink > 0 ? n_sink : end;
     jump = n_sink > 0 ? first : back;
   }
+  // BRANCH: by a branch that is taken once or twice a walk instead of selects, five instructions a tile (the dQ
+  // kernel at head_dim 128, whose waves start a tile together and wait for it; the forward gains nothing)
+  template <bool BRANCH>
   __device__ __forceinline__ void next() {
     tile++;
-    const bool at = tile == stop;
-    tile = at ? jump : tile;
-    stop = at ? end : stop;
-    jump = at ? back : jump;
+    if constexpr (BRANCH) {
+      if (__builtin_expect(tile == stop, 0)) {
+        asm volatile("");
+        tile = jump;
+        stop = end;
+        jump = back;
+      }
+    } else {
+      const bool at = tile == stop;
+      tile = at ? jump : tile;
+      stop = at ? end : stop;
+      jump = at ? back : jump;
+    }
   }
 };
 inline int walk_mask(const AttnArgs& a, int block_rows, int tile_keys) {
@@ -473,6 +485,9 @@ struct KeyRows {
         stride_bytes((int)(stride_elems * 2)) {
     bytes1 = rows1 > 0 ? (rows1 - 1) * stride_bytes + ROW_BYTES : 0;
     bytes2 = rows2 > 0 ? (rows2 - 1) * stride_bytes + ROW_BYTES : 0;
+  }
+  __device__ __forceinline__ __amdgpu_buffer_rsrc_t first_range() const {
+    return __builtin_amdgcn_make_buffer_rsrc((void*)first, 0, bytes1, 0x00020000);
   }
   template <int ROWS>
   __device__ __forceinline__ TileSrc tile(int row0) const {

@@ -115,7 +115,7 @@ void attn_fwd_kernel(const AttnArgs a) {
   const int n_tiles = n_sink_t + n_band;
   KeyWalk walk(a, n_sink_t, t_lo, n_band);
   const int t_first = walk.tile;
-  walk.next();
+  walk.next<false>();
 
   // ---- this wave's rows ----------------------------------------------------
   const int r0 = i0 + (pair ? wave & 1 : wave) * 32;
@@ -297,7 +297,7 @@ void attn_fwd_kernel(const AttnArgs a) {
   // V(t-1), last read before it: the loads of K(t+2) and V(t+1) into them follow it.
   f32x16 s_cur[2];
   int t_cur = t_first, t_next = walk.tile;  // tiles t and t + 1; the cursor: t + 2
-  walk.next();
+  walk.next<false>();
   auto prefetch = [&](int it, char* kfree, char* vn) __attribute__((always_inline)) {
     if (it + 2 < n_tiles) load_k(walk.tile, kfree);
     if (it + 1 < n_tiles) load_v(t_next, vn);
@@ -353,7 +353,7 @@ void attn_fwd_kernel(const AttnArgs a) {
     }
     t_cur = t_next;
     t_next = walk.tile;
-    walk.next();
+    walk.next<false>();
   };
 
   __syncthreads();
