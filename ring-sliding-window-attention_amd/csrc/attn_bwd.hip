@@ -180,18 +180,27 @@ __global__ __launch_bounds__(256) void attn_bwd_dkdv_kernel(const AttnArgs a) {
   // form's tiles any (422 shapes, mean 1.2 % faster, 10 % slower to 20 % faster).  Sequences of
   // more than 4096 keys keep the plain order: four of 16384 tokens lose 3 % by it, 10240 keys under
   // 8192 rows in 40 wide tiles 447 / 550.
-  int n_tile = a.n_tile, n_work = a.n_work, per_xcd = (int)gridDim.x >> 3, snake = a.snake;
+  // (which tiles an XCD takes: see tile_of_block)
+  int n_tile = a.n_tile, n_group = a.n_group, snake = a.snake;
   if (a.ktile) {
     n_tile = a.ktile[a.batch];
     snake = a.ktile[a.batch + 1];
-    n_work = n_tile * a.heads_kv;
-    per_xcd = (n_work + 7) >> 3;
+    n_group = n_tile * (a.heads_kv << a.xcd_log2 >> 3);
   }
+  const int xcd = (int)blockIdx.x & 7, in_group = (1 << a.xcd_log2) - 1;
+  int per_xcd = (n_group + in_group) >> a.xcd_log2;
+  if (a.xcd_log2 == 0) per_xcd = (n_tile * a.tile_heads + 7) >> 3;
   int in_xcd = (int)blockIdx.x >> 3;
   if (in_xcd >= per_xcd) return;
   if (snake && (in_xcd & 4) && (in_xcd | 3) < per_xcd) in_xcd ^= 3;
-  const int wid = ((int)blockIdx.x & 7) * per_xcd + in_xcd;
-  if (wid >= n_work) return;
+  int wid = xcd * per_xcd + in_xcd;
+  if (a.xcd_log2 == 0) {
+    if (wid >= n_tile * a.tile_heads) return;
+  } else {
+    const int at_group = (in_xcd << a.xcd_log2) + (xcd & in_group);
+    if (at_group >= n_group) return;
+    wid = (xcd >> a.xcd_log2) * n_group + at_group;
+  }
   const int tid = threadIdx.x;
   const int lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);  // (not WALK4: key group of 64 keys)
@@ -1212,8 +1221,6 @@ void attn_bwd_dq_kernel(const AttnArgs a) {
   __shared__ __attribute__((aligned(1024))) char v_s0[C::TILE];
   __shared__ __attribute__((aligned(1024))) char v_s1[C::TILE];
 
-  const int wid = logical_block_id(a.n_work);
-  if (wid < 0) return;
   const int tid = threadIdx.x;
   const int lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -1225,8 +1232,8 @@ void attn_bwd_dq_kernel(const AttnArgs a) {
   const bool pair = (a.group & 1) == 0;
   const int units = pair ? a.group >> 1 : a.group;
   const int bm = pair ? 16 * NW : 32 * NW;
-  int rest = quotient(wid, a.by_units);
-  const int hu = wid - rest * units;
+  int rest, hu;
+  if (!tile_of_block(a, units, rest, hu)) return;
   const int tiles_before = quotient(rest, a.by_tile);
   const int tile = rest - tiles_before * a.n_tile;
   const int slot = a.rev_q ? a.n_tile - 1 - tile : tile;
@@ -1348,7 +1355,7 @@ void attn_bwd_dq_kernel(const AttnArgs a) {
     // the elements behind the lse2 array (see attn_bwd_prep_kernel), where block 0 surely is at
     // work; for a pack, whose first slot may stand for no tile, attn_bwd_rest_kernel writes them
     const int64_t used = a.rows_q * a.heads_q;
-    if (!a.cu_q && wid == 0 && used + tid < a.delta - a.lse2) a.lse2[used + tid] = -__builtin_inff();
+    if (!a.cu_q && blockIdx.x == 0 && used + tid < a.delta - a.lse2) a.lse2[used + tid] = -__builtin_inff();
   }
 #pragma unroll
   for (int qb = 0; qb < 2; qb++) {
@@ -1610,8 +1617,6 @@ __global__ __launch_bounds__(256) void attn_bwd_dq_ds_kernel(const AttnArgs a) {
   __shared__ __attribute__((aligned(1024))) char ds_s1[4 * C::WAVE_LDS];
   __shared__ __attribute__((aligned(1024))) char ds_s2[4 * C::WAVE_LDS];
 
-  const int wid = logical_block_id(a.n_work);
-  if (wid < 0) return;
   const int tid = threadIdx.x;
   const int lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -1624,8 +1629,8 @@ __global__ __launch_bounds__(256) void attn_bwd_dq_ds_kernel(const AttnArgs a) {
   const int units = a.group >> hsh;
   const int bm_log2 = 8 - hsh;  // 64 rows x (4 >> hsh) units
   const int bm = 1 << bm_log2;
-  const int hu = wid % units;
-  int rest = wid / units;
+  int rest, hu;
+  if (!tile_of_block(a, units, rest, hu)) return;
   const int slot = a.rev_q ? a.n_tile - 1 - rest % a.n_tile : rest % a.n_tile;
   rest /= a.n_tile;
   const int hk = rest % a.heads_kv;
@@ -2002,19 +2007,12 @@ int launch_bwd(AttnArgs& a, hipStream_t stream, int phases) {
     const bool pair = (a.group & 1) == 0;
     const bool small = D == 64 || a.avg_keys <= RSWA_DQ_SMALL_AVG_KEYS;
     const int bm = (pair ? 16 : 32) * (small ? 4 : 8);
-    const int units_q = (pair ? a.group / 2 : a.group) * a.heads_kv;  // blocks per q tile
-    if (a.cu_q) {
-      a.n_tile = (int)(ceil_div(a.rows_q, bm) + a.batch);
-      a.n_work = a.n_tile * units_q;
-    } else {
-      a.n_tile = (int)ceil_div(a.seqlen_q, bm);
-      a.n_work = a.n_tile * units_q * a.batch;
-    }
-    if (a.n_work == 0) return (int)RSWA_OK;
-    set_divisors(a, units_q / a.heads_kv);
+    a.n_tile = (int)(a.cu_q ? ceil_div(a.rows_q, bm) + a.batch : ceil_div(a.seqlen_q, bm));
+    if (a.n_tile == 0) return (int)RSWA_OK;
+    const int64_t blocks = deal_blocks(a, pair ? a.group / 2 : a.group, spread_rows(a));
     a.walk_mask = walk_mask(a, bm, DqCfg<D>::BN);
     clear_launch_error();
-    const dim3 grid(padded_grid(a.n_work)), block(small ? 256 : 512);
+    const dim3 grid((unsigned)blocks), block(small ? 256 : 512);
     if constexpr (!STATS) {
       if (a.far) {
         if (small) {
@@ -2057,23 +2055,20 @@ int launch_bwd(AttnArgs& a, hipStream_t stream, int phases) {
   if (phases & RSWA_BWD_DKDV) {
     using C = DkvCfg<D>;
     const int bn = walk4 ? C::BN / 4 : C::BN;
-    if (a.cu_q) {
-      a.n_tile = (int)(ceil_div(a.rows_k, bn) + a.batch);
-      a.n_work = a.n_tile * a.heads_kv;
-    } else {
-      a.n_tile = (int)ceil_div(a.seqlen_k, bn);
-      a.n_work = a.n_tile * a.heads_kv * a.batch;
-    }
+    a.n_tile = (int)(a.cu_q ? ceil_div(a.rows_k, bn) + a.batch : ceil_div(a.seqlen_k, bn));
+    const int64_t key_blocks = a.n_tile > 0 ? deal_blocks(a, 1, spread_keys(a)) : 0;
     if (a.ktile && !(phases & RSWA_BWD_PREP)) {
       clear_launch_error();
       hipLaunchKernelGGL(attn_bwd_ktile_kernel, dim3(1), dim3(256), 0, stream, a);
       int rc = check_launch("attn_bwd key tile table");
       if (rc != RSWA_OK) return rc;
     }
-    a.snake = !a.cu_q && a.seqlen_k <= kSnakeKeys && (walk4 || a.n_tile % 4 == 0);
-    if (a.n_work > 0) {
+    // (an XCD that takes every second tile meets the same lengths again after half as many)
+    const int period = a.n_tile >> std::min<int>(a.xcd_log2, __builtin_ctz(a.n_tile | 8));
+    a.snake = !a.cu_q && a.seqlen_k <= kSnakeKeys && (walk4 || period % 4 == 0);
+    if (key_blocks > 0) {
       clear_launch_error();
-      const dim3 grid(padded_grid(a.n_work)), block(C::THREADS);
+      const dim3 grid((unsigned)key_blocks), block(C::THREADS);
       auto go = [&](auto far, auto hand, auto w4) {
         hipLaunchKernelGGL((attn_bwd_dkdv_kernel<T, D, decltype(far)::value, decltype(hand)::value, decltype(w4)::value>),
                            grid, block, 0, stream, a);
@@ -2086,7 +2081,7 @@ int launch_bwd(AttnArgs& a, hipStream_t stream, int phases) {
       int rc = check_launch("attn_bwd dkdv");
       if (rc != RSWA_OK) return rc;
     }
-    if (a.n_work > 0 && a.sink_part && a.rows_q > 0) {
+    if (key_blocks > 0 && a.sink_part && a.rows_q > 0) {
       clear_launch_error();
       const dim3 grid(a.batch * a.heads_kv * a.sink_chunks), block(256);
       if (a.n_sink == 1) hipLaunchKernelGGL((attn_bwd_sink_kernel<T, D, 1>), grid, block, 0, stream, a);
@@ -2098,17 +2093,11 @@ int launch_bwd(AttnArgs& a, hipStream_t stream, int phases) {
   if ((phases & RSWA_BWD_DQ) && a.ds) {
     const int hsh = (a.group & 3) == 0 ? 2 : (a.group & 1) == 0 ? 1 : 0;
     const int bm = 256 >> hsh;
-    const int units_q = (a.group >> hsh) * a.heads_kv;
-    if (a.cu_q) {
-      a.n_tile = (int)(ceil_div(a.rows_q, bm) + a.batch);
-      a.n_work = a.n_tile * units_q;
-    } else {
-      a.n_tile = (int)ceil_div(a.seqlen_q, bm);
-      a.n_work = a.n_tile * units_q * a.batch;
-    }
-    if (a.n_work > 0) {
+    a.n_tile = (int)(a.cu_q ? ceil_div(a.rows_q, bm) + a.batch : ceil_div(a.seqlen_q, bm));
+    if (a.n_tile > 0) {
+      const int64_t blocks = deal_blocks(a, a.group >> hsh, false);
       clear_launch_error();
-      hipLaunchKernelGGL((attn_bwd_dq_ds_kernel<T, D>), dim3(padded_grid(a.n_work)), dim3(256), 0,
+      hipLaunchKernelGGL((attn_bwd_dq_ds_kernel<T, D>), dim3((unsigned)blocks), dim3(256), 0,
                          stream, a);
       int rc = check_launch("attn_bwd dq (dS hand-off)");
       if (rc != RSWA_OK) return rc;

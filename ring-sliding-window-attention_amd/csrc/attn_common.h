@@ -76,6 +76,7 @@ struct AttnArgs {
   int32_t wide_out, wide_dq, wide_dkv, dkv_accumulate;
   int32_t n_tile;          // tiles per sequence (dense) / total tile slots (packed)
   int32_t n_work;          // logical blocks
+  int32_t xcd_log2, n_group, tile_heads;  // see tile_of_block; kv heads of all batch entries (a pack: kv heads)
   FastDiv by_tile, by_heads, by_units;  // n_tile, heads_kv, blocks per (kv head, tile)
   // Blocks are dispatched in logical order; these flags reverse the order of the query
   // tiles (forward, dQ) or key tiles (dK/dV) so that the tiles with the most visible
@@ -119,22 +120,84 @@ struct SeqInfo {
   int32_t batch_idx;
 };
 
-// XCD-aware block id: consecutive logical ids land on the same XCD (8 XCDs,
-// hardware deals physical block ids round-robin), so that blocks sharing K/V
-// tiles share an L2.  The grid is padded to a multiple of 8; returns -1 for pad.
-__device__ __forceinline__ int logical_block_id(int n_work) {
-  const int per_xcd = (int)gridDim.x >> 3;
-  const int id = ((int)blockIdx.x & 7) * per_xcd + ((int)blockIdx.x >> 3);
-  return id < n_work ? id : -1;
+// Which tile (of all: kv head after kv head, batch entry after batch entry, n_tile each) and which of its
+// `units` blocks is this block's?  Hardware deals block ids to the 8 XCDs in turn, and blocks that share K / V
+// should share an L2.  xcd_log2 = 0: every XCD takes an eighth of all blocks in a row.  Else the XCDs form groups of
+// 1 << xcd_log2, each with n_group tiles that its XCDs take in turn (see deal_blocks).  False: a block beyond the last.
+__device__ __forceinline__ bool tile_of_block(const AttnArgs& a, int units, int& tile, int& unit) {
+  const int x = (int)blockIdx.x & 7, j = (int)blockIdx.x >> 3;
+  if (a.xcd_log2 == 0) {
+    const int id = x * ((int)gridDim.x >> 3) + j;
+    tile = quotient(id, a.by_units);
+    unit = id - tile * units;
+    return id < a.n_work;
+  }
+  const int k = quotient(j, a.by_units);
+  unit = j - k * units;
+  const int at = (k << a.xcd_log2) + (x & ((1 << a.xcd_log2) - 1));
+  tile = (x >> a.xcd_log2) * a.n_group + at;
+  return at < a.n_group;
 }
 
-inline void set_divisors(AttnArgs& a, int blocks_per_tile) {
+// XCDs (as a power of two) that share kv heads where each takes an eighth of them all: 0 if each has whole ones.
+inline int xcds_per_head_log2(const AttnArgs& a) {
+  const int heads = a.heads_kv * (a.cu_q ? 1 : a.batch);
+  return 3 - std::min(3, (int)__builtin_ctz((unsigned)heads));
+}
+// Tile dealing for a.n_tile tiles per kv head (and batch entry) of `units` blocks each: sets what the kernels read
+// and returns the blocks to launch.  `spread`: XCDs that share kv heads take their tiles in turn.
+inline int64_t deal_blocks(AttnArgs& a, int units, bool spread) {
+  const int64_t heads = (int64_t)a.heads_kv * (a.cu_q ? 1 : a.batch);
+  a.xcd_log2 = spread ? xcds_per_head_log2(a) : 0;
+  a.n_work = (int)(heads * a.n_tile * units);
+  a.tile_heads = (int)heads;
+  a.n_group = (int)((heads << a.xcd_log2 >> 3) * a.n_tile);  // (whole heads; xcd_log2 = 0: read where heads % 8 == 0)
   a.by_tile = fast_div((uint32_t)a.n_tile);
   a.by_heads = fast_div((uint32_t)a.heads_kv);
-  a.by_units = fast_div((uint32_t)blocks_per_tile);
+  a.by_units = fast_div((uint32_t)units);
+  return a.xcd_log2 ? ceil_div(a.n_group, 1 << a.xcd_log2) * 8 * units : ceil_div(a.n_work, 8) * 8;
+}
+constexpr int kComputeUnits = 256;  // MI355X
+
+// Should forward and dQ blocks be spread?  Tiles in a row share their windows' K and V, so an XCD with every second
+// tile reads almost twice the bytes (12 = 12 heads, even work: 3 to 6 % slower); but where the rows of some parts of a
+// sequence see fewer keys, parts make unequal eighths (us, eighths / spread: rank step of 7298 rows, 28 / 4 heads,
+// window 5372, forward 429 / 348, dQ 651 / 524; 3958 rows, 28 / 4 heads, a sink, window 2397, 126 / 109 and 178 / 139;
+// 2 x 18605 rows, 8 / 2 heads, head_dim 64, window 3149, 277 / 253 and 329 / 300).  So: where the fullest eighth has
+// 5 % more than the average, of a dense call (of a pack the host knows too little, and both orders lost and won).  A
+// row counts as its keys and 200 for starts and ends.
+inline bool spread_rows(const AttnArgs& a) {
+  const int log2 = xcds_per_head_log2(a);
+  const int heads = (a.heads_kv * a.batch) << log2 >> 3;  // that 1 << log2 XCDs share
+  if (a.cu_q || log2 == 0 || heads > 8) return false;
+  constexpr int S = 32;  // samples per head
+  const int64_t sh = a.shift_explicit ? a.shift_val : (int64_t)a.seqlen_k - a.seqlen_q;
+  double part[8] = {0}, all = 0;
+  for (int i = 0; i < heads * S; i++) {
+    const int64_t row = (int64_t)(2 * (i % S) + 1) * a.seqlen_q / (2 * S);
+    const int64_t hi = a.wr >= 0 ? std::min<int64_t>(a.seqlen_k - 1, row + sh + a.wr) : a.seqlen_k - 1;
+    const int64_t lo = a.wl >= 0 ? std::max<int64_t>(0, row + sh - a.wl) : 0;
+    const double keys = (double)std::max<int64_t>(0, hi - lo + 1) + 200;
+    part[(i << log2) / (heads * S)] += keys;
+    all += keys;
+  }
+  return *std::max_element(part, part + (1 << log2)) * (1 << log2) > 1.05 * all;
 }
 
-static inline unsigned padded_grid(int64_t n_work) { return (unsigned)(ceil_div(n_work, 8) * 8); }
+// And dK/dV blocks?  Lengths vary more (keys at a sequence's end are seen by few rows), and with tiles in a row one
+// XCD's last blocks are those of a sequence's end, short or long, and its share of a pack's sequences is what comes (us,
+// dK/dV, eighths / spread: 28 / 4 heads, head_dim 64, 3914 rows against 5194 keys, window 1296, 122 / 90; rank step of
+// 4667 rows, 12 = 12 heads, window 5365, 107 / 96; packs of 23745 tokens, 28 / 4 heads, window 2203, 679 / 630, and of
+// 16544, 4 = 4 heads, window 1132, 99 / 92).  Not where windows are short against the sequences (even work) and the
+// launch has a second round to even out what the first leaves (25429 rows, 16 / 4 heads, window 593, 400 blocks, 183 /
+// 189; packs of long sequences, 8 / 2 heads, windows 90 and 205, 36 / 41 and 119 / 128; but 4134 rows, 28 / 4 heads,
+// window 173, 260 blocks, 64 / 53, and 20516 rows, window 568, 324 blocks, 438 / 405).
+inline bool spread_keys(const AttnArgs& a) {
+  const int64_t heads = (int64_t)a.heads_kv * (a.cu_q ? 1 : a.batch);
+  const int64_t len = a.cu_q ? a.rows_k / a.batch : a.seqlen_k;
+  const bool even = a.wl >= 0 && a.wr >= 0 && ((int64_t)a.wl + a.wr + 1) * 8 < len;
+  return !even || heads * a.n_tile <= kComputeUnits * 7 / 5;
+}
 
 // Mask bounds of one query row i (local index): visible keys are
 //   j <= hi  and  (j >= lo or j < n_sink);   hi already clipped to len_k - 1.
@@ -689,7 +752,6 @@ constexpr int kDsBlockBytes = 32 * kDkvKeysPerBlock * 2;
 constexpr int kDsUnitBytes = kDsBlockBytes / 4;
 constexpr int kMaxTileRows = 256;  // bound on the rows fetched as one tile that the stride checks assume
                                    // (today's largest tile has 64 rows: K / V in the forward and dQ kernels)
-constexpr int kComputeUnits = 256;  // MI355X
 struct BwdLayout {
   uint64_t stats_bytes;    // each of the two statistics arrays
   int n_count;             // arrival counters of the sink kernel

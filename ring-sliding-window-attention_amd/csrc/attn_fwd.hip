@@ -54,8 +54,6 @@ void attn_fwd_kernel(const AttnArgs a) {
   __shared__ __attribute__((aligned(1024))) char v_s0[C::TILE];
   __shared__ __attribute__((aligned(1024))) char v_s1[C::TILE];
 
-  const int wid = logical_block_id(a.n_work);
-  if (wid < 0) return;
   const int tid = threadIdx.x;
   const int lane = tid & 63;
   // (known to be uniform: the rows' bounds are scalars, 20 registers less; with SKIP, whose branches then
@@ -72,8 +70,8 @@ void attn_fwd_kernel(const AttnArgs a) {
   const bool pair = (a.group & 1) == 0;
   const int units = pair ? a.group >> 1 : a.group;  // blocks per (kv head, q tile)
   const int bm = pair ? 16 * NW : 32 * NW;          // query rows per block
-  int rest = quotient(wid, a.by_units);
-  const int hu = wid - rest * units;
+  int rest, hu;
+  if (!tile_of_block(a, units, rest, hu)) return;
   const int tiles_before = quotient(rest, a.by_tile);
   const int tile = rest - tiles_before * a.n_tile;
   const int slot = a.rev_q ? a.n_tile - 1 - tile : tile;
@@ -510,16 +508,9 @@ template <typename T, int D, int WAVES>
 int launch_fwd(AttnArgs& a, hipStream_t stream) {
   using C = FwdCfg<D>;
   const int bm = rows_per_block(a);
-  const int units = blocks_per_tile(a);
-  if (a.cu_q) {
-    a.n_tile = (int)(ceil_div(a.rows_q, bm) + a.batch);
-    a.n_work = a.n_tile * units;
-  } else {
-    a.n_tile = (int)ceil_div(a.seqlen_q, bm);
-    a.n_work = a.n_tile * units * a.batch;
-  }
-  if (a.n_work == 0) return RSWA_OK;
-  set_divisors(a, units / a.heads_kv);
+  a.n_tile = (int)(a.cu_q ? ceil_div(a.rows_q, bm) + a.batch : ceil_div(a.seqlen_q, bm));
+  if (a.n_tile == 0) return RSWA_OK;
+  const int64_t blocks = deal_blocks(a, blocks_per_tile(a) / a.heads_kv, spread_rows(a));
   a.walk_mask = walk_mask(a, bm, C::BN);
   // keys a row sees at most; the per-wave tile skip pays when the rows of a block beyond one
   // wave's 32 add a tenth or more to that span
@@ -528,7 +519,7 @@ int launch_fwd(AttnArgs& a, hipStream_t stream) {
   // eighteen: no difference either way, 0.435 against 0.431-0.441 ms)
   const bool skip = (bm - 32) * 10 >= span + bm;
   clear_launch_error();
-  const dim3 grid(padded_grid(a.n_work)), block(C::THREADS);
+  const dim3 grid((unsigned)blocks), block(C::THREADS);
   if (skip) {
     if (a.far) hipLaunchKernelGGL((attn_fwd_kernel<T, D, true, true, WAVES>), grid, block, 0, stream, a);
     else hipLaunchKernelGGL((attn_fwd_kernel<T, D, true, false, WAVES>), grid, block, 0, stream, a);
