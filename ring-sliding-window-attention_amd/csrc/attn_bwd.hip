@@ -331,8 +331,9 @@ __global__ __launch_bounds__(256) void attn_bwd_dkdv_kernel(const AttnArgs a) {
   Dma q_dma, do_dma;
   q_dma.init(a.q_st[1], tid);
   do_dma.init(a.do_st[1], tid);
-  const T* q_base = (const T*)a.q + b * a.q_st[0] + s.q_row0 * a.q_st[1];
-  const T* do_base = (const T*)a.dout + b * a.do_st[0] + s.q_row0 * a.do_st[1];
+  constexpr int BACK = WALK4 ? WaveTileDma<D, C::BM>::BACK : 0;  // bytes; see there
+  const T* q_base = (const T*)((const char*)a.q - BACK) + b * a.q_st[0] + s.q_row0 * a.q_st[1];
+  const T* do_base = (const T*)((const char*)a.dout - BACK) + b * a.do_st[0] + s.q_row0 * a.do_st[1];
   // statistics: one load covers both workspace arrays (lse2, then delta `stat_elems` further
   // on) through one resource, the tile's first row in the scalar offset; rows past the sequence end read
   // a neighbour's finite values, which the row mask / zero Q, dO rows void
@@ -424,7 +425,7 @@ __global__ __launch_bounds__(256) void attn_bwd_dkdv_kernel(const AttnArgs a) {
       const int row_bytes = is_q ? q_row_bytes : do_row_bytes;
       (is_q ? q_dma : do_dma)
           .template load_one<is_q ? part - 1 : part - 1 - NQD>(
-              tile_words<C::BM, FAR>(head, nxt.i0, len_q, row_bytes, C::ROWB), FAR ? 0 : nxt.i0 * row_bytes,
+              tile_words<C::BM, FAR>(head, nxt.i0, len_q, row_bytes, C::ROWB + BACK), FAR ? BACK : nxt.i0 * row_bytes + BACK,
               (uint32_t)(uintptr_t)(lds_void_t*)(is_q ? qd : dod) + w_lds, dma_chunk);
     } else if constexpr (part <= NQD) {
       const TileSrc t = tile_src<C::BM, FAR>(nxt.q_head, nxt.i0, len_q, q_row_bytes, C::ROWB);

@@ -669,11 +669,16 @@ struct WaveTileDma {
     row_off = (int)((tid & 63) / CPR * stride_elems * 2);
     step_bytes = (int)(RPI * stride_elems * 2);
   }
+  // `rsrc`: of the rows and the BACK bytes ahead of them, which no lane reads; `soff` is the tile's place among the
+  // rows.  What sharing a write of m0 takes out of the scalar offset, an unsigned number, can leave none below zero
+  // so, also where rows lie closer than their own bytes (the gradient of a sum over the rows: stride 0).
+  static constexpr int BACK = 3 * 1024;
   template <int NTH>
   __device__ __forceinline__ void load_one(u32x4 rsrc, int soff, uint32_t lds_tile, int chunk0) const {
     // rows n RPI + r, r < RPI: swz_f(n RPI + r) = swz_f(r) ^ swz_f(n RPI)
     constexpr int x = (CPR == 16 ? NTH & 3 : (NTH & 1) << 1) << 4;
     constexpr int at = (NTH & 3) * 1024;  // (the instruction's offset counts in LDS and in memory)
+    static_assert(at <= BACK, "no scalar offset below zero");
     lds_load_asm<16, at>(rsrc, (chunk0 ^ x) + row_off, soff + NTH * step_bytes - at, lds_tile + NTH * 1024 - at);
   }
 };
