@@ -1266,15 +1266,9 @@ void attn_bwd_dq_kernel(const AttnArgs a) {
 
   // ---- key tiles this block visits (same rule as the forward kernel) -----------
   const int i_last = min(i0 + bm, len_q) - 1;
-  const int lo_blk = row_bounds(a, i0, len_q, len_k).lo;
-  const int hi_blk = row_bounds(a, i_last, len_q, len_k).hi;
-  const bool band = hi_blk >= lo_blk;
-  const int t_lo = band ? lo_blk / C::BN : (1 << 29);
-  const int n_band = band ? hi_blk / C::BN - t_lo + 1 : 0;
-  const int sink_keys = max(0, min(min(a.n_sink, hi_blk + 1), lo_blk));
-  const int n_sink_t = min((sink_keys + C::BN - 1) / C::BN, t_lo);
-  const int n_tiles = n_sink_t + n_band;
-  KeyWalk walk(a, n_sink_t, t_lo, n_band);
+  const KeyTiles tiles = key_tiles<C::BN>(a, i0, i_last, len_q, len_k);
+  const int n_tiles = tiles.n_sink + tiles.n_band;
+  KeyWalk walk(a, tiles);
 
   const int r0 = i0 + (pair ? wave & ((1 << HSH) - 1) : wave) * 32;
   const bool wave_valid = r0 < len_q;
@@ -2011,7 +2005,9 @@ int launch_bwd(AttnArgs& a, hipStream_t stream, int phases) {
     a.n_tile = (int)(a.cu_q ? ceil_div(a.rows_q, bm) + a.batch : ceil_div(a.seqlen_q, bm));
     if (a.n_tile == 0) return (int)RSWA_OK;
     const int64_t blocks = deal_blocks(a, pair ? a.group / 2 : a.group, spread_rows(a));
-    a.walk_mask = walk_mask(a, bm, DqCfg<D>::BN);
+    // (rows a block may have with this window, whatever the call's lengths: no more keys a row, no block of 256)
+    const bool never_large = D == 64 || (int64_t)a.wl + a.wr + 1 + a.n_sink <= RSWA_DQ_SMALL_AVG_KEYS;
+    a.by_walk = walk_period(a, never_large ? 128 : 256, DqCfg<D>::BN);
     clear_launch_error();
     const dim3 grid((unsigned)blocks), block(small ? 256 : 512);
     if constexpr (!STATS) {

@@ -26,8 +26,8 @@ constexpr float kLog2e = 1.4426950408889634f;
 // the compiler does not know is some 30 dependent instructions, five of them ahead of a block's first
 // load).  The method is Granlund and Montgomery's ("Division by Invariant Integers using Multiplication",
 // 1994): multiplier 2^32 + mul with mul = floor(2^32 (2^shift - d) / d) + 1, shift = ceil(log2 d).
-// (`d` is not read: it keeps the kernel arguments behind where they load best -- without it a forward of
-// 2 x 333 rows, 8 / 2 heads, fp16, takes 9.44 us instead of 9.33.)
+// (`d` is read of the walk's period only; in the others it keeps the kernel arguments behind where they load best:
+// without it a forward of 2 x 333 rows, 8 / 2 heads, fp16, took 9.44 us instead of 9.33.)
 struct FastDiv {
   uint32_t d, mul, shift;
 };
@@ -36,8 +36,8 @@ inline FastDiv fast_div(uint32_t d) {  // d >= 1
   while ((1ull << s) < d) s++;
   return {d, (uint32_t)(((1ull << 32) * ((1ull << s) - d)) / d + 1), s};
 }
-__device__ __forceinline__ int quotient(int n, const FastDiv& f) {
-  return (int)((__umulhi((uint32_t)n, f.mul) + (uint32_t)n) >> f.shift);
+__host__ __device__ __forceinline__ int quotient(int n, const FastDiv& f) {
+  return (int)(((uint32_t)((uint64_t)(uint32_t)n * f.mul >> 32) + (uint32_t)n) >> f.shift);
 }
 
 // Kernel-side view of rswa_attn_params (strides in elements).
@@ -82,7 +82,7 @@ struct AttnArgs {
   // tiles (forward, dQ) or key tiles (dK/dV) so that the tiles with the most visible
   // pairs start first and the short ones fill the tail of the launch.
   int32_t rev_q, rev_k;
-  int32_t walk_mask;  // see walk_start
+  FastDiv by_walk;  // see KeyWalk
   // backward with sink keys and a bounded window: workspace of the sink kernel -- fp32 sums
   // [sequence x kv head][chunk of rows][sink][dK, dV][D] and one arrival counter per
   // (sequence, kv head); null when that kernel does not run
@@ -205,7 +205,7 @@ struct RowBounds {
   int lo, hi;
 };
 
-__device__ __forceinline__ RowBounds row_bounds(const AttnArgs& a, int i, int len_q, int len_k) {
+__host__ __device__ __forceinline__ RowBounds row_bounds(const AttnArgs& a, int i, int len_q, int len_k) {
   RowBounds r;
   const int shift = a.shift_explicit ? a.shift_val : len_k - len_q;
   r.hi = (a.wr >= 0) ? min(len_k - 1, i + shift + a.wr) : len_k - 1;
@@ -214,23 +214,35 @@ __device__ __forceinline__ RowBounds row_bounds(const AttnArgs& a, int i, int le
   return r;
 }
 
-// Offset, in a block's walk over the `n` key tiles from tile t_lo on, of the tile it starts with (the walk
-// wraps around behind the last): the first one whose number is a multiple of walk_mask + 1, the largest power
-// of two among the tiles that such blocks visit.  Blocks that start together are then on few tiles at a time
-// instead of one tile each: with as many kv heads as q heads the 64 blocks that an XCD runs at once cover
-// 8192 rows, whose K and V are as large as its L2, and every block of a window found its tiles gone again.
-// 2 x 8192 rows, 32 = 32 heads, head_dim 128, window 1000, walks from the first tile / from here: fetched beyond
-// L2 in the forward 1.89 / 0.43 GB, in dQ 1.98 / 0.72 GB; a training call 1299 / 1243 us.  Where several q heads
-// share a kv head the tiles of a window stay in L2 either way (32 / 8 heads, window 4096, 32768 rows: 0.78 /
-// 0.58 GB, 1809 / 1796 us).  A power of two, not the walk's own length (the same traffic): a block's first load
-// waits for this.  And of the mask, not of n: tiles that none of a row's keys lie in change nothing, so a
-// row's sums have the same order however many rows its block has.
-__device__ __forceinline__ int walk_start(const AttnArgs& a, int t_lo, int n) {
-  const int at = -t_lo & a.walk_mask;
-  return at < n ? at : 0;
+// The tiles of BN keys that a block of rows i0 .. i_last visits: those of the sink keys that lie before its rows'
+// windows, from tile 0 on, then n_band from tile t_lo on.
+struct KeyTiles {
+  int n_sink, t_lo, n_band;
+};
+template <int BN>
+__host__ __device__ __forceinline__ KeyTiles key_tiles(const AttnArgs& a, int i0, int i_last, int len_q, int len_k) {
+  const int lo = row_bounds(a, i0, len_q, len_k).lo, hi = row_bounds(a, i_last, len_q, len_k).hi;
+  const bool band = hi >= lo;
+  KeyTiles t;
+  t.t_lo = band ? lo / BN : (1 << 29);
+  t.n_band = band ? hi / BN - t.t_lo + 1 : 0;
+  const int sink_keys = max(0, min(min(a.n_sink, hi + 1), lo));
+  t.n_sink = min((sink_keys + BN - 1) / BN, t.t_lo);
+  return t;
 }
-// A walk's tiles in order: n_sink tiles from tile 0 on, then `n_band` from tile t_lo on, the first of these
-// being walk_start's; a cursor that is advanced beyond the last is on one of them still.  (A comparison and
+// Their order: the sinks' tiles, then the band from its first tile on whose number is a multiple of a period, around its
+// end.  Blocks that start together are then on few tiles at a time instead of one tile each: with as many kv heads as
+// q heads the 64 blocks that an XCD runs at once cover 8192 rows, whose K and V are as large as its L2, and every
+// block of a window found its tiles gone again.  2 x 8192 rows, 32 = 32 heads, head_dim 128, window 1000, walks from the
+// first tile / from here: fetched beyond L2 in the forward 1.89 / 0.43 GB, in dQ 1.98 / 0.72 GB; a training call
+// 1299 / 1243 us.
+// No block has two multiples of the period (walk_period), so a row sees its tiles in an order that its window alone
+// decides, whichever rows its block holds besides: from the multiple among them on, if there is one, else from the
+// first (tiles that none of its keys lie in change nothing).  And hardly more tiles than a block has, so that few
+// blocks have none: with the next power of two instead (no division ahead of a block's first load) the same call
+// was 1.6 % slower, a forward of 2 x 11372 rows, 32 heads, window 142, 2 %.
+//
+// A cursor; advanced beyond the last tile it is on one of them still.  (A comparison and
 // three selects a tile; computing a tile from its place in the walk, three times per tile in the forward, cost
 // the launches that gain nothing from the order 1 % (24 drawn calls with equal heads: forward 0.4 % slower than
 // with walks from the first tile that way, 1.8 % faster with the cursor; dQ 0.1 and 2.2 % faster).)
@@ -238,18 +250,19 @@ struct KeyWalk {
   int tile;        // where the cursor is
   int stop, jump;  // reaching tile `stop` it goes to tile `jump` ...
   int end, back;   // ... after which these take their place
-  __device__ __forceinline__ KeyWalk(const AttnArgs& a, int n_sink, int t_lo, int n_band) {
-    const int first = n_band > 0 ? t_lo + walk_start(a, t_lo, n_band) : 0;
-    end = n_band > 0 ? t_lo + n_band : n_sink;
-    back = n_band > 0 ? t_lo : 0;
-    tile = n_sink > 0 ? 0 : first;
-    stop = n_sink > 0 ? n_sink : end;
-    jump = n_sink > 0 ? first : back;
+  __host__ __device__ __forceinline__ KeyWalk(const AttnArgs& a, const KeyTiles& t) {
+    const int at = quotient(t.t_lo + (int)a.by_walk.d - 1, a.by_walk) * (int)a.by_walk.d - t.t_lo;
+    const int first = t.n_band > 0 ? t.t_lo + (at < t.n_band ? at : 0) : 0;
+    end = t.n_band > 0 ? t.t_lo + t.n_band : t.n_sink;
+    back = t.n_band > 0 ? t.t_lo : 0;
+    tile = t.n_sink > 0 ? 0 : first;
+    stop = t.n_sink > 0 ? t.n_sink : end;
+    jump = t.n_sink > 0 ? first : back;
   }
   // BRANCH: by a branch that is taken once or twice a walk instead of selects, five instructions a tile (the dQ
   // kernel at head_dim 128, whose waves start a tile together and wait for it; the forward gains nothing)
   template <bool BRANCH>
-  __device__ __forceinline__ void next() {
+  __host__ __device__ __forceinline__ void next() {
     tile++;
     if constexpr (BRANCH) {
       if (__builtin_expect(tile == stop, 0)) {
@@ -266,12 +279,12 @@ struct KeyWalk {
     }
   }
 };
-inline int walk_mask(const AttnArgs& a, int block_rows, int tile_keys) {
-  if (a.wl < 0 || a.wr < 0) return 0;
-  const int64_t tiles = std::min<int64_t>(((int64_t)a.wl + a.wr + block_rows) / tile_keys, 1 << 20);
-  int mask = 0;
-  while (2 * mask + 2 <= tiles) mask = 2 * mask + 1;
-  return mask;
+// The period for blocks of up to `block_rows` rows: the tiles of the largest band; and of the sinks, so that a band that
+// begins among their tiles has no multiple behind them.
+inline FastDiv walk_period(const AttnArgs& a, int block_rows, int tile_keys) {
+  if (a.wl < 0 || a.wr < 0) return fast_div(1);  // (from the first tile)
+  const int64_t band = ((int64_t)a.wl + a.wr + block_rows + tile_keys - 2) / tile_keys + 1;
+  return fast_div((uint32_t)(band + ceil_div(a.n_sink, tile_keys)));
 }
 
 // Packed mode: which sequence, and which of its tiles of `tile` = 2^tile_log2 rows, does

@@ -103,15 +103,9 @@ void attn_fwd_kernel(const AttnArgs a) {
 
   // ---- key tiles this block visits -----------------------------------------
   const int i_last = min(i0 + bm, len_q) - 1;
-  const int lo_blk = row_bounds(a, i0, len_q, len_k).lo;
-  const int hi_blk = row_bounds(a, i_last, len_q, len_k).hi;
-  const bool band = hi_blk >= lo_blk;
-  const int t_lo = band ? lo_blk / C::BN : (1 << 29);
-  const int n_band = band ? hi_blk / C::BN - t_lo + 1 : 0;
-  const int sink_keys = max(0, min(min(a.n_sink, hi_blk + 1), lo_blk));
-  const int n_sink_t = min((sink_keys + C::BN - 1) / C::BN, t_lo);
-  const int n_tiles = n_sink_t + n_band;
-  KeyWalk walk(a, n_sink_t, t_lo, n_band);
+  const KeyTiles tiles = key_tiles<C::BN>(a, i0, i_last, len_q, len_k);
+  const int n_tiles = tiles.n_sink + tiles.n_band;
+  KeyWalk walk(a, tiles);
   const int t_first = walk.tile;
   walk.next<false>();
 
@@ -511,7 +505,7 @@ int launch_fwd(AttnArgs& a, hipStream_t stream) {
   a.n_tile = (int)(a.cu_q ? ceil_div(a.rows_q, bm) + a.batch : ceil_div(a.seqlen_q, bm));
   if (a.n_tile == 0) return RSWA_OK;
   const int64_t blocks = deal_blocks(a, blocks_per_tile(a) / a.heads_kv, spread_rows(a));
-  a.walk_mask = walk_mask(a, bm, C::BN);
+  a.by_walk = walk_period(a, 128, C::BN);
   // keys a row sees at most; the per-wave tile skip pays when the rows of a block beyond one
   // wave's 32 add a tenth or more to that span
   const int64_t span = (a.wl < 0 || a.wr < 0) ? (int64_t)1 << 40 : (int64_t)a.wl + a.wr + 1;

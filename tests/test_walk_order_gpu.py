@@ -38,3 +38,42 @@ def test_wrapped_walks_match_the_oracle(rows, window, hq, hk, d, sinks):
     assert (out.float().cpu() - ref).abs().max() <= 2e-2
     for got, want in zip(grads, ref_grads):
         assert relnorm(got, want) <= GRAD_TOL
+
+
+def _run(q, k, v, do, window, *cu):
+    from ring_swa.ops import attn_bwd, attn_fwd
+
+    out, lse = attn_fwd(q, k, v, None, (window, 0), True, *cu)
+    grads = [torch.full_like(t, float("nan")) for t in (q, k, v)]
+    attn_bwd(q, k, v, out, lse, do, *grads, None, (window, 0), True, *cu)
+    return out, lse, grads[0]
+
+
+def _inputs(rows, hq, hk, d):
+    g = torch.Generator(device="cuda").manual_seed(rows)
+    return [torch.randn(1, rows, h, d, device="cuda", generator=g).bfloat16() for h in (hq, hk, hk, hq)]
+
+
+@pytest.mark.parametrize("window,d", [(350, 128), (447, 64), (1000, 128), (1950, 128), (1950, 64)])
+def test_rows_have_the_same_bits_in_blocks_of_64_and_of_128(window, d):
+    """Pairs of q heads come in blocks of 64 rows (forward; dQ), single ones in blocks of 128."""
+    q, k, v, do = _inputs(4100, 2, 1, d)
+    out, lse, dq = _run(q, k, v, do, window)
+    for h in range(2):
+        x, y, z = _run(q[:, :, h:h + 1], k, v, do[:, :, h:h + 1], window)
+        assert torch.equal(x, out[:, :, h:h + 1]) and torch.equal(y, lse[:, h:h + 1])
+        assert torch.equal(z, dq[:, :, h:h + 1])
+
+
+@pytest.mark.parametrize("hq", [1, 2])
+def test_rows_of_short_calls_and_of_long_ones_have_the_same_bits(hq):
+    """Above 3200 keys a row on average dQ takes blocks of twice as many rows: a call's first rows alone, and in a pack."""
+    window = 4000
+    q, k, v, do = _inputs(14000, hq, 1, 128)
+    whole = _run(q, k, v, do, window)
+    first = _run(*(t[:, :8000] for t in (q, k, v, do)), window)
+    cu = torch.tensor([0, 8000, 11000, 14000], device="cuda", dtype=torch.int32)
+    pack = _run(*(t[0] for t in (q, k, v, do)), window, cu, cu)
+    for a, b, c, dim in zip(whole, first, pack, (1, 2, 1)):
+        assert torch.equal(a.narrow(dim, 0, 8000), b)
+        assert torch.equal(c.narrow(dim - 1, 0, 8000), b[0])
