@@ -165,7 +165,8 @@ constexpr int kComputeUnits = 256;  // MI355X
 // window 5372, forward 429 / 348, dQ 651 / 524; 3958 rows, 28 / 4 heads, a sink, window 2397, 126 / 109 and 178 / 139;
 // 2 x 18605 rows, 8 / 2 heads, head_dim 64, window 3149, 277 / 253 and 329 / 300).  So: where the fullest eighth has
 // 5 % more than the average, of a dense call (of a pack the host knows too little, and both orders lost and won).  A
-// row counts as its keys and 200 for starts and ends.
+// row counts as its keys and 200 for starts and ends.  (123 drawn calls with such heads: forward 1.1 % and dQ 1.3 %
+// faster than eighths on average, 23 % at most; nothing slower beyond the 7 % by which single calls scatter.)
 inline bool spread_rows(const AttnArgs& a) {
   const int log2 = xcds_per_head_log2(a);
   const int heads = (a.heads_kv * a.batch) << log2 >> 3;  // that 1 << log2 XCDs share
@@ -194,7 +195,12 @@ inline bool spread_rows(const AttnArgs& a) {
 // 16544, 4 = 4 heads, window 1132, 99 / 92).  Not where windows are short against the sequences (even work) and the
 // launch has a second round to even out what the first leaves (25429 rows, 16 / 4 heads, window 593, 400 blocks, 183 /
 // 189; packs of long sequences, 8 / 2 heads, windows 90 and 205, 36 / 41 and 119 / 128; but 4134 rows, 28 / 4 heads,
-// window 173, 260 blocks, 64 / 53, and 20516 rows, window 568, 324 blocks, 438 / 405).
+// window 173, 260 blocks, 64 / 53, and 20516 rows, window 568, 324 blocks, 438 / 405).  480 drawn calls with such heads:
+// the rule is 2.0 % faster than eighths on average (ranks' chunks 7 %, packs that a rank shares 3 %, the others 0.3 to 1.1 %;
+// as many kv heads as q heads, 206 calls, 2.1 %), 100 calls by more than 3 % and 38 % at most; 42 are slower by more than
+// 3 %, mostly packs, the worst of 64 and 70 short sequences (8104 tokens, 4 = 4 heads, 26.9 / 33.1; 5423, 16 / 4,
+// head_dim 64, 21.5 / 27.0), where it depends on lengths that the host does not know.  Spreading always: 1.2 % faster on
+// 240 of them where the rule is 1.6 %; packs by their number of sequences: 1.7 % on 240 others, the rule 2.4 %.
 inline bool spread_keys(const AttnArgs& a) {
   const int64_t heads = (int64_t)a.heads_kv * (a.cu_q ? 1 : a.batch);
   const int64_t len = a.cu_q ? a.rows_k / a.batch : a.seqlen_k;
