@@ -409,9 +409,6 @@ __global__ __launch_bounds__(256) void attn_bwd_dkdv_kernel(const AttnArgs a) {
     if constexpr (part == 0) {
       if (WALK4 || wave == 0) {  // lanes 0-31: lse2 of the 32 rows, lanes 32-63: their delta
         const int first = nxt.stat_row + nxt.i0;
-        // the per-lane offset is recomputed here (opaque to the optimiser): kept in a
-        // register across the walk it could be spilled, and its reload would wait for
-        // every tile load issued before it
         if constexpr (WALK4) {
           lds_load_asm<4>(rsrc_words(a.lse2, (int)((uint32_t)stat_end * 4u)), st_voff, first * 4,
                           (uint32_t)(uintptr_t)(lds_void_t*)std_);
@@ -641,8 +638,8 @@ __global__ __launch_bounds__(256) void attn_bwd_dkdv_kernel(const AttnArgs a) {
         constexpr int m = decltype(mc)::value;
         constexpr int f = m / KB, kb = m % KB;  // fragment slot and key block of this MFMA
         if constexpr (kb == 0) fetch(std::integral_constant<int, f + AH>{});
-        // (after the last tile the cursor still names it: its rows are fetched once more, into
-        // the idle buffers, rather than branching around every load)
+        // (no branch around every load: past the last tile what the cursor is on, that tile or, where it runs
+        // on (FREE_RUN), one at the start of the head's walk, is fetched once more into idle buffers)
         // (WALK4 issues four times as many: one every other MFMA)
         constexpr int every = WALK4 ? 2 : 1;
         if constexpr (m % every == 0 && m / every < NPART) load_part(std::integral_constant<int, m / every>{}, qn, don, stn);
@@ -1279,8 +1276,8 @@ void attn_bwd_dq_kernel(const AttnArgs a) {
   // of the band and one of the sinks each, so that a tile costs a comparison or two.
   // (With this, resources kept instead of selected per tile and the walk's branch: 45 scalar instructions a tile
   // instead of 75, 60 of which both waves of a SIMD issued ahead of their first MFMA.  us, dQ with statistics: the rank
-  // step, window 4096, 677 / 667; 2 x 8192 rows, 32 heads, window 1000, 414 / 411; 4001 rows 107 / 102 to 110 / 109.6;
-  // 22 drawn and listed calls 1.0 % on average.)
+  // step, window 4096, 677 / 667; 2 x 8192 rows, 32 heads, window 1000, 414 / 411; 22 drawn and listed calls 1.0 % on
+  // average, single ones of 100 us by nothing or by 4 %.)
   const int need_lo = wb_first.lo - (C::BN - 1);
   const unsigned need_n = wave_valid ? (unsigned)max(wb_last.hi - need_lo + 1, 0) : 0u;
   const int need_sink = wave_valid ? min(a.n_sink, wb_last.hi + 1) : 0;
