@@ -30,8 +30,9 @@ def _rows(shape, stride, seed):
     (97, 6, 3, 128, 120, 8),
     (1, 4, 4, 128, 0, 0),        # a stride that no row uses
 ])
-def test_short_row_strides_equal_contiguous_rows(rows, hq, hk, d, q_stride, do_stride, packed, form, addressing, monkeypatch):
-    from ring_swa import _lib
+@pytest.mark.parametrize("route", [{}, {"num_sink": 3}, {"handoff": True}], ids=["plain", "sinks", "handoff"])
+def test_short_row_strides_equal_contiguous_rows(rows, hq, hk, d, q_stride, do_stride, route, packed, form, addressing,
+                                                   monkeypatch):
     from ring_swa.ops import attn_bwd, attn_fwd
 
     if addressing == "far":
@@ -45,9 +46,9 @@ def test_short_row_strides_equal_contiguous_rows(rows, hq, hk, d, q_stride, do_s
     cu = [torch.tensor(sorted({0, rows // 3, rows}), device="cuda", dtype=torch.int32)] * 2 if packed else []
 
     def run(q, do):
-        out, lse = attn_fwd(q, k, v, None, (50, 0), True, *cu)
+        out, lse = attn_fwd(q, k, v, None, (50, 0), True, *cu, num_sink=route.get("num_sink", 0))
         grads = [torch.full_like(t, float("nan"), memory_format=torch.contiguous_format) for t in (q, k, v)]
-        attn_bwd(q, k, v, out, lse, do, *grads, None, (50, 0), True, *cu, dkdv_form=form)
+        attn_bwd(q, k, v, out, lse, do, *grads, None, (50, 0), True, *cu, dkdv_form=form, **route)
         return [out, *grads]
 
     for got, want in zip(run(q, do), run(q.contiguous(), do.contiguous())):
